@@ -18,6 +18,7 @@
 #include "score_tiles.h"
 #include "score_narrow.h"
 #include "score_messages.h"
+#include "tiles_build.h"
 
 namespace {
 
@@ -1919,28 +1920,23 @@ int gtm_build_tiles(const gtm_config *cfg, const gtm_graphs *graphs, uint32_t *t
     TileGeom tg = geometry_for(cfg, graphs, d.K);
     if (!tg.ok) return fail(GTM_ERR_INVALID, "this data set's shape has no tile layout (gtm_tiles_bytes() == 0)");
     hipStream_t st = (hipStream_t)stream;
-    int64_t total = (int64_t)tg.n_tiles * tg.rows * tg.tw;
-    hipLaunchKernelGGL(k_build_tiles, dim3(blocks_for(total, TPB)), dim3(TPB), 0, st, graphs->X, graphs->node_type,
-                       graphs->node_index, graphs->number_of_graph_nodes, graphs->number_of_graphs, d.LA,
-                       cfg->literals, graphs->number_of_node_types, tg, total, tiles);
-    if (int rc = check_launch("build_tiles")) return rc;
     int32_t *counts = (int32_t *)(tiles + tiles_words(tg));
     hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for(tg.rows * 2, TPB)), dim3(TPB), 0, st, counts, (int64_t)tg.rows * 2, 0);
     if (int rc = check_launch("fill")) return rc;
-    int64_t total_rows = (int64_t)tg.n_tiles * tg.rows;
-    hipLaunchKernelGGL(k_row_counts, dim3(blocks_for(total_rows, TPB)), dim3(TPB), 0, st, tiles, tg, total_rows,
-                       (unsigned long long *)counts);
-    if (int rc = check_launch("row_counts")) return rc;
-    hipLaunchKernelGGL(k_row_order, dim3(blocks_for(cfg->literals, TPB)), dim3(TPB), 0, st,
+    const TileBuildShape shape = tile_build_shape(tg, d.LA);
+    const size_t lds = tile_build_lds_words(shape) * 4;
+    // (16-byte loads of a node's literal words: whole quads, from an aligned array)
+    const bool aligned = d.LA % 4 == 0 && ((uintptr_t)graphs->X & 15) == 0;
+    auto kernel = aligned ? k_build_tiles<true> : k_build_tiles<false>;
+    hipLaunchKernelGGL(kernel, dim3(shape.tile_blocks, (unsigned)shape.quad_parts, (unsigned)shape.word_parts),
+                       dim3(TILE_BUILD_BLOCK), lds, st, graphs->X, graphs->node_type, graphs->node_index,
+                       graphs->number_of_graph_nodes, graphs->number_of_graphs, d.LA, cfg->literals,
+                       graphs->number_of_node_types, tg, shape, tiles, (unsigned long long *)counts,
+                       tg.half ? tiles + tiles_xpos_offset_words(tg, cfg->literals) : nullptr);
+    if (int rc = check_launch("build_tiles")) return rc;
+    hipLaunchKernelGGL(k_row_order, dim3(blocks_for(cfg->literals, 4 * TILE_ORDER_AT_ONCE)), dim3(256), 0, st,
                        (const unsigned long long *)counts, cfg->literals, (uint32_t *)(counts + (size_t)tg.rows * 2));
     if (int rc = check_launch("row_order")) return rc;
-    if (tg.half) {
-        const int64_t slots = (int64_t)tg.n_tiles * tg.tw * 32;
-        hipLaunchKernelGGL(k_build_xpos, dim3(blocks_for(slots, TPB)), dim3(TPB), 0, st, graphs->X, graphs->node_index,
-                           graphs->number_of_graph_nodes, graphs->number_of_graphs, d.LA, tg, slots,
-                           tiles + tiles_xpos_offset_words(tg, cfg->literals));
-        if (int rc = check_launch("build_xpos")) return rc;
-    }
     remember_tiles(tiles, tg, cfg, graphs);
     return GTM_OK;
 }

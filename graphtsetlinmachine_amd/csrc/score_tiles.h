@@ -13,7 +13,7 @@
 // tiles pass from layer to layer in the same slot layout, and each layer's
 // messages are built literal-major as well.
 //
-// Tile layout in HBM (built once per data set by k_build_tiles):
+// Tile layout in HBM (built once per data set by k_build_tiles, tiles_build.h):
 //   tiles[tile][row][tw] uint32, rows = LITERALS + node_types + 1
 //     row l < LITERALS          bit-row of literal l
 //     row LITERALS + t          valid nodes of node type t
@@ -157,95 +157,6 @@ inline TileGeom tile_geometry(int literals, int n_types, int max_nodes, int n_gr
     }
     best.ok = 0;
     return best;
-}
-
-// One thread per tile word: gathers its 32 node slots.
-__global__ void k_build_tiles(const uint32_t *__restrict__ X, const uint32_t *__restrict__ node_type,
-                              const uint32_t *__restrict__ node_index, const uint32_t *__restrict__ n_nodes_arr,
-                              int G, int LA, int literals, int n_types, TileGeom tg, int64_t total,
-                              uint32_t *__restrict__ tiles) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    int w = (int)(i % tg.tw);
-    int64_t rest = i / tg.tw;
-    int row = (int)(rest % tg.rows);
-    int tile = (int)(rest / tg.rows);
-    uint32_t out = 0;
-    if (row == tg.rows - 1) {
-        // all ones over the graph slots; words that only pad the row stay 0 so
-        // that they never keep a clause alive
-        out = (tg.slot_words == 0 || w < tg.gpt * tg.slot_words) ? 0xFFFFFFFFu : 0u;
-    } else {
-        for (int b = 0; b < 32; ++b) {
-            int pos = w * 32 + b;
-            int j = pos / tg.slot_bits, n = pos % tg.slot_bits;
-            int64_t g = (int64_t)tile * tg.gpt + j;
-            if (j >= tg.gpt || g >= G) continue;
-            int count = (int)n_nodes_arr[g];
-            if (count == 0 && n == 0) {
-                // kernels.py:289-295,443-466: for a graph without nodes the reference's
-                // chunk arithmetic leaves every clause true; slot bit 0 carries that.
-                out |= 1u << b;
-                continue;
-            }
-            if (n >= count) continue;
-            int64_t node = (int64_t)node_index[g] + n;
-            uint32_t bit;
-            if (row < literals)
-                bit = (X[node * LA + (row >> 5)] >> (row & 31)) & 1u;
-            else
-                bit = (int)node_type[node] == row - literals;
-            out |= bit << b;
-        }
-    }
-    tiles[i] = out;
-}
-
-// Half tiles: the positive half of the literal words of the node in every slot (zeros where the slot
-// holds no node).  One thread per slot.
-__global__ void k_build_xpos(const uint32_t *__restrict__ X, const uint32_t *__restrict__ node_index,
-                             const uint32_t *__restrict__ n_nodes_arr, int G, int LA, TileGeom tg, int64_t slots,
-                             uint32_t *__restrict__ xpos) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= slots) return;
-    const int per_tile = tg.tw * 32;
-    const int64_t tile = i / per_tile;
-    const int pos = (int)(i - tile * per_tile);
-    const int j = pos / tg.slot_bits, n = pos - j * tg.slot_bits;
-    const int64_t g = tile * tg.gpt + j;
-    const int half = LA / 2;
-    const bool has_node = j < tg.gpt && g < G && (uint32_t)n < n_nodes_arr[g];
-    const uint32_t *row = has_node ? X + ((int64_t)node_index[g] + n) * LA : X;
-    for (int w = 0; w < half; ++w) xpos[i * half + w] = has_node ? row[w] : 0u;
-}
-
-// Number of set bits of every row over all tiles (how often a literal holds in
-// this data set); row_count[rows], zeroed by the caller.
-__global__ void k_row_counts(const uint32_t *__restrict__ tiles, TileGeom tg, int64_t total_rows,
-                             unsigned long long *__restrict__ row_count) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total_rows) return;
-    int row = (int)(i % tg.rows);
-    const uint32_t *p = tiles + i * tg.tw;
-    unsigned long long n = 0;
-    for (int w = 0; w < tg.tw; ++w) n += __popc(p[w]);
-    if (n) atomicAdd(&row_count[row], n);
-}
-
-// Literal rows ordered by how often they hold in the data set, rarest first:
-// order[r] = literal with rank r under the key (row_count, literal).  One
-// thread per literal counts the keys below its own.
-__global__ void k_row_order(const unsigned long long *__restrict__ row_count, int literals,
-                            uint32_t *__restrict__ order) {
-    int l = blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= literals) return;
-    unsigned long long mine = row_count[l];
-    int rank = 0;
-    for (int m = 0; m < literals; ++m) {
-        unsigned long long other = row_count[m];
-        rank += (other < mine) || (other == mine && m < l);
-    }
-    order[rank] = (uint32_t)l;
 }
 
 // Per call, one wave per clause: the rows the clause ANDs together, as 32-bit
