@@ -58,6 +58,18 @@ class GraphsDesc(C.Structure):
     ]
 
 
+class PackedGraphs(C.Structure):
+    _fields_ = (
+        [(name, C.c_void_p) for name in ("rows", "types", "degrees", "first_edges", "edges", "first_nodes", "node_counts",
+                                         "X", "node_type", "number_of_graph_node_edges", "edge", "node_index", "edge_index",
+                                         "number_of_graph_nodes")]
+        + [(name, C.c_int64) for name in ("total_nodes", "total_edges", "number_of_graphs")]
+        + [(name, C.c_int32) for name in ("literal_words", "hypervector_size", "rows_positive", "type_bytes", "degree_bytes",
+                                          "edge_bytes")]
+        + [("type_value", C.c_uint32), ("degree_value", C.c_uint32), ("index_follows", C.c_int32)]
+    )
+
+
 class State(C.Structure):
     _fields_ = [
         ("ta_state", C.c_void_p),
@@ -100,6 +112,7 @@ PROTOTYPES = {
     "gtm_profile_read": (C.c_int, [C.POINTER(C.c_char_p), C.POINTER(C.c_int32), C.POINTER(C.c_double)]),
     "gtm_profile_read_kernel": (C.c_int, [C.c_int32, C.POINTER(C.c_char_p), C.POINTER(C.c_int32), C.POINTER(C.c_double)]),
     "gtm_graphs_properties": (C.c_int, [_CFG, _GR, _P, _P]),
+    "gtm_unpack_graphs": (C.c_int, [C.POINTER(PackedGraphs), _P]),
     "gtm_tiles_bytes": (_SZ, [_CFG, _GR]),
     "gtm_build_tiles": (C.c_int, [_CFG, _GR, _P, _P]),
     "gtm_score_workspace_bytes": (_SZ, [_CFG, _GR, _I]),

@@ -19,13 +19,14 @@ FLAGS = [
 ]
 
 
-ENCODER_SOURCE = os.path.join(HERE, "csrc", "encode.c")
+ENCODER_SOURCES = [os.path.join(HERE, "csrc", "encode.c"), os.path.join(HERE, "csrc", "pack.c")]
 ENCODER_OUTPUT = os.path.join(HERE, "libgtm_encode.so")
 
 
 def build_encoder(verbose=True):
-    """The host-side property encoder (plain C, OpenMP) that graphs.py loads through ctypes."""
-    cmd = [os.environ.get("CC", "gcc"), "-O3", "-fopenmp", "-shared", "-fPIC", "-o", ENCODER_OUTPUT, ENCODER_SOURCE]
+    """The host-side property encoder and data-set packer (plain C, OpenMP) that graphs.py and upload.py load
+    through ctypes."""
+    cmd = [os.environ.get("CC", "gcc"), "-O3", "-fopenmp", "-shared", "-fPIC", "-o", ENCODER_OUTPUT] + ENCODER_SOURCES
     if verbose:
         print(" ".join(cmd), flush=True)
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)

@@ -19,6 +19,7 @@
 #include "score_narrow.h"
 #include "score_messages.h"
 #include "tiles_build.h"
+#include "graphs_unpack.h"
 
 namespace {
 
@@ -1900,6 +1901,31 @@ int gtm_graphs_properties(const gtm_config *cfg, const gtm_graphs *graphs, uint3
     hipLaunchKernelGGL(k_graphs_properties, dim3(blocks_for(items, TPB)), dim3(TPB), 0, st, graphs->X, graphs->total_nodes,
                        d.LA, cfg->literals, graphs->number_of_graph_nodes, graphs->number_of_graphs, properties);
     return check_launch("graphs_properties");
+}
+
+int gtm_unpack_graphs(const gtm_packed_graphs *packed, void *stream) {
+    if (!packed) return fail(GTM_ERR_INVALID, "packed is NULL");
+    const gtm_packed_graphs &p = *packed;
+    if (p.total_nodes < 1 || p.number_of_graphs < 1 || p.total_edges < 0 || p.literal_words < 1 || p.hypervector_size < 1 ||
+        (p.rows_positive && p.literal_words != (2 * p.hypervector_size - 1) / 32 + 1))
+        return fail(GTM_ERR_INVALID, "packed sizes out of range");
+    if (!p.rows || !p.first_edges || !p.first_nodes || !p.node_counts || (p.type_bytes && !p.types) ||
+        (p.degree_bytes && !p.degrees) || (p.total_edges && (!p.edges || !p.edge)) || !p.X || !p.node_type ||
+        !p.number_of_graph_node_edges || !p.node_index || !p.edge_index || !p.number_of_graph_nodes)
+        return fail(GTM_ERR_INVALID, "packed has NULL arrays");
+    auto width = [](int bytes, int least) { return bytes >= least && (bytes == 0 || bytes == 1 || bytes == 2 || bytes == 4); };
+    if (!width(p.type_bytes, 0) || !width(p.degree_bytes, 0) || (p.total_edges && !width(p.edge_bytes, 1)))
+        return fail(GTM_ERR_INVALID, "packed numbers of %d, %d and %d bytes", p.type_bytes, p.degree_bytes, p.edge_bytes);
+    UnpackShape s;
+    const int64_t nodes = p.total_nodes > p.number_of_graphs ? p.total_nodes : p.number_of_graphs;
+    s.row_blocks = blocks_for(p.total_nodes * p.literal_words, UNPACK_BLOCK * UNPACK_WORDS);
+    s.node_blocks = blocks_for(nodes, UNPACK_BLOCK);
+    s.graph_blocks = p.index_follows ? blocks_for(p.number_of_graphs, UNPACK_BLOCK / 64) : 0u;
+    s.edge_blocks = blocks_for(2 * p.total_edges, UNPACK_BLOCK * UNPACK_WORDS);
+    const unsigned blocks = blocks_for((int64_t)s.row_blocks + s.node_blocks + s.graph_blocks + s.edge_blocks, 1);
+    if (g_grid_overflow) return check_launch("unpack_graphs");
+    hipLaunchKernelGGL(k_unpack_graphs, dim3(blocks), dim3(UNPACK_BLOCK), 0, (hipStream_t)stream, p, s);
+    return check_launch("unpack_graphs");
 }
 
 size_t gtm_tiles_bytes(const gtm_config *cfg, const gtm_graphs *graphs) {

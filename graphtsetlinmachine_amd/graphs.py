@@ -51,6 +51,13 @@ def _native_encoder():
         lib.gtm_encode_membership.argtypes = [p, i64, i32, p, i32, i32, i32, p]
         lib.gtm_encode_pairs.restype = None
         lib.gtm_encode_pairs.argtypes = [p, p, i64, p, i32, i32, i32, p]
+        # csrc/pack.c, in the same library (upload.py)
+        lib.gtm_pack_plan.restype = None
+        lib.gtm_pack_plan.argtypes = [p, p, p, p, p, p, i64, i64, i64, p, p]
+        lib.gtm_pack_rows.restype = ctypes.c_int
+        lib.gtm_pack_rows.argtypes = [p, i64, i32, i32, p]
+        lib.gtm_pack_numbers.restype = None
+        lib.gtm_pack_numbers.argtypes = [p, i64, i32, p]
         _encoder = lib
     return _encoder
 

@@ -26,6 +26,7 @@ import numpy as np
 import torch
 
 from . import _abi
+from .upload import upload
 
 
 def _device():
@@ -55,17 +56,25 @@ class _DeviceGraphs:
 
     def __init__(self, graphs):
         self.signature = graphs.signature
+        self._stream = torch.cuda.current_stream()  # where the arrays and the tiles are made
         self.number_of_graphs = int(graphs.number_of_graphs)
         self.max_nodes = int(graphs.max_number_of_graph_nodes)
-        self.tensors = {
-            "X": _to_device(graphs.X),
-            "node_type": _to_device(graphs.node_type),
-            "number_of_graph_node_edges": _to_device(graphs.number_of_graph_node_edges),
-            "edge": _to_device(graphs.edge),
-            "node_index": _to_device(graphs.node_index),
-            "edge_index": _to_device(graphs.edge_index),
-            "number_of_graph_nodes": _to_device(graphs.number_of_graph_nodes),
-        }
+        # packed on the way where the arrays allow it; then it is also known whether the negated literals are the
+        # complements of the positive ones everywhere and every graph has a node (None: not looked at yet)
+        packed = upload(graphs, _device())
+        if packed is not None:
+            self.tensors, self._complementary = packed
+        else:
+            self._complementary = None
+            self.tensors = {
+                "X": _to_device(graphs.X),
+                "node_type": _to_device(graphs.node_type),
+                "number_of_graph_node_edges": _to_device(graphs.number_of_graph_node_edges),
+                "edge": _to_device(graphs.edge),
+                "node_index": _to_device(graphs.node_index),
+                "edge_index": _to_device(graphs.edge_index),
+                "number_of_graph_nodes": _to_device(graphs.number_of_graph_nodes),
+            }
         d = _abi.GraphsDesc()
         for name, t in self.tensors.items():
             setattr(d, name, _ptr(t))
@@ -78,7 +87,13 @@ class _DeviceGraphs:
         self.desc = d
         self.tiles = None
         self._tiles_key = None
-        self._complementary = None  # not looked at yet
+
+    def order_after_upload(self):
+        """Work enqueued on the current stream from now on comes after what makes the arrays and the tiles."""
+        now = torch.cuda.current_stream()
+        if now != self._stream:
+            now.wait_stream(self._stream)
+            self._stream = now
 
     def ensure_tiles(self, cfg):
         """Build the literal-major tile layout once per data set and tile
@@ -86,6 +101,7 @@ class _DeviceGraphs:
         layout keep tiles = NULL.  The geometry depends on the model's
         sizes, so a data set handed to a model of another shape is tiled
         again."""
+        self.order_after_upload()
         key = (cfg.classes, cfg.literals, cfg.depth, cfg.message_size, _abi.tuning("GTM_TILE_LANE_WORDS"),
                _abi.tuning("GTM_NO_HALF_TILES"), _abi.tuning("GTM_NO_TWO_PHASE"), _abi.tuning("GTM_HALF_LANE_WORDS"))
         if self._tiles_key == key:

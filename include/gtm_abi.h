@@ -88,6 +88,27 @@ typedef struct gtm_graphs {
     const uint32_t *tiles; /* optional: literal-major tiles from gtm_build_tiles, or NULL */
 } gtm_graphs;
 
+/* A data set's arrays in the packed form in which they cross the bus (device pointers), and where
+ * gtm_unpack_graphs writes the arrays of gtm_graphs.  `bytes` fields give the width of each packed
+ * number: 1, 2 or 4, or 0 where all are the one `value`. */
+typedef struct gtm_packed_graphs {
+    const uint32_t *rows;        /* rows_positive: [total_nodes][ceil(hypervector_size / 32)], else X itself */
+    const void *types;           /* [total_nodes] */
+    const void *degrees;         /* [total_nodes] edges of every node */
+    const uint32_t *first_edges; /* index_follows: [number_of_graphs] first edge of every graph, else edge_index itself */
+    const void *edges;           /* [total_edges][2] */
+    const uint32_t *first_nodes; /* [number_of_graphs] = node_index */
+    const uint32_t *node_counts; /* [number_of_graphs] = number_of_graph_nodes */
+    uint32_t *X, *node_type, *number_of_graph_node_edges, *edge, *node_index, *edge_index, *number_of_graph_nodes;
+    int64_t total_nodes, total_edges, number_of_graphs;
+    int32_t literal_words;    /* LA_CHUNKS */
+    int32_t hypervector_size; /* positive literals */
+    int32_t rows_positive;    /* a negated literal is the complement of its positive one, bits past the literals are 0 */
+    int32_t type_bytes, degree_bytes, edge_bytes;
+    uint32_t type_value, degree_value;
+    int32_t index_follows; /* a node's first edge = its graph's + the edges of the graph's nodes before it */
+} gtm_packed_graphs;
+
 /* The model's device buffers (tm.py:110-124). */
 typedef struct gtm_state {
     uint32_t *ta_state;                            /* [CLAUSES][LA_CHUNKS][STATE_BITS] */
@@ -165,6 +186,10 @@ int gtm_update_message(const gtm_config *cfg, uint64_t step, int32_t bank, uint3
                        const uint32_t *clause_X, const int32_t *class_clause_update, void *stream);
 
 /* ---- the driver loops --------------------------------------------------- */
+
+/* Stands where the reference uploads the arrays as they are (tm.py:528-555): one launch that widens
+ * a packed data set. */
+int gtm_unpack_graphs(const gtm_packed_graphs *packed, void *stream);
 
 /* A second, derived layout of a data set for batched depth-1 inference: per
  * tile of graphs one bit-row per literal over the tile's node slots (plus one

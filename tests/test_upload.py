@@ -1,0 +1,71 @@
+"""Data sets packed for the bus (csrc/pack.c, upload.py) and unpacked on the device (gtm_unpack_graphs)."""
+
+import copy
+
+import numpy as np
+import pytest
+
+from tests import helpers
+
+ARRAYS = ("X", "node_type", "number_of_graph_node_edges", "edge", "node_index", "edge_index", "number_of_graph_nodes")
+
+
+def graphs_of(hv, **kwargs):
+    args = dict(n_graphs=20, max_nodes=30, hv_size=hv, min_nodes=0, edge_types=("a", "b"), node_types=("x", "y"))
+    args.update(kwargs)
+    return helpers.random_graphs(hv, **args)
+
+
+@pytest.mark.parametrize("hv", [10, 16, 31, 32, 33, 50, 64, 96, 200, 1000])
+def test_rows_are_packed_and_any_flipped_bit_is_seen(hv):
+    from graphtsetlinmachine_amd.graphs import _native_encoder
+
+    lib = _native_encoder()
+    X = graphs_of(hv).X
+    N, LA = X.shape
+    out = np.full((N, (hv + 31) // 32), 0x5A5A5A5A, dtype=np.uint32)
+    pack = lambda x: lib.gtm_pack_rows(x.ctypes.data, N, LA, hv, out.ctypes.data)
+    assert pack(X) == 0
+    bits = lambda a: np.unpackbits(a.view(np.uint8), axis=1, bitorder="little")
+    assert np.array_equal(bits(out)[:, :hv], bits(X)[:, :hv]) and not bits(out)[:, hv:].any()
+    for row, bit in ((0, 0), (N - 1, hv - 1), (N // 2, hv), (1, 2 * hv - 1), (2, LA * 32 - 1)):
+        broken = X.copy()
+        broken[row, bit // 32] ^= np.uint32(1 << (bit % 32))
+        assert pack(broken) == 1, (row, bit)
+
+
+def broken_copies(g):
+    """Data sets whose public arrays a caller has changed so that some of them no longer follow from less."""
+    yield g, True
+    x = copy.deepcopy(g)
+    x.X[-1, 0] ^= np.uint32(1)
+    yield x, False
+    x = copy.deepcopy(g)
+    if x.edge.size:
+        x.edge_index[-1] += np.uint32(1)
+        x.edge[0, 1] = 70000
+        x.node_type[-1], x.number_of_graph_node_edges[-1] = 300, 256
+    yield x, True
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("piece", [128, 4096, 2 << 20])
+@pytest.mark.parametrize("shape", [
+    dict(hv=32), dict(hv=50, node_types=("x",), max_degree=0), dict(hv=96, min_nodes=1), dict(hv=200),
+    dict(hv=64, n_graphs=3, max_nodes=1), dict(hv=1000, n_graphs=70, max_nodes=130),
+], ids=lambda s: "hv%d" % s["hv"])
+def test_the_device_holds_the_arrays_as_they_are(shape, piece, monkeypatch):
+    import torch
+
+    from graphtsetlinmachine_amd import upload
+
+    monkeypatch.setattr(upload, "PIECE_BYTES", piece)
+    args = dict(shape)
+    for g, follows in broken_copies(graphs_of(args.pop("hv"), **args)):
+        tensors, complementary = upload.upload(g, torch.device("cuda"))
+        for name in ARRAYS:
+            want = getattr(g, name)
+            assert np.array_equal(tensors[name].cpu().numpy().view(np.uint32), want.reshape(-1)), name
+        assert complementary == (follows and bool((g.number_of_graph_nodes > 0).all()))
+    g.X = np.asfortranarray(g.X)
+    assert upload.upload(g, torch.device("cuda")) is None
