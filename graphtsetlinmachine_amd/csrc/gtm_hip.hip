@@ -18,6 +18,7 @@
 #include "score_tiles.h"
 #include "score_narrow.h"
 #include "score_messages.h"
+#include "score_moves.h"
 #include "tiles_build.h"
 #include "graphs_unpack.h"
 
@@ -78,6 +79,7 @@ int check_launch(const char *what) {
     X(NO_HALF_ROWS) \
     X(NO_HALF_TILES) \
     X(NO_LISTS_IN_LDS) \
+    X(NO_MESSAGE_MOVES) \
     X(NO_NARROW_TWO_PHASE) \
     X(NO_NARROW_LAYERS) \
     X(NO_PERSISTENT_FIT) \
@@ -919,6 +921,8 @@ TileGeom geometry_for(const gtm_config *cfg, const gtm_graphs *g, int classes) {
 struct TilesTag {
     TileGeom tg;
     int literals, n_types, n_graphs;
+    TileMoves moves;  // of the edges in the arrays below (n == 0: not known, or there is no such description)
+    const uint32_t *masks, *edge, *edge_index, *n_edges;
 };
 std::mutex g_tiles_mutex;
 std::unordered_map<const void *, TilesTag> &tiles_registry() {
@@ -928,7 +932,26 @@ std::unordered_map<const void *, TilesTag> &tiles_registry() {
 
 void remember_tiles(const void *tiles, const TileGeom &tg, const gtm_config *cfg, const gtm_graphs *g) {
     std::lock_guard<std::mutex> lock(g_tiles_mutex);
-    tiles_registry()[tiles] = TilesTag{tg, cfg->literals, g->number_of_node_types, g->number_of_graphs};
+    tiles_registry()[tiles] = TilesTag{tg, cfg->literals, g->number_of_node_types, g->number_of_graphs, TileMoves{}, nullptr, nullptr, nullptr, nullptr};
+}
+
+void remember_moves(const gtm_graphs *g, const TileMoves &moves, const uint32_t *masks) {
+    std::lock_guard<std::mutex> lock(g_tiles_mutex);
+    auto it = tiles_registry().find(g->tiles);
+    if (it == tiles_registry().end()) return;
+    it->second.moves = moves, it->second.masks = masks;
+    it->second.edge = g->edge, it->second.edge_index = g->edge_index, it->second.n_edges = g->number_of_graph_node_edges;
+}
+
+// The moves of the data set's edges (n == 0: they are walked).  Only for the edge arrays they were found in.
+TileMoves moves_of_tiles(const gtm_graphs *g, const uint32_t **masks) {
+    std::lock_guard<std::mutex> lock(g_tiles_mutex);
+    auto it = tiles_registry().find(g->tiles);
+    if (it == tiles_registry().end() || it->second.edge != g->edge || it->second.edge_index != g->edge_index ||
+        it->second.n_edges != g->number_of_graph_node_edges)
+        return TileMoves{};
+    *masks = it->second.masks;
+    return it->second.moves;
 }
 
 int check_tiles(const TileGeom &tg, const gtm_config *cfg, const gtm_graphs *g) {
@@ -1422,8 +1445,37 @@ int score_on_tiles(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
         }
     }
     if (in_lds.ok) fused_messages = false;
+    // Edges that are a few moves: rows shifted instead of edges walked, wherever the sent rows fit in LDS - faster
+    // than each of the kernels below on every shape measured (the passes of score_moves.h's head).  The aids that
+    // ask for one of the other kernels, and GTM_NO_MESSAGE_MOVES, switch it off.
+    TileMoves moves{};
+    const uint32_t *move_masks = nullptr;
+    size_t moved_lds = 0;
+    if (layers > 1 && !tune(T_NO_MESSAGE_MOVES) && !tune(T_MESSAGES_IN_LDS) && !tune(T_NO_FUSED_MESSAGES) &&
+        !tune(T_NODE_MESSAGES_BY_ATOMICS) && !tune(T_NO_TILE_PACK))
+        moves = moves_of_tiles(g, &move_masks);
+    for (int k = 0; k < moves.n; ++k) moves.type[k] %= d.M;
+    if (moves.n) {
+        moved_lds = tile_messages_moved_lds_words(tg, d.M, moves.n) * 4;
+        if (moved_lds > lds_limit || (int64_t)d.C * tg.tw >= (1ll << 31)) moves.n = 0;
+    }
+    if (moves.n) {
+        static thread_local size_t moved_lds_set = 48 * 1024;
+        if (moved_lds > moved_lds_set) {
+            bool raised = true;
+            for (const void *f : {(const void *)k_tile_messages_moved<0>, (const void *)k_tile_messages_moved<1>,
+                                  (const void *)k_tile_messages_moved<2>})
+                raised = raised && hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)moved_lds) == hipSuccess;
+            if (raised) {
+                moved_lds_set = moved_lds;
+            } else {
+                (void)hipGetLastError();
+                moves.n = 0;
+            }
+        }
+    }
     const bool by_bit = !tune(T_NODE_MESSAGES_BY_ATOMICS);  // tuning aid: the earlier kernel
-    if (layers > 1 && !in_lds.ok && (fused_messages || by_bit)) {
+    if (layers > 1 && !moves.n && !in_lds.ok && (fused_messages || by_bit)) {
         // the clauses of every message bit, for the kernels that build what the nodes send
         hipLaunchKernelGGL(k_message_bit_index, dim3(1), dim3(BIT_INDEX_BLOCK), 0, st, s->hypervectors, d.C, d.MB, d.M,
                            w.bit_start, w.bit_cursor, w.bit_clauses);
@@ -1457,6 +1509,22 @@ int score_on_tiles(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
         for (int l = 1; l < layers; ++l) {
             // the layer's message rows for these tiles (score_tiles.h): one graph per workgroup with its
             // vectors in LDS when they fit, else three launches with the vectors in global memory
+            if (moves.n) {
+                const int cus = compute_units();
+                const int parts = std::max(1, std::min(std::min(8, d.M / 32), cus / n_tiles));
+                auto kernel = !alive_now ? k_tile_messages_moved<0> : tg.tw <= 32 ? k_tile_messages_moved<1> : k_tile_messages_moved<2>;
+                profile_start("k_tile_messages_moved", st);
+                hipLaunchKernelGGL(kernel, dim3(n_tiles, parts), dim3(TILE_MESSAGES_LDS_BLOCK), moved_lds, st, w.tile_bitmap, d.C, tg,
+                                   t0, g->number_of_graphs, d.M, s->hypervectors, d.MB, alive_now, shape.streams(), px.alive_stride,
+                                   g->number_of_graph_nodes, moves, move_masks, w.message_rows);
+                if (int rc = check_launch("tile_messages_moved")) return rc;
+                profile_stop(st);
+                a.lists = w.message_lists + (size_t)(l - 1) * d.C * w.message_list_stride;
+                a.stride = w.message_list_stride;
+                a.longest_list = w.longest_list + (l - 1);
+                if (int rc = message_layer(n_tiles, l)) return rc;
+                continue;
+            }
             if (in_lds.ok) {
                 profile_start("k_tile_messages_in_lds", st);
                 hipLaunchKernelGGL(tg.tw > 32 ? k_tile_messages_in_lds<true> : k_tile_messages_in_lds<false>, dim3(n_tiles),
@@ -1964,6 +2032,64 @@ int gtm_build_tiles(const gtm_config *cfg, const gtm_graphs *graphs, uint32_t *t
                        (const unsigned long long *)counts, cfg->literals, (uint32_t *)(counts + (size_t)tg.rows * 2));
     if (int rc = check_launch("row_order")) return rc;
     remember_tiles(tiles, tg, cfg, graphs);
+    return GTM_OK;
+}
+
+size_t gtm_moves_bytes(const gtm_config *cfg, const gtm_graphs *graphs) {
+    Dims d;
+    if (validate(cfg, &d) || cfg->depth < 2 || !graphs || graphs->number_of_graphs < 1 || graphs->number_of_node_types < 1) return 0;
+    if (graphs->total_edges < 1) return 0;
+    TileGeom tg = geometry_for(cfg, graphs, d.K);
+    if (!tg.ok) return 0;
+    return (TILE_MOVES_HEADER_WORDS + (size_t)tg.n_tiles * TILE_MOVES_MAX * tg.tw) * 4;
+}
+
+// What was found comes back to the host once per data set, because it decides which kernels are launched: one wait of
+// this stream (10 us behind the kernels).  A stream that is being captured cannot be waited for; then the edges are walked.
+int gtm_build_moves(const gtm_config *cfg, const gtm_graphs *graphs, uint32_t *moves, void *stream) {
+    Dims d;
+    if (int rc = validate(cfg, &d)) return rc;
+    if (int rc = validate_graphs(cfg, graphs, 0, 0)) return rc;
+    if (!moves) return fail(GTM_ERR_INVALID, "moves is NULL");
+    if (!gtm_moves_bytes(cfg, graphs)) return fail(GTM_ERR_INVALID, "no moves for this model and data set (gtm_moves_bytes() == 0)");
+    if (!graphs->number_of_graph_node_edges || !graphs->edge || !graphs->edge_index)
+        return fail(GTM_ERR_INVALID, "graphs with edges need number_of_graph_node_edges, edge and edge_index");
+    TileGeom tg = geometry_for(cfg, graphs, d.K);
+    if (int rc = check_tiles(tg, cfg, graphs)) return rc;
+    hipStream_t st = (hipStream_t)stream;
+    remember_moves(graphs, TileMoves{}, nullptr);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &capture) != hipSuccess) {
+        (void)hipGetLastError();
+        return GTM_OK;
+    }
+    if (capture != hipStreamCaptureStatusNone) return GTM_OK;
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(TPB), 0, st, (int32_t *)moves, (int64_t)TILE_MOVES_HEADER_WORDS, 0);
+    if (int rc = check_launch("fill")) return rc;
+    const int64_t slots = (int64_t)tg.n_tiles * tg.tw * 32;
+    hipLaunchKernelGGL(k_edge_moves, dim3((unsigned)std::min<int64_t>(2048, (slots + TILE_MOVES_BLOCK - 1) / TILE_MOVES_BLOCK)),
+                       dim3(TILE_MOVES_BLOCK), 0, st, tg, graphs->number_of_graphs, graphs->node_index, graphs->number_of_graph_nodes,
+                       graphs->number_of_graph_node_edges, graphs->edge_index, graphs->edge, moves);
+    if (int rc = check_launch("edge_moves")) return rc;
+    hipLaunchKernelGGL(k_edge_move_masks, dim3((unsigned)std::min(tg.n_tiles, 4096)), dim3(TILE_MOVES_BLOCK),
+                       (size_t)TILE_MOVES_MAX * tg.tw * 4, st, tg, graphs->number_of_graphs, graphs->node_index,
+                       graphs->number_of_graph_nodes, graphs->number_of_graph_node_edges, graphs->edge_index, graphs->edge, moves,
+                       moves + TILE_MOVES_HEADER_WORDS);
+    if (int rc = check_launch("edge_move_masks")) return rc;
+    uint32_t found[TILE_MOVES_MAX + 1];
+    hipError_t e = hipMemcpyAsync(found, moves, sizeof found, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) return fail(GTM_ERR_HIP, "reading the edges' moves: %s", hipGetErrorString(e));
+    if (found[TILE_MOVES_MAX]) return GTM_OK;
+    TileMoves m{};
+    for (int k = 0; k < TILE_MOVES_MAX && found[k]; ++k) {
+        const int back = (int)TILE_MOVE_OFFSET - (int)(found[k] & 0xFFFFu);  // slot s receives from slot s + back
+        m.type[k] = (int)(found[k] >> 16);
+        m.words[k] = back >> 5;  // (rounded down)
+        m.bits[k] = back & 31;
+        m.n = k + 1;
+    }
+    remember_moves(graphs, m, moves + TILE_MOVES_HEADER_WORDS);
     return GTM_OK;
 }
 

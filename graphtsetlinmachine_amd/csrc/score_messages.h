@@ -67,6 +67,101 @@ inline TileMessagesPlan tile_messages_lds_plan(const TileGeom &g, int M, size_t 
     return p;
 }
 
+// The two rows after the received ones: all ones, and the graphs without nodes (slot bit 0 of each: kernels.py:443-466,
+// 505-527 leave every clause true for such a graph at every layer, which the message literals must not undo).
+__device__ __forceinline__ void tile_rows_after_messages(uint32_t *out, const TileGeom &tg, int tile, int G, int M,
+                                                         const uint32_t *__restrict__ n_nodes) {
+    const int tw = tg.tw;
+    for (int w = threadIdx.x; w < tw; w += TILE_MESSAGES_LDS_BLOCK) {
+        const int used = tg.slot_words == 0 ? tw : tg.gpt * tg.slot_words;
+        uint32_t empties = 0u;
+        for (int b = 0; b < 32; ++b) {
+            const int pos = w * 32 + b, gj = pos / tg.slot_bits;
+            const int64_t g = (int64_t)tile * tg.gpt + gj;
+            if (pos == gj * tg.slot_bits && gj < tg.gpt && g < G && n_nodes[g] == 0u) empties |= 1u << b;
+        }
+        out[(int64_t)M * tw + w] = w < used ? 0xFFFFFFFFu : 0u;
+        out[(int64_t)(M + 1) * tw + w] = empties;
+    }
+}
+
+// The rows of what is sent, literal-major: rows[p] |= truth row of every clause whose hypervector holds bit p (M rows
+// of tw words in LDS, cleared before).  Lane l of a quarter-wave fetches the number and the first two hypervector
+// bits of the stream's clause 16 k + l, a group of 16 clauses ahead of the truth rows; a clause's number and bits
+// then reach the 16 lanes by a lane move (row_share), and eight truth rows are on their way per quarter-wave.
+// WIDE: rows of 33 to 64 words, four of them per lane.
+template <bool WIDE>
+__device__ __forceinline__ void tile_sent_rows_listed(uint32_t *main_region, const uint32_t *__restrict__ bitmap, int tile_local, int C,
+                                                      int tw, int M, const uint32_t *__restrict__ hv, int MB,
+                                                      const uint32_t *__restrict__ alive, int streams, int alive_stride) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int WPL = WIDE ? 4 : 2;  // words of a truth row per lane
+    typedef uint32_t Words __attribute__((ext_vector_type(WPL)));
+    const int group = lane >> 4, gl = lane & 15;
+    // the tile's truth rows through a buffer descriptor: a row is reached by a multiply-add of 24-bit factors per
+    // lane (clause x bytes per row + the lane's place), not by a 64-bit multiply and add
+    const __amdgpu_buffer_rsrc_t truth = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t *>(bitmap + (int64_t)tile_local * C * tw), 0, C * tw * 4, 0x00020000);
+    const bool has_words = WPL * gl < tw;
+    const uint32_t place = has_words ? 4u * WPL * gl : 0u;
+    // a quarter-wave takes the streams q, q + 64, ... of the evaluation that wrote the truth rows
+    for (int q = wave * 4 + group; q < streams; q += TILE_MESSAGES_LDS_BLOCK / 16) {
+    const uint32_t *list = alive ? alive + ((int64_t)tile_local * streams + q) * alive_stride : nullptr;
+    const int n_mine = list ? (int)list[0] : (q < C ? (C - q + streams - 1) / streams : 0);
+    uint32_t id_next = 0u, bit0_next = 0u, bit1_next = 0u;
+    // (every load below is unconditional, from an address that exists, and what it brought is dropped
+    // afterwards where it was not wanted: loads under a condition would wait for one another)
+    auto fetch = [&](int i) {
+        const int at = i < n_mine ? i : n_mine - 1;
+        id_next = list ? list[1 + at] : (uint32_t)(q + streams * at);
+        bit0_next = hv[(int64_t)id_next * MB];
+        bit1_next = hv[(int64_t)id_next * MB + (MB > 1 ? 1 : 0)];
+    };
+    if (n_mine > 0) fetch(gl);
+    for (int i0 = 0; i0 < n_mine; i0 += 16) {  // (the lanes of a quarter-wave leave the loop together)
+        const uint32_t id = id_next, bit0 = bit0_next, bit1 = bit1_next;
+        fetch(i0 + 16 + gl);
+        const int n_here = n_mine - i0 < 16 ? n_mine - i0 : 16;
+        auto eight = [&](auto first_of_eight) {  // clauses u0 .. u0 + 7 of the 16
+            constexpr int u0 = decltype(first_of_eight)::value;
+            uint32_t c[8];
+            Words t[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                c[u] = tile_row_share(id, u0 + u);  // (past the stream's end: its last clause once more)
+                const int at = (int)(__umul24(c[u], (uint32_t)tw * 4u) + place);
+                if constexpr (WIDE) {
+                    t[u] = __builtin_amdgcn_raw_buffer_load_b128(truth, at, 0, 0);
+                } else {
+                    t[u] = __builtin_amdgcn_raw_buffer_load_b64(truth, at, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const uint32_t h0 = tile_row_share(bit0, u0 + u), h1 = tile_row_share(bit1, u0 + u);
+                uint32_t any = t[u][0] | t[u][1];
+                if (WIDE) any |= t[u][2] | t[u][3];
+                if (u0 + u >= n_here || !has_words || any == 0u) continue;
+                for (int j = 0; j < MB; ++j) {
+                    const uint32_t h = j == 0 ? h0 : j == 1 ? h1 : hv[(int64_t)c[u] * MB + j];
+                    if (h >= (uint32_t)M) continue;
+                    // (tw is a multiple of 4: each pair of words is one aligned 64-bit word of LDS)
+                    unsigned long long *row = reinterpret_cast<unsigned long long *>(main_region + __umul24(h, (uint32_t)tw) + WPL * gl);
+#pragma unroll
+                    for (int v = 0; v < WPL / 2; ++v) {
+                        const unsigned long long both =
+                            (unsigned long long)t[u][2 * v] | ((unsigned long long)t[u][2 * v + 1] << 32);
+                        if (both) atomicOr(&row[v], both);
+                    }
+                }
+            }
+        };
+        eight(std::integral_constant<int, 0>{});
+        if (n_here > 8) eight(std::integral_constant<int, 8>{});
+    }
+    }
+}
+
 // WIDE: rows of 33 to 64 words - a quarter-wave reads a truth row at four words per lane, and a thread owns two
 // node slots.
 template <bool WIDE>
@@ -77,7 +172,7 @@ __global__ __launch_bounds__(TILE_MESSAGES_LDS_BLOCK) void k_tile_messages_in_ld
     const uint32_t *__restrict__ edge, int has_edges, int main_words, int range_words, uint32_t *__restrict__ rows) {
     extern __shared__ uint32_t lds[];
     constexpr int NT = TILE_MESSAGES_LDS_BLOCK;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
     const int tile_local = blockIdx.x;
     const int tw = tg.tw, MW = M >> 5, VS = MW + 1, S = tw * 32;
     uint32_t *main_region = lds;
@@ -87,77 +182,8 @@ __global__ __launch_bounds__(TILE_MESSAGES_LDS_BLOCK) void k_tile_messages_in_ld
     for (int i = tid; i < M * tw; i += NT) main_region[i] = 0u;
     __syncthreads();
 
-    // 1. the rows of what is sent, literal-major.  Lane l of a quarter-wave fetches the number and the first two
-    // hypervector bits of the stream's clause 16 k + l, a group of 16 clauses ahead of the truth rows; a clause's
-    // number and bits then reach the 16 lanes by a lane move (row_share), and eight truth rows are on their way
-    // per quarter-wave.
-    {
-        constexpr int WPL = WIDE ? 4 : 2;  // words of a truth row per lane
-        typedef uint32_t Words __attribute__((ext_vector_type(WPL)));
-        const int group = lane >> 4, gl = lane & 15;
-        // the tile's truth rows through a buffer descriptor: a row is reached by a multiply-add of 24-bit factors per
-        // lane (clause x bytes per row + the lane's place), not by a 64-bit multiply and add
-        const __amdgpu_buffer_rsrc_t truth = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint32_t *>(bitmap + (int64_t)tile_local * C * tw), 0, C * tw * 4, 0x00020000);
-        const bool has_words = WPL * gl < tw;
-        const uint32_t place = has_words ? 4u * WPL * gl : 0u;
-        // a quarter-wave takes the streams q, q + 64, ... of the evaluation that wrote the truth rows
-        for (int q = wave * 4 + group; q < streams; q += TILE_MESSAGES_LDS_BLOCK / 16) {
-        const uint32_t *list = alive ? alive + ((int64_t)tile_local * streams + q) * alive_stride : nullptr;
-        const int n_mine = list ? (int)list[0] : (q < C ? (C - q + streams - 1) / streams : 0);
-        uint32_t id_next = 0u, bit0_next = 0u, bit1_next = 0u;
-        // (every load below is unconditional, from an address that exists, and what it brought is dropped
-        // afterwards where it was not wanted: loads under a condition would wait for one another)
-        auto fetch = [&](int i) {
-            const int at = i < n_mine ? i : n_mine - 1;
-            id_next = list ? list[1 + at] : (uint32_t)(q + streams * at);
-            bit0_next = hv[(int64_t)id_next * MB];
-            bit1_next = hv[(int64_t)id_next * MB + (MB > 1 ? 1 : 0)];
-        };
-        if (n_mine > 0) fetch(gl);
-        for (int i0 = 0; i0 < n_mine; i0 += 16) {  // (the lanes of a quarter-wave leave the loop together)
-            const uint32_t id = id_next, bit0 = bit0_next, bit1 = bit1_next;
-            fetch(i0 + 16 + gl);
-            const int n_here = n_mine - i0 < 16 ? n_mine - i0 : 16;
-            auto eight = [&](auto first_of_eight) {  // clauses u0 .. u0 + 7 of the 16
-                constexpr int u0 = decltype(first_of_eight)::value;
-                uint32_t c[8];
-                Words t[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    c[u] = tile_row_share(id, u0 + u);  // (past the stream's end: its last clause once more)
-                    const int at = (int)(__umul24(c[u], (uint32_t)tw * 4u) + place);
-                    if constexpr (WIDE) {
-                        t[u] = __builtin_amdgcn_raw_buffer_load_b128(truth, at, 0, 0);
-                    } else {
-                        t[u] = __builtin_amdgcn_raw_buffer_load_b64(truth, at, 0, 0);
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const uint32_t h0 = tile_row_share(bit0, u0 + u), h1 = tile_row_share(bit1, u0 + u);
-                    uint32_t any = t[u][0] | t[u][1];
-                    if (WIDE) any |= t[u][2] | t[u][3];
-                    if (u0 + u >= n_here || !has_words || any == 0u) continue;
-                    for (int j = 0; j < MB; ++j) {
-                        const uint32_t h = j == 0 ? h0 : j == 1 ? h1 : hv[(int64_t)c[u] * MB + j];
-                        if (h >= (uint32_t)M) continue;
-                        // (tw is a multiple of 4: each pair of words is one aligned 64-bit word of LDS)
-                        unsigned long long *row = reinterpret_cast<unsigned long long *>(main_region + __umul24(h, (uint32_t)tw) + WPL * gl);
-#pragma unroll
-                        for (int v = 0; v < WPL / 2; ++v) {
-                            const unsigned long long both =
-                                (unsigned long long)t[u][2 * v] | ((unsigned long long)t[u][2 * v + 1] << 32);
-                            if (both) atomicOr(&row[v], both);
-                        }
-                    }
-                }
-            };
-            eight(std::integral_constant<int, 0>{});
-            if (n_here > 8) eight(std::integral_constant<int, 8>{});
-        }
-        }
-    }
+    // 1. the rows of what is sent, literal-major
+    tile_sent_rows_listed<WIDE>(main_region, bitmap, tile_local, C, tw, M, hv, MB, alive, streams, alive_stride);
     __syncthreads();
 
     // 2. node-major in place: block (j, w) - rows 32 j .. 32 j + 31, word w - becomes word j of slots 32 w .. 32 w + 31
@@ -191,19 +217,7 @@ __global__ __launch_bounds__(TILE_MESSAGES_LDS_BLOCK) void k_tile_messages_in_ld
         }
     }
 
-    // the all-ones row and the row of graphs without nodes (slot bit 0 of each: kernels.py:443-466,505-527 leave every
-    // clause true for such a graph at every layer, which the message literals must not undo)
-    for (int w = tid; w < tw; w += NT) {
-        const int used = tg.slot_words == 0 ? tw : tg.gpt * tg.slot_words;
-        uint32_t empties = 0u;
-        for (int b = 0; b < 32; ++b) {
-            const int pos = w * 32 + b, gj = pos / tg.slot_bits;
-            const int64_t g = (int64_t)(tile0 + tile_local) * tg.gpt + gj;
-            if (pos == gj * tg.slot_bits && gj < tg.gpt && g < G && n_nodes[g] == 0u) empties |= 1u << b;
-        }
-        out[(int64_t)M * tw + w] = w < used ? 0xFFFFFFFFu : 0u;
-        out[(int64_t)(M + 1) * tw + w] = empties;
-    }
+    tile_rows_after_messages(out, tg, tile0 + tile_local, G, M, n_nodes);
 
     // this thread's source slots (tid, and tid + 1,024 on rows of more than 32 words) and their edges
     constexpr int SPT = WIDE ? 2 : 1;

@@ -51,6 +51,12 @@ def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+# Data sets of fewer edges are not looked at for moves: the look costs 33 us (three launches, a wait), and on sixteen
+# pairs scored once the launches that walk the edges hide behind the host's work (two batches 373 us, with the look
+# 439); 10,000 pairs (10,000 edges each way) gain 24 us on every pass.
+MOVES_FROM_EDGES = 8192
+
+
 class _DeviceGraphs:
     """Device copy of a Graphs object's arrays (tm.py:528-555, 759-784)."""
 
@@ -123,6 +129,11 @@ class _DeviceGraphs:
         self.tiles = torch.empty(nbytes // 4, dtype=torch.int32, device=_device())
         _abi.call("gtm_build_tiles", ctypes.byref(cfg), ctypes.byref(self.desc), _ptr(self.tiles), _stream())
         self.desc.tiles = self.tiles.data_ptr()
+        # are the edges a few moves, as in chains and grids?  (the buffer lives as long as the tiles)
+        nbytes = _abi.lib.gtm_moves_bytes(ctypes.byref(cfg), ctypes.byref(self.desc)) if self.desc.total_edges >= MOVES_FROM_EDGES else 0
+        if nbytes:
+            self.moves = torch.empty(nbytes // 4, dtype=torch.int32, device=_device())
+            _abi.call("gtm_build_moves", ctypes.byref(cfg), ctypes.byref(self.desc), _ptr(self.moves), _stream())
 
 
 class ModelState(tuple):

@@ -209,6 +209,14 @@ size_t gtm_tiles_bytes(const gtm_config *cfg, const gtm_graphs *graphs);
 int gtm_graphs_properties(const gtm_config *cfg, const gtm_graphs *graphs, uint32_t *properties, void *stream);
 int gtm_build_tiles(const gtm_config *cfg, const gtm_graphs *graphs, uint32_t *tiles, void *stream);
 
+/* No counterpart in the reference.  Optional, after gtm_build_tiles and with graphs->tiles set, for models with
+ * message layers: finds out whether the edges of the data set are a few moves (node n -> n + d with type t, as in
+ * chains and grids) and fills a caller-owned buffer of gtm_moves_bytes() with what the message kernels then use
+ * instead of walking the edges.  The buffer must stay as long as the tiles do, and the edges must not change.
+ * Waits for the stream once.  gtm_moves_bytes() is 0 where there is nothing to find. */
+size_t gtm_moves_bytes(const gtm_config *cfg, const gtm_graphs *graphs);
+int gtm_build_moves(const gtm_config *cfg, const gtm_graphs *graphs, uint32_t *moves, void *stream);
+
 /* Scratch needed by gtm_score for sub-batches of `batch` graphs. */
 size_t gtm_score_workspace_bytes(const gtm_config *cfg, const gtm_graphs *graphs, int32_t batch);
 
