@@ -1301,9 +1301,11 @@ int score_on_tiles(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
     // compiled clause: 8 words of packed 16-bit row entries (16 words of byte offsets on half tiles) + the include words
     const int stride0 = half_rows0 ? w.list_stride : tg.half ? 16 + d.LA + HALF_RECORD_EXTRA_WORDS : two_phase ? 8 + d.LA : w.list_stride;
     SegmentPlan plan{};
+    CompileBanks bank0{};
+    bank0.bank[0] = s->ta_state;
     if (half_rows0)
         // rows as k_tile_layer_narrow<ROWS_HALF> stages them: positive literals, node types, all ones
-        hipLaunchKernelGGL(k_compile_clauses, dim3(blocks_for(d.C, TPB / 64)), dim3(TPB), 0, st, s->ta_state, d.C,
+        hipLaunchKernelGGL(k_compile_clauses, dim3(blocks_for(d.C, COMPILE_WAVES)), dim3(64 * COMPILE_WAVES), 0, st, bank0, d.C,
                            d.LA, d.B, d.filter, cfg->literals, hv, g->number_of_node_types, hv, hv + g->number_of_node_types,
                            row_words0, w.list_stride, order, w.lists, d.K, layers == 1 ? s->clause_weights : nullptr, w.wt);
     else if (tg.half) {
@@ -1323,20 +1325,18 @@ int score_on_tiles(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
                            tg.rows - 1, tg.tw, order, w.lists, stride0, d.K,
                            layers == 1 ? s->clause_weights : nullptr, w.wt);
     else
-        hipLaunchKernelGGL(k_compile_clauses, dim3(blocks_for(d.C, TPB / 64)), dim3(TPB), 0, st, s->ta_state, d.C,
+        hipLaunchKernelGGL(k_compile_clauses, dim3(blocks_for(d.C, COMPILE_WAVES)), dim3(64 * COMPILE_WAVES), 0, st, bank0, d.C,
                            d.LA, d.B, d.filter, cfg->literals, 0, g->number_of_node_types, cfg->literals, tg.rows - 1,
                            tg.tw, w.list_stride, order, w.lists, d.K, layers == 1 ? s->clause_weights : nullptr, w.wt);
     if (int rc = check_launch("compile_clauses")) return rc;
     if (layers > 1) {
         hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(TPB), 0, st, (int32_t *)w.longest_list, (int64_t)(layers - 1), 0);
         if (int rc = check_launch("fill")) return rc;
-    }
-    for (int l = 1; l < layers; ++l) {
-        hipLaunchKernelGGL(k_compile_clauses, dim3(blocks_for(d.C, TPB / 64)), dim3(TPB), 0, st,
-                           s->message_ta_state[l - 1], d.C, d.MC, d.B, d.mfilter, 2 * d.M, d.M, 0, 0, d.M, row_words_m,
-                           w.message_list_stride, (const uint32_t *)nullptr,
-                           w.message_lists + (size_t)(l - 1) * d.C * w.message_list_stride, d.K,
-                           l == layers - 1 ? s->clause_weights : nullptr, w.wt, w.longest_list + (l - 1));
+        CompileBanks message_banks{};
+        for (int l = 1; l < layers; ++l) message_banks.bank[l - 1] = s->message_ta_state[l - 1];
+        hipLaunchKernelGGL(k_compile_clauses, dim3(blocks_for(d.C, COMPILE_WAVES), layers - 1), dim3(64 * COMPILE_WAVES), 0, st,
+                           message_banks, d.C, d.MC, d.B, d.mfilter, 2 * d.M, d.M, 0, 0, d.M, row_words_m, w.message_list_stride,
+                           (const uint32_t *)nullptr, w.message_lists, d.K, s->clause_weights, w.wt, w.longest_list);
         if (int rc = check_launch("compile_clauses")) return rc;
     }
     // layer 0 on narrow tiles takes its clauses by length (GTM_NARROW_IN_ORDER, tuning and test aid: by number)
