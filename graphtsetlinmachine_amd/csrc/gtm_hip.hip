@@ -2650,7 +2650,7 @@ int fit_small(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
         g->number_of_node_types < 1)
         return GTM_OK;
     const int MW = d.M / 32;
-    const size_t lds = fit_small_lds_words(cfg->depth, d.C, d.LA, d.MC, MW, d.MB, d.B, d.K) * 4;
+    size_t lds = fit_small_lds_words(cfg->depth, d.C, d.LA, d.MC, MW, d.MB, d.B, d.K) * 4;
     if (lds > FITS_MAX_LDS_BYTES) return GTM_OK;
     if (g->total_edges > 0 && (!g->number_of_graph_node_edges || !g->edge || !g->edge_index))
         return fail(GTM_ERR_INVALID, "graphs with edges need number_of_graph_node_edges, edge and edge_index");
@@ -2694,17 +2694,33 @@ int fit_small(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
     p.k0 = key.k0;
     p.k1 = key.k1;
     p.q_thr = q_threshold(cfg->q, cfg->classes);
+    p.lanes0 = fit_small_lanes(d.C, g->max_number_of_graph_nodes, d.LA);
+    p.lanes1 = fit_small_lanes(d.C, g->max_number_of_graph_nodes, d.MC);
+    p.by_LA = fits_magic((uint32_t)d.LA);
+    p.by_MC = fits_magic((uint32_t)d.MC);
+    p.by_MW = fits_magic((uint32_t)MW);
+    p.by_K = fits_magic((uint32_t)d.K);
+    p.by_types = fits_magic((uint32_t)g->number_of_node_types);
+    auto with = [&](bool draws_twice, bool inc_copy) {
+        return lds + fit_small_lds_more_words(cfg->depth, d.C, d.LA, d.MC, d.K, draws_twice, inc_copy) * 4;
+    };
+    p.draws_twice = with(true, false) <= 160 * 1024;
+    p.inc_copy = with(p.draws_twice != 0, true) <= 160 * 1024;
+    lds = with(p.draws_twice != 0, p.inc_copy != 0);
+    auto kernel = d.B == 8 ? k_fit_small<8, true> : d.B < 8 ? k_fit_small<8, false> : d.B <= 16 ? k_fit_small<16, false> : k_fit_small<32, false>;
     static thread_local size_t lds_set = 48 * 1024;
     if (lds > lds_set) {
-        if (hipFuncSetAttribute((const void *)k_fit_small, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
-            hipSuccess) {
-            (void)hipGetLastError();
-            return GTM_OK;
-        }
+        // (all forms of the kernel, so that the limit that is remembered holds for each)
+        for (const void *f : {(const void *)k_fit_small<8, true>, (const void *)k_fit_small<8, false>, (const void *)k_fit_small<16, false>,
+                              (const void *)k_fit_small<32, false>})
+            if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
+                (void)hipGetLastError();
+                return GTM_OK;
+            }
         lds_set = lds;
     }
     profile_start("k_fit_small", st);
-    hipLaunchKernelGGL(k_fit_small, dim3(1), dim3(FITS_BLOCK), lds, st, p);
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(FITS_THREADS), lds, st, p);
     profile_stop(st);
     if (int rc = check_launch("fit_small")) return rc;
     *done = true;
