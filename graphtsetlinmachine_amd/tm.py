@@ -57,12 +57,17 @@ def _stream():
 MOVES_FROM_EDGES = 8192
 
 
+# The library's switches that the tile geometry depends on.
+_GEOMETRY_SWITCHES = (b"GTM_TILE_LANE_WORDS", b"GTM_NO_HALF_TILES", b"GTM_NO_TWO_PHASE", b"GTM_HALF_LANE_WORDS")
+
+
 class _DeviceGraphs:
     """Device copy of a Graphs object's arrays (tm.py:528-555, 759-784)."""
 
     def __init__(self, graphs):
         self.signature = graphs.signature
         self._stream = torch.cuda.current_stream()  # where the arrays and the tiles are made
+        self._stream_handle, self._device_index = self._stream.cuda_stream, self._stream.device_index
         self.number_of_graphs = int(graphs.number_of_graphs)
         self.max_nodes = int(graphs.max_number_of_graph_nodes)
         # packed on the way where the arrays allow it; then it is also known whether the negated literals are the
@@ -96,10 +101,16 @@ class _DeviceGraphs:
 
     def order_after_upload(self):
         """Work enqueued on the current stream from now on comes after what makes the arrays and the tiles."""
+        # (the handle first: making a Stream object to find that nothing changed costs as much as a launch)
+        if torch._C._cuda_getCurrentRawStream(self._device_index) == self._stream_handle:
+            return
+        # (a stream under capture cannot wait for one that is not; what it captures runs later, and starting a capture
+        # has waited for the device)
+        if torch.cuda.is_current_stream_capturing():
+            return
         now = torch.cuda.current_stream()
-        if now != self._stream:
-            now.wait_stream(self._stream)
-            self._stream = now
+        now.wait_stream(self._stream)
+        self._stream, self._stream_handle = now, now.cuda_stream
 
     def ensure_tiles(self, cfg):
         """Build the literal-major tile layout once per data set and tile
@@ -108,8 +119,7 @@ class _DeviceGraphs:
         sizes, so a data set handed to a model of another shape is tiled
         again."""
         self.order_after_upload()
-        key = (cfg.classes, cfg.literals, cfg.depth, cfg.message_size, _abi.tuning("GTM_TILE_LANE_WORDS"),
-               _abi.tuning("GTM_NO_HALF_TILES"), _abi.tuning("GTM_NO_TWO_PHASE"), _abi.tuning("GTM_HALF_LANE_WORDS"))
+        key = (cfg.classes, cfg.literals, cfg.depth, cfg.message_size) + tuple(map(_abi.lib.gtm_tuning_get, _GEOMETRY_SWITCHES))
         if self._tiles_key == key:
             return
         self._tiles_key = key

@@ -86,3 +86,26 @@ def test_rows_by_moves(shape, complementary):
     assert np.array_equal(got, want)
     assert ("k_tile_messages_moved" in kernels) == taken
     assert np.array_equal(dev.score(0, n, 2), want)  # launch groups: tiles from the middle of the data set
+
+
+def test_scoring_captured_on_another_stream():
+    """Class sums of a data set that was brought to the device on the default stream, captured in a graph on the capture's own
+    stream and replayed, with eager work in between."""
+    from graphtsetlinmachine_amd.tm import MultiClassGraphTsetlinMachine
+
+    import torch
+
+    name, sizes, moves, sizing, _ = SHAPES[5]
+    graphs = _graphs(np.array(sizes * 3), moves, seed=3)  # (enough edges for the moves to be looked for)
+    tm = MultiClassGraphTsetlinMachine(60, 50, 2.0, depth=3, seed=5, **sizing)
+    tm.fit(graphs, np.arange(len(sizes) * 3) % 3, epochs=1)
+    want = tm.score_device(graphs).cpu().numpy()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = tm.score_device(graphs)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), want)
+        assert np.array_equal(tm.score_device(graphs).cpu().numpy(), want)
