@@ -46,8 +46,8 @@ void gtm_pack_plan(const uint32_t *node_type, const uint32_t *degree, const uint
     for (int64_t g = 0; g < G; ++g) {
         const int64_t first = node_index[g], n = n_nodes[g];
         empty |= n == 0;
-        /* the graphs' nodes have to follow one another from 0 to N */
-        if (first + n != (g + 1 < G ? (int64_t)node_index[g + 1] : N) || (g == 0 && first != 0)) {
+        /* the graphs' nodes have to follow one another from 0 to N (and lie inside the arrays, whatever the graphs before say) */
+        if (first + n > N || first + n != (g + 1 < G ? (int64_t)node_index[g + 1] : N) || (g == 0 && first != 0)) {
             index_bad |= 1;
             continue;
         }

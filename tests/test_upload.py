@@ -69,3 +69,22 @@ def test_the_device_holds_the_arrays_as_they_are(shape, piece, monkeypatch):
         assert complementary == (follows and bool((g.number_of_graph_nodes > 0).all()))
     g.X = np.asfortranarray(g.X)
     assert upload.upload(g, torch.device("cuda")) is None
+
+
+@pytest.mark.parametrize("node_index, node_counts", [
+    ([0, 400000000], [400000000, 0]),              # the chain of graphs holds, far past the nodes
+    ([0, 1000000, 1000002], [2, 2, 2]),            # a break, and the chain goes on behind it
+    ([0, 4294967290], [4294967290, 12]),           # sums past 32 bits
+    ([7, 3], [3, 7]),                              # graphs in another order
+], ids=["past_the_nodes", "break", "wrap", "order"])
+def test_graphs_that_do_not_follow_one_another_are_only_looked_at_inside_the_arrays(node_index, node_counts):
+    from graphtsetlinmachine_amd.graphs import _native_encoder
+
+    N = 10
+    u32 = lambda values: np.array(values, dtype=np.uint32)
+    node_type, degree, edge_index = u32([0] * N), u32([1] * N), u32(range(N))
+    first, count, edge = u32(node_index), u32(node_counts), np.zeros((N, 2), dtype=np.uint32)
+    plan, start = np.full(8, 0x5A5A5A5A, dtype=np.uint32), np.zeros(len(first), dtype=np.uint32)
+    _native_encoder().gtm_pack_plan(*(a.ctypes.data for a in (node_type, degree, edge_index, first, count, edge)), N, N, len(first),
+                                    plan.ctypes.data, start.ctypes.data)
+    assert list(plan[:3]) == [0, 0, 0] and plan[4] == 0  # all types and degrees alike; first edges do not follow
