@@ -88,3 +88,19 @@ def test_graphs_that_do_not_follow_one_another_are_only_looked_at_inside_the_arr
     _native_encoder().gtm_pack_plan(*(a.ctypes.data for a in (node_type, degree, edge_index, first, count, edge)), N, N, len(first),
                                     plan.ctypes.data, start.ctypes.data)
     assert list(plan[:3]) == [0, 0, 0] and plan[4] == 0  # all types and degrees alike; first edges do not follow
+
+
+@pytest.mark.parametrize("sizes, follows", [
+    ([1024], 1), ([1025], 0), ([1000000], 0), ([5000] + [3] * 500, 0), ([2000] * 63, 0), ([2000] * 64, 1), ([1024, 0, 7], 1),
+], ids=["1024", "1025", "million", "one_large_among_small", "63_of_2000", "64_of_2000", "ragged"])
+def test_first_edges_are_summed_on_the_device_where_graphs_are_many_or_small(sizes, follows):
+    from graphtsetlinmachine_amd.graphs import _native_encoder
+
+    count = np.array(sizes, dtype=np.uint32)
+    first = (np.cumsum(count) - count).astype(np.uint32)
+    N, G = int(count.sum()), len(count)
+    zeros, edge = np.zeros(N, dtype=np.uint32), np.zeros((1, 2), dtype=np.uint32)
+    plan, start = np.zeros(8, dtype=np.uint32), np.zeros(G, dtype=np.uint32)
+    _native_encoder().gtm_pack_plan(*(a.ctypes.data for a in (zeros, zeros, zeros, first, count, edge)), N, 0, G, plan.ctypes.data,
+                                    start.ctypes.data)
+    assert plan[4] == follows
