@@ -411,11 +411,12 @@ class CommonTsetlinMachine:
         elif incremental == False:  # noqa: E712  (the reference re-initialises layer 0 only, tm.py:524-526)
             self._prepare(self._config(graphs.max_number_of_graph_nodes), False)
         if self._train_graphs is None or not np.array_equal(self.graphs_signature_train, graphs.signature):
-            self.graphs_signature_train = graphs.signature
+            # (first the data, then its name: a construction that fails leaves the resident set under its own)
             self._train_graphs = _DeviceGraphs(graphs)
+            self.graphs_signature_train = graphs.signature
         if self._encoded_Y_gpu is None or not np.array_equal(self.encoded_Y, encoded_Y):
-            self.encoded_Y = encoded_Y
             self._encoded_Y_gpu = _to_device(np.ascontiguousarray(encoded_Y, dtype=np.int32))
+            self.encoded_Y = encoded_Y
 
     def _fit(self, graphs, encoded_Y, epochs=100, incremental=False, examples=None):
         """tm.py:664-752; each epoch is one gtm_fit call.  ``examples=(first, count)`` (not in
@@ -450,8 +451,8 @@ class CommonTsetlinMachine:
         if self._train_graphs is not None and np.array_equal(self.graphs_signature_train, graphs.signature):
             return self._train_graphs  # same data already resident
         if self._test_graphs is None or not np.array_equal(self.graphs_signature_test, graphs.signature):
-            self.graphs_signature_test = graphs.signature
             self._test_graphs = _DeviceGraphs(graphs)
+            self.graphs_signature_test = graphs.signature
         return self._test_graphs
 
     def _score(self, graphs, batch=None):

@@ -216,3 +216,55 @@ def test_subsetting_copies_only_the_edges_added_so_far():
     g.encode()
     sub = g[[1]]
     assert sub.edge.tolist() == [[1, 0], [0, 1], [0, 0]]
+
+
+class _Resident:
+    """Stands in for a data set on the device; the construction of some fails, as when memory runs out."""
+
+    refused = set()
+
+    def __init__(self, graphs):
+        if id(graphs) in self.refused:
+            raise MemoryError("no room")
+        self.graphs = graphs
+
+
+class _Signed:
+    def __init__(self, name):
+        self.signature = np.array([name])
+        self.max_number_of_graph_nodes = 2
+
+
+def test_a_data_set_that_did_not_reach_the_device_is_not_taken_for_the_one_that_did(monkeypatch):
+    monkeypatch.setattr(tm_module, "_DeviceGraphs", _Resident)
+    monkeypatch.setattr(_Resident, "refused", set())
+    monkeypatch.setattr(tm_module, "_to_device", lambda a: a.copy())
+    tm = MultiClassGraphTsetlinMachine(4, 10, 1.0, depth=2, message_size=32, seed=1)
+    tm.initialized = True
+    first, second, labels = _Signed(b"first"), _Signed(b"second"), np.arange(3)
+    # scoring
+    assert tm._score_init(first).graphs is first
+    _Resident.refused.add(id(second))
+    for _ in range(2):
+        with pytest.raises(MemoryError):
+            tm._score_init(second)
+    assert tm._score_init(first).graphs is first
+    _Resident.refused.clear()
+    assert tm._score_init(second).graphs is second
+    # training, and its labels
+    tm._init_fit(first, labels, True)
+    _Resident.refused.add(id(second))
+    for _ in range(2):
+        with pytest.raises(MemoryError):
+            tm._init_fit(second, labels, True)
+    _Resident.refused.clear()
+    tm._init_fit(second, labels, True)
+    assert tm._train_graphs.graphs is second
+    with monkeypatch.context() as m:
+        def refuse(a):
+            raise MemoryError("no room")
+        m.setattr(tm_module, "_to_device", refuse)
+        with pytest.raises(MemoryError):
+            tm._init_fit(second, labels + 1, True)
+    tm._init_fit(second, labels + 1, True)
+    assert np.array_equal(tm._encoded_Y_gpu, labels + 1)
