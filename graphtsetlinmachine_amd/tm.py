@@ -66,8 +66,6 @@ class _DeviceGraphs:
 
     def __init__(self, graphs):
         self.signature = graphs.signature
-        self._stream = torch.cuda.current_stream()  # where the arrays and the tiles are made
-        self._stream_handle, self._device_index = self._stream.cuda_stream, self._stream.device_index
         self.number_of_graphs = int(graphs.number_of_graphs)
         self.max_nodes = int(graphs.max_number_of_graph_nodes)
         # packed on the way where the arrays allow it; then it is also known whether the negated literals are the
@@ -96,21 +94,12 @@ class _DeviceGraphs:
         d.total_edges = int(graphs.edge.shape[0])
         d.tiles = None
         self.desc = d
-        self.tiles = None
+        self.tiles = self.moves = None
         self._tiles_key = None
 
-    def order_after_upload(self):
-        """Work enqueued on the current stream from now on comes after what makes the arrays and the tiles."""
-        # (the handle first: making a Stream object to find that nothing changed costs as much as a launch)
-        if torch._C._cuda_getCurrentRawStream(self._device_index) == self._stream_handle:
-            return
-        # (a stream under capture cannot wait for one that is not; what it captures runs later, and starting a capture
-        # has waited for the device)
-        if torch.cuda.is_current_stream_capturing():
-            return
-        now = torch.cuda.current_stream()
-        now.wait_stream(self._stream)
-        self._stream, self._stream_handle = now, now.cuda_stream
+    def buffers(self):
+        """Every tensor that the device reads this data set from."""
+        return list(self.tensors.values()) + [t for t in (self.tiles, self.moves) if t is not None]
 
     def ensure_tiles(self, cfg):
         """Build the literal-major tile layout once per data set and tile
@@ -118,12 +107,11 @@ class _DeviceGraphs:
         layout keep tiles = NULL.  The geometry depends on the model's
         sizes, so a data set handed to a model of another shape is tiled
         again."""
-        self.order_after_upload()
         key = (cfg.classes, cfg.literals, cfg.depth, cfg.message_size) + tuple(map(_abi.lib.gtm_tuning_get, _GEOMETRY_SWITCHES))
         if self._tiles_key == key:
             return
         self._tiles_key = key
-        self.tiles = None
+        self.tiles = self.moves = None
         self.desc.tiles = None
         if self._complementary is None and cfg.literals % 2 == 0:
             # one look at the data on the device: are the negated literals the complements of the
@@ -308,6 +296,38 @@ class CommonTsetlinMachine:
         self._test_graphs = None
         self._workspace = None
         self._encoded_Y_gpu = None
+        self._stream = self._stream_handle = self._device_index = None
+
+    # ------------------------------------------------------------ streams
+
+    def _take_stream(self):
+        """What this model does on the device happens in the order of the calls, whichever streams they are made
+        on: a call on another stream than the last one's waits for what the last one enqueued (the workspace, the
+        resident data sets and the automata are shared), and memory that is then given up is not used again
+        before both streams are done with it."""
+        # (the handle first: making a Stream object to find that nothing changed costs as much as a launch)
+        if self._stream is not None and torch._C._cuda_getCurrentRawStream(self._device_index) == self._stream_handle:
+            return
+        _device()
+        # (a stream under capture cannot wait for one that is not; what it captures runs later, and starting a capture
+        # has waited for the device)
+        if self._stream is not None and torch.cuda.is_current_stream_capturing():
+            return
+        now = torch.cuda.current_stream()
+        if self._stream is not None:
+            now.wait_stream(self._stream)
+            for t in self._device_buffers():
+                t.record_stream(now)
+        self._stream, self._stream_handle, self._device_index = now, now.cuda_stream, now.device_index
+
+    def _device_buffers(self):
+        out = [t for t in (self._workspace, self._encoded_Y_gpu) if t is not None]
+        if self.initialized:
+            out += [self.ta_state_gpu, self.clause_weights_gpu, self.hypervectors_gpu] + self.message_ta_state_gpu
+        for dg in (self._train_graphs, self._test_graphs):
+            if dg is not None:
+                out += dg.buffers()
+        return out
 
     # ------------------------------------------------------------ sizing
 
@@ -422,6 +442,7 @@ class CommonTsetlinMachine:
         """tm.py:664-752; each epoch is one gtm_fit call.  ``examples=(first, count)`` (not in
         the reference) restricts an epoch to that run of the data set's graphs, so that a
         resident data set can be trained on piece by piece without being cut up."""
+        self._take_stream()
         self._init_fit(graphs, encoded_Y, incremental)
         dg = self._train_graphs
         cfg = self._config(max(dg.max_nodes, 1))
@@ -463,6 +484,7 @@ class CommonTsetlinMachine:
     def score_device(self, graphs, batch=None):
         """Class sums as a flat int32 device tensor [graphs * outputs]; work is
         only enqueued on the current stream."""
+        self._take_stream()
         dg = self._score_init(graphs)
         cfg = self._config(max(dg.max_nodes, 1))
         n = dg.number_of_graphs
@@ -484,6 +506,7 @@ class CommonTsetlinMachine:
 
     def _transform(self, graphs, nodewise, batch=None):
         """tm.py:814-900 as one gtm_transform call."""
+        self._take_stream()
         dg = self._score_init(graphs)
         cfg = self._config(max(dg.max_nodes, 1))
         n, C = dg.number_of_graphs, self.number_of_clauses
@@ -517,6 +540,7 @@ class CommonTsetlinMachine:
     # ------------------------------------------------------------- state I/O
 
     def _download(self):
+        self._take_stream()
         C, B = self.number_of_clauses, self.number_of_state_bits
         self.ta_state = self.ta_state_gpu.cpu().numpy().view(np.uint32).reshape(C * self.number_of_ta_chunks * B)
         self.message_ta_state = [t.cpu().numpy().view(np.uint32) for t in self.message_ta_state_gpu]
@@ -538,6 +562,7 @@ class CommonTsetlinMachine:
         else:
             bank = self.message_ta_state_gpu[depth - 1]
             chunks, literals = self.number_of_message_chunks, self.number_of_message_literals
+        self._take_stream()
         cfg = self._config(max(self._max_nodes_seen(), 1))
         out = torch.empty(self.number_of_clauses * literals, dtype=torch.int32, device=_device())
         _abi.call(entry, ctypes.byref(cfg), _ptr(bank), chunks, literals, _ptr(out), _stream())
@@ -586,6 +611,7 @@ class CommonTsetlinMachine:
     def get_weights(self):
         """tm.py:207-211."""
         if np.array_equal(self.clause_weights, np.array([])):
+            self._take_stream()
             self.clause_weights = self.clause_weights_gpu.cpu().numpy()
         return self.clause_weights.reshape((self.number_of_outputs, self.number_of_clauses))
 
@@ -636,6 +662,7 @@ class CommonTsetlinMachine:
         if ta_state.size < bank_words or weights.size != int(outputs) * int(clauses) or int(ta_chunks) != chunks:
             raise _abi.GtmError("set_state: array sizes do not match the sizes in the tuple")
         banks = getattr(state, "message_ta_state", None)
+        self._take_stream()
         if not same_shape:
             if int(clauses) != self.number_of_clauses and int(depth) > 1:
                 raise _abi.GtmError("set_state cannot change the number of clauses of a model with message layers "
@@ -783,6 +810,7 @@ class CommonTsetlinMachine:
             if np.asarray(array).size != size:
                 raise _abi.GtmError("state's %s has %d elements, expected %d" % (name, np.asarray(array).size, size))
         self.hypervectors = np.ascontiguousarray(self.hypervectors, dtype=np.uint32).reshape(C, self.message_bits)
+        self._take_stream()
         self._allocate()
         self.ta_state_gpu.copy_(_to_device(np.asarray(self.ta_state, dtype=np.uint32)))
         for t, host in zip(self.message_ta_state_gpu, self.message_ta_state):

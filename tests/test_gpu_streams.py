@@ -1,0 +1,62 @@
+"""One model called on several streams, without a device-wide wait between the calls."""
+
+import numpy as np
+import pytest
+
+from tests.test_gpu_message_moves import GRID, _graphs
+
+pytestmark = pytest.mark.gpu
+
+
+def _model_and_sets():
+    from graphtsetlinmachine_amd.tm import MultiClassGraphTsetlinMachine
+
+    sets = [_graphs(np.array([841] * n), GRID, seed=n) for n in (40, 60, 50)]
+    tm = MultiClassGraphTsetlinMachine(120, 100, 2.0, depth=3, message_size=256, seed=5)
+    tm.fit(sets[0], np.arange(40) % 3, epochs=1)
+    want = [tm.score(s) for s in sets]
+    return tm, sets, want
+
+
+def test_data_sets_scored_in_turn_on_two_streams():
+    import torch
+
+    tm, sets, want = _model_and_sets()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    # the training set stays resident; the other two replace one another: brought to the device on one stream, scored on
+    # it and on the other, and given up while that pass may be running, with the memory wanted again at once
+    got = []
+    for turn in range(12):
+        here, there = streams[turn % 2], streams[1 - turn % 2]
+        which = 1 + turn % 2
+        with torch.cuda.stream(here):
+            got.append((which, tm.score_device(sets[which])))
+        with torch.cuda.stream(there):
+            got.append((which, tm.score_device(sets[which])))
+            got.append((0, tm.score_device(sets[0])))
+        with torch.cuda.stream(here):
+            other = 3 - which
+            got.append((other, tm.score_device(sets[other])))
+            torch.full((1 << 20,), 0x5A5A5A5A, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    for which, sums in got:
+        assert np.array_equal(sums.cpu().numpy().reshape(want[which].shape), want[which]), which
+
+
+def test_trained_on_one_stream_from_an_upload_on_another():
+    import torch
+
+    tm, sets, _ = _model_and_sets()
+    twin, _, _ = _model_and_sets()
+    y = np.arange(60) % 3
+    tm.fit(sets[1], y, epochs=2, incremental=True)
+    want = tm.score(sets[2])
+    with torch.cuda.stream(torch.cuda.Stream()):
+        twin.score_device(sets[1])
+        sums = twin.score_device(sets[2])
+    with torch.cuda.stream(torch.cuda.Stream()):
+        twin.fit(sets[1], y, epochs=2, incremental=True)
+        assert np.array_equal(twin.get_weights(), tm.get_weights())
+    assert np.array_equal(twin.get_state()[0], tm.get_state()[0])
+    assert np.array_equal(twin.score(sets[2]), want)
+    del sums

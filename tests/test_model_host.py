@@ -268,3 +268,58 @@ def test_a_data_set_that_did_not_reach_the_device_is_not_taken_for_the_one_that_
             tm._init_fit(second, labels + 1, True)
     tm._init_fit(second, labels + 1, True)
     assert np.array_equal(tm._encoded_Y_gpu, labels + 1)
+
+
+def test_calls_on_different_streams_wait_for_one_another(monkeypatch):
+    """Which stream waits for which, and which tensors are held for which stream, without a device."""
+    log = []
+
+    class Stream:
+        device_index = 0
+
+        def __init__(self, handle):
+            self.cuda_stream = handle
+
+        def wait_stream(self, other):
+            log.append((self.cuda_stream, "waits for", other.cuda_stream))
+
+    class Tensor:
+        def __init__(self, name):
+            self.name = name
+
+        def record_stream(self, stream):
+            log.append((self.name, "held for", stream.cuda_stream))
+
+    class Data:
+        def __init__(self, graphs):
+            self.graphs = graphs
+
+        def buffers(self):
+            return [Tensor(self.graphs)]
+
+    at, capturing = [Stream(11)], [False]
+    monkeypatch.setattr(tm_module, "_device", lambda: None)
+    monkeypatch.setattr(tm_module.torch._C, "_cuda_getCurrentRawStream", lambda device: at[0].cuda_stream, raising=False)
+    monkeypatch.setattr(tm_module.torch.cuda, "current_stream", lambda: at[0])
+    monkeypatch.setattr(tm_module.torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    tm = MultiClassGraphTsetlinMachine(4, 10, 1.0, depth=2, message_size=32, seed=1)
+    tm._take_stream()
+    tm._take_stream()
+    assert log == []
+    tm.initialized, tm._workspace, tm._train_graphs, tm._test_graphs = True, Tensor("workspace"), Data("train"), Data("test")
+    tm.ta_state_gpu, tm.clause_weights_gpu, tm.hypervectors_gpu = Tensor("automata"), Tensor("weights"), Tensor("hypervectors")
+    tm.message_ta_state_gpu = [Tensor("messages")]
+    held = {"workspace", "train", "test", "automata", "weights", "hypervectors", "messages"}
+    at[0] = Stream(22)
+    tm._take_stream()
+    assert log[0] == (22, "waits for", 11)
+    assert {name for name, what, _ in log[1:]} == held and all(s == 22 for _, _, s in log[1:])
+    del log[:]
+    tm._take_stream()
+    assert log == []
+    at[0], capturing[0] = Stream(33), True  # a stream under capture can wait for none that is not
+    tm._take_stream()
+    assert log == []
+    at[0], capturing[0] = Stream(11), False
+    tm._take_stream()
+    assert log[0] == (11, "waits for", 22)
