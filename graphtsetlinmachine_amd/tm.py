@@ -61,10 +61,18 @@ MOVES_FROM_EDGES = 8192
 _GEOMETRY_SWITCHES = (b"GTM_TILE_LANE_WORDS", b"GTM_NO_HALF_TILES", b"GTM_NO_TWO_PHASE", b"GTM_HALF_LANE_WORDS")
 
 
+def _refuse_capture(what):
+    """Uploads and tiles are made once and then taken to be there; recorded in a graph they would be made at each replay,
+    from host memory that is long given back."""
+    if torch.cuda.is_current_stream_capturing():
+        raise _abi.GtmError("%s cannot be used on a stream under capture: score it once before" % what)
+
+
 class _DeviceGraphs:
     """Device copy of a Graphs object's arrays (tm.py:528-555, 759-784)."""
 
     def __init__(self, graphs):
+        _refuse_capture("a data set that is not on the device yet")
         self.signature = graphs.signature
         self.number_of_graphs = int(graphs.number_of_graphs)
         self.max_nodes = int(graphs.max_number_of_graph_nodes)
@@ -96,6 +104,7 @@ class _DeviceGraphs:
         self.desc = d
         self.tiles = self.moves = None
         self._tiles_key = None
+        self._made = None  # event after what made the arrays and the tiles
 
     def buffers(self):
         """Every tensor that the device reads this data set from."""
@@ -110,7 +119,21 @@ class _DeviceGraphs:
         key = (cfg.classes, cfg.literals, cfg.depth, cfg.message_size) + tuple(map(_abi.lib.gtm_tuning_get, _GEOMETRY_SWITCHES))
         if self._tiles_key == key:
             return
+        _refuse_capture("a data set without the tiles of this model's sizes")
         self._tiles_key = key
+        try:
+            self._build_tiles(cfg)
+        finally:
+            self._made = torch.cuda.Event()
+            self._made.record()
+
+    def require_made(self):
+        """For a call that is captured on another stream than the one that made the arrays and the tiles: a stream under
+        capture cannot wait for that one, so it has to be done."""
+        if self._made is None or not self._made.query():
+            raise _abi.GtmError("the data set is still on its way to the device: synchronize before capturing on another stream")
+
+    def _build_tiles(self, cfg):
         self.tiles = self.moves = None
         self.desc.tiles = None
         if self._complementary is None and cfg.literals % 2 == 0:
@@ -304,21 +327,21 @@ class CommonTsetlinMachine:
         """What this model does on the device happens in the order of the calls, whichever streams they are made
         on: a call on another stream than the last one's waits for what the last one enqueued (the workspace, the
         resident data sets and the automata are shared), and memory that is then given up is not used again
-        before both streams are done with it."""
+        before both streams are done with it.  Returns True where it could not wait: on another stream that is being
+        captured (a stream under capture cannot wait for one that is not; what it captures runs later)."""
         # (the handle first: making a Stream object to find that nothing changed costs as much as a launch)
         if self._stream is not None and torch._C._cuda_getCurrentRawStream(self._device_index) == self._stream_handle:
-            return
+            return False
         _device()
-        # (a stream under capture cannot wait for one that is not; what it captures runs later, and starting a capture
-        # has waited for the device)
         if self._stream is not None and torch.cuda.is_current_stream_capturing():
-            return
+            return True
         now = torch.cuda.current_stream()
         if self._stream is not None:
             now.wait_stream(self._stream)
             for t in self._device_buffers():
                 t.record_stream(now)
         self._stream, self._stream_handle, self._device_index = now, now.cuda_stream, now.device_index
+        return False
 
     def _device_buffers(self):
         out = [t for t in (self._workspace, self._encoded_Y_gpu) if t is not None]
@@ -484,11 +507,13 @@ class CommonTsetlinMachine:
     def score_device(self, graphs, batch=None):
         """Class sums as a flat int32 device tensor [graphs * outputs]; work is
         only enqueued on the current stream."""
-        self._take_stream()
+        captured_elsewhere = self._take_stream()
         dg = self._score_init(graphs)
         cfg = self._config(max(dg.max_nodes, 1))
         n = dg.number_of_graphs
         dg.ensure_tiles(cfg)
+        if captured_elsewhere:
+            dg.require_made()
         if batch is None:
             # as many graphs per launch group as fit in 4 GiB of workspace beyond its fixed part
             size = lambda b: _abi.lib.gtm_score_workspace_bytes(ctypes.byref(cfg), ctypes.byref(dg.desc), b)

@@ -60,3 +60,47 @@ def test_trained_on_one_stream_from_an_upload_on_another():
     assert np.array_equal(twin.get_state()[0], tm.get_state()[0])
     assert np.array_equal(twin.score(sets[2]), want)
     del sums
+
+
+def test_a_data_set_that_is_not_on_the_device_is_refused_under_capture():
+    """... with an error, and the model goes on; so is one without this model's tiles, and one whose upload is under way."""
+    import torch
+
+    from graphtsetlinmachine_amd import _abi
+
+    tm, sets, want = _model_and_sets()
+    new = _graphs(np.array([841] * 30), GRID, seed=30)
+    resident = tm._test_graphs
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        here = torch.zeros(1, device="cuda")
+        with pytest.raises(_abi.GtmError, match="not on the device yet"):
+            tm.score_device(new)
+    assert tm._test_graphs is resident and here is not None
+    resident._tiles_key = None
+    with torch.cuda.graph(torch.cuda.CUDAGraph()):
+        here = torch.zeros(1, device="cuda")
+        with pytest.raises(_abi.GtmError, match="tiles of this model's sizes"):
+            tm.score_device(sets[2])
+    want_new = tm.score(new)
+    # resident and done: captured, on another stream than the default one where it was made
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = tm.score_device(new)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy().reshape(want_new.shape), want_new)
+        assert np.array_equal(tm.score(sets[0]), want[0])
+
+    class Unfinished:
+        def query(self):
+            return False
+
+    tm._test_graphs._made = Unfinished()
+    with torch.cuda.graph(torch.cuda.CUDAGraph()):
+        here = torch.zeros(1, device="cuda")
+        with pytest.raises(_abi.GtmError, match="on its way"):
+            tm.score_device(new)
+    assert np.array_equal(tm.score(new), want_new)
