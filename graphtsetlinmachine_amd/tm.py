@@ -103,6 +103,7 @@ class _DeviceGraphs:
         d.tiles = None
         self.desc = d
         self.tiles = self.moves = None
+        self._moves_known = False
         self._tiles_key = None
         self._made = None  # event after what made the arrays and the tiles
 
@@ -135,6 +136,7 @@ class _DeviceGraphs:
 
     def _build_tiles(self, cfg):
         self.tiles = self.moves = None
+        self._moves_known = False
         self.desc.tiles = None
         if self._complementary is None and cfg.literals % 2 == 0:
             # one look at the data on the device: are the negated literals the complements of the
@@ -150,7 +152,13 @@ class _DeviceGraphs:
         self.tiles = torch.empty(nbytes // 4, dtype=torch.int32, device=_device())
         _abi.call("gtm_build_tiles", ctypes.byref(cfg), ctypes.byref(self.desc), _ptr(self.tiles), _stream())
         self.desc.tiles = self.tiles.data_ptr()
-        # are the edges a few moves, as in chains and grids?  (the buffer lives as long as the tiles)
+
+    def ensure_moves(self, cfg):
+        """Are the edges a few moves, as in chains and grids?  Looked at once per layout of tiles, by the first call that
+        has a use for the answer: training has none.  (The buffer lives as long as the tiles.)"""
+        if self._moves_known or self.tiles is None or torch.cuda.is_current_stream_capturing():
+            return
+        self._moves_known = True
         nbytes = _abi.lib.gtm_moves_bytes(ctypes.byref(cfg), ctypes.byref(self.desc)) if self.desc.total_edges >= MOVES_FROM_EDGES else 0
         if nbytes:
             self.moves = torch.empty(nbytes // 4, dtype=torch.int32, device=_device())
@@ -506,7 +514,8 @@ class CommonTsetlinMachine:
 
     def score_device(self, graphs, batch=None):
         """Class sums as a flat int32 device tensor [graphs * outputs]; work is
-        only enqueued on the current stream."""
+        only enqueued on the current stream.  (The first call on a data set may
+        wait for the stream once: what it finds decides which kernels follow.)"""
         captured_elsewhere = self._take_stream()
         dg = self._score_init(graphs)
         cfg = self._config(max(dg.max_nodes, 1))
@@ -514,6 +523,7 @@ class CommonTsetlinMachine:
         dg.ensure_tiles(cfg)
         if captured_elsewhere:
             dg.require_made()
+        dg.ensure_moves(cfg)
         if batch is None:
             # as many graphs per launch group as fit in 4 GiB of workspace beyond its fixed part
             size = lambda b: _abi.lib.gtm_score_workspace_bytes(ctypes.byref(cfg), ctypes.byref(dg.desc), b)
@@ -536,6 +546,7 @@ class CommonTsetlinMachine:
         cfg = self._config(max(dg.max_nodes, 1))
         n, C = dg.number_of_graphs, self.number_of_clauses
         dg.ensure_tiles(cfg)
+        dg.ensure_moves(cfg)
         width = max(int(np.max(graphs.number_of_graph_nodes)), 1) if nodewise else 0
         if batch is None:
             size = lambda b: _abi.lib.gtm_transform_workspace_bytes(ctypes.byref(cfg), ctypes.byref(dg.desc), b)

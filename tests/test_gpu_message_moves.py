@@ -109,3 +109,24 @@ def test_scoring_captured_on_another_stream():
         torch.cuda.synchronize()
         assert np.array_equal(out.cpu().numpy(), want)
         assert np.array_equal(tm.score_device(graphs).cpu().numpy(), want)
+
+
+def test_moves_are_looked_for_by_the_first_call_that_uses_them():
+    """Training has no use for them; scoring the training set has, and so has every layout of its tiles."""
+    from graphtsetlinmachine_amd.tm import MultiClassGraphTsetlinMachine
+
+    name, sizes, moves, sizing, _ = SHAPES[5]
+    graphs = _graphs(np.array(sizes * 3), moves, seed=3)
+    tm = MultiClassGraphTsetlinMachine(60, 50, 2.0, depth=3, seed=5, **sizing)
+    tm.fit(graphs, np.arange(len(sizes) * 3) % 3, epochs=1)
+    dg = tm._train_graphs
+    assert dg.tiles is not None and dg.moves is None
+    want = tm.score(graphs)
+    assert tm._train_graphs is dg and dg.moves is not None
+    dg._tiles_key = None
+    tm.fit(graphs, np.arange(len(sizes) * 3) % 3, epochs=0, incremental=True)
+    assert dg.moves is None
+    features, sums = tm.transform(graphs)
+    assert dg.moves is not None and np.array_equal(sums, want)
+    words = dg.moves[:9].cpu().numpy()  # the (type, offset) keys found, then whether there were too many
+    assert sorted(int(v) for v in words[:4]) == sorted((t << 16) | (32768 + d) for t, d in GRID) and not words[4:].any()
