@@ -38,7 +38,11 @@ class _Image:
     def _buffer(self):
         if self.open is None:
             if self.turn < PIECES:
-                self.ring.append((torch.empty(self.piece, dtype=torch.uint8, pin_memory=True), torch.cuda.Event()))
+                try:
+                    buffer = torch.empty(self.piece, dtype=torch.uint8, pin_memory=True)
+                except RuntimeError as e:
+                    raise torch.OutOfMemoryError("no pinned memory") from e
+                self.ring.append((buffer, torch.cuda.Event()))
             self.open = self.ring[self.turn % PIECES]
             if self.turn >= PIECES:
                 self.open[1].synchronize()
@@ -80,7 +84,8 @@ def _align(n):
 
 def upload(graphs, device):
     """(tensors by name, True when every negated literal is the complement of its positive one and every graph has
-    a node) or None when the arrays are not as the packer addresses them (then they are copied as they are)."""
+    a node) or None when the arrays are not as the packer addresses them, or when there is no room for the packed image
+    beside them (half as much again) or for pinned memory.  Then they are copied as they are."""
     lib = _native_encoder()
     arrays = {name: getattr(graphs, name) for name in _ARRAYS}
     if lib is None or any(
@@ -95,6 +100,16 @@ def upload(graphs, device):
     if edge.shape != (E, 2) or any(arrays[n].shape != (N,) for n in ("node_type", "number_of_graph_node_edges", "edge_index")) \
             or arrays["node_index"].shape != (G,):
         return None
+    try:
+        return _upload(lib, arrays, hv, device)
+    except torch.OutOfMemoryError:
+        pass  # (and the image is given back here, with the exception)
+    return None
+
+
+def _upload(lib, arrays, hv, device):
+    X, edge = arrays["X"], arrays["edge"]
+    N, G, E = X.shape[0], arrays["number_of_graph_nodes"].shape[0], edge.shape[0]
     at = {name: a.ctypes.data for name, a in arrays.items()}
     LA, words = X.shape[1], (hv + 31) // 32
     plan = np.empty(8, dtype=np.uint32)

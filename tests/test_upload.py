@@ -104,3 +104,46 @@ def test_first_edges_are_summed_on_the_device_where_graphs_are_many_or_small(siz
     _native_encoder().gtm_pack_plan(*(a.ctypes.data for a in (zeros, zeros, zeros, first, count, edge)), N, 0, G, plan.ctypes.data,
                                     start.ctypes.data)
     assert plan[4] == follows
+
+
+def _refusing(monkeypatch, is_refused):
+    import torch
+
+    empty = torch.empty
+
+    def refuse(*size, **kwargs):
+        if is_refused(kwargs):
+            raise torch.OutOfMemoryError("no room")
+        return empty(*size, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", refuse)
+
+
+@pytest.mark.parametrize("refused", [lambda k: True, lambda k: False], ids=["image", "pinned"])
+def test_without_room_the_arrays_are_left_to_plain_copies(refused, monkeypatch):
+    import torch
+
+    from graphtsetlinmachine_amd import upload
+
+    _refusing(monkeypatch, refused)
+    if torch.cuda.is_available():
+        _refusing(monkeypatch, lambda k: refused(k) or k.get("pin_memory"))  # (without a device there is no pinned memory)
+    assert upload.upload(graphs_of(32), torch.device("cpu")) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("piece", [128, 2 << 20])
+@pytest.mark.parametrize("refused", [
+    lambda k: k.get("dtype") is not None and str(k["dtype"]) == "torch.int32", lambda k: k.get("pin_memory")], ids=["arrays", "pinned"])
+def test_without_room_the_device_still_holds_the_arrays(refused, piece, monkeypatch):
+    from graphtsetlinmachine_amd import upload
+    from graphtsetlinmachine_amd.tm import _DeviceGraphs
+
+    g = graphs_of(64, n_graphs=70, max_nodes=130)
+    monkeypatch.setattr(upload, "PIECE_BYTES", piece)
+    with monkeypatch.context() as m:
+        _refusing(m, refused)
+        dg = _DeviceGraphs(g)
+    assert dg._complementary is None  # (plain copies: not looked at)
+    for name in ARRAYS:
+        assert np.array_equal(dg.tensors[name].cpu().numpy().view(np.uint32), getattr(g, name).reshape(-1)), name
