@@ -29,7 +29,8 @@ class _Image:
 
     def __init__(self, nbytes, largest_item, device):
         self.device = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        self.piece = min(nbytes, max(PIECE_BYTES, 16 * largest_item))
+        # (one size for whatever data set: pinned memory of a new size takes 100 to 200 us the first time)
+        self.piece = max(PIECE_BYTES, 16 * largest_item)
         self.ring = []  # [pinned buffer, event after its last transfer]
         self.turn = 0
         self.open = None  # the ring's entry that is being filled

@@ -147,3 +147,22 @@ def test_without_room_the_device_still_holds_the_arrays(refused, piece, monkeypa
     assert dg._complementary is None  # (plain copies: not looked at)
     for name in ARRAYS:
         assert np.array_equal(dg.tensors[name].cpu().numpy().view(np.uint32), getattr(g, name).reshape(-1)), name
+
+
+@pytest.mark.gpu
+def test_small_data_sets_of_any_size_share_their_pinned_memory(monkeypatch):
+    import torch
+
+    from graphtsetlinmachine_amd import upload
+
+    asked, empty = set(), torch.empty
+
+    def watch(*size, **kwargs):
+        if kwargs.get("pin_memory"):
+            asked.add(size)
+        return empty(*size, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", watch)
+    for n in (1, 3, 20, 150):
+        upload.upload(graphs_of(64, n_graphs=n), torch.device("cuda"))
+    assert asked == {(upload.PIECE_BYTES,)}
