@@ -295,6 +295,9 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
             if (!p.has_edges || nodes == 0) return;
             first_edge = (uint32_t)__builtin_amdgcn_readfirstlane((int)offset);
             graph_edges = __builtin_amdgcn_readlane((int)(offset + count), nodes - 1) - (int)first_edge;
+            // edges that do not lie node after node are not parked but read where they are
+            const uint32_t next_offset = (uint32_t)__shfl_down((int)offset, 1);
+            if (__ballot(lane < nodes - 1 && next_offset != offset + count) != 0ull) graph_edges = FITS_EDGES_LDS + 1;
             const uint2 *from = (const uint2 *)p.edge + first_edge;
             if (graph_edges <= FITS_EDGES_LDS) {
 #pragma unroll

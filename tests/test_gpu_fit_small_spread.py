@@ -48,3 +48,41 @@ def test_every_spread_trains_as_the_oracle(shape, s):
         assert np.array_equal(ta, model.ta_state), "layer-0 automata after epoch %d" % epoch
         for layer in range(depth - 1):
             assert np.array_equal(banks[layer], model.message_ta_state[layer]), "bank %d epoch %d" % (layer, epoch)
+
+
+def _trains_as_the_oracle(model, dev, graphs, classes, seed, epochs=2):
+    G = graphs.number_of_graphs
+    Y = o.encode_labels(np.random.default_rng(seed).integers(0, classes, size=G), classes, model.cfg.threshold)
+    for epoch in range(epochs):
+        o.fit(model, graphs, Y)
+        dev.fit(Y, 0, G, epoch * G)
+        ta, banks, w = dev.download()
+        assert np.array_equal(w, model.clause_weights), "weights after epoch %d" % epoch
+        assert np.array_equal(ta, model.ta_state), "layer-0 automata after epoch %d" % epoch
+        for layer in range(model.depth - 1):
+            assert np.array_equal(banks[layer], model.message_ta_state[layer]), "bank %d epoch %d" % (layer, epoch)
+
+
+@pytest.mark.parametrize("degree", [2, 9], ids=["few", "many"])
+@pytest.mark.parametrize("order", ["reversed", "shuffled", "gap"])
+def test_edges_that_do_not_lie_node_after_node(order, degree):
+    """The same graphs with a node's edges anywhere in the edge array: edge_index says where."""
+    import copy
+
+    from tests.gpu_harness import Device
+
+    graphs = helpers.random_graphs(11, n_graphs=30, max_nodes=20, max_degree=degree, edge_types=("a", "b"))
+    cfg = helpers.oracle_config(graphs, classes=2, clauses=8, depth=2, T=15, message_size=64)
+    model = helpers.random_model(11, cfg, 2, s=2.0, include_density=0.03)
+    moved = copy.deepcopy(graphs)
+    N, gap = len(graphs.node_type), 5 if order == "gap" else 0
+    nodes = np.arange(N)[::-1] if order == "reversed" else np.random.default_rng(3).permutation(N) if order == "shuffled" else np.arange(N)
+    edges, at = [], 0
+    for n in nodes:
+        a, k = int(graphs.edge_index[n]), int(graphs.number_of_graph_node_edges[n])
+        moved.edge_index[n] = at
+        edges.append(graphs.edge[a:a + k])
+        edges.append(np.zeros((gap, 2), dtype=np.uint32))
+        at += k + gap
+    moved.edge = np.ascontiguousarray(np.concatenate(edges))
+    _trains_as_the_oracle(model, Device(model, moved), graphs, 2, 11)
