@@ -42,7 +42,8 @@ constexpr int FITS_MAX_NODES = 64;
 constexpr size_t FITS_MAX_LDS_BYTES = 128 * 1024;  // of the 160 KB a workgroup can have
 constexpr int FITS_X_AHEAD = 16;                   // literal words per helper lane fetched ahead; the rest is read at the step's end
 constexpr int FITS_EDGES_LDS = FITS_BLOCK;         // edges of a graph parked in LDS (more: read in place)
-constexpr int FITS_DIRECT = 4;                     // LDS atomics per thread up to which messages skip the nodes' vectors
+constexpr int FITS_DIRECT = 4;                     // (clause, edge, bit)s per thread up to which messages skip the nodes' vectors
+constexpr uint32_t FITS_IS_DIRECT = 1u << 16;      // in what is told of an example's nodes
 constexpr int FITS_Y_LDS = 64;                     // classes whose labels are fetched ahead (K <= this, else read in place)
 
 struct FitSmallParams {
@@ -90,7 +91,7 @@ inline size_t fit_small_lds_words(int depth, int C, int LA, int MC, int MW, int 
 // example (twice); where there is room, the second half of the random draws and the include planes' copy (else the
 // planes are read where they are).
 inline size_t fit_small_lds_more_words(int depth, int C, int LA, int MC, int K, bool draws_twice, bool inc_copy) {
-    return (size_t)C + FITS_MAX_NODES + 1 + 8 + (draws_twice ? (size_t)C + 2 * (size_t)C * K : 0) +
+    return (size_t)C + FITS_EDGES_LDS + 1 + 8 + (draws_twice ? (size_t)C + 2 * (size_t)C * K : 0) +
            (inc_copy ? (size_t)C * (LA + (size_t)(depth - 1) * MC) : 0);
 }
 
@@ -200,10 +201,10 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
     int32_t *upd = incl_both + 2 * C;              // [C][K]
     const int draw_words = p.draws_twice ? C + 2 * C * K : 0;  // (from an example's to the next one's)
     uint32_t *draw_both = (uint32_t *)(upd + C * K);  // [C] node picks, [C][K][2] decisions
-    uint32_t *info_both = draw_both + C + 2 * C * K + draw_words;  // twice: an example's nodes, edges, first edge, magic of its nodes
-    uint32_t *magic_of = info_both + 8;            // [FITS_MAX_NODES + 1]
+    uint32_t *info_both = draw_both + C + 2 * C * K + draw_words;  // twice: an example's nodes, edges, first edge (or the edges' magic), magic of its nodes
+    uint32_t *magic_of = info_both + 8;            // [FITS_EDGES_LDS + 1]
     // the include planes, every bank's words in order: a copy, so that lanes read neighbouring words, or in place
-    uint32_t *inc_copy = magic_of + FITS_MAX_NODES + 1;
+    uint32_t *inc_copy = magic_of + FITS_EDGES_LDS + 1;
     const uint32_t *inc_words = p.inc_copy ? inc_copy : lds + (B - 1);
     const int inc_stride = p.inc_copy ? 1 : B;
     const int all_words = C * (LA + layers * MC);
@@ -224,11 +225,6 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
             if (!pick) to[1] = r.v[1];
         }
     };
-    // Few edges: a true clause's bits go straight to the far ends of its node's edges (at most FITS_DIRECT atomics
-    // per thread); else through the vectors that the nodes send, one phase more.
-    auto goes_direct = [&](int graph_edges) {
-        return graph_edges <= FITS_EDGES_LDS && (int64_t)graph_edges * C * p.MB <= FITS_DIRECT * FITS_BLOCK;
-    };
     struct Example {  // where example i's data are
         uint32_t *x_rows, *types, *ne, *ei, *labels, *header;
     };
@@ -240,9 +236,11 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
         e.labels = e.types + 3 * FITS_MAX_NODES, e.header = e.labels + FITS_Y_LDS;
         return e;
     };
-    auto tell = [&](int i, int nodes, int edges, uint32_t first_edge) {  // (one lane)
+    auto tell = [&](int i, int nodes, int edges, bool direct, uint32_t first_edge) {  // (one lane)
         uint32_t *info = info_both + 4 * (i & 1);
-        info[0] = (uint32_t)nodes, info[1] = (uint32_t)edges, info[2] = first_edge, info[3] = magic_of[nodes > 0 ? nodes : 1];
+        info[0] = (uint32_t)nodes | (direct ? FITS_IS_DIRECT : 0u);
+        info[1] = (uint32_t)edges, info[2] = direct ? magic_of[edges > 0 ? edges : 1] : first_edge;
+        info[3] = magic_of[nodes > 0 ? nodes : 1];
     };
 
     // state -> LDS
@@ -256,7 +254,7 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
             const int first = l == 0 ? 0 : C * LA + (l - 1) * C * MC;
             for (int i = tid; i < C * (l == 0 ? LA : MC); i += FITS_THREADS) inc_copy[first + i] = p.bank[l][(int64_t)i * B + B - 1];
         }
-    for (int i = tid; i <= FITS_MAX_NODES; i += FITS_THREADS) magic_of[i] = fits_magic((uint32_t)i);
+    for (int i = tid; i <= FITS_EDGES_LDS; i += FITS_THREADS) magic_of[i] = fits_magic((uint32_t)i);
     for (int i = tid; i < 2 * C; i += FITS_THREADS) incl_both[i] = 0;
     draw(0, tid, draws, FITS_THREADS);
     for (int i = tid; i < K * C; i += FITS_THREADS) wts[i] = p.weights[i];
@@ -289,15 +287,19 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
         // requested at its top): the edge counts and offsets that say where they are came with the example's other data.
         uint32_t first_edge = 0u;
         int graph_edges = 0;
+        bool direct = true;
         uint2 edge_ahead[FITS_EDGES_LDS / 64];
         auto request_edges = [&](int nodes, uint32_t count, uint32_t offset) {  // count, offset: of node `lane`
-            first_edge = 0u, graph_edges = 0;
+            first_edge = 0u, graph_edges = 0, direct = true;
             if (!p.has_edges || nodes == 0) return;
             first_edge = (uint32_t)__builtin_amdgcn_readfirstlane((int)offset);
             graph_edges = __builtin_amdgcn_readlane((int)(offset + count), nodes - 1) - (int)first_edge;
             // edges that do not lie node after node are not parked but read where they are
             const uint32_t next_offset = (uint32_t)__shfl_down((int)offset, 1);
             if (__ballot(lane < nodes - 1 && next_offset != offset + count) != 0ull) graph_edges = FITS_EDGES_LDS + 1;
+            // Few edges: a true clause's bits go straight to the far ends of the edges, a thread per (clause, edge); else
+            // through the vectors that the nodes send, one phase more.
+            direct = graph_edges <= FITS_EDGES_LDS && (int64_t)graph_edges * C * p.MB <= FITS_DIRECT * FITS_BLOCK;
             const uint2 *from = (const uint2 *)p.edge + first_edge;
             if (graph_edges <= FITS_EDGES_LDS) {
 #pragma unroll
@@ -305,24 +307,42 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
                     if (64 * r < graph_edges && lane + 64 * r < graph_edges) edge_ahead[r] = from[lane + 64 * r];
             }
         };
+        // ... and, where messages go straight along them, the node that each starts from (the last one whose first edge is
+        // not behind it), in the upper half of the word with the far end
+        uint32_t source_ahead[FITS_EDGES_LDS / 64];
+        auto find_sources = [&](const Example &e, int nodes) {
+#pragma unroll
+            for (int r = 0; r < FITS_EDGES_LDS / 64; ++r) {
+                source_ahead[r] = 0u;
+                if (!direct || 64 * r >= graph_edges) continue;
+                uint32_t from = 0u;
+                for (int step = nodes > 1 ? 1 << (31 - __clz(nodes - 1)) : 0; step > 0; step >>= 1) {
+                    const uint32_t n = from + (uint32_t)step;
+                    if (n < (uint32_t)nodes && e.ei[n] - first_edge <= (uint32_t)(lane + 64 * r)) from = n;
+                }
+                source_ahead[r] = from << 16;
+            }
+        };
         {
             const Example e = example(0);
             request_edges(n_nodes, lane < n_nodes ? e.ne[lane] : 0u, lane < n_nodes ? e.ei[lane] : 0u);
-            if (lane == 0) tell(0, n_nodes, graph_edges, first_edge);
+            find_sources(e, n_nodes);
+            if (lane == 0) tell(0, n_nodes, graph_edges, direct, first_edge);
         }
         lds_barrier();
         for (int i = 0; i < p.n_examples; ++i) {
             const int ex = p.first_example + i;
             const int nn = n_nodes > 0 ? n_nodes : 1;
             const Example e = example(i), to = example(i + 1);
-            const bool direct = goes_direct(graph_edges);
+            const bool direct_now = direct;  // (this example's: the next one's edges are asked for below)
             for (int l = 0; l < layers; ++l)  // (what arrives is ORed in)
                 for (int j = lane; j < nn * MW; j += 64) got_all[l * FITS_MAX_NODES * MW + j] = 0u;
             if (graph_edges <= FITS_EDGES_LDS) {
 #pragma unroll
                 for (int r = 0; r < FITS_EDGES_LDS / 64; ++r) {
                     const int j = lane + 64 * r;
-                    if (64 * r < graph_edges && j < graph_edges) edges_lds[2 * j] = edge_ahead[r].x, edges_lds[2 * j + 1] = edge_ahead[r].y;
+                    if (64 * r < graph_edges && j < graph_edges)
+                        edges_lds[2 * j] = (edge_ahead[r].x & 0xFFFFu) | source_ahead[r], edges_lds[2 * j + 1] = edge_ahead[r].y;
                 }
             }
             // what lands at the step's end: example i + 1 (its node count and offset came with example i), the header of i + 2
@@ -347,8 +367,8 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
                 if (l > 0)
                     for (int j = lane; j < 2 * C; j += 64) truth[(l & 1) ^ 1][j] = 0u;
                 lds_barrier();  // sent
-                if (!direct) lds_barrier();  // along the edges
-                if (!direct)
+                if (!direct_now) lds_barrier();  // along the edges
+                if (!direct_now)
                     for (int j = lane; j < nn * MW; j += 64) sent[j] = 0u;
                 lds_barrier();  // K2
             }
@@ -373,7 +393,8 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
             to.types[lane] = field_ahead[0], to.ne[lane] = field_ahead[1], to.ei[lane] = field_ahead[2];
             to.labels[lane] = label_ahead;
             if (lane < 2) to.header[lane] = header_ahead;
-            if (lane == 0) tell(i + 1, n_next, graph_edges, first_edge);
+            find_sources(to, n_next);
+            if (lane == 0) tell(i + 1, n_next, graph_edges, direct, first_edge);
             n_nodes = n_next;
             lds_barrier();
         }
@@ -385,15 +406,17 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
         const uint32_t step = p.first_step + (uint32_t)i;
         const uint32_t *info = info_both + 4 * (i & 1);
         const int graph_edges = __builtin_amdgcn_readfirstlane((int)info[1]);
-        const uint32_t first_edge = info[2], by_nn = info[3];
+        const uint32_t first_edge = info[2], by_edges = info[2], by_nn = info[3];
         n_nodes = __builtin_amdgcn_readfirstlane((int)info[0]);
+        const bool direct = ((uint32_t)n_nodes & FITS_IS_DIRECT) != 0u;
+        n_nodes &= (int)(FITS_IS_DIRECT - 1u);
         const int nn = n_nodes > 0 ? n_nodes : 1;  // a graph without nodes: one stand-in pair per clause
         const Example e_now = example(i);
         const uint32_t *x_rows = e_now.x_rows, *types = e_now.types, *ne_lds = e_now.ne, *ei_lds = e_now.ei;
         const int32_t *y = (const int32_t *)e_now.labels;
         const uint32_t *draw_node = draw_both + (i & 1) * draw_words, *draw_update = draw_node + C;
         int32_t *incl_of = incl_both + (i & 1) * C;
-        const bool edges_parked = graph_edges <= FITS_EDGES_LDS, direct = goes_direct(graph_edges);
+        const bool edges_parked = graph_edges <= FITS_EDGES_LDS;
 
         // ---- layer 0 (K1), 2^lanes0 lanes per (clause, node); truth[0] is all zero here
         uint32_t *cur = truth[0], *nxt = truth[1];
@@ -425,19 +448,16 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
         for (int l = 0; l < layers; ++l) {
             uint32_t *got = got_all + (size_t)l * FITS_MAX_NODES * MW;
             if (direct) {
-                for (int j = tid; j < C * n_nodes; j += FITS_BLOCK) {
-                    const int c = fits_div(j, nn, by_nn), n = j - c * nn;
+                for (int j = tid; j < C * graph_edges; j += FITS_BLOCK) {
+                    const int c = fits_div(j, graph_edges, by_edges), e = j - c * graph_edges;
+                    const uint32_t ends = edges_lds[2 * e], n = ends >> 16, dst = ends & (FITS_MAX_NODES - 1);
+                    uint32_t type = edges_lds[2 * e + 1];
                     if (!((cur[2 * c + (n >> 5)] >> (n & 31)) & 1u)) continue;
-                    const uint32_t ne = ne_lds[n], at = ei_lds[n] - (uint32_t)first_edge;
-                    for (uint32_t e = 0; e < ne; ++e) {
-                        const uint32_t dst = edges_lds[2 * (at + e)];
-                        uint32_t type = edges_lds[2 * (at + e) + 1];
-                        if (type >= (uint32_t)(MW * 32)) type %= (uint32_t)(MW * 32);
-                        for (int b = 0; b < p.MB; ++b) {
-                            uint32_t h = hv[c * p.MB + b] + type;
-                            h -= h >= (uint32_t)(MW * 32) ? (uint32_t)(MW * 32) : 0u;
-                            atomicOr(&got[dst * MW + (h >> 5)], 1u << (h & 31));
-                        }
+                    if (type >= (uint32_t)(MW * 32)) type %= (uint32_t)(MW * 32);
+                    for (int b = 0; b < p.MB; ++b) {
+                        uint32_t h = hv[c * p.MB + b] + type;
+                        h -= h >= (uint32_t)(MW * 32) ? (uint32_t)(MW * 32) : 0u;
+                        atomicOr(&got[dst * MW + (h >> 5)], 1u << (h & 31));
                     }
                 }
                 lds_barrier();

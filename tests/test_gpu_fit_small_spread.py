@@ -86,3 +86,44 @@ def test_edges_that_do_not_lie_node_after_node(order, degree):
         at += k + gap
     moved.edge = np.ascontiguousarray(np.concatenate(edges))
     _trains_as_the_oracle(model, Device(model, moved), graphs, 2, 11)
+
+
+# out-degrees of every graph's nodes: edges shared out evenly among the threads whichever node they start from - one node with all of
+# them, at either end or in the middle, nodes without any between them, as many as are parked and one more, one node only
+DEGREES = [
+    dict(degrees=[40] + [0] * 63, clauses=10, bits=2),
+    dict(degrees=[0] * 30 + [17, 0, 0, 3] + [0] * 6, clauses=4, bits=4),
+    dict(degrees=[0] * 63 + [256], clauses=1, bits=4),
+    dict(degrees=[0] * 63 + [257], clauses=1, bits=2),
+    dict(degrees=[64, 64, 64, 64], clauses=2, bits=2),
+    dict(degrees=[1, 0] * 16, clauses=16, bits=4),
+    dict(degrees=[6], clauses=33, bits=1),
+    dict(degrees=[1] * 32 + [0] + [1] * 31, clauses=3, bits=3),
+]
+
+
+@pytest.mark.parametrize("shape", DEGREES, ids=lambda s: "%dx%d" % (len(s["degrees"]), sum(s["degrees"])))
+def test_edges_of_a_few_nodes_or_of_all(shape):
+    from graphtsetlinmachine_amd.graphs import Graphs
+    from tests.gpu_harness import Device
+
+    G, degrees, rng = 12, np.array(shape["degrees"]), np.random.default_rng(len(shape["degrees"]))
+    N = len(degrees)
+    np.random.seed(N)
+    g = Graphs(G, symbols=list(range(5)), hypervector_size=16, hypervector_bits=2)
+    g.number_of_graph_nodes[:] = N
+    g.prepare_node_configuration()
+    g.add_graph_nodes(np.tile(degrees, G).astype(np.uint32))
+    g.prepare_edge_configuration()
+    source = np.tile(np.repeat(np.arange(N), degrees), G)
+    graph, to, kind = np.repeat(np.arange(G), degrees.sum()), rng.integers(0, N, size=source.size), rng.integers(0, 3, size=source.size)
+    for t in range(3):
+        m = kind == t
+        g.add_graph_node_edges(graph[m], source[m], to[m], "type%d" % t)
+    for _ in range(2):
+        nodes = np.flatnonzero(rng.random(G * N) < 0.7)
+        g.add_graph_node_properties(nodes, rng.integers(0, 5, size=nodes.size))
+    g.encode()
+    cfg = helpers.oracle_config(g, classes=2, clauses=shape["clauses"], depth=3, T=15, message_size=96, message_bits=shape["bits"])
+    model = helpers.random_model(N, cfg, 3, s=2.0, include_density=0.01)
+    _trains_as_the_oracle(model, Device(model, g), g, 2, N)
