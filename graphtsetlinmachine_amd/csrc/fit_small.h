@@ -40,7 +40,9 @@ constexpr int FITS_BLOCK = 256;                    // threads that work
 constexpr int FITS_THREADS = FITS_BLOCK + 64;      // and the helper wave
 constexpr int FITS_MAX_NODES = 64;
 constexpr size_t FITS_MAX_LDS_BYTES = 128 * 1024;  // of the 160 KB a workgroup can have
-constexpr int FITS_X_AHEAD = 16;                   // literal words per helper lane fetched ahead; the rest is read at the step's end
+// Literal words per helper lane fetched ahead; the rest is read at the step's end, by the four waves that work: graphs of
+// 64 nodes of 64 words 14.0 us per example before there was a helper, 17.3 when it read the rest by itself, 9.2 now.
+constexpr int FITS_X_AHEAD = 16;
 constexpr int FITS_EDGES_LDS = FITS_BLOCK;         // edges of a graph parked in LDS (more: read in place)
 constexpr int FITS_DIRECT = 4;                     // (clause, edge, bit)s per thread up to which messages skip the nodes' vectors
 constexpr uint32_t FITS_IS_DIRECT = 1u << 16;      // in what is told of an example's nodes
@@ -389,7 +391,6 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
 #pragma unroll
             for (int r = 0; r < FITS_X_AHEAD; ++r)
                 if (64 * r < x_words && lane + 64 * r < x_words) to.x_rows[lane + 64 * r] = x_ahead[r];
-            for (int j = lane + 64 * FITS_X_AHEAD; j < x_words; j += 64) to.x_rows[j] = x_from[j];
             to.types[lane] = field_ahead[0], to.ne[lane] = field_ahead[1], to.ei[lane] = field_ahead[2];
             to.labels[lane] = label_ahead;
             if (lane < 2) to.header[lane] = header_ahead;
@@ -414,6 +415,7 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
         const Example e_now = example(i);
         const uint32_t *x_rows = e_now.x_rows, *types = e_now.types, *ne_lds = e_now.ne, *ei_lds = e_now.ei;
         const int32_t *y = (const int32_t *)e_now.labels;
+        const int x_words_next = __builtin_amdgcn_readfirstlane((int)e_now.header[0]) * LA;  // (of no use in the last example)
         const uint32_t *draw_node = draw_both + (i & 1) * draw_words, *draw_update = draw_node + C;
         int32_t *incl_of = incl_both + (i & 1) * C;
         const bool edges_parked = graph_edges <= FITS_EDGES_LDS;
@@ -629,7 +631,15 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
             if (p.inc_copy) inc_copy[j] = word.top();
         }
         // the next example's random numbers: the first 64 are the helper's
-        if (i + 1 < p.n_examples) draw(i + 1, 64 + FITS_BLOCK - 1 - tid, draws, FITS_BLOCK);
+        if (i + 1 < p.n_examples) {
+            draw(i + 1, 64 + FITS_BLOCK - 1 - tid, draws, FITS_BLOCK);
+            // ... and the literal words that the helper does not fetch ahead
+            if (x_words_next > 64 * FITS_X_AHEAD) {
+                const uint32_t *x_from = p.X + (int64_t)e_now.header[1] * LA;
+                uint32_t *to = example(i + 1).x_rows;
+                for (int j = tid + 64 * FITS_X_AHEAD; j < x_words_next; j += FITS_BLOCK) to[j] = x_from[j];
+            }
+        }
         lds_barrier();
     }
     }

@@ -127,3 +127,15 @@ def test_edges_of_a_few_nodes_or_of_all(shape):
     cfg = helpers.oracle_config(g, classes=2, clauses=shape["clauses"], depth=3, T=15, message_size=96, message_bits=shape["bits"])
     model = helpers.random_model(N, cfg, 3, s=2.0, include_density=0.01)
     _trains_as_the_oracle(model, Device(model, g), g, 2, N)
+
+
+@pytest.mark.parametrize("hv, nodes", [(256, 64), (272, 64), (520, 31), (1000, 64)], ids=["1024", "1088", "1023", "4032"])
+def test_graphs_of_more_literal_words_than_are_fetched_ahead(hv, nodes):
+    """At most 1,024 literal words of the next graph wait in registers; ragged sizes in turn, so that a graph with more follows
+    one with fewer and the other way round."""
+    from tests.gpu_harness import Device
+
+    graphs = helpers.random_graphs(hv, sizes=[nodes, 3, nodes, nodes - 1, 0, nodes, nodes], n_graphs=7, hv_size=hv, max_degree=2)
+    cfg = helpers.oracle_config(graphs, classes=2, clauses=3, depth=2, T=15, message_size=64)
+    model = helpers.random_model(hv, cfg, 2, s=2.0, include_density=0.005)
+    _trains_as_the_oracle(model, Device(model, graphs), graphs, 2, hv)
