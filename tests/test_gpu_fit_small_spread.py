@@ -139,3 +139,18 @@ def test_graphs_of_more_literal_words_than_are_fetched_ahead(hv, nodes):
     cfg = helpers.oracle_config(graphs, classes=2, clauses=3, depth=2, T=15, message_size=64)
     model = helpers.random_model(hv, cfg, 2, s=2.0, include_density=0.005)
     _trains_as_the_oracle(model, Device(model, graphs), graphs, 2, hv)
+
+
+# message words per half and lanes that share a pair: 4 and 1, 16 and 4, 64 and 16 (each lane's words come in fours: the form that
+# takes a half at a time), 4 and 2, 12 and 2, 3 and 1, 2 and 8 (the general form); every number of state bits has its own kernels
+@pytest.mark.parametrize("state_bits", [6, 8, 12, 20])
+@pytest.mark.parametrize("message_size, clauses, nodes", [
+    (128, 40, 12), (512, 12, 5), (2048, 1, 3), (128, 20, 5), (384, 12, 10), (96, 30, 14), (64, 5, 5),
+], ids=lambda v: str(v))
+def test_message_words_a_half_at_a_time_and_one_by_one(message_size, clauses, nodes, state_bits):
+    from tests.gpu_harness import Device
+
+    graphs = helpers.random_graphs(message_size, n_graphs=10, max_nodes=nodes, min_nodes=max(1, nodes - 2), hv_size=16, edge_types=("a", "b"))
+    cfg = helpers.oracle_config(graphs, classes=2, clauses=clauses, depth=3, T=15, message_size=message_size, state_bits=state_bits)
+    model = helpers.random_model(message_size + clauses, cfg, 3, s=2.0, include_density=0.02, message_density=0.5 / message_size)
+    _trains_as_the_oracle(model, Device(model, graphs), graphs, 2, clauses)
