@@ -326,26 +326,9 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
                     if (64 * r < graph_edges && lane + 64 * r < graph_edges) edge_ahead[r] = from[lane + 64 * r];
             }
         };
-        // ... and, where messages go straight along them, the node that each starts from (the last one whose first edge is
-        // not behind it), in the upper half of the word with the far end
-        uint32_t source_ahead[FITS_EDGES_LDS / 64];
-        auto find_sources = [&](const Example &e, int nodes) {
-#pragma unroll
-            for (int r = 0; r < FITS_EDGES_LDS / 64; ++r) {
-                source_ahead[r] = 0u;
-                if (!direct || 64 * r >= graph_edges) continue;
-                uint32_t from = 0u;
-                for (int step = nodes > 1 ? 1 << (31 - __clz(nodes - 1)) : 0; step > 0; step >>= 1) {
-                    const uint32_t n = from + (uint32_t)step;
-                    if (n < (uint32_t)nodes && e.ei[n] - first_edge <= (uint32_t)(lane + 64 * r)) from = n;
-                }
-                source_ahead[r] = from << 16;
-            }
-        };
         {
             const Example e = example(0);
             request_edges(n_nodes, lane < n_nodes ? e.ne[lane] : 0u, lane < n_nodes ? e.ei[lane] : 0u);
-            find_sources(e, n_nodes);
             if (lane == 0) tell(0, n_nodes, graph_edges, direct, first_edge);
         }
         lds_barrier();
@@ -360,8 +343,17 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
 #pragma unroll
                 for (int r = 0; r < FITS_EDGES_LDS / 64; ++r) {
                     const int j = lane + 64 * r;
-                    if (64 * r < graph_edges && j < graph_edges)
-                        edges_lds[2 * j] = edge_ahead[r].x | source_ahead[r], edges_lds[2 * j + 1] = edge_ahead[r].y;
+                    if (64 * r < graph_edges && j < graph_edges) {
+                        // where messages go straight along the edges, the node that each starts from - the last one whose
+                        // first edge is not behind it - in the upper half of the word with the far end
+                        uint32_t source = 0u;
+                        if (direct_now)
+                            for (int ahead = n_nodes > 1 ? 1 << (31 - __clz(n_nodes - 1)) : 0; ahead > 0; ahead >>= 1) {
+                                const uint32_t n = source + (uint32_t)ahead;
+                                if (n < (uint32_t)n_nodes && e.ei[n] - first_edge <= (uint32_t)j) source = n;
+                            }
+                        edges_lds[2 * j] = edge_ahead[r].x | (source << 16), edges_lds[2 * j + 1] = edge_ahead[r].y;
+                    }
                 }
             }
             // what lands at the step's end: example i + 1 (its node count and offset came with example i), the header of i + 2
@@ -411,7 +403,6 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
             to.types[lane] = field_ahead[0], to.ne[lane] = field_ahead[1], to.ei[lane] = field_ahead[2];
             to.labels[lane] = label_ahead;
             if (lane < 2) to.header[lane] = header_ahead;
-            find_sources(to, n_next);
             if (lane == 0) tell(i + 1, n_next, graph_edges, direct, first_edge);
             n_nodes = n_next;
             lds_barrier();
