@@ -105,7 +105,9 @@ class _DeviceGraphs:
         self.tiles = self.moves = None
         self._moves_known = False
         self._tiles_key = None
-        self._made = None  # event after what made the arrays and the tiles
+        # whether what made the arrays and the tiles is known to be done: True after a wait for the stream, an event
+        # after a call that did not wait, None before either
+        self._made = None
 
     def buffers(self):
         """Every tensor that the device reads this data set from."""
@@ -122,16 +124,13 @@ class _DeviceGraphs:
             return
         _refuse_capture("a data set without the tiles of this model's sizes")
         self._tiles_key = key
-        try:
-            self._build_tiles(cfg)
-        finally:
-            self._made = torch.cuda.Event()
-            self._made.record()
+        self._made = None
+        self._build_tiles(cfg)
 
     def require_made(self):
         """For a call that is captured on another stream than the one that made the arrays and the tiles: a stream under
         capture cannot wait for that one, so it has to be done."""
-        if self._made is None or not self._made.query():
+        if self._made is None or not (self._made is True or self._made.query()):
             raise _abi.GtmError("the data set is still on its way to the device: synchronize before capturing on another stream")
 
     def _build_tiles(self, cfg):
@@ -490,6 +489,7 @@ class CommonTsetlinMachine:
             )
             self.step += count
         torch.cuda.current_stream().synchronize()
+        dg._made = True
         self.ta_state = np.array([])
         self.clause_weights = np.array([])
 
@@ -510,12 +510,22 @@ class CommonTsetlinMachine:
     def _score(self, graphs, batch=None):
         """tm.py:786-812 as one gtm_score call."""
         n = int(graphs.number_of_graphs)
-        return self.score_device(graphs, batch).cpu().numpy().reshape(n, self.number_of_outputs)
+        dg, out = self._enqueue_score(graphs, batch)
+        out = out.cpu().numpy().reshape(n, self.number_of_outputs)
+        dg._made = True
+        return out
 
     def score_device(self, graphs, batch=None):
         """Class sums as a flat int32 device tensor [graphs * outputs]; work is
         only enqueued on the current stream.  (The first call on a data set may
         wait for the stream once: what it finds decides which kernels follow.)"""
+        dg, out = self._enqueue_score(graphs, batch)
+        if dg._made is None:
+            dg._made = torch.cuda.Event()
+            dg._made.record()
+        return out
+
+    def _enqueue_score(self, graphs, batch):
         captured_elsewhere = self._take_stream()
         dg = self._score_init(graphs)
         cfg = self._config(max(dg.max_nodes, 1))
@@ -537,7 +547,7 @@ class CommonTsetlinMachine:
             "gtm_score", ctypes.byref(cfg), ctypes.byref(dg.desc), ctypes.byref(self._state), 0, n, batch,
             _ptr(ws), ws.numel(), _ptr(out), _stream(),
         )
-        return out
+        return dg, out
 
     def _transform(self, graphs, nodewise, batch=None):
         """tm.py:814-900 as one gtm_transform call."""
@@ -563,6 +573,7 @@ class CommonTsetlinMachine:
             _ptr(ws), ws.numel(), _ptr(flat), _ptr(wide) if nodewise else None, width, _ptr(sums), _stream(),
         )
         out = wide.cpu().numpy().reshape(n, C, width) if nodewise else flat.cpu().numpy().reshape(n, C)
+        dg._made = True
         return out, sums.cpu().numpy().reshape(n, self.number_of_outputs)
 
     def transform(self, graphs):
