@@ -10,9 +10,9 @@
 //   layer 0  K1: a few lanes per (clause, node): (include & ~X[node]) == 0 and the
 //            node-type gate (kernels.py:443-466)
 //   per message layer
-//     send   K3-K5: the hypervector bits of the true clauses, rotated, straight to the far ends
-//            of their nodes' edges; with many edges in two phases, per-node bit vectors
-//            (kernels.py:565-588) and the vectors rotated along the edges
+//     send   K3-K5: a thread per (clause, edge), the hypervector bits of a clause true where the
+//            edge starts, rotated, straight to its far end; with many edges in two phases,
+//            per-node bit vectors (kernels.py:565-588) and the vectors rotated along the edges
 //     K2     a few lanes per (clause, node) against the message bank's include
 //            words; the negated message literals are the complement of the
 //            received vector (kernels.py:505-527)
@@ -26,11 +26,12 @@
 // A fifth wave helps, in a loop of its own with the same barriers: it fetches the next example (literal
 // words, node types, edge counts and offsets, labels; the node count and offset of the one after) and, as soon as
 // the offsets are there, its edges - memory latency that nobody waits for -, clears what the phases add to, and
-// draws the random numbers of K7 and K8 while the others pick and decide.  The barriers order LDS traffic only.
+// draws the first 64 random numbers of K7 and K8 while the others pick and decide (where LDS has no room for two
+// examples' draws, after that); the four draw the rest after their feedback.  The barriers order LDS traffic only.
 //
 // Measured on pairs of nodes (10 clauses, 2 + 16 include words each, 2 classes), per example: 5.5 us with one thread
 // per pair, run-time divisions and every wave doing all of this; 4.9 with the helper wave, divisions as
-// multiplications, the planes of an automaton word known to the compiler and one pass that counts up and down; 3.5
+// multiplications, the planes of an automaton word known to the compiler and one pass that counts up and down; 3.6
 // with the edges requested a step ahead, the draws where the helper idles, and votes and decisions by the same
 // threads on values requested together (by clock64, cycles before that: layer 0 3,500 - the edges' latency -, send
 // 1,440, K2 1,620, pick to decisions 3,900, feedback 2,600).
@@ -41,10 +42,12 @@ constexpr int FITS_THREADS = FITS_BLOCK + 64;      // and the helper wave
 constexpr int FITS_MAX_NODES = 64;
 constexpr size_t FITS_MAX_LDS_BYTES = 128 * 1024;  // of the 160 KB a workgroup can have
 // Literal words per helper lane fetched ahead; the rest is read at the step's end, by the four waves that work: graphs of
-// 64 nodes of 64 words 14.0 us per example before there was a helper, 17.3 when it read the rest by itself, 9.2 now.
+// 64 nodes of 64 words 14.0 us per example before there was a helper, 17.3 when it read the rest by itself, 9.5 now.
 constexpr int FITS_X_AHEAD = 16;
 constexpr int FITS_EDGES_LDS = FITS_BLOCK;         // edges of a graph parked in LDS (more: read in place)
-constexpr int FITS_DIRECT = 4;                     // (clause, edge, bit)s per thread up to which messages skip the nodes' vectors
+// (clause, edge, bit)s per thread up to which messages skip the nodes' vectors.  Chains, us per example, straight | through the
+// vectors: 280 in all 5.3 | 6.3, 600 5.7 | 6.1, 1,240 6.7 | 6.7, 2,500 8.0 to 8.2 | 8.0.
+constexpr int FITS_DIRECT = 4;
 constexpr uint32_t FITS_IS_DIRECT = 1u << 16;      // in what is told of an example's nodes
 constexpr int FITS_Y_LDS = 64;                     // classes whose labels are fetched ahead (K <= this, else read in place)
 
@@ -64,7 +67,7 @@ struct FitSmallParams {
     int depth, C, LA, MC, MW, MB, B, K, T, negative, boost, max_included;
     uint32_t k0, k1;
     uint64_t q_thr;
-    // how the work is spread (fit_small_spread)
+    // how the work is spread (fit_small_lanes)
     int lanes0, lanes1;         // log2 of the lanes that share a (clause, node): layer 0, message layers
     int inc_copy;               // the include planes have a copy of their own in LDS
     int draws_twice;            // the random draws of two examples have room in LDS: the next one's need not wait
@@ -220,7 +223,8 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
     int32_t *upd = incl_both + 2 * C;              // [C][K]
     const int draw_words = p.draws_twice ? C + 2 * C * K : 0;  // (from an example's to the next one's)
     uint32_t *draw_both = (uint32_t *)(upd + C * K);  // [C] node picks, [C][K][2] decisions
-    uint32_t *info_both = draw_both + C + 2 * C * K + draw_words;  // twice: an example's nodes, edges, first edge (or the edges' magic), magic of its nodes
+    // twice: an example's nodes and FITS_IS_DIRECT, edges, first edge (of direct ones the edges' magic), magic of its nodes
+    uint32_t *info_both = draw_both + C + 2 * C * K + draw_words;
     uint32_t *magic_of = info_both + 8;            // [FITS_EDGES_LDS + 1]
     // the include planes, every bank's words in order: a copy, so that lanes read neighbouring words, or in place
     uint32_t *inc_copy = magic_of + FITS_EDGES_LDS + 1;

@@ -213,7 +213,7 @@ int gtm_build_tiles(const gtm_config *cfg, const gtm_graphs *graphs, uint32_t *t
  * message layers: finds out whether the edges of the data set are a few moves (node n -> n + d with type t, as in
  * chains and grids) and fills a caller-owned buffer of gtm_moves_bytes() with what the message kernels then use
  * instead of walking the edges.  The buffer must stay as long as the tiles do, and the edges must not change.
- * Waits for the stream once.  gtm_moves_bytes() is 0 where there is nothing to find. */
+ * Waits for the stream once; on a stream under capture it looks at nothing.  gtm_moves_bytes() is 0 where there is nothing to find. */
 size_t gtm_moves_bytes(const gtm_config *cfg, const gtm_graphs *graphs);
 int gtm_build_moves(const gtm_config *cfg, const gtm_graphs *graphs, uint32_t *moves, void *stream);
 
