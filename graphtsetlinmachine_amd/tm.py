@@ -527,7 +527,7 @@ class CommonTsetlinMachine:
         return out
 
     def _enqueue_score(self, graphs, batch):
-        captured_elsewhere = self._take_stream()
+        captured_elsewhere = self.initialized and self._take_stream()
         dg = self._score_init(graphs)
         cfg = self._config(max(dg.max_nodes, 1))
         n = dg.number_of_graphs
@@ -552,7 +552,8 @@ class CommonTsetlinMachine:
 
     def _transform(self, graphs, nodewise, batch=None):
         """tm.py:814-900 as one gtm_transform call."""
-        self._take_stream()
+        if self.initialized:
+            self._take_stream()
         dg = self._score_init(graphs)
         cfg = self._config(max(dg.max_nodes, 1))
         n, C = dg.number_of_graphs, self.number_of_clauses

@@ -323,3 +323,16 @@ def test_calls_on_different_streams_wait_for_one_another(monkeypatch):
     at[0], capturing[0] = Stream(11), False
     tm._take_stream()
     assert log[0] == (11, "waits for", 22)
+
+
+@pytest.mark.parametrize("call", ["score", "predict", "transform", "transform_nodewise", "score_device"])
+def test_a_model_that_was_never_trained_ends_the_program_with_or_without_a_device(call, monkeypatch):
+    """tm.py:755-757: before anything asks for a device."""
+    def no_device():
+        raise AssertionError("a device was asked for")
+
+    monkeypatch.setattr(tm_module, "_device", no_device)
+    tm = MultiClassGraphTsetlinMachine(4, 10, 1.0, seed=1)
+    graphs = Graphs(1, symbols=["a"], hypervector_size=8, hypervector_bits=1)
+    with pytest.raises(SystemExit):
+        getattr(tm, call)(graphs)
