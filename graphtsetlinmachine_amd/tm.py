@@ -521,7 +521,7 @@ class CommonTsetlinMachine:
         only enqueued on the current stream.  (The first call on a data set may
         wait for the stream once: what it finds decides which kernels follow.)"""
         dg, out = self._enqueue_score(graphs, batch)
-        if dg._made is None:
+        if dg._made is None and not torch.cuda.is_current_stream_capturing():
             dg._made = torch.cuda.Event()
             dg._made.record()
         return out

@@ -104,3 +104,27 @@ def test_a_data_set_that_is_not_on_the_device_is_refused_under_capture():
         with pytest.raises(_abi.GtmError, match="on its way"):
             tm.score_device(new)
     assert np.array_equal(tm.score(new), want_new)
+
+
+def test_what_is_recorded_in_a_graph_does_not_stand_for_the_upload():
+    """An event recorded under capture tells nothing about the upload, and cannot be asked."""
+    import torch
+
+    tm, sets, want = _model_and_sets()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        tm.score(sets[1])
+        tm._test_graphs._made = None  # as after a call that failed between the tiles and its end
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        graph.capture_begin()
+        out = tm.score_device(sets[1])
+        graph.capture_end()
+    assert tm._test_graphs._made is None
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy().reshape(want[1].shape), want[1])
+        assert np.array_equal(tm.score(sets[0]), want[0])
