@@ -156,13 +156,20 @@ class _DeviceGraphs:
     def ensure_moves(self, cfg):
         """Are the edges a few moves, as in chains and grids?  Looked at once per layout of tiles, by the first call that
         has a use for the answer: training has none.  (The buffer lives as long as the tiles.)"""
-        if self._moves_known or self.tiles is None or torch.cuda.is_current_stream_capturing():
+        if self._moves_known or self.tiles is None:
             return
+        if self.desc.total_edges >= MOVES_FROM_EDGES:
+            if torch.cuda.is_current_stream_capturing():
+                return  # (the look waits for the stream; a later call makes it)
+            self._moves_known = True
+            nbytes = _abi.lib.gtm_moves_bytes(ctypes.byref(cfg), ctypes.byref(self.desc))
+            if nbytes:
+                try:
+                    self.moves = torch.empty(nbytes // 4, dtype=torch.int32, device=_device())
+                except torch.OutOfMemoryError:
+                    return  # (the edges are walked)
+                _abi.call("gtm_build_moves", ctypes.byref(cfg), ctypes.byref(self.desc), _ptr(self.moves), _stream())
         self._moves_known = True
-        nbytes = _abi.lib.gtm_moves_bytes(ctypes.byref(cfg), ctypes.byref(self.desc)) if self.desc.total_edges >= MOVES_FROM_EDGES else 0
-        if nbytes:
-            self.moves = torch.empty(nbytes // 4, dtype=torch.int32, device=_device())
-            _abi.call("gtm_build_moves", ctypes.byref(cfg), ctypes.byref(self.desc), _ptr(self.moves), _stream())
 
 
 class ModelState(tuple):

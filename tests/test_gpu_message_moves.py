@@ -130,3 +130,27 @@ def test_moves_are_looked_for_by_the_first_call_that_uses_them():
     assert dg.moves is not None and np.array_equal(sums, want)
     words = dg.moves[:9].cpu().numpy()  # the (type, offset) keys found, then whether there were too many
     assert sorted(int(v) for v in words[:4]) == sorted((t << 16) | (32768 + d) for t, d in GRID) and not words[4:].any()
+
+
+def test_without_room_for_the_moves_the_edges_are_walked(monkeypatch):
+    import torch
+
+    from graphtsetlinmachine_amd.tm import MultiClassGraphTsetlinMachine
+
+    name, sizes, moves, sizing, _ = SHAPES[5]
+    graphs = _graphs(np.array(sizes * 3), moves, seed=3)
+    tm = MultiClassGraphTsetlinMachine(60, 50, 2.0, depth=3, seed=5, **sizing)
+    tm.fit(graphs, np.arange(len(sizes) * 3) % 3, epochs=1)
+    want, dg, empty = tm.score(graphs), tm._train_graphs, torch.empty
+    assert dg.moves is not None
+    words = dg.moves.numel()
+    dg._tiles_key = None
+
+    def refuse(*size, **kwargs):
+        if size == (words,):
+            raise torch.OutOfMemoryError("no room")
+        return empty(*size, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", refuse)
+    assert np.array_equal(tm.score(graphs), want) and dg.moves is None
+    assert np.array_equal(tm.score(graphs), want)
