@@ -3,14 +3,19 @@
 //
 // Each workgroup owns a contiguous range of clauses for the whole run and keeps
 // their automata (all bit planes) and weights in LDS; they go back to global
-// memory once, at the end.  Per example a workgroup
+// memory once, at the end.  (Small clauses: fit_waves.h.)  Per example a workgroup
 //   1. evaluates its clauses on the graph's literal-major rows (staged in LDS;
-//      the next graph's rows, literal words and labels are loaded straight into
-//      the other LDS buffers while waiting at the barrier), picks the nodes, and
-//      adds its clauses' votes to the class sums in global memory;
+//      the next graph's rows and labels are loaded straight into the other LDS
+//      buffers while waiting at the barrier) by the clauses' lists of rows
+//      (fit_lists.h), picks the nodes, and adds its clauses' votes to the class
+//      sums in global memory;
 //   2. meets the other workgroups at a device-wide barrier (the class sums are
 //      the only thing that crosses clause boundaries, kernels.py:310-315);
-//   3. decides the feedback and updates its automata and weights in LDS.
+//   3. decides the feedback and updates its automata and weights in LDS: the
+//      (clause, class) pairs that need Type I bits and the clauses that get any
+//      feedback are listed, so that every thread has a byte to draw or a word to update.
+// Single-node images of 128 literal words, 2,500 clauses: 9.4 us per example before the lists, with every
+// (clause, word) looking at all its classes and a word's four generator calls in one thread; now 6.0.
 // Class sums and barrier are one thing: class k has a 64-bit word (kept as
 // FITP_SUM_PARTS partial words that a reader adds up, since the memory system
 // carries out the adds to one word one after the other) to which every
@@ -79,36 +84,12 @@ struct FitPersistParams {
     int clauses_per_group;
     int rows_words;       // LDS words of one staged graph: (literals + n_types + 1) * max slot words
     int max_words;        // words per graph slot that can hold nodes
-    const uint32_t *order;  // literals sorted by how often they hold in the data set, rarest first
-    int x_words;          // LDS words of one graph's node-major literal words: max nodes * LA
+    int x_words;          // LDS words of one graph's node-major literal words: max nodes * LA (DIRECT, else 0)
     const uint32_t *node_type;  // [total nodes]
-    int direct;           // graphs of at most FITP_DIRECT_NODES nodes: every node is tested on its own literal words, no rows are staged
+    int lanes_log;        // log2 of the lanes that a row takes (fit_lists.h)
+    int lists;            // entries of a clause's list of rows
+    int ahead;            // the picked nodes' literal words have a place in LDS
 };
-
-__device__ __forceinline__ void fitp_stage_rows(const FitPersistParams &p, const FitGraph &fg, uint32_t *dst, int tid) {
-    const uint32_t *tile = p.tiles + (int64_t)fg.tile * p.tg.rows * p.tg.tw + fg.word0;
-    const int words = fg.words;
-    const int total = (p.literals + p.n_types + 1) * words;
-    // element i = r * words + w; a thread visits i = tid, tid + FITP_BLOCK, ...: (r, w) advance without dividing
-    const int dr = FITP_BLOCK / words, dw = FITP_BLOCK - dr * words;
-    int r = tid / words, w = tid - r * words;
-    for (int base = tid; base < total; base += FITP_BLOCK * 8) {
-        uint32_t v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            v[u] = base + u * FITP_BLOCK < total ? tile[(int64_t)r * p.tg.tw + w] : 0u;
-            r += dr;
-            w += dw;
-            if (w >= words) {
-                w -= words;
-                ++r;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (base + u * FITP_BLOCK < total) dst[base + u * FITP_BLOCK] = v[u];
-    }
-}
 
 constexpr unsigned long long FITP_HALF = 1ull << 47;      // class sums are smaller than this in magnitude
 constexpr unsigned long long FITP_ARRIVED = 1ull << 48;   // one arrival in bits 48..63
@@ -117,10 +98,7 @@ constexpr int FITP_SUM_STRIDE = 16;                      // 64-bit words between
 // reader adds the parts up (the protocol is linear in the word). Adds to one word are carried out
 // one after the other by the memory system, so fewer groups per word shorten the exchange.
 constexpr int FITP_SUM_PARTS = 16;
-constexpr int FITP_WALK_ALL = 24;   // clauses with at most this many literals AND all their rows
-constexpr int FITP_FILTER_ROWS = 16;  // rows the others AND before testing the surviving nodes
 constexpr int FITP_DIRECT_NODES = 2;  // data sets whose graphs have at most this many nodes skip the literal rows altogether
-constexpr int FITP_FEW_NODES = 2;     // up to this many surviving nodes are tested one by one, more are filtered further
 
 // One 32-bit word per lane from global memory straight into LDS (no register holds it meanwhile):
 // lane l's word lands at dst_of_wave[l]; dst_of_wave must be the same for the whole wave. The words
@@ -138,41 +116,83 @@ __device__ __forceinline__ void fitp_wave_lds_sync() {
 }
 constexpr int FITP_WAIT_VMEM = 0x0F70;  // s_waitcnt vmcnt(0) (export and LDS counters left alone)
 
-// MAXB: bit planes of an automaton the kernel keeps in registers while updating a word (>= B).
-template <int MAXB>
+
+// The rows of a graph's slot -> LDS, fitl_stride(words) words apart, straight from memory (no register holds them meanwhile; they are
+// there once the wave has waited for its vector-memory counter and, for other waves, after the barrier that follows).
+// Threads tid < loaders (a multiple of 64) take part.
+struct FitRowLoader {
+    int stride, dr, dw, r0, w0;  // a thread's elements are `loaders` apart: (row, word) advance without dividing
+    __device__ __forceinline__ void prepare(int words, int loaders, int tid) {
+        stride = fitl_stride(words);
+        dr = loaders / stride, dw = loaders - dr * stride;
+        r0 = tid / stride, w0 = tid - r0 * stride;
+    }
+    __device__ __forceinline__ void request(const uint32_t *tile, int tw, int rows, int words, uint32_t *dst_of_wave, int loaders, int tid) const {
+        if (tid >= loaders) return;
+        const int total = rows * stride;
+        int w = w0, row = r0 * tw;
+        for (int at = 0; at < total; at += loaders) {
+            if (at + tid < total) fitp_load_to_lds(tile + (row + (w < words ? w : 0)), dst_of_wave + at);
+            w += dw, row += dr * tw;
+            if (w >= stride) w -= stride, row += tw;
+        }
+    }
+};
+
+// LDS words of the kernel: `lists` = room for the clauses' lists of rows (entries per clause, a whole number of batches, 0 without),
+// `ahead` = room for the literal words of the nodes that the clauses learn from.
+inline size_t fit_persistent_lds_words(int per_group, int LA, int B, int K, int rows_words, int x_words, int lists, bool ahead) {
+    const size_t own = (size_t)per_group, KW = (size_t)(K + 31) / 32;
+    return (own * LA * B + 7) / 8 * 8 + (own * lists / 2 + 3) / 4 * 4 + 2 * (size_t)rows_words + own * K + 5 * own + 2 * (size_t)K + 2 * own * K +
+           own * LA * K + own * K + 2 * own * KW + 2 * (size_t)x_words + (ahead ? own * LA : 0) + 8 * (size_t)K;
+}
+
+// MAXB: bit planes of an automaton the kernel keeps in registers while updating a word (>= B; EXACT: B itself).
+// DIRECT: graphs of at most FITP_DIRECT_NODES nodes: every node is tested on its own literal words, no rows are staged.
+template <int MAXB, bool EXACT, bool DIRECT>
 __global__ __launch_bounds__(FITP_BLOCK) void k_fit_persistent(FitPersistParams p) {
-    extern __shared__ uint32_t lds[];
+    extern __shared__ __align__(16) uint32_t lds[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int WAVES = FITP_BLOCK / 64;
     const int c0 = blockIdx.x * p.clauses_per_group;
     const int n_own = min(p.clauses_per_group, p.C - c0);
-    const int LA = p.LA, B = p.B, K = p.K;
+    const int LA = p.LA, B = EXACT ? MAXB : p.B, K = p.K, KW = (K + 31) / 32;
     const int own_max = p.clauses_per_group;
 
     // LDS carve-up
-    uint32_t *rows_buf[2] = {lds, lds + p.rows_words};
-    uint32_t *ta = lds + 2 * p.rows_words;                     // [own][LA][B]
-    int32_t *wts = (int32_t *)(ta + (size_t)own_max * LA * B);  // [own][K]
-    int32_t *upd = wts + (size_t)own_max * K;                  // [own][K]
-    int32_t *node_of = upd + (size_t)own_max * K;              // [own]
-    int32_t *incl_of = node_of + own_max;                      // [own]
-    int32_t *sums = incl_of + own_max;                         // [K] class sums of the example
+    uint32_t *ta = lds;                                               // [own][LA][B]
+    uint16_t *lists = (uint16_t *)(ta + ((size_t)own_max * LA * B + 7) / 8 * 8);  // [own][p.lists] rows that a clause ANDs
+    // (buffers of this and the next example: addressed from the first one, a choice between two pointers would make the
+    // reads flat ones)
+    uint32_t *rows_both = (uint32_t *)lists + ((size_t)own_max * p.lists / 2 + 3) / 4 * 4;  // [2][p.rows_words] literal-major rows
+    int32_t *wts = (int32_t *)(rows_both + 2 * p.rows_words);  // [own][K]
+    int32_t *node_of = wts + (size_t)own_max * K;              // [own]
+    int32_t *incl_of = node_of + own_max;                      // [own] included literals
+    uint32_t *stale = (uint32_t *)(incl_of + own_max);         // [own] bit 0: the include plane has changed since list and count were made; bit 1: on the busy list
+    uint32_t *pick_of = stale + own_max;                       // [own] random word of the node pick, drawn a step ahead
+    int32_t *busy_list = (int32_t *)(pick_of + own_max);       // [own] clauses with feedback
+    int32_t *sums = busy_list + own_max;                       // [K] class sums of the example
     int32_t *votes = sums + K;                                 // [K] this group's share of the class sums
     uint32_t *gate = (uint32_t *)(votes + K);                  // [own][K][2] random words of the feedback gates
     uint32_t *fbits = gate + 2 * (size_t)own_max * K;          // [own][LA][K] Type I feedback bits
     int32_t *pair_list = (int32_t *)(fbits + (size_t)own_max * LA * K);  // [own * K] (clause, class) pairs with Type I feedback
-    uint32_t *x_buf[2] = {(uint32_t *)(pair_list + (size_t)own_max * K),
-                          (uint32_t *)(pair_list + (size_t)own_max * K) + p.x_words};  // [nodes][LA] of the graph
-    uint32_t *order_lds = x_buf[1] + p.x_words;                 // [literals]
+    uint32_t *pos_of = (uint32_t *)(pair_list + (size_t)own_max * K);    // [own][KW] classes with Type I feedback
+    uint32_t *neg_of = pos_of + (size_t)own_max * KW;                    // [own][KW] classes with Type II feedback
+    uint32_t *x_both = neg_of + (size_t)own_max * KW;          // DIRECT: [2][nodes][LA] literal words of the graph
+    uint32_t *x_ahead = x_both + 2 * p.x_words;                // [own][LA] literal words of the picked nodes (p.ahead)
     // thread k < K: its class-sum word as it stood when each of the three
     // slots was last complete (all zero before the first use): [slot][low, high][K]
-    uint32_t *seen = order_lds + p.literals;
-    uint32_t *y_buf[2] = {seen + 6 * K, seen + 7 * K};        // [K] labels of this and the next example
-    __shared__ int go_on, n_pairs;
+    uint32_t *seen = x_ahead + (p.ahead ? (size_t)own_max * LA : 0);
+    uint32_t *y_both = seen + 6 * K;                          // [2][K] labels
+    __shared__ int go_on, n_pairs, n_busy;
     __shared__ uint32_t after_lds[2];
     __shared__ uint32_t types_lds[2][FITP_DIRECT_NODES];  // node types of this and the next graph (direct evaluation)
+
+    auto draw_pick = [&](int cl, uint32_t step) {
+        return philox4x32_10((uint32_t)(c0 + cl), 0u, step, GTM_TAG_CLAUSE_NODE, p.k0, p.k1).v[0];
+    };
 
     // own state -> LDS
     for (int k = tid; k < K; k += FITP_BLOCK) votes[k] = 0;
@@ -181,226 +201,111 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_persistent(FitPersistParams 
         int cl = i / K, k = i - cl * K;
         wts[i] = p.weights[(int64_t)k * p.C + c0 + cl];
     }
+    for (int cl = tid; cl < n_own; cl += FITP_BLOCK) stale[cl] = 1u, pick_of[cl] = draw_pick(cl, p.first_step);
     const int last = p.first_example + p.n_examples - 1;
     int n_now = 0, n_next = 0;          // node counts of example i and i + 1
     uint32_t base_now = 0, base_next = 0;  // node_index of example i and i + 1
+    FitGraph fg{};                      // the slot of example i
     if (p.n_examples > 0) {
         n_now = (int)p.n_nodes[p.first_example];
         base_now = p.node_index[p.first_example];
         const int e1 = min(p.first_example + 1, last);
         n_next = (int)p.n_nodes[e1];
         base_next = p.node_index[e1];
-        FitGraph fg0 = fit_graph_slot(p.tg, p.first_example, n_now);
-        if (!p.direct) fitp_stage_rows(p, fg0, rows_buf[0], tid);
-        for (int at = tid; at < n_now * LA; at += FITP_BLOCK) x_buf[0][at] = p.X[(int64_t)base_now * LA + at];
-        if (p.direct && tid < n_now) types_lds[0][tid] = p.node_type[base_now + tid];
-        for (int k = tid; k < K; k += FITP_BLOCK) y_buf[0][k] = (uint32_t)p.encoded_Y[(int64_t)p.first_example * K + k];
+        fg = fit_graph_slot(p.tg, p.first_example, n_now);
+        if (!DIRECT) {
+            FitRowLoader all;
+            all.prepare(fg.words, FITP_BLOCK, tid);
+            all.request(p.tiles + (int64_t)fg.tile * p.tg.rows * p.tg.tw + fg.word0, p.tg.tw, p.literals + p.n_types + 1, fg.words,
+                        rows_both + wave * 64, FITP_BLOCK, tid);
+            __builtin_amdgcn_s_waitcnt(FITP_WAIT_VMEM);
+        }
+        if (DIRECT) {
+            for (int at = tid; at < n_now * LA; at += FITP_BLOCK) x_both[at] = p.X[(int64_t)base_now * LA + at];
+            if (tid < n_now) types_lds[0][tid] = p.node_type[base_now + tid];
+        }
+        for (int k = tid; k < K; k += FITP_BLOCK) y_both[k] = (uint32_t)p.encoded_Y[(int64_t)p.first_example * K + k];
     }
-    for (int l = tid; l < p.literals; l += FITP_BLOCK) order_lds[l] = p.order[l];
     for (int j = tid; j < 6 * K; j += FITP_BLOCK) seen[j] = 0u;
     lds_barrier();
 
     const int ones_row = p.literals + p.n_types;
-    // one small clause per wave: the feedback of a step runs inside the clause's wave
-    const bool wave_local = own_max <= WAVES && K * LA <= 256;
-    int div_words = 0, div_dr = 0, div_r0 = 0;
+    int quarter_log = 2, word_log = 0;  // 2^quarter_log >= 4 LA lanes draw a clause's Type I bytes for one class, 2^word_log >= LA update its words
+    while ((1 << word_log) < LA && word_log < 10) ++word_log;
+    while ((1 << quarter_log) < 4 * LA && quarter_log < 10) ++quarter_log;
+    FitRowLoader loader{};
+    int loader_words = 0;
     // The threads that add the group's votes to the device-wide class sums and then poll for them are the first K
     // of the LAST wave when K <= 64; that wave requests none of the next graph's words and draws no random
     // numbers, so its polling starts at once and runs beside the other waves' work instead of after its own share.
     const bool poll_apart = K <= 64;
     const int poll0 = poll_apart ? (WAVES - 1) * 64 : 0;         // the first polling thread
     const int loaders = poll_apart ? poll0 : FITP_BLOCK;        // threads 0 .. loaders - 1 request the next graph's words
+    const int place = lane & ((1 << p.lanes_log) - 1);
+    const bool one_type = p.n_types == 1;
+    int slot = 0;  // i modulo 3
     for (int i = 0; i < p.n_examples; ++i) {
-        const int ex = p.first_example + i;
         const uint32_t step = p.first_step + (uint32_t)i;
-        const FitGraph fg = fit_graph_slot(p.tg, ex, n_now);
-        const uint32_t *rows = rows_buf[i & 1];
-        unsigned long long *slot_now = p.class_sum + (size_t)(i % 3) * K * FITP_SUM_PARTS * FITP_SUM_STRIDE;
-
-        // ---- 0. the next graph's slot; the sizes of the graph after it are requested
-        const bool has_next = i + 1 < p.n_examples;
-        const FitGraph fn = fit_graph_slot(p.tg, has_next ? ex + 1 : ex, has_next ? n_next : n_now);
-        const int next_total = has_next && !p.direct ? (p.literals + p.n_types + 1) * fn.words : 0;
-        const uint32_t *x_now = x_buf[i & 1];
-        // node count and first node of the graph after the next, fetched by two threads with vector
-        // loads (scalar loads share their counter with LDS: the evaluation's first LDS read would wait
-        // for them) and handed over through LDS at the end of the step
-        const int e2 = min(ex + 2, last);
-        uint32_t after = 0u;
-        if (tid < 2) after = (tid == 0 ? p.n_nodes : p.node_index)[e2];
-        uint32_t type_ahead = 0u;
-        if (p.direct && has_next && tid < n_next) type_ahead = p.node_type[base_next + tid];
+        const uint32_t *rows = rows_both + (i & 1) * p.rows_words;
+        const uint32_t *x_now = x_both + (i & 1) * p.x_words;
 
         // ---- 1. evaluate own clauses (K1 + K7), votes (K6)
-        const bool active = lane < fg.words;
-        const uint32_t *col = rows + (active ? lane : 0);
-        const int stride = fg.words;
+        const int stride = fitl_stride(fg.words);
+        const uint32_t *col = rows + (2 * place < stride ? 2 * place : 0);  // every group of lanes reads whole rows
         for (int cl = wave; cl < n_own; cl += WAVES) {
             const int c = c0 + cl;
             const uint32_t *inc = ta + (size_t)cl * LA * B + (B - 1);
-            uint32_t acc = active && !p.direct ? col[(p.literals + c % p.n_types) * stride] : 0u;
-            int included = 0;
-            uint32_t first_words = 0;
-            for (int w0 = 0; w0 < LA; w0 += 64) {
-                uint32_t mine = w0 + lane < LA ? inc[(w0 + lane) * B] : 0u;
-                if (w0 + lane == LA - 1) mine &= p.filter;
-                if (w0 == 0) first_words = mine;
-                included += wave_sum_small(__popc(mine));
-            }
-            // A clause with many literals ANDs only the rows of its FITP_FILTER_ROWS rarest ones and then
-            // tests the few nodes that are left against its whole include mask on the nodes' own words.
-            const bool filter_only = included > FITP_WALK_ALL && n_now > 0 && !p.direct;
-            bool all_rows = false;  // every included literal's row has been applied: acc is the clause's truth
-            if (filter_only) {
-                int budget = FITP_FILTER_ROWS;
-                bool stop = false;
-                // The included literals in rarest-first order, 256 ranks at a time: the four LDS reads
-                // of the ranks and the four of the include words are each issued together (a clause
-                // whose rare literals are few would otherwise pay two LDS round trips per 64 ranks).
-                for (int g0 = 0; g0 < p.literals && !stop; g0 += 256) {
-                    uint32_t lit4[4];
-                    unsigned long long m4[4];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const int r = g0 + 64 * u + lane;
-                        lit4[u] = r < p.literals ? order_lds[r] : 0u;
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const int r = g0 + 64 * u + lane;
-                        uint32_t word = inc[(lit4[u] >> 5) * B];
-                        if ((int)(lit4[u] >> 5) == LA - 1) word &= p.filter;
-                        m4[u] = __ballot(r < p.literals && ((word >> (lit4[u] & 31u)) & 1u));
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        unsigned long long picked = m4[u];  // lanes whose literal is included and not applied yet
-                        const uint32_t lit = lit4[u];
-                        while (picked != 0ull && !stop) {
-                            if (budget <= 0) {
-                                // a few surviving nodes are cheapest tested one by one; more than that, and 8 more
-                                // rows (one LDS round trip) remove most of them at the price of testing one
-                                // (counted as lanes with a survivor, twice those with several: an estimate is enough)
-                                if (n_now <= FITP_FEW_NODES) {
-                                    stop = true;
-                                    break;
-                                }
-                                const int mine = active ? __popc((acc >> fg.shift) & fg.mask) : 0;
-                                const int left = __popcll(__ballot(mine > 0)) + __popcll(__ballot(mine > 1));
-                                if (left <= FITP_FEW_NODES) {
-                                    stop = true;
-                                    break;
-                                }
-                                budget = 8;
-                            }
-                            int row[8];
-#pragma unroll
-                            for (int v8 = 0; v8 < 8; ++v8) {
-                                row[v8] = picked ? (int)__builtin_amdgcn_readlane(lit, __ffsll((long long)picked) - 1) : ones_row;
-                                picked &= picked - 1;
-                            }
-                            uint32_t r8[8];
-#pragma unroll
-                            for (int v8 = 0; v8 < 8; ++v8) r8[v8] = col[row[v8] * stride];
-#pragma unroll
-                            for (int v8 = 0; v8 < 8; ++v8) acc &= r8[v8];
-                            budget -= 8;
-                        }
-                    }
+            uint16_t *list = lists + (size_t)cl * p.lists;
+            const uint32_t stale_now = stale[cl];
+            const int listed = incl_of[cl];
+            const uint32_t state = __builtin_amdgcn_readfirstlane(stale_now);
+            int included = __builtin_amdgcn_readfirstlane(listed);
+            if (state & 1u) {
+                int n = 0;
+                if constexpr (!DIRECT) {
+                    if (lane == 0 && p.lists > 0) list[0] = (uint16_t)(p.literals + (one_type ? 0 : c % p.n_types));
+                    n = 1;
                 }
-                all_rows = !stop;  // every included literal's row has been applied
-            } else if (!p.direct) {
                 for (int w0 = 0; w0 < LA; w0 += 64) {
-                    uint32_t mine = w0 == 0 ? first_words : (w0 + lane < LA ? inc[(w0 + lane) * B] : 0u);
-                    if (w0 != 0 && w0 + lane == LA - 1) mine &= p.filter;
-                    unsigned long long nonzero = __ballot(mine != 0);
-                    while (nonzero) {
-                        const int wl = __ffsll((long long)nonzero) - 1;
-                        nonzero &= nonzero - 1;
-                        uint32_t m = __builtin_amdgcn_readlane(mine, wl);
-                        const int base = (w0 + wl) << 5;
-                        while (m) {
-                            int row[8];
-#pragma unroll
-                            for (int u = 0; u < 8; ++u) {
-                                row[u] = m ? base + __builtin_ctz(m) : ones_row;
-                                m &= m - 1;
-                            }
-                            uint32_t r[8];
-#pragma unroll
-                            for (int u = 0; u < 8; ++u) r[u] = col[row[u] * stride];
-#pragma unroll
-                            for (int u = 0; u < 8; ++u) acc &= r[u];
-                        }
-                    }
+                    uint32_t mine = w0 + lane < LA ? inc[(w0 + lane) * B] : 0u;
+                    if (w0 + lane == LA - 1) mine &= p.filter;
+                    if constexpr (DIRECT)
+                        n += wave_sum_small(__popc(mine));
+                    else
+                        n = fitl_append(mine, min(64, LA - w0), 32 * w0, list, p.lists, n, lane);
                 }
+                if constexpr (!DIRECT) fitl_finish(list, p.lists, n, ones_row, p.lanes_log, lane);
+                included = DIRECT ? n : n - 1;
+                if (lane == 0) incl_of[cl] = included, stale[cl] = 0u;
+                fitp_wave_lds_sync();
+            } else if (state != 0u && lane == 0) {
+                stale[cl] = 0u;
             }
-            uint32_t v = active ? (acc >> fg.shift) & fg.mask : 0u;
-            if (p.direct) {
+            uint2 v;
+            if constexpr (DIRECT) {
                 // one or two nodes: the clause against each node's own literal words (kernels.py:443-466 as
                 // it stands), lane w on word w; no literal-major rows are read or staged
                 uint32_t bits = 0u;
                 for (int node = 0; node < n_now; ++node) {
                     bool violated = false;
                     for (int w0 = 0; w0 < LA; w0 += 64) {
-                        uint32_t mine = w0 == 0 ? first_words : (w0 + lane < LA ? inc[(w0 + lane) * B] : 0u);
-                        if (w0 != 0 && w0 + lane == LA - 1) mine &= p.filter;
+                        uint32_t mine = w0 + lane < LA ? inc[(w0 + lane) * B] : 0u;
+                        if (w0 + lane == LA - 1) mine &= p.filter;
                         const uint32_t xs = w0 + lane < LA ? x_now[node * LA + w0 + lane] : 0xFFFFFFFFu;
                         violated |= __ballot((mine & ~xs) != 0) != 0;
                     }
-                    if (!violated && (int)types_lds[i & 1][node] == c % p.n_types) bits |= 1u << node;
+                    if (!violated && (int)types_lds[i & 1][node] == (one_type ? 0 : c % p.n_types)) bits |= 1u << node;
                 }
-                v = lane == 0 ? bits : 0u;
+                v = make_uint2(lane == 0 ? bits : 0u, 0u);
+            } else {
+                const uint2 acc = included < p.lists ? fitl_truth(list, included + 1, col, stride, p.lanes_log, lane)
+                                                     : fitl_walk(inc, B, LA, p.filter, p.literals + (one_type ? 0 : c % p.n_types),
+                                                                 ones_row, col, stride, lane);
+                v = fitl_nodes(acc, fg, p.lanes_log, lane);
             }
-            if (filter_only && !all_rows) {
-                // lane L holds nodes 32 L .. 32 L + 31: the surviving ones are walked on the scalar unit; lane w
-                // compares include word w with the node's literal word w (LDS copy of the graph's X rows)
-                unsigned long long live = __ballot(v != 0);
-                while (live) {
-                    const int L = __ffsll((long long)live) - 1;
-                    live &= live - 1;
-                    uint32_t word = __builtin_amdgcn_readlane(v, L);
-                    uint32_t cleared = 0;
-                    while (word) {
-                        const int b = __builtin_ctz(word);
-                        word &= word - 1;
-                        const uint32_t *x = x_now + (L * 32 + b) * LA;
-                        bool violated = false;
-                        for (int w0 = 0; w0 < LA; w0 += 64) {
-                            uint32_t mine = w0 == 0 ? first_words : (w0 + lane < LA ? inc[(w0 + lane) * B] : 0u);
-                            if (w0 != 0 && w0 + lane == LA - 1) mine &= p.filter;
-                            const uint32_t xs = w0 + lane < LA ? x[w0 + lane] : 0xFFFFFFFFu;
-                            violated |= __ballot((mine & ~xs) != 0) != 0;
-                        }
-                        if (violated) cleared |= 1u << b;
-                    }
-                    if (lane == L) v &= ~cleared;
-                }
-            }
-            const int pc = __popc(v);
-            int true_nodes, before;
-            wave_count_scan(pc, lane, &true_nodes, &before);
-            bool fired = true_nodes > 0;
-            int node = -1;
-            if (n_now == 0) {
-                fired = true;  // the reference's arithmetic for a graph without nodes (kernels.py:289-295)
-            } else if (fired) {
-                philox_out r = philox4x32_10((uint32_t)c, 0u, step, GTM_TAG_CLAUSE_NODE, p.k0, p.k1);
-                const int pick = (int)(((uint64_t)r.v[0] * (uint64_t)true_nodes) >> 32);
-                const bool mine_is = pick >= before && pick < before + pc;
-                int candidate = 0;
-                if (mine_is) {
-                    uint32_t t = v;
-                    for (int j = before; j < pick; ++j) t &= t - 1;
-                    candidate = lane * 32 + __ffs(t) - 1;
-                }
-                const unsigned long long owner = __ballot(mine_is);
-                node = __builtin_amdgcn_readlane(candidate, __ffsll((long long)owner) - 1);
-            }
-            if (lane == 0) {
-                node_of[cl] = node;
-                incl_of[cl] = included;
-            }
+            const int node = n_now == 0 ? -1 : fitl_pick_node(v, pick_of[cl], lane);
+            const bool fired = n_now == 0 || node >= 0;  // (the reference's arithmetic for a graph without nodes, kernels.py:289-295)
+            if (lane == 0) node_of[cl] = node;
             if (fired)
                 for (int k = lane; k < K; k += 64) atomicAdd(&votes[k], wts[cl * K + k]);  // LDS
         }
@@ -408,6 +313,7 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_persistent(FitPersistParams 
         // ---- 2. class sums across the device (see the header comment)
         if (tid == 0) go_on = 1;
         lds_barrier();  // the group's votes are complete
+        unsigned long long *slot_now = p.class_sum + (size_t)slot * K * FITP_SUM_PARTS * FITP_SUM_STRIDE;
         if (tid >= poll0 && tid - poll0 < K) {  // (K <= FITP_BLOCK: one class per thread)
             const int k = tid - poll0;
             __hip_atomic_fetch_add(&slot_now[(k * FITP_SUM_PARTS + (int)(blockIdx.x % FITP_SUM_PARTS)) * FITP_SUM_STRIDE], FITP_ARRIVED + (unsigned long long)(long long)votes[k], __ATOMIC_RELAXED,
@@ -416,81 +322,73 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_persistent(FitPersistParams 
         }
         // Work that does not need the class sums is done while the other groups arrive: the next
         // graph's rows, literal words and labels are requested (straight into the other LDS
-        // buffers; they are waited for at the end of the step)
-        {
-            // element at = row * words + w; a thread's elements are FITP_BLOCK apart: step (row, w) without dividing
-            const uint32_t *tile = p.tiles + (int64_t)fn.tile * p.tg.rows * p.tg.tw + fn.word0;
-            if (fn.words != div_words) {  // the divisions are redone only when the slot width changes
-                div_words = fn.words;
-                div_dr = loaders / fn.words;
-                div_r0 = tid / fn.words;
+        // buffers; they are waited for at the end of the step). Nothing is requested before the barrier above: what is
+        // under way into LDS has to land before a barrier, and the literal words of the picked nodes, requested as soon as
+        // the nodes were known, held that barrier up by their memory latency (6.8 -> 5.9 us per example on 361 nodes).
+        const bool has_next = i + 1 < p.n_examples;
+        const int ex = p.first_example + i;
+        const FitGraph fn = fit_graph_slot(p.tg, has_next ? ex + 1 : ex, has_next ? n_next : n_now);
+        // node count and first node of the graph after the next, fetched by two threads and handed over through LDS
+        uint32_t after = 0u;
+        if (tid < 2) after = (tid == 0 ? p.n_nodes : p.node_index)[min(ex + 2, last)];
+        uint32_t type_ahead = 0u;
+        if (DIRECT && has_next && tid < n_next) type_ahead = p.node_type[base_next + tid];
+        // the literal words of the nodes that the wave's clauses learn from
+        if (!DIRECT && p.ahead)
+            for (int cl = wave; cl < n_own; cl += WAVES) {
+                const int node = __builtin_amdgcn_readfirstlane(node_of[cl]);
+                if (node < 0) continue;
+                for (int w0 = 0; w0 < LA; w0 += 64)
+                    if (w0 + lane < LA) fitp_load_to_lds(p.X + ((int64_t)base_now + node) * LA + w0 + lane, x_ahead + (size_t)cl * LA + w0);
             }
-            const int dr = div_dr, dw = loaders - dr * fn.words;
-            int r = div_r0, w = tid - r * fn.words;
-            uint32_t *dst = rows_buf[(i + 1) & 1] + wave * 64;
-            for (int at0 = 0; at0 < next_total && tid < loaders; at0 += loaders) {
-                if (at0 + tid < next_total) fitp_load_to_lds(tile + (int64_t)r * p.tg.tw + w, dst + at0);
-                r += dr;
-                w += dw;
-                if (w >= fn.words) {
-                    w -= fn.words;
-                    ++r;
-                }
-            }
-        }
-        const int next_x_total = has_next ? n_next * LA : 0;
-        {
+        if constexpr (!DIRECT) {
+            if (fn.words != loader_words) loader_words = fn.words, loader.prepare(fn.words, loaders, tid);
+            if (has_next)
+                loader.request(p.tiles + (int64_t)fn.tile * p.tg.rows * p.tg.tw + fn.word0, p.tg.tw, p.literals + p.n_types + 1, fn.words,
+                               rows_both + (~i & 1) * p.rows_words + wave * 64, loaders, tid);
+        } else {
+            const int next_x_total = has_next ? n_next * LA : 0;
             const uint32_t *src = p.X + (int64_t)base_next * LA + tid;
-            uint32_t *dst = x_buf[(i + 1) & 1] + wave * 64;
+            uint32_t *dst = x_both + (~i & 1) * p.x_words + wave * 64;
             for (int at0 = 0; at0 < next_x_total && tid < loaders; at0 += loaders)
                 if (at0 + tid < next_x_total) fitp_load_to_lds(src + at0, dst + at0);
         }
         if (has_next) {
             const uint32_t *src = (const uint32_t *)p.encoded_Y + (int64_t)(ex + 1) * K + tid;
-            uint32_t *dst = y_buf[(i + 1) & 1] + wave * 64;
+            uint32_t *dst = y_both + (~i & 1) * K + wave * 64;
             for (int at0 = 0; at0 < K && tid < loaders; at0 += loaders)
                 if (at0 + tid < K) fitp_load_to_lds(src + at0, dst + at0);
         }
-        if (p.direct && has_next && tid < n_next) types_lds[(i + 1) & 1][tid] = type_ahead;
-        // The random words of the feedback gates are drawn by the waves that do not poll, while the
-        // class sums are on their way. (Drawing the Type I feedback bits of every (clause, class,
+        // The random words of the feedback gates and of the next step's node picks are drawn by the waves that
+        // do not poll, while the class sums are on their way. (Drawing the Type I feedback bits of every (clause, class,
         // word) here as well costs more generator work than the exchange hides: they are drawn
         // afterwards, for the pairs that turn out to need them.)
         const int pollers = (K + 63) & ~63, helpers = FITP_BLOCK - pollers;
-        if (helpers >= FITP_BLOCK / 2) {
-            // (the polling threads are the first `pollers`, or - set apart - within the last 64)
-            if (poll_apart ? tid < poll0 : tid >= pollers)
-                for (int j = poll_apart ? tid : tid - pollers; j < n_own * K; j += helpers) {
-                    const int cl = j / K, k = j - cl * K;
-                    philox_out r = philox4x32_10((uint32_t)(c0 + cl), (uint32_t)k, step, GTM_TAG_CLAUSE_UPDATES, p.k0, p.k1);
-                    gate[2 * j] = r.v[0];
-                    gate[2 * j + 1] = r.v[1];
+        const bool helped = helpers >= FITP_BLOCK / 2;
+        // (the polling threads are the first `pollers`, or - set apart - within the last 64)
+        if (!helped || (poll_apart ? tid < poll0 : tid >= pollers)) {
+            const int first = !helped || poll_apart ? tid : tid - pollers, every = helped ? helpers : FITP_BLOCK;
+            for (int j = first; j < n_own * KW; j += every) pos_of[j] = 0u, neg_of[j] = 0u;
+            if (first == 0) n_pairs = 0, n_busy = 0;
+            for (int j = first; j < n_own * (K + 1); j += every) {
+                if (j >= n_own * K) {
+                    pick_of[j - n_own * K] = draw_pick(j - n_own * K, step + 1u);
+                    continue;
                 }
-        } else {
-            for (int j = tid; j < n_own * K; j += FITP_BLOCK) {
                 const int cl = j / K, k = j - cl * K;
                 philox_out r = philox4x32_10((uint32_t)(c0 + cl), (uint32_t)k, step, GTM_TAG_CLAUSE_UPDATES, p.k0, p.k1);
                 gate[2 * j] = r.v[0];
                 gate[2 * j + 1] = r.v[1];
             }
-            lds_barrier();
         }
+        if (!helped) lds_barrier();
         if (tid >= poll0 && tid - poll0 < K) {
             const int k = tid - poll0;
             const unsigned long long everyone = (unsigned long long)gridDim.x;
-            auto read_sum = [](const unsigned long long *slot, int k) {
-                unsigned long long part[FITP_SUM_PARTS], all = 0ull;
-#pragma unroll
-                for (int s = 0; s < FITP_SUM_PARTS; ++s)
-                    part[s] = __hip_atomic_load(&slot[(k * FITP_SUM_PARTS + s) * FITP_SUM_STRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-                for (int s = 0; s < FITP_SUM_PARTS; ++s) all += part[s];
-                return all;
-            };
             auto arrivals = [](unsigned long long now, unsigned long long before) {
                 return ((now - before + FITP_HALF) >> 48) & 0xFFFFull;
             };
-            uint32_t *seen_slot = seen + (size_t)(i % 3) * 2 * K;
+            uint32_t *seen_slot = seen + (size_t)slot * 2 * K;
             const unsigned long long seen_own = ((unsigned long long)seen_slot[K + k] << 32) | seen_slot[k];
             uint32_t polls = 0;
             unsigned long long waiting_since = 0ull;
@@ -498,15 +396,21 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_persistent(FitPersistParams 
             bool ok = !p.force_abort;
             if (!ok) __hip_atomic_store(p.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             while (ok) {
-                word = read_sum(slot_now, k);
+                // the abort flag travels with the parts: asked for after a look in vain it was a second round trip per look
+                unsigned long long part[FITP_SUM_PARTS];
+#pragma unroll
+                for (int s = 0; s < FITP_SUM_PARTS; ++s)
+                    part[s] = __hip_atomic_load(&slot_now[(k * FITP_SUM_PARTS + s) * FITP_SUM_STRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t aborted = __hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                word = 0ull;
+#pragma unroll
+                for (int s = 0; s < FITP_SUM_PARTS; ++s) word += part[s];
                 if (arrivals(word, seen_own) == everyone) break;
-                if (__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ||
-                    fit_wait_is_over(polls, p.spin_limit, waiting_since, p.wait_ticks)) {
+                if (aborted != 0 || fit_wait_is_over(polls, p.spin_limit, waiting_since, p.wait_ticks)) {
                     __hip_atomic_store(p.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     ok = false;
                     break;
                 }
-                __builtin_amdgcn_s_sleep(1);
             }
             if (!ok) go_on = 0;
             sums[k] = (int32_t)(long long)(word - seen_own - (everyone << 48));
@@ -515,14 +419,14 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_persistent(FitPersistParams 
         }
         __builtin_amdgcn_s_waitcnt(FITP_WAIT_VMEM);  // the next graph's words are in LDS
         if (tid < 2) after_lds[tid] = after;
+        if (DIRECT && has_next && tid < n_next) types_lds[(i + 1) & 1][tid] = type_ahead;
         lds_barrier();
         if (!go_on) break;  // uniform over the group; every group leaves at its next check
 
         // ---- 3. feedback (K8) and automaton updates (K9) on the LDS copies
-        const int32_t *y = (const int32_t *)y_buf[i & 1];
-        const uint32_t *X_rows = x_now;  // the graph's literal words, node-major, in LDS
-        auto decide = [&](int j, int k) {  // K8 for (clause, class) pair j = cl * K + k
-            const int cl = j / K;
+        const int32_t *y = (const int32_t *)(y_both + (i & 1) * K);
+        auto decide = [&](int cl, int k) {  // K8 for a (clause, class) pair
+            const int j = cl * K + k;
             int cs = sums[k];
             cs = cs > p.T ? p.T : (cs < -p.T ? -p.T : cs);
             const int yk = y[k];
@@ -542,86 +446,57 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_persistent(FitPersistParams 
                 if (p.negative == 0 && w < 1) w = 1;
                 wts[j] = w;
             }
-            upd[j] = u;
             return u;
         };
-        if (wave_local) {
-            // One clause per wave and few (class, word) pairs per clause: the wave decides for the clause's classes, draws the Type I feedback
-            // bits of the (class, word) pairs that need them and updates the clause's automata, with
-            // no barrier in between (a wave's LDS accesses are carried out in order).
-            if (wave < n_own) {
-                const int cl = wave;
-                bool any = false;
-                for (int k0 = 0; k0 < K; k0 += 64) {
-                    const int k = k0 + lane;
-                    const int u = k < K ? decide(cl * K + k, k) : 0;
-                    any |= __ballot(u != 0) != 0ull;
-                    const unsigned long long type1 = __ballot(u > 0);
-                    const int n_items = __popcll(type1) * LA;
-                    for (int t = lane; t < n_items; t += 64) {
-                        const int nth = t / LA, w = t - nth * LA;
-                        unsigned long long m = type1;
-                        for (int skip = 0; skip < nth; ++skip) m &= m - 1;
-                        const int kk = k0 + __ffsll((long long)m) - 1;
-                        fbits[((size_t)cl * LA + w) * K + kk] =
-                            gtm_feedback_bits(p.k0, p.k1, (uint32_t)(c0 + cl), (uint32_t)w, step, 0u, (uint32_t)kk, p.thr16);
-                    }
-                }
-                fitp_wave_lds_sync();
-                if (any) {
-                    const int node = node_of[cl];
-                    const bool fired = node != -1;
-                    const bool within = incl_of[cl] <= p.max_included;
-                    for (int w = lane; w < LA; w += 64) {
-                        const uint32_t x = fired ? X_rows[node * LA + w] : 0u;
-                        feedback_word<MAXB>(ta + ((size_t)cl * LA + w) * B, B, K, upd + cl * K, 1, fired, within, p.boost, x, p.k0,
-                                            p.k1, (uint32_t)(c0 + cl), (uint32_t)w, step, 0u, p.thr16,
-                                            fbits + ((size_t)cl * LA + w) * K);
-                    }
-                }
-            }
-        } else {
-            for (int j = tid; j < n_own * K; j += FITP_BLOCK) decide(j, j % K);
-            lds_barrier();
-            // Type I feedback bits for the (clause, class) pairs that need them: the pairs are listed
-            // first (wave 0, ballots), then one thread per (listed pair, word) draws the bits, so that
-            // the lanes that run the generator are (nearly) all busy
-            if (wave == 0) {
-                int n_listed = 0;
-                for (int j0 = 0; j0 < n_own * K; j0 += 64) {
-                    const int j = j0 + lane;
-                    const bool need = j < n_own * K && upd[j] > 0;
-                    const unsigned long long m = __ballot(need);
-                    if (need) pair_list[n_listed + __popcll(m & ((1ull << lane) - 1ull))] = j;
-                    n_listed += __popcll(m);
-                }
-                if (lane == 0) n_pairs = n_listed;
-            }
-            lds_barrier();
-            for (int t = tid; t < n_pairs * LA; t += FITP_BLOCK) {
-                const int j = pair_list[t / LA], w = t % LA;
-                const int cl = j / K, k = j - cl * K;
-                fbits[((size_t)cl * LA + w) * K + k] =
-                    gtm_feedback_bits(p.k0, p.k1, (uint32_t)(c0 + cl), (uint32_t)w, step, 0u, (uint32_t)k, p.thr16);
-            }
-            lds_barrier();
-            for (int j = tid; j < n_own * LA; j += FITP_BLOCK) {
-                const int cl = j / LA, w = j - cl * LA;
-                const int32_t *u_of = upd + cl * K;
-                bool any = false;
-                for (int k = 0; k < K; ++k) any |= u_of[k] != 0;
-                if (!any) continue;
-                const int node = node_of[cl];
-                const bool fired = node != -1;
-                const bool within = incl_of[cl] <= p.max_included;
-                const uint32_t x = fired ? X_rows[node * LA + w] : 0u;
-                feedback_word<MAXB>(ta + (size_t)j * B, B, K, u_of, 1, fired, within, p.boost, x, p.k0, p.k1,
-                                  (uint32_t)(c0 + cl), (uint32_t)w, step, 0u, p.thr16, fbits + (size_t)j * K);
+        // word w of the literals of the node that clause cl learns from
+        auto literal_word = [&](int cl, int node, int w) {
+            if constexpr (DIRECT) return x_now[node * LA + w];
+            if (p.ahead) return x_ahead[(size_t)cl * LA + w];
+            // (an atomic load, so that the compiler does not make one flat load of the two)
+            return __hip_atomic_load(&p.X[((int64_t)base_now + node) * LA + w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+        auto planes_of = [&](int cl, int w) {
+            return (uint32_t *)__builtin_assume_aligned(ta + ((size_t)cl * LA + w) * B, EXACT && MAXB == 8 ? 16 : 4);
+        };
+        for (int j = tid; j < n_own * K; j += FITP_BLOCK) {
+            const int cl = j / K, k = j - cl * K;
+            const int u = decide(cl, k);
+            if (u == 0) continue;
+            // listed: the pairs that need Type I bits, and the clauses that get any feedback (once)
+            if (u > 0) pair_list[atomicAdd(&n_pairs, 1)] = j;
+            atomicOr(&(u > 0 ? pos_of : neg_of)[cl * KW + (k >> 5)], 1u << (k & 31));
+            if (atomicOr(&stale[cl], 2u) < 2u) busy_list[atomicAdd(&n_busy, 1)] = cl;
+        }
+        lds_barrier();
+        // a thread per byte of Type I bits, 2^quarter_log threads per pair
+        for (int t = tid; t < n_pairs << quarter_log; t += FITP_BLOCK) {
+            const int j = pair_list[t >> quarter_log], cl = j / K, k = j - cl * K;
+            for (int item = t & ((1 << quarter_log) - 1); item < 4 * LA; item += 1 << quarter_log) {
+                const int w = item >> 2, q = item & 3;
+                ((uint8_t *)&fbits[((size_t)cl * LA + w) * K + k])[q] =
+                    (uint8_t)fitl_feedback_byte(p.k0, p.k1, (uint32_t)(c0 + cl), (uint32_t)w, (uint32_t)q, step, 0u, (uint32_t)k, p.thr16);
             }
         }
-        // With the feedback inside the clause's wave, the wave goes on to evaluate its clause on the
-        // next graph (everything that evaluation reads was complete at the barrier above).
-        if (!wave_local) lds_barrier();
+        lds_barrier();
+        for (int t = tid; t < n_busy << word_log; t += FITP_BLOCK) {
+            const int cl = busy_list[t >> word_log];
+            const int node = node_of[cl];
+            const bool fired = node != -1;
+            const bool learns = fired && incl_of[cl] <= p.max_included;
+            for (int w = t & ((1 << word_log) - 1); w < LA; w += 1 << word_log) {
+                const uint32_t x = fired ? literal_word(cl, node, w) : 0u;
+                fits_word<MAXB, EXACT> word(planes_of(cl, w), B);
+                const uint32_t was = word.top();
+                const uint32_t *fb_of = fbits + ((size_t)cl * LA + w) * K;
+                for (int kw = 0; kw < KW; ++kw)
+                    fitl_feedback(word, pos_of[cl * KW + kw], neg_of[cl * KW + kw], fired, learns, p.boost, x, fb_of + 32 * kw);
+                word.store(planes_of(cl, w));
+                if (word.top() != was) atomicOr(&stale[cl], 1u);
+            }
+        }
+        lds_barrier();
+        slot = slot == 2 ? 0 : slot + 1;
+        fg = fn;
         n_now = n_next;
         base_now = base_next;
         n_next = (int)after_lds[0];

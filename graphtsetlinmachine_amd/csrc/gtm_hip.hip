@@ -65,6 +65,7 @@ int check_launch(const char *what) {
     X(FIT_DEEP_WINDOW_ROWS) \
     X(FIT_FACTOR_MIN) \
     X(FIT_PER_GROUP) \
+    X(FIT_LIST_ROWS) \
     X(FIT_SPIN_LIMIT) \
     X(HALF_LANE_WORDS) \
     X(MESSAGES_IN_LDS) \
@@ -75,6 +76,7 @@ int check_launch(const char *what) {
     X(NO_DEEP_FIT) \
     X(NO_DEEP_PERSISTENT_FIT) \
     X(NO_DIRECT_FIT) \
+    X(NO_FIT_WAVES) \
     X(NO_FUSED_MESSAGES) \
     X(NO_HALF_ROWS) \
     X(NO_HALF_TILES) \
@@ -508,7 +510,9 @@ __global__ void k_select_clause_updates(int32_t *weights, const int32_t *__restr
 #include "fit_fused.h"
 #include "fit_deep.h"
 #include "fit_small.h"
+#include "fit_lists.h"
 #include "fit_persistent.h"
+#include "fit_waves.h"
 #include "fit_deep_persistent.h"
 
 // K9 / K10: one thread per (clause, automaton word); the classes are applied
@@ -2233,38 +2237,56 @@ int fit_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
     FitPersistParams p{};
     p.max_words = tg.slot_words > 0 ? tg.slot_words : 1;
     // graphs of one or two nodes: the nodes are tested on their own literal words, no rows are staged
-    p.direct = g->max_number_of_graph_nodes <= FITP_DIRECT_NODES && !tune(T_NO_DIRECT_FIT);
+    const bool direct = g->max_number_of_graph_nodes <= FITP_DIRECT_NODES && !tune(T_NO_DIRECT_FIT);
     p.node_type = g->node_type;
-    p.rows_words = p.direct ? 0 : (cfg->literals + g->number_of_node_types + 1) * p.max_words;
-    p.x_words = (g->max_number_of_graph_nodes > 0 ? g->max_number_of_graph_nodes : 1) * d.LA;
-    p.order = g->tiles + tiles_words(tg) + (size_t)tg.rows * 2;
+    p.rows_words = direct ? 0 : (cfg->literals + g->number_of_node_types + 1) * fitl_stride(p.max_words);
+    p.x_words = direct ? (g->max_number_of_graph_nodes > 0 ? g->max_number_of_graph_nodes : 1) * d.LA : 0;
     // One clause per wave and step. Few clauses per group keep a step's feedback short, few groups
     // keep the exchange of the class sums short: the clauses are spread over all CUs (8 to 12 per
     // group measured best on 2,000 and 2,500 clauses), but a group gets at least 8 where their
     // automata fit in LDS.
-    auto lds_bytes = [&](int per_group) {
-        return (2 * (size_t)p.rows_words + (size_t)per_group * d.LA * d.B + 2 * (size_t)per_group +
-                2 * (size_t)d.K + 5 * (size_t)per_group * d.K + (size_t)per_group * d.LA * d.K + 2 * (size_t)p.x_words +
-                (size_t)cfg->literals + 8 * (size_t)d.K) * 4;
+    auto lds_bytes = [&](int per_group, int lists, bool ahead) {
+        return fit_persistent_lds_words(per_group, d.LA, d.B, d.K, p.rows_words, p.x_words, lists, ahead) * 4;
     };
-    const size_t lds_limit = 150 * 1024;
+    const size_t lds_limit = 158 * 1024;  // of 160 KiB; the kernel has a few words of its own
     int per_group = (d.C + cus - 1) / cus;
     const int preferred = 8;
-    if (per_group < preferred && lds_bytes(preferred) <= lds_limit) per_group = preferred;
+    if (per_group < preferred && lds_bytes(preferred, 0, false) <= lds_limit) per_group = preferred;
     if (const char *e = tune(T_FIT_PER_GROUP)) {  // tuning: clauses per group, at least C / CUs
         const int asked = atoi(e);
         if (asked >= (d.C + cus - 1) / cus && asked <= FITP_BLOCK) per_group = asked;
     }
-    if (lds_bytes(per_group) > lds_limit) return GTM_OK;
     const int groups = (d.C + per_group - 1) / per_group;
     p.clauses_per_group = per_group;
-    const size_t lds = lds_bytes(per_group);
+    p.lanes_log = fitl_lanes_log(p.max_words);
+    p.lists = direct ? 0 : fitl_entries(cfg->literals, p.lanes_log);
+    // A wave per clause with its state in registers where the clauses are small enough (us per example, waves against
+    // state in LDS: 361 nodes, 2,500 clauses of 8 words, 10 classes 5.2 against 6.3; 81 nodes, 250 clauses of 4 words 3.3
+    // against 5.1; ragged chains of up to 300 nodes, 150 clauses 4.1 against 6.3); else the state in LDS, and as much of the lists
+    // and of the picked nodes' literal words as it has room for (a clause with more literals than its list holds walks
+    // its include plane instead).
+    const bool waves = !direct && per_group <= FITP_BLOCK / 64 && d.K <= FITV_MAX_CLASSES && d.LA <= FITV_MAX_WORDS &&
+                       fit_waves_lds_words(per_group, p.rows_words, p.lists) * 4 <= lds_limit && !tune(T_NO_FIT_WAVES);
+    size_t lds = fit_waves_lds_words(per_group, p.rows_words, p.lists) * 4;
+    if (!waves) {
+        if (lds_bytes(per_group, 0, false) > lds_limit) return GTM_OK;
+        p.ahead = !direct && lds_bytes(per_group, 0, true) <= lds_limit;
+        const int batch = 1 << (FITL_BATCH_LOG + 6 - p.lanes_log);
+        if (const char *e = tune(T_FIT_LIST_ROWS)) p.lists = std::min(p.lists, std::max(0, atoi(e)) / batch * batch);  // (tests)
+        while (p.lists > 0 && lds_bytes(per_group, p.lists, p.ahead != 0) > lds_limit) p.lists -= batch;
+        lds = lds_bytes(per_group, p.lists, p.ahead != 0);
+    }
     // one instance per width of the automata in registers (the widest would cost the others registers)
-    const int variant = d.B <= 8 ? 0 : d.B <= 16 ? 1 : 2;
-    const void *kernel = variant == 0   ? (const void *)k_fit_persistent<8>
-                         : variant == 1 ? (const void *)k_fit_persistent<16>
-                                        : (const void *)k_fit_persistent<32>;
-    static thread_local size_t lds_set_of[3] = {48 * 1024, 48 * 1024, 48 * 1024};
+    const int variant = (d.B == 8 ? 0 : d.B < 8 ? 1 : d.B <= 16 ? 2 : 3) + (waves ? 8 : direct ? 4 : 0);
+    const void *kernels[12] = {(const void *)k_fit_persistent<8, true, false>,   (const void *)k_fit_persistent<8, false, false>,
+                              (const void *)k_fit_persistent<16, false, false>, (const void *)k_fit_persistent<32, false, false>,
+                              (const void *)k_fit_persistent<8, true, true>,    (const void *)k_fit_persistent<8, false, true>,
+                              (const void *)k_fit_persistent<16, false, true>,  (const void *)k_fit_persistent<32, false, true>,
+                              (const void *)k_fit_waves<8, true>,               (const void *)k_fit_waves<8, false>,
+                              (const void *)k_fit_waves<16, false>,             (const void *)k_fit_waves<32, false>};
+    const void *kernel = kernels[variant];
+    static thread_local size_t lds_set_of[12] = {48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024,
+                                                 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024};
     size_t &lds_set = lds_set_of[variant];
     if (lds > lds_set) {
         if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
@@ -2323,7 +2345,7 @@ int fit_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
                        (unsigned long long *)w.class_sum, (int64_t)0, 0ull, (int64_t)d.K * 3 * FITP_SUM_PARTS * FITP_SUM_STRIDE + 1);
     if (int rc = check_launch("fill")) return rc;
     void *args[] = {&p};
-    profile_start("k_fit_persistent", st);
+    profile_start(waves ? "k_fit_waves" : "k_fit_persistent", st);
     e = hipLaunchCooperativeKernel(kernel, dim3(groups), dim3(FITP_BLOCK), args, (unsigned)lds, st);
     if (e != hipSuccess) return fail(GTM_ERR_HIP, "cooperative launch of the training kernel: %s", hipGetErrorString(e));
     profile_stop(st);
