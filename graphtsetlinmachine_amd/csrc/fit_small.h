@@ -242,7 +242,7 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
         for (int j = first; j < end; j += stride) {
             const bool pick = j < C;
             const int ck = pick ? 0 : j - C, c = pick ? j : fits_div(ck, K, p.by_K), k = pick ? 0 : ck - c * K;
-            const philox_out r = philox4x32_10((uint32_t)c, (uint32_t)k, at_step, pick ? GTM_TAG_CLAUSE_NODE : GTM_TAG_CLAUSE_UPDATES, p.k0, p.k1);
+            const philox_out r = philox4x32_10<false>((uint32_t)c, (uint32_t)k, at_step, pick ? GTM_TAG_CLAUSE_NODE : GTM_TAG_CLAUSE_UPDATES, p.k0, p.k1);
             uint32_t *to = pick ? draw_node + j : draw_update + 2 * ck;
             to[0] = r.v[0];
             if (!pick) to[1] = r.v[1];
@@ -633,7 +633,7 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
                 // Type I where u > 0 (kernels.py:141-173), Type II where u < 0 (:174-183): bits to count up and down
                 uint32_t up = fired ? ~x & ~word.top() : 0u, down = 0u;
                 if (now > 0) {
-                    const uint32_t fb = gtm_feedback_bits(p.k0, p.k1, (uint32_t)c, (uint32_t)w, step, (uint32_t)l, (uint32_t)k, thr16);
+                    const uint32_t fb = gtm_feedback_bits<false>(p.k0, p.k1, (uint32_t)c, (uint32_t)w, step, (uint32_t)l, (uint32_t)k, thr16);
                     up = learns ? (p.boost == 1 ? x : x & ~fb) : 0u;
                     down = learns ? ~x & fb : fb;
                 }

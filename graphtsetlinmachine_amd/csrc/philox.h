@@ -33,13 +33,23 @@ GTM_HD uint32_t gtm_mulhi32(uint32_t a, uint32_t b) {
 #endif
 }
 
+// WHOLE: a product's halves by one instruction (v_mad_u64_u32); else by two, as slow each but sooner done when nothing
+// else is there to issue.  Many waves per SIMD gain from the first (361-node images at depth 1 5.23 -> 5.10 us per example, ragged chains
+// 4.11 -> 3.98), the one workgroup of k_fit_small from the second (3.61 against 3.69).
+template <bool WHOLE = true>
 GTM_HD philox_out philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0, uint32_t k1) {
     const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u;
     const uint32_t W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
 #pragma unroll
     for (int round = 0; round < 10; ++round) {
-        uint32_t hi0 = gtm_mulhi32(M0, c0), lo0 = M0 * c0;
-        uint32_t hi1 = gtm_mulhi32(M1, c2), lo1 = M1 * c2;
+        uint32_t hi0, lo0, hi1, lo1;
+        if constexpr (WHOLE) {
+            const uint64_t p0 = (uint64_t)M0 * c0, p1 = (uint64_t)M1 * c2;
+            hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0, hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
+        } else {
+            hi0 = gtm_mulhi32(M0, c0), lo0 = M0 * c0;
+            hi1 = gtm_mulhi32(M1, c2), lo1 = M1 * c2;
+        }
         uint32_t n0 = hi1 ^ c1 ^ k0;
         uint32_t n2 = hi0 ^ c3 ^ k1;
         c0 = n0;
@@ -61,6 +71,7 @@ GTM_HD philox_out philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t 
 // the b-th 16-bit slice of four Philox blocks is below threshold16
 // (threshold16 = min(65536, floor(65536 / s)), so s = 1 gives all ones).
 // Stands for the 32 `curand_uniform <= 1/s` draws of kernels.py:113-118,157-162.
+template <bool WHOLE = true>
 GTM_HD uint32_t gtm_feedback_bits(uint32_t k0, uint32_t k1, uint32_t clause, uint32_t word, uint32_t step,
                                   uint32_t bank, uint32_t class_id, uint32_t threshold16) {
     if (threshold16 >= 65536u) return 0xFFFFFFFFu;  // s <= 1: every 16-bit value is below the threshold
@@ -68,7 +79,7 @@ GTM_HD uint32_t gtm_feedback_bits(uint32_t k0, uint32_t k1, uint32_t clause, uin
     uint32_t bits = 0;
 #pragma unroll
     for (uint32_t j = 0; j < 4; ++j) {
-        philox_out r = philox4x32_10(clause, word * 4u + j, step, c3, k0, k1);
+        philox_out r = philox4x32_10<WHOLE>(clause, word * 4u + j, step, c3, k0, k1);
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) {
             uint32_t lo = r.v[i] & 0xFFFFu, hi = r.v[i] >> 16;
