@@ -76,6 +76,7 @@ int check_launch(const char *what) {
     X(NO_DEEP_FIT) \
     X(NO_DEEP_PERSISTENT_FIT) \
     X(NO_DIRECT_FIT) \
+    X(NO_FIT_MOVES) \
     X(NO_FIT_WAVES) \
     X(NO_FUSED_MESSAGES) \
     X(NO_HALF_ROWS) \
@@ -514,6 +515,7 @@ __global__ void k_select_clause_updates(int32_t *weights, const int32_t *__restr
 #include "fit_persistent.h"
 #include "fit_waves.h"
 #include "fit_deep_persistent.h"
+#include "fit_moves.h"
 
 // K9 / K10: one thread per (clause, automaton word); the classes are applied
 // in ascending order to that word, as kernels.py:205-207,236-238 do per clause
@@ -768,8 +770,23 @@ struct FitWs {
     size_t coop_words;                      // words of coop_got
     int *coop_perm;                         // [C + 2,048] which clause sits in which workgroup's slots (k_fit_deep_deal)
     uint32_t *coop_cost;                    // [C]
+    uint32_t *move_masks;                   // [FITM_CHUNK][TILE_MOVES_MAX][even NC] where a graph's edges end (k_fit_moves)
+    uint16_t *lists;                        // [C + 2,048][entries] the clauses' rows (k_fit_moves; NULL: too large)
     size_t bytes;
 };
+
+// What k_fit_moves takes whatever the data: whole words of message bits, a lane per pair of truth words, 16-bit row numbers
+// (15 bits and a sign for messages), classes that one wave polls for.
+bool fit_moves_takes(const Dims &d, const gtm_config *cfg) {
+    return cfg->depth > 1 && d.M % 32 == 0 && d.M < 32768 && d.NC <= 64 && d.K <= FITM_MAX_CLASSES && d.B <= 16 && cfg->literals < 32768;
+}
+int fit_moves_list0(const gtm_config *cfg) { return (cfg->literals + 1 + 7) / 8 * 8; }
+int fit_moves_listm(const Dims &d) { return 2 * d.M; }  // (both halves whole octets)
+// The lists of the clauses whose automata stay in memory.
+constexpr size_t FITM_LISTS_MAX = (size_t)256 << 20;
+size_t fit_moves_list_bytes(const Dims &d, const gtm_config *cfg) {
+    return ((size_t)d.C + 2048) * (fit_moves_list0(cfg) + (size_t)(cfg->depth - 1) * fit_moves_listm(d)) * 2;
+}
 
 FitWs carve_fit(const Dims &d, const gtm_config *cfg, char *base) {
     FitWs w;
@@ -797,12 +814,15 @@ FitWs carve_fit(const Dims &d, const gtm_config *cfg, char *base) {
     w.got = cfg->depth > 1 ? (uint32_t *)take(vector_bytes) : nullptr;
     w.bank_backup = (uint32_t *)take(((size_t)d.C * d.LA + (size_t)(cfg->depth - 1) * d.C * d.MC) * d.B * 4);
     w.weights_backup = (int32_t *)take((size_t)d.K * d.C * 4);
-    w.coop_words = cfg->depth > 1 ? (size_t)3 * (cfg->depth - 1) * d.M * d.NC : 0;
+    w.coop_words = cfg->depth > 1 ? (size_t)3 * (cfg->depth - 1) * d.M * fitl_stride(d.NC) : 0;
     w.coop_got = cfg->depth > 1 ? (uint32_t *)take(w.coop_words * 4) : nullptr;
     w.coop_vec = cfg->depth > 1 ? (uint32_t *)take((size_t)(cfg->depth - 1) * cfg->max_nodes * d.MC * 2) : nullptr;
     w.coop_arrived = cfg->depth > 1 ? (unsigned long long *)take((size_t)(cfg->depth - 1) * FITD_PARTS * FITD_STRIDE * 8) : nullptr;
     w.coop_perm = cfg->depth > 1 ? (int *)take(((size_t)d.C + 2048) * 4) : nullptr;
     w.coop_cost = cfg->depth > 1 ? (uint32_t *)take((size_t)d.C * 4) : nullptr;
+    const bool moves = cfg->depth > 1 && fit_moves_takes(d, cfg);
+    w.move_masks = moves ? (uint32_t *)take((size_t)FITM_CHUNK * TILE_MOVES_MAX * fitl_stride(d.NC) * 4) : nullptr;
+    w.lists = moves && fit_moves_list_bytes(d, cfg) <= FITM_LISTS_MAX ? (uint16_t *)take(fit_moves_list_bytes(d, cfg)) : nullptr;
     w.bytes = off;
     return w;
 }
@@ -2603,6 +2623,215 @@ int fit_deep_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *
     return GTM_OK;
 }
 
+// The same for data sets whose edges are a few moves (fit_moves.h).
+int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const gtm_state *s, const TileGeom &tg, const FitWs &w,
+              const int32_t *encoded_Y, int first_example, int n_examples, uint64_t first_step, hipStream_t st, bool *done,
+              int *examples_done) {
+    *done = false;
+    *examples_done = 0;
+    if (tune(T_NO_FIT_MOVES) || tune(T_NO_DEEP_PERSISTENT_FIT) || tune(T_NO_PERSISTENT_FIT) || !w.move_masks) return GTM_OK;
+    int dev = 0, coop = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return GTM_OK;
+    if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !coop) return GTM_OK;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) return GTM_OK;
+    if (g->total_edges == 0 || cfg->max_nodes < 2) return GTM_OK;  // nothing to shift: as before
+    if (!g->number_of_graph_node_edges || !g->edge || !g->edge_index)
+        return fail(GTM_ERR_INVALID, "graphs with edges need number_of_graph_node_edges, edge and edge_index");
+
+    const int layers = cfg->depth - 1, S = fitl_stride(d.NC);
+    int per_group = (d.C + cus - 1) / cus;
+    if (const char *e = tune(T_FIT_DEEP_CLAUSES_PER_GROUP)) per_group = std::max(per_group, atoi(e));  // tuning aid
+    const int groups = (d.C + per_group - 1) / per_group, words = d.LA + layers * d.MC;
+    if (per_group > 512 || (size_t)groups * per_group > (size_t)d.C + 2048) return GTM_OK;
+    FitMovesParams p{};
+    p.S = S;
+    p.list0 = fit_moves_list0(cfg), p.listm = fit_moves_listm(d);
+    const int rows_words = ((cfg->literals + g->number_of_node_types + 1) * fitl_stride(tg.slot_words > 0 ? tg.slot_words : 1) + 3) / 4 * 4;
+    // Automata in registers and lists in LDS, with the graph's rows staged in LDS where there is room; else automata and lists in
+    // memory, rows in place.
+    const size_t lds_limit = 158 * 1024;  // of 160 KiB; the kernel has a few words of its own
+    auto lds_bytes = [&](bool regs, bool rows_lds, int n_moves) {
+        return fit_moves_lds_words(regs, rows_lds, cfg->depth, per_group, d.LA, d.MC, d.MB, d.M, d.K, S, rows_words, p.list0, p.listm, n_moves) * 4;
+    };
+    const bool in_memory = tune(T_FIT_DEEP_IN_MEMORY) != nullptr;  // (tests)
+    auto layout_of = [&](int n_moves) {  // 0: registers and staged rows, 1: registers, 2: memory, -1: none
+        if (!in_memory && per_group * words <= FITP_BLOCK) {
+            if (lds_bytes(true, true, n_moves) <= lds_limit) return 0;
+            if (lds_bytes(true, false, n_moves) <= lds_limit) return 1;
+        }
+        return w.lists && lds_bytes(false, false, n_moves) <= lds_limit ? 2 : -1;
+    };
+    if (layout_of(0) < 0) return GTM_OK;
+
+    uint32_t found[TILE_MOVES_HEADER_WORDS] = {};
+    uint32_t *header = w.coop_got;
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(TPB), 0, st, (int32_t *)header, (int64_t)TILE_MOVES_HEADER_WORDS, 0);
+    if (int rc = check_launch("fill")) return rc;
+    hipLaunchKernelGGL(k_fit_edge_moves, dim3(n_examples), dim3(256), 0, st, g->number_of_graph_nodes, g->node_index,
+                       g->number_of_graph_node_edges, g->edge_index, g->edge, first_example, header);
+    if (int rc = check_launch("k_fit_edge_moves")) return rc;
+    hipError_t looked = hipMemcpyAsync(found, header, sizeof found, hipMemcpyDeviceToHost, st);
+    if (looked == hipSuccess) looked = hipStreamSynchronize(st);
+    if (looked != hipSuccess) return fail(GTM_ERR_HIP, "reading the edges' moves: %s", hipGetErrorString(looked));
+    if (found[TILE_MOVES_MAX] != 0u || found[0] == 0u) return GTM_OK;
+    while (p.moves.n < TILE_MOVES_MAX && found[p.moves.n] != 0u) {
+        const uint32_t key = found[p.moves.n];
+        const int off = (int)(key & 0xFFFFu) - (int)TILE_MOVE_OFFSET;  // node n sends to n + off: node v receives from v - off
+        p.moves.type[p.moves.n] = (int)((key >> 16) % (uint32_t)d.M);
+        p.moves.words[p.moves.n] = (-off) >> 5;
+        p.moves.bits[p.moves.n] = (-off) & 31;
+        ++p.moves.n;
+    }
+    const int layout = layout_of(p.moves.n);
+    if (layout < 0) return GTM_OK;
+    const bool rows_lds = layout == 0;
+    const size_t lds = lds_bytes(layout < 2, rows_lds, p.moves.n);
+    const int variant = (d.B == 8 ? 0 : 3) + layout;
+    const void *kernels[6] = {(const void *)k_fit_moves<8, true, true, true>,    (const void *)k_fit_moves<8, true, true, false>,
+                              (const void *)k_fit_moves<8, true, false, false>,  (const void *)k_fit_moves<16, false, true, true>,
+                              (const void *)k_fit_moves<16, false, true, false>, (const void *)k_fit_moves<16, false, false, false>};
+    const void *kernel = kernels[variant];
+    static thread_local size_t lds_set_of[6] = {48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024};
+    if (lds > lds_set_of[variant]) {
+        if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
+            (void)hipGetLastError();
+            return GTM_OK;
+        }
+        lds_set_of[variant] = lds;
+    }
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, FITP_BLOCK, lds) != hipSuccess || per_cu < 1 || groups > per_cu * cus) {
+        (void)hipGetLastError();
+        return GTM_OK;
+    }
+
+    Key key = key_of(cfg);
+    p.tiles = g->tiles;
+    p.X = g->X;
+    p.node_index = g->node_index;
+    p.n_nodes = g->number_of_graph_nodes;
+    p.encoded_Y = encoded_Y;
+    p.tg = tg;
+    p.masks = w.move_masks;
+    p.bank[0] = s->ta_state;
+    p.thr16[0] = feedback_threshold(cfg->s[0]);
+    for (int l = 1; l < cfg->depth; ++l) {
+        p.bank[l] = s->message_ta_state[l - 1];
+        p.thr16[l] = feedback_threshold(cfg->s[l]);
+    }
+    p.weights = s->clause_weights;
+    p.hv = s->hypervectors;
+    p.depth = cfg->depth;
+    p.literals = cfg->literals;
+    p.n_types = g->number_of_node_types;
+    p.C = d.C, p.LA = d.LA, p.MC = d.MC, p.MW = d.M / 32, p.M = d.M, p.MB = d.MB, p.B = d.B, p.K = d.K;
+    p.T = cfg->threshold;
+    p.negative = cfg->negative_clauses;
+    p.boost = cfg->boost_true_positive_feedback;
+    p.max_included = cfg->max_included_literals;
+    p.filter = d.filter;
+    p.k0 = key.k0, p.k1 = key.k1;
+    p.q_thr = q_threshold(cfg->q, cfg->classes);
+    p.got = w.coop_got;
+    p.vec = w.coop_vec;
+    p.arrived = w.coop_arrived;
+    p.class_sum = (unsigned long long *)w.class_sum;
+    p.abort_flag = (uint32_t *)((unsigned long long *)w.class_sum + (size_t)d.K * 3 * FITP_SUM_PARTS * FITP_SUM_STRIDE);
+    const WaitBound bound = wait_bound(dev);
+    p.spin_limit = bound.spin_limit, p.wait_ticks = bound.wait_ticks, p.force_abort = bound.force_abort;
+    p.clauses_per_group = per_group;
+    p.lists = w.lists;
+    p.lanes_log = fitl_lanes_log(S);
+    p.rows_words = rows_lds ? rows_words : 0;
+    p.max_nodes = cfg->max_nodes;
+
+    // Clauses dealt out by their cost before each launch, as fit_deep_persistent does.
+    const bool deal = per_group >= 2 && d.C <= FITD_DEAL_MAX && w.coop_perm && w.coop_cost && !tune(T_FIT_DEEP_NO_DEAL);
+    int chunk = deal ? 256 : FITM_CHUNK;
+    if (const char *e = tune(T_FIT_DEEP_CHUNK)) chunk = std::min(FITM_CHUNK, std::max(1, atoi(e)));
+    const bool chunk_grows = deal && !tune(T_FIT_DEEP_CHUNK);
+    static thread_local bool deal_lds_raised = false;
+    if (deal && !deal_lds_raised) {
+        if (hipFuncSetAttribute((const void *)k_fit_deep_deal, hipFuncAttributeMaxDynamicSharedMemorySize, FITD_DEAL_MAX * 8) != hipSuccess)
+            return fail(GTM_ERR_HIP, "raising the LDS limit of the dealing kernel");
+        deal_lds_raised = true;
+    }
+    for (int at = 0; at < n_examples;) {
+        const int n_now = std::min(chunk, n_examples - at);
+        p.first_example = first_example + at;
+        p.n_examples = n_now;
+        p.first_step = (uint32_t)(first_step + (uint64_t)at);
+        p.perm = nullptr;
+        if (deal) {
+            FitDeepBanks banks{};
+            for (int l = 0; l < cfg->depth; ++l) banks.bank[l] = p.bank[l];
+            hipLaunchKernelGGL(k_fit_deep_cost, dim3(blocks_for(d.C, TPB / 64)), dim3(TPB), 0, st, banks, cfg->depth, d.C, d.LA, d.MC,
+                               d.B, w.coop_cost);
+            if (int rc = check_launch("fit_deep_cost")) return rc;
+            int pow2 = 1;
+            while (pow2 < d.C) pow2 <<= 1;
+            hipLaunchKernelGGL(k_fit_deep_deal, dim3(1), dim3(1024), (size_t)pow2 * 8, st, w.coop_cost, d.C, groups, per_group, w.coop_perm);
+            if (int rc = check_launch("fit_deep_deal")) return rc;
+            p.perm = w.coop_perm;
+        }
+        {
+            if (at > 0) {  // (the header lies in the rows that the launch before exchanged)
+                hipError_t e = hipMemcpyAsync(header, found, sizeof found, hipMemcpyHostToDevice, st);
+                if (e != hipSuccess) return fail(GTM_ERR_HIP, "the edges' moves: %s", hipGetErrorString(e));
+            }
+            hipLaunchKernelGGL(k_fit_move_masks, dim3(n_now), dim3(256), (size_t)p.moves.n * S * 4, st, g->number_of_graph_nodes, g->node_index,
+                               g->number_of_graph_node_edges, g->edge_index, g->edge, p.first_example, header, p.moves.n, S, w.move_masks);
+            if (int rc = check_launch("k_fit_move_masks")) return rc;
+        }
+        // the exchange buffers start at zero; the model is kept as it was in case the run gives up
+        hipLaunchKernelGGL(k_fill_u64, dim3(blocks_for((int64_t)d.K * 3 * FITP_SUM_PARTS * FITP_SUM_STRIDE + 1, TPB)), dim3(TPB), 0, st,
+                           (unsigned long long *)w.class_sum, (int64_t)0, 0ull, (int64_t)d.K * 3 * FITP_SUM_PARTS * FITP_SUM_STRIDE + 1);
+        if (int rc = check_launch("fill")) return rc;
+        hipLaunchKernelGGL(k_fill_u64, dim3(blocks_for((int64_t)layers * FITD_PARTS * FITD_STRIDE, TPB)), dim3(TPB), 0, st,
+                           w.coop_arrived, (int64_t)0, 0ull, (int64_t)layers * FITD_PARTS * FITD_STRIDE);
+        if (int rc = check_launch("fill")) return rc;
+        hipLaunchKernelGGL(k_fill_i32, dim3(blocks_for((int64_t)w.coop_words, TPB)), dim3(TPB), 0, st, (int32_t *)w.coop_got,
+                           (int64_t)w.coop_words, 0);
+        if (int rc = check_launch("fill")) return rc;
+        const size_t bank0_bytes = (size_t)d.C * d.LA * d.B * 4, bankm_bytes = (size_t)d.C * d.MC * d.B * 4;
+        const size_t weights_bytes = (size_t)d.K * d.C * 4;
+        hipError_t e = hipMemcpyAsync(w.bank_backup, s->ta_state, bank0_bytes, hipMemcpyDeviceToDevice, st);
+        for (int l = 0; l < layers && e == hipSuccess; ++l)
+            e = hipMemcpyAsync((char *)w.bank_backup + bank0_bytes + (size_t)l * bankm_bytes, s->message_ta_state[l], bankm_bytes,
+                               hipMemcpyDeviceToDevice, st);
+        if (e == hipSuccess) e = hipMemcpyAsync(w.weights_backup, s->clause_weights, weights_bytes, hipMemcpyDeviceToDevice, st);
+        if (e != hipSuccess) return fail(GTM_ERR_HIP, "keeping a copy of the model state: %s", hipGetErrorString(e));
+        void *args[] = {&p};
+        profile_start("k_fit_moves", st);
+        e = hipLaunchCooperativeKernel(kernel, dim3(groups), dim3(FITP_BLOCK), args, (unsigned)lds, st);
+        if (e != hipSuccess) return fail(GTM_ERR_HIP, "cooperative launch of the training kernel: %s", hipGetErrorString(e));
+        profile_stop(st);
+        uint32_t flag = 0;
+        e = hipMemcpyAsync(&flag, p.abort_flag, 4, hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
+        if (e != hipSuccess) return fail(GTM_ERR_HIP, "training kernel: %s", hipGetErrorString(e));
+        if (flag != 0) {
+            e = hipMemcpyAsync(s->ta_state, w.bank_backup, bank0_bytes, hipMemcpyDeviceToDevice, st);
+            for (int l = 0; l < layers && e == hipSuccess; ++l)
+                e = hipMemcpyAsync(s->message_ta_state[l], (char *)w.bank_backup + bank0_bytes + (size_t)l * bankm_bytes, bankm_bytes,
+                                   hipMemcpyDeviceToDevice, st);
+            if (e == hipSuccess) e = hipMemcpyAsync(s->clause_weights, w.weights_backup, weights_bytes, hipMemcpyDeviceToDevice, st);
+            if (e == hipSuccess) e = hipStreamSynchronize(st);
+            if (e != hipSuccess)
+                return fail(GTM_ERR_HIP, "training kernel gave up waiting at a device-wide barrier (%d workgroups) and the "
+                                         "model state could not be restored: %s", groups, hipGetErrorString(e));
+            if (!p.force_abort) return GTM_OK;  // as in fit_persistent: the launches per example take over
+            return fail(GTM_ERR_HIP, "training kernel gave up waiting at a device-wide barrier (%d workgroups); "
+                                     "the model state is as it was before the call", groups);
+        }
+        at += n_now;
+        *examples_done = at;
+        if (chunk_grows && chunk < 2048) chunk *= 2;
+    }
+    *done = true;
+    return GTM_OK;
+}
+
 // `_fit`'s inner loop for a depth-1 model on a data set that has tiles: two
 // launches per example (fit_fused.h).
 int fit_on_tiles(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const gtm_state *s, const TileGeom &tg,
@@ -2962,6 +3191,9 @@ int gtm_fit(const gtm_config *cfg, const gtm_graphs *graphs, const gtm_state *st
         if (tg.ok && tg.slot_words <= 64 && cfg->max_nodes <= 2048) {  // one lane per word of the graph's nodes
             bool done = false;
             int so_far = 0;  // examples that launches which did not give up have trained on
+            if (int rc = fit_moves(d, cfg, graphs, state, tg, w, encoded_Y, first_example, n_examples, first_step, st, &done, &so_far)) return rc;
+            if (done) return GTM_OK;
+            first_example += so_far, n_examples -= so_far, first_step += (uint64_t)so_far, h_n += so_far, h_base += so_far;
             if (int rc = fit_deep_persistent(d, cfg, graphs, state, tg, w, encoded_Y, first_example, n_examples, first_step, st,
                                              &done, &so_far))
                 return rc;

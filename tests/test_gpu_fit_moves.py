@@ -1,0 +1,97 @@
+"""Training with message layers on data sets whose edges are a few moves (k_fit_moves): automata of every bank and the
+weights follow the oracle bit for bit in every layout, and other data sets keep the kernel that walks the edges."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import gtm_oracle as o
+from tests import helpers
+from tests.test_gpu_message_moves import GRID, _graphs
+
+pytestmark = pytest.mark.gpu
+
+CHAIN = [(0, -1), (1, 1)]
+SHAPES = [
+    # name, nodes per graph, moves, hypervector size, model, taken
+    ("tiny_with_loops", [1, 16, 0, 7, 2] * 4, [(0, 0), (1, 3), (0, -2)], 20, dict(classes=2, clauses=33, depth=2, message_size=32, message_bits=3), True),
+    ("chains_of_one_word", [31, 17, 32, 0, 24, 20] * 2, CHAIN, 40, dict(classes=64, clauses=40, depth=3, message_size=96), True),
+    ("ragged_chains", [3, 41, 17, 33, 32, 64, 1, 200], CHAIN, 20, dict(classes=3, clauses=300, depth=4, message_size=64, message_bits=1), True),
+    ("long_chains", [1000, 999, 513, 1], CHAIN, 64, dict(classes=2, clauses=200, depth=2, message_size=512), True),
+    ("longest_rows", [2048, 1025, 2000], CHAIN, 16, dict(classes=2, clauses=60, depth=2, message_size=256), True),
+    ("grid", [841] * 3, GRID, 128, dict(classes=10, clauses=70, depth=3, message_size=288), True),
+    ("grid_of_many_clauses", [841] * 2, GRID, 40, dict(classes=4, clauses=1500, depth=2, message_size=64), True),
+    ("far_moves", [300, 257, 290], [(0, 32), (1, -64), (2, 96), (3, -33), (0, 255), (1, -250), (2, 63), (3, 0)], 33,
+     dict(classes=3, clauses=50, depth=3, message_size=64), True),
+    ("no_edges", [70, 31, 65, 0], [], 20, dict(classes=3, clauses=20, depth=3, message_size=32), False),
+    ("too_many", [90, 84, 70], [(0, d) for d in range(-4, 5)], 20, dict(classes=3, clauses=40, depth=2, message_size=64), False),
+]
+LAYOUTS = {
+    "as_it_comes": {},
+    "in_memory": {"GTM_FIT_DEEP_IN_MEMORY": "1"},
+    "7_a_workgroup_dealt_every_3_examples": {"GTM_FIT_DEEP_CLAUSES_PER_GROUP": "7", "GTM_FIT_DEEP_CHUNK": "3"},
+    "40_a_workgroup_in_memory": {"GTM_FIT_DEEP_CLAUSES_PER_GROUP": "40", "GTM_FIT_DEEP_IN_MEMORY": "1"},
+    "17_a_workgroup": {"GTM_FIT_DEEP_CLAUSES_PER_GROUP": "17"},
+}
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: s[0])
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("boost,max_included,state_bits", [(1, None, 8), (0, 9, 5), (1, None, 12)])
+def test_training_by_moves(shape, layout, boost, max_included, state_bits, tune):
+    from graphtsetlinmachine_amd import _abi
+    from tests.gpu_harness import Device
+
+    name, sizes, moves, hv, sizing, taken = shape
+    for switch, value in LAYOUTS[layout].items():
+        tune(switch, value)
+    tune("GTM_NO_SMALL_FIT", "1")
+    graphs = _graphs(np.array(sizes), moves, seed=len(name), hv=hv)
+    depth = sizing["depth"]
+    cfg = helpers.oracle_config(graphs, T=30, boost=boost, max_included=max_included, state_bits=state_bits, **sizing)
+    model = helpers.random_model(5, cfg, depth, s=(3.0, 2.0, 1.5, 1.2)[:depth], include_density=0.02, message_density=0.02)
+    dev = Device(model, graphs)
+    assert dev.build_tiles()
+    G = graphs.number_of_graphs
+    Y = o.encode_labels(np.random.default_rng(1).integers(0, cfg.classes, size=G), cfg.classes, cfg.threshold)
+    kernel, launches, total = ctypes.c_char_p(), ctypes.c_int32(), ctypes.c_double()
+    for epoch in range(2):
+        o.fit(model, graphs, Y)
+        _abi.call("gtm_profile_enable", 1)
+        dev.fit(Y, 0, G // 3, epoch * G)  # the restart from memory is covered, too
+        dev.fit(Y, G // 3, G - G // 3, epoch * G + G // 3)
+        _abi.call("gtm_profile_read", ctypes.byref(kernel), ctypes.byref(launches), ctypes.byref(total))
+        _abi.call("gtm_profile_enable", 0)
+        assert (kernel.value == b"k_fit_moves") == taken, kernel.value
+        ta, banks, w = dev.download()
+        assert np.array_equal(w, model.clause_weights), "weights after epoch %d" % epoch
+        assert np.array_equal(ta, model.ta_state), "layer-0 automata after epoch %d" % epoch
+        for layer in range(depth - 1):
+            assert np.array_equal(banks[layer], model.message_ta_state[layer]), "bank %d epoch %d" % (layer, epoch)
+
+
+@pytest.mark.parametrize("in_memory", [False, True])
+def test_giving_up_leaves_the_model_as_it_was(in_memory, tune):
+    from graphtsetlinmachine_amd import _abi
+    from tests.gpu_harness import Device
+
+    if in_memory:
+        tune("GTM_FIT_DEEP_IN_MEMORY", "1")
+    graphs = _graphs(np.array([100, 90, 110]), CHAIN, seed=2)
+    cfg = helpers.oracle_config(graphs, classes=3, clauses=40, depth=3, message_size=64, T=30)
+    model = helpers.random_model(5, cfg, 3, s=(3.0, 2.0, 1.5), include_density=0.02, message_density=0.02)
+    dev = Device(model, graphs)
+    assert dev.build_tiles()
+    Y = o.encode_labels(np.arange(3) % 3, 3, cfg.threshold)
+    tune("GTM_FIT_SPIN_LIMIT", "abort")
+    with pytest.raises(_abi.GtmError, match="gave up waiting.*as it was before the call"):
+        dev.fit(Y, 0, 3, 0)
+    tune("GTM_FIT_SPIN_LIMIT", None)
+    for trained in (False, True):
+        if trained:
+            o.fit(model, graphs, Y)
+            dev.fit(Y, 0, 3, 0)
+        ta, banks, w = dev.download()
+        assert np.array_equal(w, model.clause_weights) and np.array_equal(ta, model.ta_state)
+        assert all(np.array_equal(a, b) for a, b in zip(banks, model.message_ta_state))
