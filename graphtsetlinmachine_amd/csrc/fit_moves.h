@@ -9,19 +9,20 @@
 //     ends: no edge is staged or walked;
 //   - clauses are lists of rows per bank (fit_lists.h), remade when an include plane changes.  A message literal's
 //     row is the received row, negated literals their complements: lists are octets of one sign;
-//   - with at most 1,024 automaton words a workgroup, a thread (or, up to 256, a quad of lanes, each with a quarter of the
-//     Type I bits) keeps a word's planes in registers for the whole run (REGS); else they stay in memory and the words
+//   - where a clause's words fit its share of the workgroup's 16 waves, its automata live in the lanes' registers for the
+//     whole run and every one of its waves decides its feedback for itself (REGS); else they stay in memory and the words
 //     of the clauses that get feedback are shared out;
 //   - random words of the gates and of the next node pick are drawn, and the words of the picked nodes fetched, while
 //     the class sums travel.
 // Bound by the two or three device-wide exchanges per example (few clauses), or by the generator calls of the Type I
 // feedback and the copies of the received rows (thousands of clauses).  us per example, edges walked and clauses' include
-// planes walked (fit_deep_persistent.h) -> here: 1,000-node chains, 200 clauses 20.5 -> 14.1; chains of 10 to 40 nodes, 333 clauses,
-// three layers 26 -> 17.8; 324-node grids, 2,000 clauses, three layers 54 -> 24.7; 841-node grids, 8,000 clauses, three layers
-// 170 -> 70, of which the slowest workgroup's evaluation, for which all others waited, was more than half.
+// planes walked (fit_deep_persistent.h) -> here: 1,000-node chains, 200 clauses 20.5 -> 11.8; chains of 10 to 40 nodes, 333 clauses,
+// three layers 26 -> 15.9; 324-node grids, 2,000 clauses, three layers 54 -> 22.4; 841-node grids, 8,000 clauses, three layers
+// 170 -> 64, of which the slowest workgroup's evaluation, for which all others waited, was more than half.
 #pragma once
 
 constexpr int FITM_MAX_CLASSES = 64;
+constexpr int FITM_REGS_CLASSES = 63;  // lane 63 draws for the node pick
 constexpr int FITM_CHUNK = 4096;  // examples of a launch, for which the moves' masks are kept
 
 struct FitMovesParams {
@@ -63,7 +64,7 @@ inline size_t fit_moves_lds_words(bool regs, bool rows_lds, int depth, int own, 
                                   int list0, int listm, int n_moves) {
     const size_t o = (size_t)own, words = (size_t)LA + (size_t)(depth - 1) * MC;
     return (size_t)M * S + (rows_lds ? 2 * (size_t)rows_words : 0) + (regs ? o * (list0 + (depth - 1) * listm) / 2 : 0) + o * S +
-           2 * (size_t)n_moves * S + o * words + 3 * o * K + 4 * o + 4 * o * depth + 6 * o + o * n_moves * MB + o * (MC / 2) + (regs ? o * LA : 0);
+           2 * (size_t)n_moves * S + o * words + 3 * o * K + 4 * o + 4 * o * depth + 6 * o + o * n_moves * MB + o * (MC / 2);
 }
 
 // The (type, offset) pairs of a run's edges -> header (zero on entry; as k_edge_moves).  One workgroup per example.
@@ -178,7 +179,7 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
     __shared__ int32_t votes[64], sums[64], labels[2][64];
     __shared__ int go_on, n_own_shared, n_busy, n_stale, next_unit;
     constexpr int WAVES = FITP_BLOCK / 64, POLL = WAVES - 1;  // the last wave announces, adds and polls
-    const int tid = threadIdx.x, lane = tid & 63;
+    int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int G = (int)gridDim.x, g = (int)blockIdx.x, own_max = p.clauses_per_group;
     const int LA = p.LA, MC = p.MC, MW = p.MW, M = p.M, B = EXACT ? MAXB : p.B, K = p.K, S = p.S, depth = p.depth, L = depth - 1, NM = p.moves.n;
@@ -209,7 +210,6 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
     int32_t *own_id = (int32_t *)(busy_of + own_max);                   // [own] the clause in a slot
     uint32_t *send_row = (uint32_t *)(own_id + own_max);                // [own][NM][MB] rows that a clause sends to along a move
     uint32_t *mlit = send_row + (size_t)own_max * NM * p.MB;            // [own][MW] what the picked node received in the last layer
-    uint32_t *x_ahead = mlit + (size_t)own_max * MW;                    // REGS: [own][LA] literal words of the picked node
 
     if (tid == 0) {
         int n = 0;
@@ -247,38 +247,43 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
         else
             return p.lists + ((int64_t)g * own_max * list_entries + at);
     };
-    // one wave: the list of a slot's bank from its include words
+    // one wave: the list of a slot's bank from its include words, a lane per word: as many turns as the fullest word has literals
     auto make_list = [&](int cl, int bank) {
         uint16_t *list = list_of(cl, bank);
         const uint32_t *from = inc + (size_t)cl * words_all + (bank == 0 ? 0 : LA + (bank - 1) * MC);
-        int n = 0, included = 0;
-        for (int half = 0; half < (bank == 0 ? 1 : 2); ++half) {
-            const int words = bank == 0 ? LA : MW, first = half ? 0x8000 : 0, was = n;
-            if (bank == 0) {
-                if (lane == 0) list[0] = (uint16_t)(p.literals + own_id[cl] % p.n_types);
-                n = 1;
-            }
-            for (int w0 = 0; w0 < words; w0 += 64) {
-                uint32_t mine = w0 + lane < words ? from[half * MW + w0 + lane] : 0u;
-                if (bank == 0 && w0 + lane == LA - 1) mine &= p.filter;
-                n = fitl_append(mine, min(64, words - w0), first + 32 * w0, list, 0x7FFFFFFF, n, lane);
-            }
-            included += n - was;
-            // the last octet is filled up with an entry of its own sign
-            const int full = (n + 7) & ~7;
-            if (n > was && n < full) {
-                if constexpr (REGS) {
-                    fitp_wave_lds_sync();
-                } else {
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-                }
-                const uint16_t again = list[was];
-                if (n + lane < full) list[n + lane] = again;
-            }
-            n = full;
+        int n = 0, included = 0;  // n: entries so far, whole octets before the negated half
+        if (bank == 0) {
+            if (lane == 0) list[0] = (uint16_t)(p.literals + own_id[cl] % p.n_types);
+            n = 1;
         }
-        if (lane == 0) octets_of[cl * depth + bank] = n >> 3, incl_of[cl * depth + bank] = included - (bank == 0), stale[cl * depth + bank] = 0u;
+        const int words = bank == 0 ? LA : MC, half = bank == 0 ? LA : MW;
+        int again = bank == 0 ? p.literals + own_id[cl] % p.n_types : -1;  // an entry of the sign at hand, to fill an octet up with
+        auto fill_up = [&]() {
+            const int full = (n + 7) & ~7;
+            if (n + lane < full) list[n + lane] = (uint16_t)again;
+            n = full;
+        };
+        for (int w0 = 0; w0 < words;) {
+            const int w1 = min(words, w0 < half ? min(half, w0 + 64) : w0 + 64);  // (a pass holds words of one sign)
+            uint32_t mine = w0 + lane < w1 ? from[w0 + lane] : 0u;
+            if (bank == 0 && w0 + lane == LA - 1) mine &= p.filter;
+            const int first = w0 < half ? 32 * w0 : 0x8000 | (32 * (w0 - half)), own = __popc(mine), up_to = fitl_sum_up_to(own);
+            const unsigned long long some = __ballot(mine != 0u);
+            if (some != 0ull) {
+                const int at = __ffsll((long long)some) - 1;
+                if (again < 0) again = first + 32 * at + __builtin_ctz(__builtin_amdgcn_readlane(mine, at));
+                uint16_t *to = list + (n + up_to - own);
+                for (uint32_t m = mine; m; m &= m - 1) *to++ = (uint16_t)(first + 32 * lane + __builtin_ctz(m));
+                const int more = __builtin_amdgcn_readlane(up_to, 63);
+                n += more, included += more;
+            }
+            w0 = w1;
+            if (w0 == half || w0 == words) {
+                fill_up();
+                again = -1;
+            }
+        }
+        if (lane == 0) octets_of[cl * depth + bank] = n >> 3, incl_of[cl * depth + bank] = included, stale[cl * depth + bank] = 0u;
     };
 
     // own state -> LDS and registers
@@ -303,22 +308,56 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
         return philox4x32_10((uint32_t)own_id[cl], 0u, step, GTM_TAG_CLAUSE_NODE, p.k0, p.k1).v[0];
     };
     for (int cl = tid; cl < n_own; cl += FITP_BLOCK) pick_of[cl] = draw_pick(cl, p.first_step);
-    // REGS: the automaton word of this thread, or of its quad
-    const int quad_log = REGS && own_max * words_all * 4 <= FITP_BLOCK ? 2 : 0;
-    const int my_word = tid >> quad_log, my_cl = my_word / words_all, my_w = my_word - my_cl * words_all;
-    const bool has_word = REGS && my_word < n_own * words_all;
-    const int my_bank = my_w < LA ? 0 : 1 + (my_w - LA) / MC, my_wl = my_w < LA ? my_w : (my_w - LA) % MC;
-    const uint32_t my_threshold = threshold_of(my_bank);
-    uint32_t planes[MAXB] = {};
-    if (has_word) {
-        const uint32_t *from = planes_in_memory(own_id[my_cl], my_bank, my_wl);
+    int parts_log = 0;  // waves that share a clause
+    while ((2 << parts_log) * own_max <= WAVES) ++parts_log;
+    const int parts = 1 << parts_log, part = wave & (parts - 1);
+    const int wave_cl = wave >> parts_log;  // the wave's clause, where a workgroup has at most as many clauses as waves
+    // REGS: a lane keeps one automaton word of the wave's clause, or two; or four lanes keep one, each drawing a quarter of its
+    // Type I bits.  What the decisions take, every wave of the clause keeps as well: lane k the weight of class k and
+    // its random words, lane 63 the one of the next node pick.
+    const bool owns = REGS && wave_cl < n_own;
+    const int clause_lanes = 64 << parts_log, quad_log = words_all * 4 <= clause_lanes ? 2 : 0;
+    const bool two_words = words_all > clause_lanes;
+    struct Place {
+        int w, bank, wl;
+        bool there;
+    };
+    auto place_of = [&](int r) {
+        Place at;
+        at.w = (((part << 6) | lane) >> quad_log) + r * clause_lanes;
+        at.there = owns && at.w < words_all;
+        at.bank = 0, at.wl = at.w;
+        if (at.w >= LA) {
+            at.bank = 1, at.wl = at.w - LA;
+            while (at.wl >= MC) at.wl -= MC, ++at.bank;
+        }
+        return at;
+    };
+    const int my_id = owns ? own_id[wave_cl] : 0;
+    uint32_t planes[2][MAXB] = {};
+    int32_t weight = 0;
+    philox_out drawn = {};
+    auto draw = [&](uint32_t step) {
+        const bool pick = lane == 63;
+        drawn = philox4x32_10((uint32_t)my_id, pick ? 0u : (uint32_t)lane, pick ? step + 1u : step,
+                              pick ? (uint32_t)GTM_TAG_CLAUSE_NODE : (uint32_t)GTM_TAG_CLAUSE_UPDATES, p.k0, p.k1);
+    };
+    if (owns) {
 #pragma unroll
-        for (int b = 0; b < MAXB; ++b)
-            if (EXACT || b < B) planes[b] = from[b];
+        for (int r = 0; r < 2; ++r) {
+            const Place at = place_of(r);
+            if (!at.there || (r == 1 && !two_words)) continue;
+            const uint32_t *from = planes_in_memory(my_id, at.bank, at.wl);
+#pragma unroll
+            for (int b = 0; b < MAXB; ++b)
+                if (EXACT || b < B) planes[r][b] = from[b];
+        }
+        if (lane < K) weight = p.weights[(int64_t)lane * p.C + my_id];
+        draw(p.first_step - 1u);  // (the pick of the first step)
     }
-    fits_word<MAXB, EXACT> word(planes, B);
-    // the (clause, class) pair that this thread decides first
-    const int pair_cl = tid / K, pair_k = tid - pair_cl * K;
+    fits_word<MAXB, EXACT> word0(planes[0], B), word1(planes[1], B);
+    // the (clause, class) pair that this thread decides first, and the word of the listed clauses that it updates first (not REGS)
+    const int pair_cl = tid / K, pair_k = tid - pair_cl * K, my_cl = tid / words_all, my_w = tid - my_cl * words_all;
 
     int n_now = (int)p.n_nodes[p.first_example], n_next = (int)p.n_nodes[min(p.first_example + 1, last)];
     uint32_t base_now = p.node_index[p.first_example], base_next = p.node_index[min(p.first_example + 1, last)];
@@ -334,9 +373,6 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
     if (tid < K) labels[0][tid] = p.encoded_Y[(int64_t)p.first_example * K + tid];
     __syncthreads();
     for (int u = wave; u < n_own * depth; u += WAVES) make_list(u / depth, u % depth);
-    int parts_log = 0;  // waves that share a clause
-    while ((2 << parts_log) * own_max <= WAVES) ++parts_log;
-    const int parts = 1 << parts_log;
     if (parts > 1)
         for (int i = tid; i < n_own * S; i += FITP_BLOCK) truth[i] = 0xFFFFFFFFu;
     __builtin_amdgcn_s_waitcnt(FITP_WAIT_VMEM);
@@ -346,7 +382,13 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
     FitRowLoader loader{};
     int loader_words = 0;
     const uint32_t *sizes = lane & 1 ? p.node_index : p.n_nodes;  // (a value per lane: nothing waits for it before it is used)
-    const int place = 2 * (lane & ((1 << lg) - 1));
+    int place = 2 * (lane & ((1 << lg) - 1));
+    // Per-lane addresses are worked out anew in every phase: kept over the whole loop, as the compiler would, sixty of them were
+    // spilled to memory and fetched back one by one on the step's longest path (14.1 -> 13.7 us per example on the chains).
+    auto refresh = [&]() {
+        asm volatile("" : "+v"(tid));
+        lane = tid & 63, place = 2 * (lane & ((1 << lg) - 1));
+    };
     int row_log = 3;  // 2^row_log >= S lanes send a row
     while ((1 << row_log) < S) ++row_log;
     const int by_moves = NM > 0 ? (65536 + NM - 1) / NM : 0;
@@ -357,14 +399,15 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
 
     // what a wave does with a clause on the rows of layer `bank` (0: the graph's literals); `last_layer`: node and votes as well
     auto pick_and_vote = [&](int cl, uint2 v) {
-        const int node = n_now > 0 ? fitl_pick_node(v, pick_of[cl], lane) : -1;
+        const uint32_t random = REGS ? (uint32_t)__builtin_amdgcn_readlane(drawn.v[0], 63) : pick_of[cl];
+        const int node = n_now > 0 ? fitl_pick_node(v, random, lane) : -1;
         const bool fired = n_now == 0 || node >= 0;  // (the reference's arithmetic for a graph without nodes, kernels.py:289-295)
         if (lane == 0) {
             int included = 0;
             for (int b = 0; b < depth; ++b) included += incl_of[cl * depth + b];
             node_of[cl] = node, learns_of[cl] = node >= 0 && included <= p.max_included;
         }
-        if (fired && lane < K) atomicAdd(&votes[lane], wts[cl * K + lane]);
+        if (fired && lane < K) atomicAdd(&votes[lane], REGS ? weight : wts[cl * K + lane]);
     };
     auto truth_row = [&](int cl) {
         const uint2 v = *reinterpret_cast<const uint2 *>(truth + cl * S + (place < S ? place : 0));
@@ -404,8 +447,7 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
     };
     auto evaluate_all = [&](int bank, int i) {
         if (own_max <= WAVES) {
-            const int cl = wave >> parts_log;
-            if (cl < n_own) evaluate(cl, wave & (parts - 1), bank, i);
+            if (wave_cl < n_own) evaluate(wave_cl, part, bank, i);
         } else {  // (clauses differ a lot in what they cost: the waves take them from a queue)
             for (;;) {
                 int u = 0;
@@ -420,6 +462,7 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
     for (int i = 0; i < p.n_examples; ++i) {
         const uint32_t step = p.first_step + (uint32_t)i;
         const int ex = p.first_example + i;
+        refresh();
         uint32_t *got_now = p.got + (size_t)slot * L * layer_words, *got_next = p.got + (size_t)(slot == 2 ? 0 : slot + 1) * L * layer_words;
         // ---- 1. layer 0 (K1)
         evaluate_all(0, i);
@@ -430,6 +473,7 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
         // ---- 2. the message layers
         for (int l = 0; l < L; ++l) {
             lds_barrier();  // the truth rows are complete, and nobody reads the received rows of the layer before
+            refresh();
             uint32_t *got_l = got_now + (size_t)l * layer_words;
             if (tid == 0) next_unit = 0;
             // a. what the own clauses make the nodes receive: their truth rows, shifted, where an edge of the move ends
@@ -449,6 +493,7 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
             __builtin_amdgcn_s_waitcnt(FITP_WAIT_VMEM);  // the ORs have been carried out where every workgroup sees them
             asm volatile("" ::: "memory");
             lds_barrier();
+            refresh();
             unsigned long long *arrived = p.arrived + (size_t)l * FITD_PARTS * FITD_STRIDE;
             if (wave == POLL) {
                 if (lane == 0)
@@ -494,6 +539,7 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
                 break;
             }
             // b. the received rows -> LDS
+            refresh();
             {
                 const unsigned long long *from = (const unsigned long long *)got_l;
                 unsigned long long *to = (unsigned long long *)mrows;
@@ -510,6 +556,7 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
                 }
             }
             lds_barrier();
+            refresh();
             // c. K2 for the own clauses; what the nodes of this group's share received, node-major, for the feedback
             evaluate_all(l + 1, i);
             if (l < L - 1) {
@@ -528,9 +575,9 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
         if (!alive) break;
         if (parts > 1) {  // ---- 3. node pick (K7) and votes (K6) of clauses that several waves share
             lds_barrier();
-            if ((wave & (parts - 1)) == 0 && (wave >> parts_log) < n_own) {
-                const uint2 v = truth_row(wave >> parts_log);
-                pick_and_vote(wave >> parts_log, lane < (1 << lg) ? v : make_uint2(0u, 0u));
+            if (part == 0 && wave_cl < n_own) {
+                const uint2 v = truth_row(wave_cl);
+                pick_and_vote(wave_cl, lane < (1 << lg) ? v : make_uint2(0u, 0u));
             }
         }
         // the next slot's share is cleared (and the node-major words are out) before this group arrives
@@ -539,6 +586,7 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
         lds_barrier();
 
         // ---- 4. class sums across the device (the protocol of fit_persistent.h); meanwhile all that does not need them
+        refresh();
         unsigned long long *slot_sum = p.class_sum + (size_t)slot * K * FITP_SUM_PARTS * FITP_SUM_STRIDE;
         if (wave == POLL) {
             if (lane < K) {
@@ -557,18 +605,12 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
                 const unsigned long long got = __ballot(r < M && ((mrows[r * S + (node >> 5)] >> (node & 31)) & 1u));
                 if (lane < 2 && 2 * j + lane < MW) mlit[cl * MW + 2 * j + lane] = (uint32_t)(got >> (32 * lane));
             }
-            if constexpr (REGS)
-                for (int cl = wave; cl < n_own; cl += POLL) {
-                    const int node = __builtin_amdgcn_readfirstlane(node_of[cl]);
-                    if (node < 0) continue;
-                    for (int w0 = 0; w0 < LA; w0 += 64)
-                        if (w0 + lane < LA) fitp_load_to_lds(p.X + ((int64_t)base_now + node) * LA + w0 + lane, x_ahead + cl * LA + w0);
-                }
             if (parts > 1)
                 for (int at = tid; at < n_own * S; at += LOADERS) truth[at] = 0xFFFFFFFFu;
-            for (int at = tid; at < 2 * n_own; at += LOADERS) type1[at] = 0u, type2[at] = 0u, busy_of[at >> 1] = 0u;
             if (tid == 0) n_busy = 0, n_stale = 0, next_unit = 0;
-            for (int j = tid; j < n_own * (K + 1); j += LOADERS) {
+            if constexpr (!REGS)
+                for (int at = tid; at < 2 * n_own; at += LOADERS) type1[at] = 0u, type2[at] = 0u, busy_of[at >> 1] = 0u;
+            for (int j = tid; !REGS && j < n_own * (K + 1); j += LOADERS) {
                 if (j >= n_own * K) {
                     pick_of[j - n_own * K] = draw_pick(j - n_own * K, step + 1u);
                     continue;
@@ -576,6 +618,19 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
                 const int cl = j == tid ? pair_cl : j / K, k = j - cl * K;
                 const philox_out r = philox4x32_10((uint32_t)own_id[cl], (uint32_t)k, step, GTM_TAG_CLAUSE_UPDATES, p.k0, p.k1);
                 gate[2 * j] = r.v[0], gate[2 * j + 1] = r.v[1];
+            }
+        }
+        uint32_t x0 = 0u, x1 = 0u;  // REGS: the literal words of the picked node for this lane's words
+        if constexpr (REGS) {
+            if (owns) {
+                const int node = __builtin_amdgcn_readfirstlane(node_of[wave_cl]);
+                if (node >= 0) {
+                    const uint32_t *from = p.X + ((int64_t)base_now + node) * LA;
+                    const int w = ((part << 6) | lane) >> quad_log;
+                    if (w < LA) x0 = from[w];
+                    if (w + clause_lanes < LA) x1 = from[w + clause_lanes];
+                }
+                draw(step);
             }
         }
         fn = fit_graph_slot(p.tg, min(ex + 1, last), n_next);
@@ -611,34 +666,40 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
         if (!go_on) break;
 
         // ---- 5. feedback decisions (K8) and weights
-        for (int j = tid; j < n_own * K; j += FITP_BLOCK) {
-            const int cl = j == tid ? pair_cl : j / K, k = j == tid ? pair_k : j - cl * K;
+        refresh();
+        auto decide = [&](int k, int32_t &w, uint32_t r0, uint32_t r1, bool fired) {
             int cs = sums[k];
             cs = cs > p.T ? p.T : (cs < -p.T ? -p.T : cs);
             const int y = labels[i & 1][k];
             const int target = 1 - 2 * (cs > y);
-            int w = wts[j];
             const int sign = w >= 0 ? 1 : -1;
             int err = y - cs;
             err = err < 0 ? -err : err;
-            const bool skip = (target == -1 && (uint64_t)gate[2 * j] >= p.q_thr) ||
-                              ((uint64_t)gate[2 * j + 1] * (uint64_t)(2 * (int64_t)p.T) >= ((uint64_t)err << 32));
+            const bool skip = (target == -1 && (uint64_t)r0 >= p.q_thr) || ((uint64_t)r1 * (uint64_t)(2 * (int64_t)p.T) >= ((uint64_t)err << 32));
             const int u = skip ? 0 : target * sign;
-            const bool fired = node_of[cl] >= 0;
             if (u > 0 && fired && (w < 0 ? -(int64_t)w : (int64_t)w) < 2147483647) {
-                wts[j] = w + sign;
+                w += sign;
             } else if (u < 0 && fired) {
                 w -= sign;
                 if (p.negative == 0 && w < 1) w = 1;
-                wts[j] = w;
             }
-            if (u == 0) continue;
-            atomicOr(&type1[(u > 0 ? 0 : 2 * own_max) + 2 * cl + (k >> 5)], 1u << (k & 31));
-            if (!REGS && atomicOr(&busy_of[cl], 1u) == 0u) busy_list[atomicAdd(&n_busy, 1)] = cl;
+            return u;
+        };
+        if constexpr (!REGS) {
+            for (int j = tid; j < n_own * K; j += FITP_BLOCK) {
+                const int cl = j == tid ? pair_cl : j / K, k = j == tid ? pair_k : j - cl * K;
+                int32_t w = wts[j];
+                const int u = decide(k, w, gate[2 * j], gate[2 * j + 1], node_of[cl] >= 0);
+                if (u == 0) continue;
+                wts[j] = w;
+                atomicOr(&type1[(u > 0 ? 0 : 2 * own_max) + 2 * cl + (k >> 5)], 1u << (k & 31));
+                if (atomicOr(&busy_of[cl], 1u) == 0u) busy_list[atomicAdd(&n_busy, 1)] = cl;
+            }
+            lds_barrier();
         }
-        lds_barrier();
 
         // ---- 6. Type I / II feedback on every bank (K9, K10)
+        refresh();
         // the literal word of a clause's picked node (kernels.py:592-615: the negated half of a message is the complement)
         auto message_word = [&](int cl, int node, int bank, int wl) {
             const int w = wl < MW ? wl : wl - MW;
@@ -649,51 +710,64 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
                 v = fitd_load(&p.vec[((size_t)(bank - 1) * p.max_nodes + node) * MW + w]);
             return wl < MW ? v : ~v;
         };
-        auto changed = [&](int cl, int bank) {
-            if (atomicOr(&stale[cl * depth + bank], 1u) == 0u) stale_list[atomicAdd(&n_stale, 1)] = cl * depth + bank;
-        };
         if constexpr (REGS) {
-            if (has_word) {
-                const uint32_t pos[2] = {type1[2 * my_cl], type1[2 * my_cl + 1]}, neg[2] = {type2[2 * my_cl], type2[2 * my_cl + 1]};
-                if ((pos[0] | pos[1] | neg[0] | neg[1]) != 0u) {
-                    const int node = node_of[my_cl];
-                    const bool fired = node >= 0, learns = learns_of[my_cl] != 0;
-                    uint32_t x = 0u;
-                    if (fired) {
-                        if (my_bank == 0)
-                            x = x_ahead[my_cl * LA + my_wl];
-                        else
-                            x = message_word(my_cl, node, my_bank, my_wl);
-                    }
-                    const uint32_t was = word.top(), c = (uint32_t)own_id[my_cl];
-#pragma unroll
-                    for (int h = 0; h < 2; ++h)
-                        for (uint32_t m = pos[h] | neg[h]; m; m &= m - 1) {
-                            const int k = 32 * h + __builtin_ctz(m);
+            if (owns) {
+                const int node = __builtin_amdgcn_readfirstlane(node_of[wave_cl]);
+                const bool fired = node >= 0;
+                const int u = lane < K ? decide(lane, weight, drawn.v[0], drawn.v[1], fired) : 0;
+                const unsigned long long pos = __ballot(u > 0), neg = __ballot(u < 0);
+                if ((pos | neg) != 0ull) {
+                    const bool learns = __builtin_amdgcn_readfirstlane(learns_of[wave_cl]) != 0;
+                    const Place at0 = place_of(0);
+                    if (fired && at0.there && at0.bank != 0) x0 = message_word(wave_cl, node, at0.bank, at0.wl);
+                    const uint32_t was0 = word0.top();
+                    auto update = [&](fits_word<MAXB, EXACT> &word, const Place &at, uint32_t x, uint32_t threshold) {
+                        for (unsigned long long m = pos | neg; m != 0ull; m &= m - 1) {
+                            const int k = __ffsll((long long)m) - 1;
                             uint32_t up = fired ? ~x & ~word.top() : 0u, down = 0u;
-                            if ((pos[h] >> (k & 31)) & 1u) {
+                            if ((pos >> k) & 1ull) {
                                 uint32_t fb;
                                 if (quad_log == 2) {
-                                    fb = fitl_feedback_byte(p.k0, p.k1, c, (uint32_t)my_wl, (uint32_t)tid & 3u, step, (uint32_t)my_bank, (uint32_t)k,
-                                                            my_threshold)
-                                         << (8 * (tid & 3));
+                                    fb = fitl_feedback_byte(p.k0, p.k1, (uint32_t)my_id, (uint32_t)at.wl, (uint32_t)lane & 3u, step, (uint32_t)at.bank,
+                                                            (uint32_t)k, threshold)
+                                         << (8 * (lane & 3));
                                     fb |= (uint32_t)__builtin_amdgcn_mov_dpp((int)fb, 0xB1, 0xF, 0xF, true);  // lanes of a quad: [1, 0, 3, 2]
                                     fb |= (uint32_t)__builtin_amdgcn_mov_dpp((int)fb, 0x4E, 0xF, 0xF, true);  // [2, 3, 0, 1]
                                 } else {
-                                    fb = gtm_feedback_bits(p.k0, p.k1, c, (uint32_t)my_wl, step, (uint32_t)my_bank, (uint32_t)k, my_threshold);
+                                    fb = gtm_feedback_bits(p.k0, p.k1, (uint32_t)my_id, (uint32_t)at.wl, step, (uint32_t)at.bank, (uint32_t)k, threshold);
                                 }
                                 up = learns ? (p.boost == 1 ? x : x & ~fb) : 0u;
                                 down = learns ? ~x & fb : fb;
                             }
                             word.count(up, down);
                         }
-                    if (word.top() != was && (tid & ((1 << quad_log) - 1)) == 0) {
-                        inc[my_word] = word.top();
-                        changed(my_cl, my_bank);
+                    };
+                    auto note = [&](const Place &at, uint32_t top) {
+                        inc[wave_cl * words_all + at.w] = top;
+                        stale[wave_cl * depth + at.bank] = 1u;
+                        n_stale = 1;
+                    };
+                    if (at0.there) {
+                        update(word0, at0, x0, threshold_of(at0.bank));
+                        if (word0.top() != was0) note(at0, word0.top());
+                    }
+                    if (two_words) {
+                        const Place at1 = place_of(1);
+                        if (at1.there) {
+                            if (fired && at1.bank != 0) x1 = message_word(wave_cl, node, at1.bank, at1.wl);
+                            const uint32_t was1 = word1.top();
+                            update(word1, at1, x1, threshold_of(at1.bank));
+                            if (word1.top() != was1) note(at1, word1.top());
+                        }
                     }
                 }
             }
             lds_barrier();
+            if (n_stale != 0) {
+                for (int bank = part; owns && bank < depth; bank += parts)
+                    if (__builtin_amdgcn_readfirstlane(stale[wave_cl * depth + bank]) != 0u) make_list(wave_cl, bank);
+                lds_barrier();
+            }
         } else {
             // the words of the clauses that get feedback, shared out; a thread's next word is fetched while it works on one
             struct Fetched {
@@ -753,19 +827,17 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
                 state.store(planes_in_memory(own_id[now.cl], now.bank, now.wl));
                 if (state.top() != was) {
                     inc[now.cl * words_all + now.w] = state.top();
-                    changed(now.cl, now.bank);
+                    if (atomicOr(&stale[now.cl * depth + now.bank], 1u) == 0u) stale_list[atomicAdd(&n_stale, 1)] = now.cl * depth + now.bank;
                 }
                 now = next;
             }
             __syncthreads();
-        }
-        const int n_changed = n_stale;
-        if (n_changed != 0) {
-            for (int u = wave; u < n_changed; u += WAVES) make_list(stale_list[u] / depth, stale_list[u] % depth);
-            if constexpr (REGS)
-                lds_barrier();
-            else
+            refresh();
+            const int n_changed = n_stale;
+            if (n_changed != 0) {
+                for (int u = wave; u < n_changed; u += WAVES) make_list(stale_list[u] / depth, stale_list[u] % depth);
                 __syncthreads();
+            }
         }
         slot = slot == 2 ? 0 : slot + 1;
         fg = fn;
@@ -776,9 +848,17 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
     __builtin_amdgcn_s_waitcnt(FITP_WAIT_VMEM);  // no load into LDS is left in flight when the group ends
     lds_barrier();
     // own state -> global memory (also after an abort: the host puts the model back as it was)
-    if (has_word && (tid & ((1 << quad_log) - 1)) == 0) word.store(planes_in_memory(own_id[my_cl], my_bank, my_wl));
-    for (int i = tid; i < n_own * K; i += FITP_BLOCK) {
-        const int cl = i / K, k = i - cl * K;
-        p.weights[(int64_t)k * p.C + own_id[cl]] = wts[i];
+    if constexpr (REGS) {
+        if (owns) {
+            const Place at0 = place_of(0), at1 = place_of(1);
+            if (at0.there && (lane & ((1 << quad_log) - 1)) == 0) word0.store(planes_in_memory(my_id, at0.bank, at0.wl));
+            if (two_words && at1.there) word1.store(planes_in_memory(my_id, at1.bank, at1.wl));
+            if (part == 0 && lane < K) p.weights[(int64_t)lane * p.C + my_id] = weight;
+        }
+    } else {
+        for (int i = tid; i < n_own * K; i += FITP_BLOCK) {
+            const int cl = i / K, k = i - cl * K;
+            p.weights[(int64_t)k * p.C + own_id[cl]] = wts[i];
+        }
     }
 }

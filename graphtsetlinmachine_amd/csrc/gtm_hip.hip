@@ -2655,7 +2655,9 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
     };
     const bool in_memory = tune(T_FIT_DEEP_IN_MEMORY) != nullptr;  // (tests)
     auto layout_of = [&](int n_moves) {  // 0: registers and staged rows, 1: registers, 2: memory, -1: none
-        if (!in_memory && per_group * words <= FITP_BLOCK) {
+        int parts = 1;  // waves of a clause
+        while (2 * parts * per_group <= FITP_BLOCK / 64) parts *= 2;
+        if (!in_memory && per_group <= FITP_BLOCK / 64 && words <= 2 * 64 * parts && d.K <= FITM_REGS_CLASSES) {
             if (lds_bytes(true, true, n_moves) <= lds_limit) return 0;
             if (lds_bytes(true, false, n_moves) <= lds_limit) return 1;
         }
