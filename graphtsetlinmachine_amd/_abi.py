@@ -117,6 +117,7 @@ PROTOTYPES = {
     "gtm_build_tiles": (C.c_int, [_CFG, _GR, _P, _P]),
     "gtm_moves_bytes": (_SZ, [_CFG, _GR]),
     "gtm_build_moves": (C.c_int, [_CFG, _GR, _P, _P]),
+    "gtm_score_needs_tiles": (C.c_int, [_CFG, _GR]),
     "gtm_score_workspace_bytes": (_SZ, [_CFG, _GR, _I]),
     "gtm_score": (C.c_int, [_CFG, _GR, _ST, _I, _I, _I, _P, _SZ, _P, _P]),
     "gtm_score_static_scratch_bytes": (_SZ, []),

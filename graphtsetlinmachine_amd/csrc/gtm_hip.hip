@@ -19,6 +19,7 @@
 #include "score_narrow.h"
 #include "score_messages.h"
 #include "score_moves.h"
+#include "score_small.h"
 #include "tiles_build.h"
 #include "graphs_unpack.h"
 
@@ -87,6 +88,7 @@ int check_launch(const char *what) {
     X(NO_NARROW_LAYERS) \
     X(NO_PERSISTENT_FIT) \
     X(NO_SMALL_FIT) \
+    X(NO_SMALL_SCORE) \
     X(NO_TILE_LINE) \
     X(TILE_LINE_GROUPS) \
     X(NO_TILE_PACK) \
@@ -2131,6 +2133,46 @@ size_t gtm_score_workspace_bytes(const gtm_config *cfg, const gtm_graphs *graphs
     return carve_score(d, cfg, batch, nullptr, tiles ? &tg : nullptr).bytes;
 }
 
+// A data set and a model that k_score_small takes.  Everything but the last two lines is what the kernel's registers and LDS hold.
+static bool score_small_takes(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, ScoreSmallParams *p, size_t *lds) {
+    const int nodes = std::max(g->max_number_of_graph_nodes, 1), slots = std::max(nodes, (d.K + SCORE_SMALL_VOTES - 1) / SCORE_SMALL_VOTES);
+    const bool layers = cfg->depth > 1;
+    if (nodes > SCORE_SMALL_NODES || slots > SCORE_SMALL_SLOTS || d.LA > 4 * SCORE_SMALL_QUADS) return false;
+    if (layers && (d.M % 32 != 0 || d.M / 32 > 4 * SCORE_SMALL_QUADS)) return false;
+    if (layers && g->total_edges > 0 && (!g->number_of_graph_node_edges || !g->edge || !g->edge_index)) return false;
+    p->slots = slots, p->graphs = 64 / slots;
+    *lds = score_small_lds_words(d.C, d.K, d.MB, cfg->depth, (d.LA + 3) / 4, layers ? (d.M / 32 + 3) / 4 : 1, p->graphs) * 4;
+    if (*lds > SCORE_SMALL_LDS) return false;
+    const int64_t groups = ((int64_t)g->number_of_graphs + p->graphs - 1) / p->graphs;
+    return groups * d.C * (d.LA + (layers ? (cfg->depth - 1) * d.MC : 0)) <= SCORE_SMALL_WORK && !tune(T_NO_SMALL_SCORE);
+}
+
+static int score_small(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const gtm_state *s, ScoreSmallParams p, size_t lds,
+                       int first_graph, int n_graphs, int32_t *class_sum, hipStream_t st) {
+    p.X = g->X, p.node_type = g->node_type, p.node_index = g->node_index, p.n_nodes = g->number_of_graph_nodes;
+    if (g->total_edges > 0) p.n_edges = g->number_of_graph_node_edges, p.edge_index = g->edge_index, p.edge = g->edge;
+    p.bank[0] = s->ta_state;
+    for (int l = 1; l < cfg->depth; ++l) p.bank[l] = s->message_ta_state[l - 1];
+    p.weights = s->clause_weights, p.hv = s->hypervectors, p.class_sum = class_sum;
+    p.first = first_graph, p.n_graphs = n_graphs, p.depth = cfg->depth;
+    p.C = d.C, p.LA = d.LA, p.MW = d.M / 32, p.M = d.M, p.MB = d.MB, p.B = d.B, p.K = d.K, p.n_types = g->number_of_node_types;
+    p.filter = d.filter;
+    const bool wide_x = d.LA > 4, wide_m = cfg->depth > 1 && d.M / 32 > 4;
+    const auto kernel = wide_x ? (wide_m ? k_score_small<2, 2> : k_score_small<2, 1>) : (wide_m ? k_score_small<1, 2> : k_score_small<1, 1>);
+    profile_start("k_score_small", st);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((n_graphs + p.graphs - 1) / p.graphs)), dim3(64 * SCORE_SMALL_WAVES), lds, st, p);
+    if (int rc = check_launch("k_score_small")) return rc;
+    profile_stop(st);
+    return GTM_OK;
+}
+
+int gtm_score_needs_tiles(const gtm_config *cfg, const gtm_graphs *graphs) {
+    Dims d;
+    ScoreSmallParams p{};
+    size_t lds = 0;
+    return !(graphs && !validate(cfg, &d) && score_small_takes(d, cfg, graphs, &p, &lds));
+}
+
 int gtm_score(const gtm_config *cfg, const gtm_graphs *graphs, const gtm_state *state, int32_t first_graph,
               int32_t n_graphs, int32_t batch, void *workspace, size_t workspace_bytes, int32_t *class_sum,
               void *stream) {
@@ -2147,6 +2189,10 @@ int gtm_score(const gtm_config *cfg, const gtm_graphs *graphs, const gtm_state *
         return fail(GTM_ERR_INVALID, "workspace of %zu bytes needed, %zu given", w.bytes, workspace_bytes);
     hipStream_t st = (hipStream_t)stream;
     if (n_graphs == 0) return GTM_OK;
+    ScoreSmallParams small{};
+    size_t small_lds = 0;
+    if (!graphs->tiles && score_small_takes(d, cfg, graphs, &small, &small_lds))
+        return score_small(d, cfg, graphs, state, small, small_lds, first_graph, n_graphs, class_sum, st);
     if (tiles) {
         if (int rc = check_tiles(tg, cfg, graphs)) return rc;
         return score_on_tiles(d, cfg, graphs, state, tg, w, first_graph, n_graphs, batch, class_sum, st);

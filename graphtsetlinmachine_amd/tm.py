@@ -538,21 +538,27 @@ class CommonTsetlinMachine:
         dg = self._score_init(graphs)
         cfg = self._config(max(dg.max_nodes, 1))
         n = dg.number_of_graphs
-        dg.ensure_tiles(cfg)
+        desc, tiles = dg.desc, _abi.lib.gtm_score_needs_tiles(ctypes.byref(cfg), ctypes.byref(dg.desc)) != 0
+        if tiles:
+            dg.ensure_tiles(cfg)
+        else:  # (training and transform may have made some)
+            desc = _abi.GraphsDesc.from_buffer_copy(desc)
+            desc.tiles = None
         if captured_elsewhere:
             dg.require_made()
-        dg.ensure_moves(cfg)
+        if tiles:
+            dg.ensure_moves(cfg)
         if batch is None:
             # as many graphs per launch group as fit in 4 GiB of workspace beyond its fixed part
-            size = lambda b: _abi.lib.gtm_score_workspace_bytes(ctypes.byref(cfg), ctypes.byref(dg.desc), b)
+            size = lambda b: _abi.lib.gtm_score_workspace_bytes(ctypes.byref(cfg), ctypes.byref(desc), b)
             fixed = size(1)
             per_graph = max(1.0, (size(1025) - fixed) / 1024.0)
             batch = int(max(1, min(n, ((4 << 30) - fixed) // per_graph, 1 << 16)))
-        need = _abi.lib.gtm_score_workspace_bytes(ctypes.byref(cfg), ctypes.byref(dg.desc), batch)
+        need = _abi.lib.gtm_score_workspace_bytes(ctypes.byref(cfg), ctypes.byref(desc), batch)
         ws = self._workspace_of(need)
         out = torch.empty(n * self.number_of_outputs, dtype=torch.int32, device=_device())
         _abi.call(
-            "gtm_score", ctypes.byref(cfg), ctypes.byref(dg.desc), ctypes.byref(self._state), 0, n, batch,
+            "gtm_score", ctypes.byref(cfg), ctypes.byref(desc), ctypes.byref(self._state), 0, n, batch,
             _ptr(ws), ws.numel(), _ptr(out), _stream(),
         )
         return dg, out

@@ -217,6 +217,10 @@ int gtm_build_tiles(const gtm_config *cfg, const gtm_graphs *graphs, uint32_t *t
 size_t gtm_moves_bytes(const gtm_config *cfg, const gtm_graphs *graphs);
 int gtm_build_moves(const gtm_config *cfg, const gtm_graphs *graphs, uint32_t *moves, void *stream);
 
+/* No counterpart in the reference.  0 where gtm_score is faster with graphs->tiles NULL: small models on graphs of a few
+ * nodes are then scored in one launch straight from the arrays.  (Other entry points may still want tiles.) */
+int gtm_score_needs_tiles(const gtm_config *cfg, const gtm_graphs *graphs);
+
 /* Scratch needed by gtm_score for sub-batches of `batch` graphs. */
 size_t gtm_score_workspace_bytes(const gtm_config *cfg, const gtm_graphs *graphs, int32_t batch);
 
