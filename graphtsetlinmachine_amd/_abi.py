@@ -105,6 +105,7 @@ PROTOTYPES = {
     "gtm_get_hyperliterals": (C.c_int, [_CFG, _P, _I, _I, _P, _P]),
     "gtm_transform_workspace_bytes": (_SZ, [_CFG, _GR, _I]),
     "gtm_transform": (C.c_int, [_CFG, _GR, _ST, _I, _I, _I, _P, _SZ, _P, _P, _I, _P, _P]),
+    "gtm_pack_outputs": (C.c_int, [_P, C.c_int64, _P, _P]),
     "gtm_tuning_set": (C.c_int, [C.c_char_p, C.c_char_p]),
     "gtm_tuning_get": (C.c_char_p, [C.c_char_p]),
     "gtm_tuning_reload": (C.c_int, []),

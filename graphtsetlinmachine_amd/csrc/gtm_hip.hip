@@ -585,15 +585,15 @@ __global__ void k_transform_nodewise(const uint32_t *__restrict__ bitmap, int C,
     out[i] = node < n ? (bitmap[gc * NC + (node >> 5)] >> (node & 31)) & 1u : 0;
 }
 
-// `transform` and `transform_nodewise` (kernels.py:666-710) from the truth rows that the tile kernels
+// `transform` (kernels.py:666-691) from the truth rows that the tile kernels
 // leave behind ([tiles of the launch][C][tw]), and the class sums (kernels.py:297-315) from the same
-// rows: one workgroup per graph.  A graph without nodes gives zeros in both outputs (the reference
+// rows: one workgroup per graph.  A graph without nodes gives zeros (the reference
 // loops over the nodes) while its class sums count every clause, as `evaluate` does.
 constexpr int TILE_TRANSFORM_BLOCK = 256;
 __global__ __launch_bounds__(TILE_TRANSFORM_BLOCK) void k_tile_transform(
     const uint32_t *__restrict__ bitmap, TileGeom tg, int tile0, int graph0, int first_graph, int C, int K,
     const uint32_t *__restrict__ n_nodes_arr, const int32_t *__restrict__ weights, int32_t *__restrict__ transformed,
-    int32_t *__restrict__ nodewise, int width, int32_t *__restrict__ class_sum) {
+    int32_t *__restrict__ class_sum) {
     extern __shared__ uint32_t fired[];  // one bit per clause, then a partial sum per wave
     int32_t *partial = (int32_t *)(fired + (C + 31) / 32);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -610,13 +610,6 @@ __global__ __launch_bounds__(TILE_TRANSFORM_BLOCK) void k_tile_transform(
         if (any) atomicOr(&fired[c >> 5], 1u << (c & 31));
         transformed[out0 + c] = n > 0 && any != 0u;
     }
-    if (nodewise)
-        for (int64_t i = tid; i < (int64_t)C * width; i += TILE_TRANSFORM_BLOCK) {
-            const int c = (int)(i / width), node = (int)(i - (int64_t)c * width);
-            uint32_t bit = 0u;
-            if (node < n) bit = (((rows[(int64_t)c * tg.tw + (node >> 5)] >> f.shift) & f.mask) >> (node & 31)) & 1u;
-            nodewise[out0 * width + i] = (int32_t)bit;
-        }
     __syncthreads();
     for (int k = 0; k < K; ++k) {
         int sum = 0;
@@ -632,6 +625,49 @@ __global__ __launch_bounds__(TILE_TRANSFORM_BLOCK) void k_tile_transform(
             class_sum[(int64_t)(g - first_graph) * K + k] = total;
         }
         __syncthreads();
+    }
+}
+
+// `transform_nodewise` (kernels.py:693-710) from the same truth rows: a workgroup per graph and range of `per` clauses, whose
+// outputs lie one after the other.  Bound by writing them.  TILE_NODEWISE outputs a workgroup fill the chip from a handful of graphs
+// on; per * width stays below 2^31, so that an output's clause is a 32-bit multiplication by the width's inverse, one too low at most.
+constexpr int64_t TILE_NODEWISE = 16384;
+__global__ __launch_bounds__(TILE_TRANSFORM_BLOCK) void k_tile_nodewise(const uint32_t *__restrict__ bitmap, TileGeom tg, int tile0,
+                                                                        int graph0, int first_graph, int C, int per, uint32_t inverse,
+                                                                        const uint32_t *__restrict__ n_nodes_arr,
+                                                                        int32_t *__restrict__ nodewise, int width) {
+    const int g = graph0 + (int)blockIdx.x, c0 = (int)blockIdx.y * per;
+    const int n = (int)n_nodes_arr[g];
+    const FitGraph f = fit_graph_slot(tg, g, n);
+    const uint32_t *rows = bitmap + ((int64_t)(f.tile - tile0) * C + c0) * tg.tw + f.word0;
+    int32_t *out = nodewise + ((int64_t)(g - first_graph) * C + c0) * width;
+    const int items = min(per, C - c0) * width;
+    for (int i = threadIdx.x; i < items; i += TILE_TRANSFORM_BLOCK) {
+        int c = (int)__umulhi((uint32_t)i, inverse), node = i - c * width;
+        if (node >= width) ++c, node -= width;
+        uint32_t bit = 0u;
+        if (node < n) bit = (((rows[(int64_t)c * tg.tw + (node >> 5)] >> f.shift) & f.mask) >> (node & 31)) & 1u;
+        out[i] = (int32_t)bit;
+    }
+}
+
+// Outputs (0 or 1) as bits, 64 to a wave, for their way to the host: 4 bytes read per bit, a 32nd of them sent.  Bound by reading them.
+__global__ void k_pack_outputs(const int32_t *__restrict__ outputs, int64_t n, uint32_t *__restrict__ bits) {
+    const int lane = threadIdx.x & 63;
+    const int64_t words = (n + 31) / 32, waves = (int64_t)gridDim.x * (blockDim.x >> 6);
+    for (int64_t at = 64 * ((int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)); at < n; at += 256 * waves) {
+        int32_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t i = at + 64 * waves * u + lane;
+            v[u] = i < n ? outputs[i] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const unsigned long long m = __ballot(v[u] != 0);
+            const int64_t word = (at + 64 * waves * u) / 32 + lane;
+            if (lane < 2 && word < words) bits[word] = (uint32_t)(m >> (32 * lane));
+        }
     }
 }
 
@@ -1622,9 +1658,15 @@ int score_on_tiles(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
                 profile_start("k_tile_transform", st);
                 hipLaunchKernelGGL(k_tile_transform, dim3(g_hi - g_lo), dim3(TILE_TRANSFORM_BLOCK),
                                    ((size_t)(d.C + 31) / 32 + TILE_TRANSFORM_BLOCK / 64) * 4, st, w.tile_bitmap, tg, t0, g_lo, first,
-                                   d.C, d.K, g->number_of_graph_nodes, s->clause_weights, tr->transformed, tr->nodewise, tr->width,
-                                   class_sum);
+                                   d.C, d.K, g->number_of_graph_nodes, s->clause_weights, tr->transformed, class_sum);
                 if (int rc = check_launch("tile_transform")) return rc;
+                if (tr->nodewise) {
+                    const int per = (int)std::max<int64_t>({1, TILE_NODEWISE / tr->width, ((int64_t)d.C + 65534) / 65535});
+                    hipLaunchKernelGGL(k_tile_nodewise, dim3(g_hi - g_lo, (d.C + per - 1) / per), dim3(TILE_TRANSFORM_BLOCK), 0, st,
+                                       w.tile_bitmap, tg, t0, g_lo, first, d.C, per, 0xFFFFFFFFu / (uint32_t)tr->width,
+                                       g->number_of_graph_nodes, tr->nodewise, tr->width);
+                    if (int rc = check_launch("tile_nodewise")) return rc;
+                }
                 profile_stop(st);
             }
         }
@@ -1899,6 +1941,15 @@ int gtm_transform(const gtm_config *cfg, const gtm_graphs *graphs, const gtm_sta
         }
     }
     return GTM_OK;
+}
+
+int gtm_pack_outputs(const int32_t *outputs, int64_t n, uint32_t *bits, void *stream) {
+    if (n < 0) return fail(GTM_ERR_INVALID, "n=%lld", (long long)n);
+    if (n == 0) return GTM_OK;
+    if (!outputs || !bits) return fail(GTM_ERR_INVALID, "NULL buffer");
+    const int64_t blocks = std::min<int64_t>(2048, (n + 4 * TPB - 1) / (4 * TPB));
+    hipLaunchKernelGGL(k_pack_outputs, dim3((unsigned)blocks), dim3(TPB), 0, (hipStream_t)stream, outputs, n, bits);
+    return check_launch("pack_outputs");
 }
 
 int gtm_tuning_set(const char *name, const char *value) {

@@ -136,3 +136,17 @@ void gtm_pack_numbers(const uint32_t *in, int64_t n, int32_t bytes, void *out) {
         for (int64_t a = 0; a < n; a += piece) memcpy((uint32_t *)out + a, in + a, (size_t)(n - a < piece ? n - a : piece) * 4);
     }
 }
+
+/* Clause outputs, which cross the bus as bits: out[i] = bit i % 32 of word i / 32.  Eight outputs per table look-up; from
+ * PACK_PARALLEL words on by all threads (a new array's pages are then also touched by all of them). */
+void gtm_unpack_outputs(const uint32_t *bits, int64_t n, int32_t *out) {
+    static int32_t of_byte[256][8]; /* (every call writes the same values: two at once do no harm) */
+    for (int b = 0; b < 256; ++b)
+        for (int j = 0; j < 8; ++j) of_byte[b][j] = (b >> j) & 1;
+    const int64_t piece = 1 << 10, words = n / 32;
+#pragma omp parallel for schedule(static) if (words > PACK_PARALLEL / 4)
+    for (int64_t a = 0; a < words; a += piece)
+        for (int64_t w = a; w < words && w < a + piece; ++w)
+            for (int q = 0; q < 4; ++q) memcpy(out + 32 * w + 8 * q, of_byte[(bits[w] >> (8 * q)) & 0xFF], 32);
+    for (int64_t i = 32 * words; i < n; ++i) out[i] = (bits[words] >> (i % 32)) & 1;
+}

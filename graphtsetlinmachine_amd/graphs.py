@@ -58,6 +58,9 @@ def _native_encoder():
         lib.gtm_pack_rows.argtypes = [p, i64, i32, i32, p]
         lib.gtm_pack_numbers.restype = None
         lib.gtm_pack_numbers.argtypes = [p, i64, i32, p]
+        # (tm.py)
+        lib.gtm_unpack_outputs.restype = None
+        lib.gtm_unpack_outputs.argtypes = [p, i64, p]
         _encoder = lib
     return _encoder
 

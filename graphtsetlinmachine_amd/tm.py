@@ -26,6 +26,7 @@ import numpy as np
 import torch
 
 from . import _abi
+from .graphs import _native_encoder
 from .upload import upload
 
 
@@ -45,6 +46,27 @@ def _to_device(array):
 
 def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None and t.numel() > 0 else ctypes.c_void_p(0)
+
+
+# Clause outputs from this many on cross the bus as bits and are made numbers again by all threads of the host; below, the launch
+# and the threads' waking take longer than what they save (us per call, bits and numbers: 100,000 outputs 139 and 122, 333,000 149
+# and 208, 1.3 million 265 and 539, 20 million per node 1,617 and 19,720).
+OUTPUTS_AS_BITS = 1 << 18
+# Bytes that are fetched through pinned memory, which torch keeps for the next call.
+PINNED_RESULT = 16 << 20
+
+
+def _to_host(t):
+    """t on the host, complete; through pinned memory where it is small and there is some."""
+    if t.numel() * t.element_size() <= PINNED_RESULT:
+        try:
+            out = torch.empty(t.shape, dtype=t.dtype, pin_memory=True)
+        except RuntimeError:
+            return t.cpu()
+        out.copy_(t, non_blocking=True)
+        torch.cuda.current_stream().synchronize()
+        return out
+    return t.cpu()
 
 
 def _stream():
@@ -580,16 +602,28 @@ class CommonTsetlinMachine:
             batch = int(max(1, min(n, ((1 << 30) - fixed) // per_graph, 1 << 16)))
         need = _abi.lib.gtm_transform_workspace_bytes(ctypes.byref(cfg), ctypes.byref(dg.desc), batch)
         ws = self._workspace_of(need)
-        sums = torch.empty(n * self.number_of_outputs, dtype=torch.int32, device=_device())
         flat = torch.empty(n * C, dtype=torch.int32, device=_device())
         wide = torch.empty(n * C * width, dtype=torch.int32, device=_device()) if nodewise else None
+        outputs = wide if nodewise else flat
+        native = _native_encoder() if outputs.numel() >= OUTPUTS_AS_BITS else None
+        words = (outputs.numel() + 31) // 32 if native else 0
+        result = torch.empty(words + n * self.number_of_outputs, dtype=torch.int32, device=_device())  # bits, class sums
+        sums = result[words:]
         _abi.call(
             "gtm_transform", ctypes.byref(cfg), ctypes.byref(dg.desc), ctypes.byref(self._state), 0, n, batch,
             _ptr(ws), ws.numel(), _ptr(flat), _ptr(wide) if nodewise else None, width, _ptr(sums), _stream(),
         )
-        out = wide.cpu().numpy().reshape(n, C, width) if nodewise else flat.cpu().numpy().reshape(n, C)
+        shape = (n, C, width) if nodewise else (n, C)
+        if native:
+            _abi.call("gtm_pack_outputs", _ptr(outputs), outputs.numel(), _ptr(result), _stream())
+            result = _to_host(result)
+            out = np.empty(shape, dtype=np.int32)
+            native.gtm_unpack_outputs(result.data_ptr(), out.size, out.ctypes.data)
+            sums = result[words:].numpy().copy()
+        else:
+            out, sums = outputs.cpu().numpy().reshape(shape), sums.cpu().numpy()
         dg._made = True
-        return out, sums.cpu().numpy().reshape(n, self.number_of_outputs)
+        return out, sums.reshape(n, self.number_of_outputs)
 
     def transform(self, graphs):
         """tm.py:814-851: (int32 [graphs][clauses] = the clause is true at some node, class sums)."""

@@ -292,6 +292,10 @@ int gtm_transform(const gtm_config *cfg, const gtm_graphs *graphs, const gtm_sta
                   int32_t n_graphs, int32_t batch, void *workspace, size_t workspace_bytes, int32_t *transformed,
                   int32_t *nodewise, int32_t width, int32_t *class_sum, void *stream);
 
+/* No counterpart in the reference.  n outputs of gtm_transform as bits for the way to the host: bit i % 32 of
+ * bits[i / 32] = output i is not 0, bits past the last output are 0. */
+int gtm_pack_outputs(const int32_t *outputs, int64_t n, uint32_t *bits, void *stream);
+
 /* No counterpart in the reference (its tuning knobs are the `grid` and `block` constructor
  * arguments, tm.py:53-54).  The library's tuning and test switches - the GTM_* names listed in its
  * documentation - are read from the process environment once, when the library is loaded, and
