@@ -16,9 +16,9 @@
 //     the class sums travel.
 // Bound by the two or three device-wide exchanges per example (few clauses), or by the generator calls of the Type I
 // feedback and the copies of the received rows (thousands of clauses).  us per example, edges walked and clauses' include
-// planes walked (fit_deep_persistent.h) -> here: 1,000-node chains, 200 clauses 20.5 -> 11.8; chains of 10 to 40 nodes, 333 clauses,
+// planes walked (fit_deep_persistent.h) -> here: 1,000-node chains, 200 clauses 20.5 -> 11.1; chains of 10 to 40 nodes, 333 clauses,
 // three layers 26 -> 15.9; 324-node grids, 2,000 clauses, three layers 54 -> 22.4; 841-node grids, 8,000 clauses, three layers
-// 170 -> 64, of which the slowest workgroup's evaluation, for which all others waited, was more than half.
+// 170 -> 61, of which the slowest workgroup's evaluation, for which all others waited, was more than half.
 #pragma once
 
 constexpr int FITM_MAX_CLASSES = 64;
@@ -177,7 +177,7 @@ template <int MAXB, bool EXACT, bool REGS, bool ROWS_LDS>
 __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
     extern __shared__ __align__(16) uint32_t lds[];
     __shared__ int32_t votes[64], sums[64], labels[2][64];
-    __shared__ int go_on, n_own_shared, n_busy, n_stale, next_unit;
+    __shared__ int go_on, n_own_shared, n_busy, n_stale, next_unit, next_words;
     constexpr int WAVES = FITP_BLOCK / 64, POLL = WAVES - 1;  // the last wave announces, adds and polls
     int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -356,8 +356,9 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
         draw(p.first_step - 1u);  // (the pick of the first step)
     }
     fits_word<MAXB, EXACT> word0(planes[0], B), word1(planes[1], B);
-    // the (clause, class) pair that this thread decides first, and the word of the listed clauses that it updates first (not REGS)
-    const int pair_cl = tid / K, pair_k = tid - pair_cl * K, my_cl = tid / words_all, my_w = tid - my_cl * words_all;
+    // the (clause, class) pair that this thread decides first (not REGS)
+    const int pair_cl = tid / K, pair_k = tid - pair_cl * K;
+    const uint32_t by_words = 0xFFFFFFFFu / (uint32_t)words_all;  // (a quotient from it is one too low at most)
 
     int n_now = (int)p.n_nodes[p.first_example], n_next = (int)p.n_nodes[min(p.first_example + 1, last)];
     uint32_t base_now = p.node_index[p.first_example], base_next = p.node_index[min(p.first_example + 1, last)];
@@ -389,8 +390,8 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
         asm volatile("" : "+v"(tid));
         lane = tid & 63, place = 2 * (lane & ((1 << lg) - 1));
     };
-    int row_log = 3;  // 2^row_log >= S lanes send a row
-    while ((1 << row_log) < S) ++row_log;
+    int row_log = 2;  // 2^row_log >= S / 2 lanes send a row
+    while ((2 << row_log) < S) ++row_log;
     const int by_moves = NM > 0 ? (65536 + NM - 1) / NM : 0;
     const int layer_words = M * S;
     const int share_lo = (int)((int64_t)g * layer_words / G), share_hi = (int)((int64_t)(g + 1) * layer_words / G);
@@ -475,20 +476,26 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
             lds_barrier();  // the truth rows are complete, and nobody reads the received rows of the layer before
             refresh();
             uint32_t *got_l = got_now + (size_t)l * layer_words;
-            if (tid == 0) next_unit = 0;
-            // a. what the own clauses make the nodes receive: their truth rows, shifted, where an edge of the move ends
+            if (tid == 0) next_unit = 0, next_words = 0;
+            // a. what the own clauses make the nodes receive: their truth rows, shifted, where an edge of the move ends; two words per
+            // atomic (841-node grids: 1.7 million of one word per layer took 2.9 us a workgroup to hand over, 2.0 as pairs)
             for (int u = tid >> row_log; u < n_own * NM; u += FITP_BLOCK >> row_log) {
-                const int cl = (u * by_moves) >> 16, k = u - cl * NM, w = tid & ((1 << row_log) - 1);
+                const int cl = (u * by_moves) >> 16, k = u - cl * NM, w = 2 * (tid & ((1 << row_log) - 1));
                 int shift_words = 0, shift_bits = 0;
 #pragma unroll
                 for (int m = 0; m < TILE_MOVES_MAX; ++m)
                     if (m == k) shift_words = p.moves.words[m], shift_bits = p.moves.bits[m];
-                const int q = w + shift_words;
-                const uint32_t lo = q >= 0 && q < S ? truth[cl * S + q] : 0u, hi = q + 1 >= 0 && q + 1 < S ? truth[cl * S + q + 1] : 0u;
-                const uint32_t v = w < fg.words ? __builtin_amdgcn_alignbit(hi, lo, shift_bits) & ends[((i & 1) * NM + k) * S + w] : 0u;
-                if (v != 0u)
+                const uint32_t *row = truth + cl * S;
+                auto word = [&](int q) { return q >= 0 && q < S ? row[q] : 0u; };
+                const uint32_t t0 = word(w + shift_words), t1 = word(w + shift_words + 1), t2 = word(w + shift_words + 2);
+                const uint32_t *to = ends + ((i & 1) * NM + k) * S + w;  // (S is even)
+                const uint32_t v0 = w < fg.words ? __builtin_amdgcn_alignbit(t1, t0, shift_bits) & to[0] : 0u;
+                const uint32_t v1 = w + 1 < fg.words ? __builtin_amdgcn_alignbit(t2, t1, shift_bits) & to[1] : 0u;
+                const unsigned long long v = (unsigned long long)v1 << 32 | v0;
+                if (v != 0ull)
                     for (int j = 0; j < p.MB; ++j)
-                        __hip_atomic_fetch_or(&got_l[send_row[u * p.MB + j] * (uint32_t)S + w], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        __hip_atomic_fetch_or((unsigned long long *)(got_l + send_row[u * p.MB + j] * (uint32_t)S + w), v, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
             }
             __builtin_amdgcn_s_waitcnt(FITP_WAIT_VMEM);  // the ORs have been carried out where every workgroup sees them
             asm volatile("" ::: "memory");
@@ -798,15 +805,25 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
                         f.x = message_word(f.cl, node, f.bank, f.wl);
                 }
             };
-            const int total = n_busy * words_all, step_b = FITP_BLOCK / words_all, step_w = FITP_BLOCK - step_b * words_all;
-            int b = my_cl, w = my_w;
-            Fetched now;
-            if (tid < total) fetch(now, b, w);
-            for (int at = tid; at < total; at += FITP_BLOCK) {
-                b += step_b, w += step_w;
-                if (w >= words_all) w -= words_all, ++b;
-                Fetched next = now;
-                if (at + FITP_BLOCK < total) fetch(next, b, w);
+            // 64 words at a time off a queue: what a word costs depends on its clause's feedback (in turns of all threads 15.6 us
+            // on the 841-node grids, the last of five turns nearly empty; 14.5)
+            const int total = n_busy * words_all;
+            auto take = [&](Fetched &f) {
+                int at = 0;
+                if (lane == 0) at = atomicAdd(&next_words, 64);
+                at = __builtin_amdgcn_readfirstlane(at) + lane;
+                f.cl = -1;
+                if (at < total) {
+                    int b = (int)__umulhi((uint32_t)at, by_words), w = at - b * words_all;
+                    if (w >= words_all) w -= words_all, ++b;
+                    fetch(f, b, w);
+                }
+                return at - lane < total;
+            };
+            Fetched now, next;
+            for (bool more = take(now); more; now = next) {
+                more = take(next);
+                if (now.cl < 0) continue;
                 fits_word<MAXB, EXACT> state(now.planes, B);
                 const uint32_t was = state.top(), c = (uint32_t)own_id[now.cl];
                 const bool fired = node_of[now.cl] >= 0, learns = learns_of[now.cl] != 0;
@@ -829,7 +846,6 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
                     inc[now.cl * words_all + now.w] = state.top();
                     if (atomicOr(&stale[now.cl * depth + now.bank], 1u) == 0u) stale_list[atomicAdd(&n_stale, 1)] = now.cl * depth + now.bank;
                 }
-                now = next;
             }
             __syncthreads();
             refresh();
