@@ -16,7 +16,7 @@
 //     the class sums travel.
 // Bound by the two or three device-wide exchanges per example (few clauses), or by the generator calls of the Type I
 // feedback and the copies of the received rows (thousands of clauses).  us per example, edges walked and clauses' include
-// planes walked (fit_deep_persistent.h) -> here: 1,000-node chains, 200 clauses 20.5 -> 11.1; chains of 10 to 40 nodes, 333 clauses,
+// planes walked (fit_deep_persistent.h) -> here: 1,000-node chains, 200 clauses 20.5 -> 11; chains of 10 to 40 nodes, 333 clauses,
 // three layers 26 -> 15.9; 324-node grids, 2,000 clauses, three layers 54 -> 22.4; 841-node grids, 8,000 clauses, three layers
 // 170 -> 61, of which the slowest workgroup's evaluation, for which all others waited, was more than half.
 #pragma once
@@ -390,8 +390,12 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
         asm volatile("" : "+v"(tid));
         lane = tid & 63, place = 2 * (lane & ((1 << lg) - 1));
     };
-    int row_log = 2;  // 2^row_log >= S / 2 lanes send a row
-    while ((2 << row_log) < S) ++row_log;
+    // Words that a lane sends by one atomic.  Two where a workgroup has many clauses: on the 841-node grids, 128 rows a workgroup and
+    // layer, sending took 2.9 us word by word, 2.0 in pairs.  With few (REGS) one turn of the threads sends all, and a lane is done sooner with
+    // one word (1,000-node chains, 2 rows: 0.71 against 0.76 us).
+    constexpr int SENT = REGS ? 1 : 2;
+    int row_log = 2;  // 2^row_log lanes send a row
+    while ((SENT << row_log) < S) ++row_log;
     const int by_moves = NM > 0 ? (65536 + NM - 1) / NM : 0;
     const int layer_words = M * S;
     const int share_lo = (int)((int64_t)g * layer_words / G), share_hi = (int)((int64_t)(g + 1) * layer_words / G);
@@ -477,25 +481,28 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
             refresh();
             uint32_t *got_l = got_now + (size_t)l * layer_words;
             if (tid == 0) next_unit = 0, next_words = 0;
-            // a. what the own clauses make the nodes receive: their truth rows, shifted, where an edge of the move ends; two words per
-            // atomic (841-node grids: 1.7 million of one word per layer took 2.9 us a workgroup to hand over, 2.0 as pairs)
+            // a. what the own clauses make the nodes receive: their truth rows, shifted, where an edge of the move ends
             for (int u = tid >> row_log; u < n_own * NM; u += FITP_BLOCK >> row_log) {
-                const int cl = (u * by_moves) >> 16, k = u - cl * NM, w = 2 * (tid & ((1 << row_log) - 1));
+                const int cl = (u * by_moves) >> 16, k = u - cl * NM, w = SENT * (tid & ((1 << row_log) - 1));
                 int shift_words = 0, shift_bits = 0;
 #pragma unroll
                 for (int m = 0; m < TILE_MOVES_MAX; ++m)
                     if (m == k) shift_words = p.moves.words[m], shift_bits = p.moves.bits[m];
                 const uint32_t *row = truth + cl * S;
                 auto word = [&](int q) { return q >= 0 && q < S ? row[q] : 0u; };
-                const uint32_t t0 = word(w + shift_words), t1 = word(w + shift_words + 1), t2 = word(w + shift_words + 2);
-                const uint32_t *to = ends + ((i & 1) * NM + k) * S + w;  // (S is even)
-                const uint32_t v0 = w < fg.words ? __builtin_amdgcn_alignbit(t1, t0, shift_bits) & to[0] : 0u;
-                const uint32_t v1 = w + 1 < fg.words ? __builtin_amdgcn_alignbit(t2, t1, shift_bits) & to[1] : 0u;
-                const unsigned long long v = (unsigned long long)v1 << 32 | v0;
-                if (v != 0ull)
-                    for (int j = 0; j < p.MB; ++j)
-                        __hip_atomic_fetch_or((unsigned long long *)(got_l + send_row[u * p.MB + j] * (uint32_t)S + w), v, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t *to = ends + ((i & 1) * NM + k) * S + w;
+                const uint32_t t0 = word(w + shift_words), t1 = word(w + shift_words + 1);
+                uint64_t v = w < fg.words ? __builtin_amdgcn_alignbit(t1, t0, shift_bits) & to[0] : 0u;
+                if (SENT == 2 && w + 1 < fg.words)  // (S is even)
+                    v |= (uint64_t)(__builtin_amdgcn_alignbit(word(w + shift_words + 2), t1, shift_bits) & to[SENT - 1]) << 32;
+                if (v != 0u)
+                    for (int j = 0; j < p.MB; ++j) {
+                        uint32_t *at = got_l + send_row[u * p.MB + j] * (uint32_t)S + w;
+                        if constexpr (SENT == 2)
+                            __hip_atomic_fetch_or((unsigned long long *)at, (unsigned long long)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        else
+                            __hip_atomic_fetch_or(at, (uint32_t)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
             }
             __builtin_amdgcn_s_waitcnt(FITP_WAIT_VMEM);  // the ORs have been carried out where every workgroup sees them
             asm volatile("" ::: "memory");
@@ -806,7 +813,7 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
                 }
             };
             // 64 words at a time off a queue: what a word costs depends on its clause's feedback (in turns of all threads 15.6 us
-            // on the 841-node grids, the last of five turns nearly empty; 14.5)
+            // on the 841-node grids, the last of five turns nearly empty; 14.5 off the queue)
             const int total = n_busy * words_all;
             auto take = [&](Fetched &f) {
                 int at = 0;
