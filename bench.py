@@ -338,9 +338,11 @@ def roofline_of(tm, test, run, steps, graphs):
         b_msg = message_layer_bytes_per_graph(n_nodes, tm.number_of_message_chunks, tm.number_of_clauses,
                                               node_chunks, edges_per_graph)
         layer_groups = []
-        for label, wanted, group_bytes in (("layer 0", lambda k: "messages" not in k, b_eval),
-                                          ("message layers (%d)" % (tm.depth - 1), lambda k: "messages" in k,
-                                           b_msg * (tm.depth - 1))):
+        groups = [("layer 0", lambda k: "messages" not in k, b_eval),
+                  ("message layers (%d)" % (tm.depth - 1), lambda k: "messages" in k, b_msg * (tm.depth - 1))]
+        if any(k["kernel"] == "k_score_small" for k in run["kernels"]):  # one launch for all layers
+            groups = [("all layers", lambda k: True, b_eval + b_msg * (tm.depth - 1))]
+        for label, wanted, group_bytes in groups:
             members = [k for k in run["kernels"] if wanted(k["kernel"])]
             ms = sum(k["ms_per_step"] for k in members)
             gbs = group_bytes * graphs / (ms * 1e-3) / 1e9 if ms > 0 else 0.0
