@@ -2732,6 +2732,7 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
     if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !coop) return GTM_OK;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) return GTM_OK;
     if (g->total_edges == 0 || cfg->max_nodes < 2) return GTM_OK;  // nothing to shift: as before
+    if (cfg->literals + std::min(d.C, g->number_of_node_types) > 65536) return GTM_OK;  // (the last type row's 16-bit number)
     if (!g->number_of_graph_node_edges || !g->edge || !g->edge_index)
         return fail(GTM_ERR_INVALID, "graphs with edges need number_of_graph_node_edges, edge and edge_index");
 

@@ -95,3 +95,25 @@ def test_giving_up_leaves_the_model_as_it_was(in_memory, tune):
         ta, banks, w = dev.download()
         assert np.array_equal(w, model.clause_weights) and np.array_equal(ta, model.ta_state)
         assert all(np.array_equal(a, b) for a, b in zip(banks, model.message_ta_state))
+
+
+def test_more_rows_than_a_list_can_number():
+    """65,600 node types and as many clauses: the type rows of the last of them have numbers of 17 bits, lists hold 16."""
+    from oracle import gtm_oracle_c as oc
+    from tests.gpu_harness import Device
+
+    graphs = _graphs(np.array([7, 4, 9, 1, 16]), CHAIN, seed=4, hv=32)
+    types = 65600
+    graphs.node_type_id = {"type %d" % t: t for t in range(types)}
+    graphs.node_type[:] = np.random.default_rng(2).choice([0, 3, 65471, 65472, 65500, 65535, 65536, 65599], size=graphs.node_type.size)
+    cfg = helpers.oracle_config(graphs, classes=2, clauses=types, message_size=32, T=30000)
+    model = helpers.random_model(5, cfg, 2, s=(3.0, 2.0), include_density=0.0, message_density=0.0)
+    dev = Device(model, graphs)
+    assert dev.build_tiles()
+    Y = o.encode_labels(np.arange(5) % 2, 2, cfg.threshold)
+    for epoch in range(2):
+        oc.fit(model, graphs, Y)
+        dev.fit(Y, 0, 5, epoch * 5)
+        ta, banks, w = dev.download()
+        assert np.array_equal(w, model.clause_weights) and np.array_equal(ta, model.ta_state)
+        assert np.array_equal(banks[0], model.message_ta_state[0])
