@@ -137,16 +137,17 @@ void gtm_pack_numbers(const uint32_t *in, int64_t n, int32_t bytes, void *out) {
     }
 }
 
-/* Clause outputs, which cross the bus as bits: out[i] = bit i % 32 of word i / 32.  Eight outputs per table look-up; from
+#define OUTPUTS_4(v) { (v) & 1, ((v) >> 1) & 1, ((v) >> 2) & 1, ((v) >> 3) & 1 }
+/* Clause outputs, which cross the bus as bits: out[i] = bit i % 32 of word i / 32.  Four outputs per table look-up; from
  * PACK_PARALLEL words on by all threads (a new array's pages are then also touched by all of them). */
 void gtm_unpack_outputs(const uint32_t *bits, int64_t n, int32_t *out) {
-    static int32_t of_byte[256][8]; /* (every call writes the same values: two at once do no harm) */
-    for (int b = 0; b < 256; ++b)
-        for (int j = 0; j < 8; ++j) of_byte[b][j] = (b >> j) & 1;
+    static const int32_t of_half_byte[16][4] = {OUTPUTS_4(0), OUTPUTS_4(1), OUTPUTS_4(2), OUTPUTS_4(3), OUTPUTS_4(4), OUTPUTS_4(5),
+                                                OUTPUTS_4(6), OUTPUTS_4(7), OUTPUTS_4(8), OUTPUTS_4(9), OUTPUTS_4(10), OUTPUTS_4(11),
+                                                OUTPUTS_4(12), OUTPUTS_4(13), OUTPUTS_4(14), OUTPUTS_4(15)};
     const int64_t piece = 1 << 10, words = n / 32;
 #pragma omp parallel for schedule(static) if (words > PACK_PARALLEL / 4)
     for (int64_t a = 0; a < words; a += piece)
         for (int64_t w = a; w < words && w < a + piece; ++w)
-            for (int q = 0; q < 4; ++q) memcpy(out + 32 * w + 8 * q, of_byte[(bits[w] >> (8 * q)) & 0xFF], 32);
+            for (int q = 0; q < 8; ++q) memcpy(out + 32 * w + 4 * q, of_half_byte[(bits[w] >> (4 * q)) & 0xF], 16);
     for (int64_t i = 32 * words; i < n; ++i) out[i] = (bits[words] >> (i % 32)) & 1;
 }

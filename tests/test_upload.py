@@ -166,3 +166,19 @@ def test_small_data_sets_of_any_size_share_their_pinned_memory(monkeypatch):
     for n in (1, 3, 20, 150):
         upload.upload(graphs_of(64, n_graphs=n), torch.device("cuda"))
     assert asked == {(upload.PIECE_BYTES,)}
+
+
+def test_the_packer_keeps_no_data_of_its_own(tmp_path):
+    """Calls from several threads run side by side (ctypes releases the interpreter lock): no static that one writes and another reads."""
+    import shutil
+    import subprocess
+
+    from graphtsetlinmachine_amd import build
+
+    if not (shutil.which("gcc") and shutil.which("nm")):
+        pytest.skip("needs gcc and nm")
+    source = [s for s in build.ENCODER_SOURCES if s.endswith("pack.c")][0]
+    subprocess.run(["gcc", "-O3", "-fopenmp", "-fPIC", "-c", "-o", str(tmp_path / "pack.o"), source], check=True)
+    symbols = subprocess.run(["nm", str(tmp_path / "pack.o")], check=True, capture_output=True, text=True).stdout.splitlines()
+    assert any(line.endswith(" T gtm_unpack_outputs") for line in symbols)
+    assert not [line for line in symbols if line.split()[-2] in "bBdDC"]
