@@ -2176,14 +2176,6 @@ static bool score_uses_tiles(const gtm_config *cfg, const gtm_graphs *graphs, in
     return tiles_usable(cfg, graphs, classes, tg);
 }
 
-size_t gtm_score_workspace_bytes(const gtm_config *cfg, const gtm_graphs *graphs, int32_t batch) {
-    Dims d;
-    if (validate(cfg, &d) || batch < 1) return 0;
-    TileGeom tg;
-    bool tiles = score_uses_tiles(cfg, graphs, d.K, &tg);
-    return carve_score(d, cfg, batch, nullptr, tiles ? &tg : nullptr).bytes;
-}
-
 // A data set and a model that k_score_small takes.  Everything but the last two lines is what the kernel's registers and LDS hold.
 static bool score_small_takes(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, ScoreSmallParams *p, size_t *lds) {
     const int nodes = std::max(g->max_number_of_graph_nodes, 1), slots = std::max(nodes, (d.K + SCORE_SMALL_VOTES - 1) / SCORE_SMALL_VOTES);
@@ -2196,6 +2188,25 @@ static bool score_small_takes(const Dims &d, const gtm_config *cfg, const gtm_gr
     if (*lds > SCORE_SMALL_LDS) return false;
     const int64_t groups = ((int64_t)g->number_of_graphs + p->graphs - 1) / p->graphs;
     return groups * d.C * (d.LA + (layers ? (cfg->depth - 1) * d.MC : 0)) <= SCORE_SMALL_WORK && !tune(T_NO_SMALL_SCORE);
+}
+
+// ... and that gtm_score hands to it: tiles, where they are given, are used.
+static bool score_small_runs(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, ScoreSmallParams *p, size_t *lds) {
+    return g && !g->tiles && score_small_takes(d, cfg, g, p, lds);
+}
+
+// The kernel keeps what it needs in registers and LDS; 0 bytes would mean an invalid configuration.
+constexpr size_t SCORE_SMALL_WORKSPACE = 256;
+
+size_t gtm_score_workspace_bytes(const gtm_config *cfg, const gtm_graphs *graphs, int32_t batch) {
+    Dims d;
+    if (validate(cfg, &d) || batch < 1) return 0;
+    ScoreSmallParams small{};
+    size_t small_lds = 0;
+    if (score_small_runs(d, cfg, graphs, &small, &small_lds)) return SCORE_SMALL_WORKSPACE;
+    TileGeom tg;
+    bool tiles = score_uses_tiles(cfg, graphs, d.K, &tg);
+    return carve_score(d, cfg, batch, nullptr, tiles ? &tg : nullptr).bytes;
 }
 
 static int score_small(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const gtm_state *s, ScoreSmallParams p, size_t lds,
@@ -2233,17 +2244,20 @@ int gtm_score(const gtm_config *cfg, const gtm_graphs *graphs, const gtm_state *
     if (int rc = validate_state(cfg, state)) return rc;
     if (batch < 1) return fail(GTM_ERR_INVALID, "batch=%d", batch);
     if (!class_sum) return fail(GTM_ERR_INVALID, "class_sum is NULL");
+    hipStream_t st = (hipStream_t)stream;
+    ScoreSmallParams small{};
+    size_t small_lds = 0;
+    if (score_small_runs(d, cfg, graphs, &small, &small_lds)) {
+        if (!workspace || workspace_bytes < SCORE_SMALL_WORKSPACE)
+            return fail(GTM_ERR_INVALID, "workspace of %zu bytes needed, %zu given", SCORE_SMALL_WORKSPACE, workspace_bytes);
+        return n_graphs == 0 ? GTM_OK : score_small(d, cfg, graphs, state, small, small_lds, first_graph, n_graphs, class_sum, st);
+    }
     TileGeom tg;
     bool tiles = score_uses_tiles(cfg, graphs, d.K, &tg);
     ScoreWs w = carve_score(d, cfg, batch, (char *)workspace, tiles ? &tg : nullptr);
     if (!workspace || workspace_bytes < w.bytes)
         return fail(GTM_ERR_INVALID, "workspace of %zu bytes needed, %zu given", w.bytes, workspace_bytes);
-    hipStream_t st = (hipStream_t)stream;
     if (n_graphs == 0) return GTM_OK;
-    ScoreSmallParams small{};
-    size_t small_lds = 0;
-    if (!graphs->tiles && score_small_takes(d, cfg, graphs, &small, &small_lds))
-        return score_small(d, cfg, graphs, state, small, small_lds, first_graph, n_graphs, class_sum, st);
     if (tiles) {
         if (int rc = check_tiles(tg, cfg, graphs)) return rc;
         return score_on_tiles(d, cfg, graphs, state, tg, w, first_graph, n_graphs, batch, class_sum, st);

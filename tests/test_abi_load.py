@@ -154,3 +154,21 @@ def test_buffer_sizes_are_computed_in_64_bits_at_and_beyond_the_largest_configur
     rows_part = n_tiles * 258 * 256 * 4 + 258 * 8 + 256 * 4
     assert rows_part % 16 == 0
     assert _abi.lib.gtm_tiles_bytes(ctypes.byref(conv), ctypes.byref(d)) == rows_part + n_tiles * 256 * 32 * 16
+
+
+def test_scoring_in_one_launch_asks_for_no_general_workspace(tune):
+    """10,000 pairs and 200 clauses: the kernel that scores them from the arrays uses no scratch, whatever the batch."""
+    from graphtsetlinmachine_amd import _abi
+
+    cfg = _abi.make_config(classes=2, clauses=200, literals=64, state_bits=8, boost_true_positive_feedback=1, threshold=10, q=1.0,
+                           max_included_literals=64, negative_clauses=1, max_nodes=2, message_size=256, message_bits=2, depth=2,
+                           s=(1.0, 1.0), seed=1)
+    d = _desc(10000, 2)
+    size = lambda: _abi.lib.gtm_score_workspace_bytes(ctypes.byref(cfg), ctypes.byref(d), 10000)
+    assert not _abi.lib.gtm_score_needs_tiles(ctypes.byref(cfg), ctypes.byref(d))
+    assert 0 < size() <= 4096
+    d.tiles = 4096  # (an address: tiles that are given are used)
+    assert size() > 1 << 20
+    d.tiles = 0
+    tune("GTM_NO_SMALL_SCORE", "1")
+    assert size() > 1 << 20
