@@ -2176,18 +2176,21 @@ static bool score_uses_tiles(const gtm_config *cfg, const gtm_graphs *graphs, in
     return tiles_usable(cfg, graphs, classes, tg);
 }
 
-// A data set and a model that k_score_small takes.  Everything but the last two lines is what the kernel's registers and LDS hold.
+// A data set and a model that k_score_small takes: what its registers and LDS hold, and where it is the faster way (score_small.h).
 static bool score_small_takes(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, ScoreSmallParams *p, size_t *lds) {
     const int nodes = std::max(g->max_number_of_graph_nodes, 1), slots = std::max(nodes, (d.K + SCORE_SMALL_VOTES - 1) / SCORE_SMALL_VOTES);
     const bool layers = cfg->depth > 1;
     if (nodes > SCORE_SMALL_NODES || slots > SCORE_SMALL_SLOTS || d.LA > 4 * SCORE_SMALL_QUADS) return false;
     if (layers && (d.M % 32 != 0 || d.M / 32 > 4 * SCORE_SMALL_QUADS)) return false;
     if (layers && g->total_edges > 0 && (!g->number_of_graph_node_edges || !g->edge || !g->edge_index)) return false;
+    const int literal_quads = (d.LA + 3) / 4, message_quads = layers ? (d.M / 32 + 3) / 4 : 1;
     p->slots = slots, p->graphs = 64 / slots;
-    *lds = score_small_lds_words(d.C, d.K, d.MB, cfg->depth, (d.LA + 3) / 4, layers ? (d.M / 32 + 3) / 4 : 1, p->graphs) * 4;
-    if (*lds > SCORE_SMALL_LDS) return false;
-    const int64_t groups = ((int64_t)g->number_of_graphs + p->graphs - 1) / p->graphs;
-    return groups * d.C * (d.LA + (layers ? (cfg->depth - 1) * d.MC : 0)) <= SCORE_SMALL_WORK && !tune(T_NO_SMALL_SCORE);
+    *lds = score_small_lds_words(d.C, d.K, d.MB, cfg->depth, literal_quads, message_quads, p->graphs) * 4;
+    if (*lds > SCORE_SMALL_LDS || tune(T_NO_SMALL_SCORE)) return false;
+    const int64_t groups = ((int64_t)g->number_of_graphs + p->graphs - 1) / p->graphs, clauses = d.C;
+    if (!layers) return groups <= SCORE_SMALL_GROUPS && clauses * literal_quads <= SCORE_SMALL_CLAUSE_QUADS;
+    const int64_t tested = literal_quads + (cfg->depth - 1) * 2 * message_quads + (d.K + slots - 1) / slots - 1;
+    return (nodes <= 2 || groups <= SCORE_SMALL_LAYER_GROUPS) && groups * clauses * tested <= SCORE_SMALL_TESTED[std::min(nodes, 3) - 1];
 }
 
 // ... and that gtm_score hands to it: tiles, where they are given, are used.

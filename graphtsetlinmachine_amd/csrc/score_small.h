@@ -17,11 +17,21 @@ constexpr int SCORE_SMALL_VOTES = 4;     // classes that a lane counts for its g
 constexpr int SCORE_SMALL_SLOTS = 16;    // slots of a graph, to have lanes for its classes
 constexpr int SCORE_SMALL_QUADS = 2;     // 128-bit reads of literal words, and of message words of one sign
 constexpr size_t SCORE_SMALL_LDS = 64 * 1024;
-// Include words tested for 64 nodes, over all graphs.  On tiles the launches and their latencies come to some 60 us, but a clause then
-// takes 2,048 nodes at a time, its included literals only.  us per call here and on tiles: 0.06 million words (10 clauses, 10,000 pairs)
-// 47 and 85, 2.5 million (200 clauses, three layers, 10,000 pairs) 94 and 200, 7.5 million (30,000 pairs) 140 and 208, 7.9 million
-// (100 clauses, two layers, 140,000 pairs) 208 and 308; beyond, the two come together.
-constexpr int64_t SCORE_SMALL_WORK = 8000000;
+// Where the kernel is the faster way also for clauses that hold at few nodes, which on tiles cost little beyond the launches.
+// A workgroup's time grows with its clauses, the quads that it tests of each and the turns in which its lanes count votes, and about
+// a thousand workgroups run at once; on tiles a clause takes 2,048 nodes at a time and its included literals only.  us per call on
+// a resident data set, here and on tiles, clauses of ten random literals (those of one literal hold at more nodes, where tiles
+// take up to five times as long):
+//   depth 1, one launch on tiles, too.  20,000 nodes: 10 clauses 31 and 35, 200 clauses of one quad 41 and 42, of two 45
+//   and 42, 1,000 clauses 90 and 83; 200,000 nodes: 10 clauses 45 and 35, 200 clauses 96 and 45.
+//   message layers.  Graphs of four and eight nodes, 20,000 nodes, 200 clauses, two layers of 256 bits (560,000) 69 and 94;
+//   200,000 nodes, 10 clauses 50 and 61, 65 and 52, 200 clauses (1.9 million) 133 and 100.  Two nodes, 200,000 in all: 10 clauses
+//   49 and 77, 50 clauses 67 and 84, 200 clauses (1.9 million) 132 and 109; 800,000, two layers, 10 clauses (1.1 million) 151 and 265.
+//   Single nodes, 200,000, 200 clauses (2.5 million) 136 and 333; 800,000, 50 clauses (2.5 million) 172 and 722.
+constexpr int64_t SCORE_SMALL_GROUPS = 640, SCORE_SMALL_CLAUSE_QUADS = 200;  // depth 1: workgroups, clauses times quads
+constexpr int64_t SCORE_SMALL_LAYER_GROUPS = 1300;                           // message layers, more than two nodes: workgroups
+// ... for single nodes, two, more: workgroups times clauses times (quads + turns of votes after the first)
+constexpr int64_t SCORE_SMALL_TESTED[3] = {2500000, 1250000, 750000};
 
 struct ScoreSmallParams {
     const uint32_t *X, *node_type, *node_index, *n_nodes, *n_edges, *edge_index, *edge;  // n_edges NULL: no edges

@@ -63,15 +63,23 @@ def test_class_sums_in_one_launch(sizes, hv, node_types, edge_types, degree, siz
     assert np.array_equal(dev.score(0, n_graphs, n_graphs), want)
 
 
-def test_large_data_sets_stay_on_tiles():
+@pytest.mark.parametrize("nodes,hv,classes,depth,clauses,most", [
+    (2, 32, 2, 2, 100, 32 * (1250000 // (100 * 5))),                # pairs: 32 to a workgroup, a quad of literals and four of a layer
+    (1, 32, 2, 2, 100, 64 * (2500000 // (100 * 6))),                # single nodes count their second class in a turn of its own
+    (8, 128, 2, 3, 10, 8 * 1300),                                   # graphs of eight: workgroups ...
+    (8, 128, 2, 3, 200, 8 * (750000 // (200 * 10))),                # ... and quads
+    (4, 16, 2, 1, 200, 16 * 640), (1, 128, 1, 1, 100, 64 * 640),    # depth 1: workgroups
+    (4, 16, 2, 1, 201, 0), (1, 128, 1, 1, 101, 0),                  # ... and quads of clauses
+])
+def test_large_data_sets_stay_on_tiles(nodes, hv, classes, depth, clauses, most):
     from graphtsetlinmachine_amd import _abi
 
-    cfg = _abi.make_config(classes=2, clauses=100, literals=64, state_bits=8, boost_true_positive_feedback=1, threshold=10, q=1.0,
-                           max_included_literals=64, negative_clauses=1, max_nodes=2, message_size=256, message_bits=2, depth=2,
-                           s=(1.0, 1.0), seed=1)
+    cfg = _abi.make_config(classes=classes, clauses=clauses, literals=2 * hv, state_bits=8, boost_true_positive_feedback=1, threshold=10, q=1.0,
+                           max_included_literals=64, negative_clauses=1, max_nodes=nodes, message_size=256, message_bits=2, depth=depth,
+                           s=(1.0,) * depth, seed=1)
     d = _abi.GraphsDesc()
-    d.number_of_node_types, d.max_number_of_graph_nodes = 1, 2
-    d.number_of_graphs = 32 * (8000000 // (100 * 18))
-    assert not _abi.lib.gtm_score_needs_tiles(ctypes.byref(cfg), ctypes.byref(d))
+    d.number_of_node_types, d.max_number_of_graph_nodes = 1, nodes
+    d.number_of_graphs = most
+    assert most == 0 or not _abi.lib.gtm_score_needs_tiles(ctypes.byref(cfg), ctypes.byref(d))
     d.number_of_graphs += 1
     assert _abi.lib.gtm_score_needs_tiles(ctypes.byref(cfg), ctypes.byref(d))
