@@ -808,10 +808,29 @@ struct FitWs {
     size_t coop_words;                      // words of coop_got
     int *coop_perm;                         // [C + 2,048] which clause sits in which workgroup's slots (k_fit_deep_deal)
     uint32_t *coop_cost;                    // [C]
-    uint32_t *move_masks;                   // [FITM_CHUNK][TILE_MOVES_MAX][even NC] where a graph's edges end (k_fit_moves)
-    uint16_t *lists;                        // [C + 2,048][entries] the clauses' rows (k_fit_moves; NULL: too large)
-    size_t bytes;
+    size_t bytes;                           // what no path can do without
+    uint32_t *move_masks;                   // [examples of a launch][TILE_MOVES_MAX][even NC] where a graph's edges end (NULL: no k_fit_moves)
+    uint16_t *lists;                        // [workgroups][clauses of one][entries] the clauses' rows (k_fit_moves with automata in memory)
+    size_t bytes_by_moves;                  // ... with these two
 };
+
+int compute_units() {
+    static thread_local int cus_of[64] = {0};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    if (cus_of[dev] == 0) {
+        int cus = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+            (void)hipGetLastError();
+            return 0;
+        }
+        cus_of[dev] = cus;
+    }
+    return cus_of[dev];
+}
 
 // What k_fit_moves takes whatever the data: whole words of message bits, a lane per pair of truth words, 16-bit row numbers
 // (15 bits and a sign for messages), classes that one wave polls for.
@@ -820,13 +839,31 @@ bool fit_moves_takes(const Dims &d, const gtm_config *cfg) {
 }
 int fit_moves_list0(const gtm_config *cfg) { return (cfg->literals + 1 + 7) / 8 * 8; }
 int fit_moves_listm(const Dims &d) { return 2 * d.M; }  // (both halves whole octets)
+int fit_moves_per_group(const Dims &d, int cus) {
+    const int per_group = (d.C + cus - 1) / cus;
+    const char *e = tune(T_FIT_DEEP_CLAUSES_PER_GROUP);  // tuning aid
+    return e ? std::max(per_group, atoi(e)) : per_group;
+}
+constexpr size_t FITM_LDS_LIMIT = 158 * 1024;  // of 160 KiB; the kernel has a few words of its own
+size_t fit_moves_lds_bytes(const Dims &d, const gtm_config *cfg, int per_group, bool regs, int staged_rows_words, int n_moves) {
+    return fit_moves_lds_words(regs, staged_rows_words > 0, cfg->depth, per_group, d.LA, d.MC, d.MB, d.M, d.K, fitl_stride(d.NC), staged_rows_words,
+                               fit_moves_list0(cfg), fit_moves_listm(d), n_moves) * 4;
+}
+// Automata in registers and lists in LDS (the graph's rows in place)?
+bool fit_moves_in_registers(const Dims &d, const gtm_config *cfg, int per_group, int n_moves) {
+    int parts = 1;  // waves of a clause
+    while (2 * parts * per_group <= FITP_BLOCK / 64) parts *= 2;
+    return !tune(T_FIT_DEEP_IN_MEMORY) /* (tests) */ && per_group <= FITP_BLOCK / 64 && d.LA + (cfg->depth - 1) * d.MC <= 2 * 64 * parts &&
+           d.K <= FITM_REGS_CLASSES && fit_moves_lds_bytes(d, cfg, per_group, true, 0, n_moves) <= FITM_LDS_LIMIT;
+}
 // The lists of the clauses whose automata stay in memory.
 constexpr size_t FITM_LISTS_MAX = (size_t)256 << 20;
-size_t fit_moves_list_bytes(const Dims &d, const gtm_config *cfg) {
-    return ((size_t)d.C + 2048) * (fit_moves_list0(cfg) + (size_t)(cfg->depth - 1) * fit_moves_listm(d)) * 2;
+size_t fit_moves_list_bytes(const Dims &d, const gtm_config *cfg, int per_group) {
+    return (size_t)((d.C + per_group - 1) / per_group) * per_group * (fit_moves_list0(cfg) + (size_t)(cfg->depth - 1) * fit_moves_listm(d)) * 2;
 }
 
-FitWs carve_fit(const Dims &d, const gtm_config *cfg, char *base) {
+// `graphs` NULL: for any data set.
+FitWs carve_fit(const Dims &d, const gtm_config *cfg, const gtm_graphs *graphs, char *base) {
     FitWs w;
     size_t off = 0;
     auto take = [&](size_t bytes) {
@@ -858,10 +895,18 @@ FitWs carve_fit(const Dims &d, const gtm_config *cfg, char *base) {
     w.coop_arrived = cfg->depth > 1 ? (unsigned long long *)take((size_t)(cfg->depth - 1) * FITD_PARTS * FITD_STRIDE * 8) : nullptr;
     w.coop_perm = cfg->depth > 1 ? (int *)take(((size_t)d.C + 2048) * 4) : nullptr;
     w.coop_cost = cfg->depth > 1 ? (uint32_t *)take((size_t)d.C * 4) : nullptr;
-    const bool moves = cfg->depth > 1 && fit_moves_takes(d, cfg);
-    w.move_masks = moves ? (uint32_t *)take((size_t)FITM_CHUNK * TILE_MOVES_MAX * fitl_stride(d.NC) * 4) : nullptr;
-    w.lists = moves && fit_moves_list_bytes(d, cfg) <= FITM_LISTS_MAX ? (uint16_t *)take(fit_moves_list_bytes(d, cfg)) : nullptr;
     w.bytes = off;
+    // what only k_fit_moves wants, last: gtm_fit goes on without where the caller has no room for it
+    w.move_masks = nullptr, w.lists = nullptr;
+    const int cus = compute_units();
+    if (fit_moves_takes(d, cfg) && cus > 0 && (!graphs || graphs->total_edges > 0) && !tune(T_NO_FIT_MOVES)) {
+        const int per_group = fit_moves_per_group(d, cus);
+        const size_t examples = graphs ? (size_t)std::min(std::max(graphs->number_of_graphs, 0), FITM_CHUNK) : FITM_CHUNK;
+        w.move_masks = (uint32_t *)take(examples * TILE_MOVES_MAX * fitl_stride(d.NC) * 4);
+        const size_t list_bytes = fit_moves_list_bytes(d, cfg, per_group);
+        if (!fit_moves_in_registers(d, cfg, per_group, TILE_MOVES_MAX) && list_bytes <= FITM_LISTS_MAX) w.lists = (uint16_t *)take(list_bytes);
+    }
+    w.bytes_by_moves = off;
     return w;
 }
 
@@ -1138,21 +1183,6 @@ int launch_two_phase(const TileLayerArgs &a, int n_tiles, int la4, bool last, hi
 }
 
 // Compute units of the current device (0 if it cannot be told).
-int compute_units() {
-    static thread_local int cus_of[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-    if (cus_of[dev] == 0) {
-        int cus = 0;
-        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-            (void)hipGetLastError();
-            return 0;
-        }
-        cus_of[dev] = cus;
-    }
-    return cus_of[dev];
-}
-
 // The tiles of a launch of k_tile_two_phase_half shared out among the compute units (tile_segments_part
 // in score_tiles.h) - when they do not fill a whole number of rounds of the chip, and a share is at least 64
 // clauses (a share stages its tile).  GTM_NO_TILE_LINE turns it off; GTM_TILE_LINE_GROUPS = n (tests) cuts the
@@ -2753,10 +2783,7 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
     if (!g->number_of_graph_node_edges || !g->edge || !g->edge_index)
         return fail(GTM_ERR_INVALID, "graphs with edges need number_of_graph_node_edges, edge and edge_index");
 
-    const int layers = cfg->depth - 1, S = fitl_stride(d.NC);
-    int per_group = (d.C + cus - 1) / cus;
-    if (const char *e = tune(T_FIT_DEEP_CLAUSES_PER_GROUP)) per_group = std::max(per_group, atoi(e));  // tuning aid
-    const int groups = (d.C + per_group - 1) / per_group, words = d.LA + layers * d.MC;
+    const int layers = cfg->depth - 1, S = fitl_stride(d.NC), per_group = fit_moves_per_group(d, cus), groups = (d.C + per_group - 1) / per_group;
     if (per_group > 512 || (size_t)groups * per_group > (size_t)d.C + 2048) return GTM_OK;
     FitMovesParams p{};
     p.S = S;
@@ -2764,19 +2791,10 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
     const int rows_words = ((cfg->literals + g->number_of_node_types + 1) * fitl_stride(tg.slot_words > 0 ? tg.slot_words : 1) + 3) / 4 * 4;
     // Automata in registers and lists in LDS, with the graph's rows staged in LDS where there is room; else automata and lists in
     // memory, rows in place.
-    const size_t lds_limit = 158 * 1024;  // of 160 KiB; the kernel has a few words of its own
-    auto lds_bytes = [&](bool regs, bool rows_lds, int n_moves) {
-        return fit_moves_lds_words(regs, rows_lds, cfg->depth, per_group, d.LA, d.MC, d.MB, d.M, d.K, S, rows_words, p.list0, p.listm, n_moves) * 4;
-    };
-    const bool in_memory = tune(T_FIT_DEEP_IN_MEMORY) != nullptr;  // (tests)
     auto layout_of = [&](int n_moves) {  // 0: registers and staged rows, 1: registers, 2: memory, -1: none
-        int parts = 1;  // waves of a clause
-        while (2 * parts * per_group <= FITP_BLOCK / 64) parts *= 2;
-        if (!in_memory && per_group <= FITP_BLOCK / 64 && words <= 2 * 64 * parts && d.K <= FITM_REGS_CLASSES) {
-            if (lds_bytes(true, true, n_moves) <= lds_limit) return 0;
-            if (lds_bytes(true, false, n_moves) <= lds_limit) return 1;
-        }
-        return w.lists && lds_bytes(false, false, n_moves) <= lds_limit ? 2 : -1;
+        if (fit_moves_in_registers(d, cfg, per_group, n_moves))
+            return fit_moves_lds_bytes(d, cfg, per_group, true, rows_words, n_moves) <= FITM_LDS_LIMIT ? 0 : 1;
+        return w.lists && fit_moves_lds_bytes(d, cfg, per_group, false, 0, n_moves) <= FITM_LDS_LIMIT ? 2 : -1;
     };
     if (layout_of(0) < 0) return GTM_OK;
 
@@ -2802,7 +2820,7 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
     const int layout = layout_of(p.moves.n);
     if (layout < 0) return GTM_OK;
     const bool rows_lds = layout == 0;
-    const size_t lds = lds_bytes(layout < 2, rows_lds, p.moves.n);
+    const size_t lds = fit_moves_lds_bytes(d, cfg, per_group, layout < 2, rows_lds ? rows_words : 0, p.moves.n);
     const int variant = (d.B == 8 ? 0 : 3) + layout;
     const void *kernels[6] = {(const void *)k_fit_moves<8, true, true, true>,    (const void *)k_fit_moves<8, true, true, false>,
                               (const void *)k_fit_moves<8, true, false, false>,  (const void *)k_fit_moves<16, false, true, true>,
@@ -3253,8 +3271,13 @@ extern "C" {
 size_t gtm_fit_workspace_bytes(const gtm_config *cfg, const gtm_graphs *graphs) {
     Dims d;
     if (validate(cfg, &d)) return 0;
-    (void)graphs;
-    return carve_fit(d, cfg, nullptr).bytes;
+    return carve_fit(d, cfg, graphs, nullptr).bytes_by_moves;
+}
+
+size_t gtm_fit_workspace_least_bytes(const gtm_config *cfg, const gtm_graphs *graphs) {
+    Dims d;
+    if (validate(cfg, &d)) return 0;
+    return carve_fit(d, cfg, graphs, nullptr).bytes;
 }
 
 int gtm_fit(const gtm_config *cfg, const gtm_graphs *graphs, const gtm_state *state, const int32_t *encoded_Y,
@@ -3265,9 +3288,10 @@ int gtm_fit(const gtm_config *cfg, const gtm_graphs *graphs, const gtm_state *st
     if (int rc = validate_graphs(cfg, graphs, first_example, n_examples)) return rc;
     if (int rc = validate_state(cfg, state)) return rc;
     if (!encoded_Y) return fail(GTM_ERR_INVALID, "encoded_Y is NULL");
-    FitWs w = carve_fit(d, cfg, (char *)workspace);
+    FitWs w = carve_fit(d, cfg, graphs, (char *)workspace);
     if (!workspace || workspace_bytes < w.bytes)
         return fail(GTM_ERR_INVALID, "workspace of %zu bytes needed, %zu given", w.bytes, workspace_bytes);
+    if (workspace_bytes < w.bytes_by_moves) w.move_masks = nullptr, w.lists = nullptr;  // (the edges are walked)
     if (n_examples == 0) return GTM_OK;
     hipStream_t st = (hipStream_t)stream;
     // node counts and offsets of the examples, read once

@@ -507,8 +507,10 @@ class CommonTsetlinMachine:
         dg = self._train_graphs
         cfg = self._config(max(dg.max_nodes, 1))
         dg.ensure_tiles(cfg)
-        need = _abi.lib.gtm_fit_workspace_bytes(ctypes.byref(cfg), ctypes.byref(dg.desc))
-        ws = self._workspace_of(need)
+        try:
+            ws = self._workspace_of(_abi.lib.gtm_fit_workspace_bytes(ctypes.byref(cfg), ctypes.byref(dg.desc)))
+        except torch.OutOfMemoryError:  # (a slower kernel takes less)
+            ws = self._workspace_of(_abi.lib.gtm_fit_workspace_least_bytes(ctypes.byref(cfg), ctypes.byref(dg.desc)))
         first, count = (0, dg.number_of_graphs) if examples is None else (int(examples[0]), int(examples[1]))
         if first < 0 or count < 0 or first + count > dg.number_of_graphs:
             raise _abi.GtmError("examples=(%d, %d) outside the data set's %d graphs" % (first, count, dg.number_of_graphs))

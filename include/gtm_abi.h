@@ -246,8 +246,10 @@ size_t gtm_score_static_scratch_bytes(void);
 int gtm_score_static(const gtm_config *cfg, const gtm_graphs *graphs, const gtm_state *state, int32_t first_graph,
                      int32_t n_graphs, int32_t batch, int32_t *class_sum, void *stream);
 
-/* Scratch needed by gtm_fit. */
+/* Scratch that gtm_fit has a use for (graphs NULL: for any data set).  With less, down to
+ * gtm_fit_workspace_least_bytes(), it still trains, models with message layers more slowly where the edges are a few moves. */
 size_t gtm_fit_workspace_bytes(const gtm_config *cfg, const gtm_graphs *graphs);
+size_t gtm_fit_workspace_least_bytes(const gtm_config *cfg, const gtm_graphs *graphs);
 
 /* The inner loop of `_fit` (tm.py:669-747) over examples
  * [first_example, first_example + n_examples), strictly in order (online

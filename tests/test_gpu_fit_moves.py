@@ -117,3 +117,69 @@ def test_more_rows_than_a_list_can_number():
         ta, banks, w = dev.download()
         assert np.array_equal(w, model.clause_weights) and np.array_equal(ta, model.ta_state)
         assert np.array_equal(banks[0], model.message_ta_state[0])
+
+
+@pytest.mark.parametrize("in_memory", [False, True])
+def test_without_room_for_masks_and_lists_the_edges_are_walked(in_memory, tune, monkeypatch):
+    """What only k_fit_moves uses is asked for where it can run - not for data sets without edges, lists not where they stay in LDS - and
+    a caller that has no more than the rest trains all the same."""
+    import torch
+
+    from graphtsetlinmachine_amd import _abi, tm as tm_module
+    from tests.gpu_harness import Device
+
+    clauses = 41
+    if in_memory:
+        tune("GTM_FIT_DEEP_CLAUSES_PER_GROUP", "20")
+    graphs = _graphs(np.array([100, 90, 110, 64]), CHAIN, seed=2)
+    size = lambda name, dev: getattr(_abi.lib, name)(ctypes.byref(dev.acfg), ctypes.byref(dev.dg.desc))
+    extra = lambda dev: size("gtm_fit_workspace_bytes", dev) - size("gtm_fit_workspace_least_bytes", dev)
+    cfg = helpers.oracle_config(graphs, classes=3, clauses=clauses, depth=3, message_size=64, T=30)
+    make = lambda g: Device(helpers.random_model(5, cfg, 3, s=(3.0, 2.0, 1.5), include_density=0.02, message_density=0.02), g)
+    dev = make(graphs)
+    masks = 4 * 8 * 4 * 4  # examples, moves, words of the longest rows, bytes
+    lists = 60 * (48 + 2 * 128) * 2 if in_memory else 0  # clauses of whole workgroups, entries of their three lists, bytes
+    assert masks + lists <= extra(dev) < masks + lists + 512
+    tune("GTM_NO_FIT_MOVES", "1")
+    assert extra(dev) == 0
+    tune("GTM_NO_FIT_MOVES", None)
+    assert extra(make(_graphs(np.array([100, 90]), [], seed=2))) == 0
+
+    assert dev.build_tiles()
+    least, st = size("gtm_fit_workspace_least_bytes", dev), dev.state()
+    Y = o.encode_labels(np.arange(4) % 3, 3, cfg.threshold)
+    y = tm_module._to_device(np.ascontiguousarray(Y, dtype=np.int32))
+    ws = torch.empty(least, dtype=torch.uint8, device="cuda")
+    fit = lambda nbytes: _abi.call("gtm_fit", ctypes.byref(dev.acfg), ctypes.byref(dev.dg.desc), ctypes.byref(st), tm_module._ptr(y), 0, 4, 0,
+                                   tm_module._ptr(ws), nbytes, tm_module._stream())
+    with pytest.raises(_abi.GtmError, match="workspace of"):
+        fit(least - 1)
+    _abi.call("gtm_profile_enable", 1)
+    fit(least)
+    kernel, launches, total = ctypes.c_char_p(), ctypes.c_int32(), ctypes.c_double()
+    _abi.call("gtm_profile_read", ctypes.byref(kernel), ctypes.byref(launches), ctypes.byref(total))
+    _abi.call("gtm_profile_enable", 0)
+    assert kernel.value.startswith(b"k_fit_deep_persistent"), kernel.value
+    o.fit(dev.model, graphs, Y)
+    ta, banks, w = dev.download()
+    assert np.array_equal(w, dev.model.clause_weights) and np.array_equal(ta, dev.model.ta_state)
+    assert all(np.array_equal(a, b) for a, b in zip(banks, dev.model.message_ta_state))
+
+    asked = []
+
+    def no_room(self, nbytes):
+        asked.append(nbytes)
+        if len(asked) == 1:
+            raise torch.OutOfMemoryError("no room")
+        return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device="cuda")
+
+    monkeypatch.setattr(tm_module.CommonTsetlinMachine, "_workspace_of", no_room)
+    states = []
+    for attempt in range(2):  # (the second has room at once)
+        asked[:] = [0] * attempt
+        np.random.seed(3)
+        tm = tm_module.MultiClassGraphTsetlinMachine(clauses, 30, 2.0, depth=3, message_size=64, message_bits=2, seed=3)
+        tm.fit(graphs, np.array([0, 1, 2, 0]), epochs=2)
+        states.append(tm.get_state())
+        assert attempt == 1 or asked[1] < asked[0]
+    assert np.array_equal(states[0][0], states[1][0]) and np.array_equal(states[0][1], states[1][1])
