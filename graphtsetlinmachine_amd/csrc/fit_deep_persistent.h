@@ -119,29 +119,47 @@ inline size_t fit_deep_lds_words(bool big, int depth, int literals, int per_grou
            (big ? (size_t)(FITD_BLOCK / 64) * FIT_QUEUE : 0) + 64;
 }
 
-// What the cooperative kernel has to know about the edges of a run of examples: [0] most edges of
-// one graph, [1] largest edge type, [2] != 0 when some graph's edges are not stored node after node
-// (edge_index[n + 1] == edge_index[n] + number_of_graph_node_edges[n]) or point outside the graph.
-// One workgroup per example.
-__global__ void k_edge_limits(const uint32_t *__restrict__ n_nodes, const uint32_t *__restrict__ node_index,
-                              const uint32_t *__restrict__ n_edges, const uint32_t *__restrict__ edge_index,
-                              const uint32_t *__restrict__ edge, int first_example, uint32_t *out) {
+// What the one-launch kernels have to know about the edges of a run of examples, in the words of a header that are zero on entry:
+// the (type, offset) pairs and whether they are all (as k_edge_moves, if `moves`), then what FITD_EDGES_* name.  One look for
+// k_fit_moves and k_fit_deep_persistent: a look of its own for each cost a data set that is no moves a launch and a wait more
+// per call (16 examples of 200 nodes with random edges 655 us, with one look 625).  One workgroup per example.
+constexpr int FITD_EDGES_MOST = TILE_MOVES_MAX + 1;       // most edges of one graph
+constexpr int FITD_EDGES_TYPE = TILE_MOVES_MAX + 2;       // largest edge type
+constexpr int FITD_EDGES_IRREGULAR = TILE_MOVES_MAX + 3;  // != 0: some graph's edges are not stored node after node, or point outside the graph
+static_assert(FITD_EDGES_IRREGULAR < TILE_MOVES_HEADER_WORDS, "");
+__global__ __launch_bounds__(256) void k_fit_edge_look(const uint32_t *__restrict__ n_nodes, const uint32_t *__restrict__ node_index,
+                                                       const uint32_t *__restrict__ n_edges, const uint32_t *__restrict__ edge_index,
+                                                       const uint32_t *__restrict__ edge, int first_example, int moves, uint32_t *header) {
+    __shared__ uint32_t keys[TILE_MOVES_MAX], too_many;
+    if (threadIdx.x < TILE_MOVES_MAX) keys[threadIdx.x] = 0u;
+    // (another workgroup may have found too many already)
+    if (threadIdx.x == 0) too_many = moves ? __hip_atomic_load(&header[TILE_MOVES_MAX], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 1u;
+    __syncthreads();
     const int ex = first_example + (int)blockIdx.x;
-    const int n = (int)n_nodes[ex];
-    if (n == 0) return;
+    const uint32_t n = n_nodes[ex];
+    if (n == 0u) return;
     const int64_t base = node_index[ex];
     const uint32_t e0 = edge_index[base];
     const uint32_t total = edge_index[base + n - 1] + n_edges[base + n - 1] - e0;
     uint32_t irregular = 0u, top = 0u;
-    for (int j = threadIdx.x; j < n - 1; j += blockDim.x)
-        irregular |= edge_index[base + j + 1] != edge_index[base + j] + n_edges[base + j];
+    for (uint32_t j = threadIdx.x; j + 1 < n; j += blockDim.x) irregular |= edge_index[base + j + 1] != edge_index[base + j] + n_edges[base + j];
     for (uint32_t e = threadIdx.x; e < total && total < (1u << 24); e += blockDim.x) {
-        irregular |= edge[(int64_t)(e0 + e) * 2] >= (uint32_t)n;
+        irregular |= edge[(int64_t)(e0 + e) * 2] >= n;
         top = max(top, edge[(int64_t)(e0 + e) * 2 + 1]);
     }
-    if (threadIdx.x == 0) atomicMax(&out[0], total);
-    if (top) atomicMax(&out[1], top);
-    if (irregular) atomicOr(&out[2], 1u);
+    if (threadIdx.x == 0) atomicMax(&header[FITD_EDGES_MOST], total);
+    if (top) atomicMax(&header[FITD_EDGES_TYPE], top);
+    if (irregular) atomicOr(&header[FITD_EDGES_IRREGULAR], 1u);
+    for (uint32_t v = threadIdx.x; v < n; v += blockDim.x) {
+        const uint32_t count = n_edges[base + v];
+        const uint2 *out_edges = reinterpret_cast<const uint2 *>(edge) + edge_index[base + v];
+        for (uint32_t e = 0; e < count; ++e) {
+            if (*(volatile uint32_t *)&too_many) break;
+            if (!tile_move_noted(keys, tile_move_key(v, out_edges[e].x, out_edges[e].y, n))) too_many = 1u;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) tile_moves_publish(keys, too_many, header);
 }
 
 __device__ __forceinline__ uint32_t fitd_load(const uint32_t *p) {

@@ -59,55 +59,11 @@ struct FitMovesParams {
     int max_nodes;
 };
 
-inline int fitm_octets(int entries) { return (entries + 7) / 8; }
 inline size_t fit_moves_lds_words(bool regs, bool rows_lds, int depth, int own, int LA, int MC, int MB, int M, int K, int S, int rows_words,
                                   int list0, int listm, int n_moves) {
     const size_t o = (size_t)own, words = (size_t)LA + (size_t)(depth - 1) * MC;
     return (size_t)M * S + (rows_lds ? 2 * (size_t)rows_words : 0) + (regs ? o * (list0 + (depth - 1) * listm) / 2 : 0) + o * S +
            2 * (size_t)n_moves * S + o * words + 3 * o * K + 4 * o + 4 * o * depth + 6 * o + o * n_moves * MB + o * (MC / 2);
-}
-
-// The (type, offset) pairs of a run's edges -> header (zero on entry; as k_edge_moves).  One workgroup per example.
-__global__ void k_fit_edge_moves(const uint32_t *__restrict__ n_nodes, const uint32_t *__restrict__ node_index,
-                                 const uint32_t *__restrict__ n_edges, const uint32_t *__restrict__ edge_index,
-                                 const uint32_t *__restrict__ edge, int first_example, uint32_t *header) {
-    __shared__ uint32_t keys[TILE_MOVES_MAX], too_many;
-    if (threadIdx.x < TILE_MOVES_MAX) keys[threadIdx.x] = 0u;
-    if (threadIdx.x == 0) too_many = 0u;
-    __syncthreads();
-    const int ex = first_example + (int)blockIdx.x;
-    const uint32_t n = n_nodes[ex];
-    const int64_t base = node_index[ex];
-    for (uint32_t v = threadIdx.x; v < n; v += blockDim.x) {
-        const uint32_t count = n_edges[base + v];
-        const uint2 *out_edges = reinterpret_cast<const uint2 *>(edge) + edge_index[base + v];
-        for (uint32_t e = 0; e < count; ++e) {
-            if (*(volatile uint32_t *)&too_many) break;
-            const uint32_t key = tile_move_key(v, out_edges[e].x, out_edges[e].y, n);
-            int k = 0;
-            if (key)
-                for (; k < TILE_MOVES_MAX; ++k) {
-                    uint32_t held = *(volatile uint32_t *)&keys[k];
-                    if (held == 0u) held = atomicCAS(&keys[k], 0u, key);
-                    if (held == key || held == 0u) break;
-                }
-            if (key == 0u || k == TILE_MOVES_MAX) too_many = 1u;
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t lost = too_many;
-        for (int j = 0; j < TILE_MOVES_MAX && keys[j] && !lost; ++j) {
-            int k = 0;
-            for (; k < TILE_MOVES_MAX; ++k) {
-                uint32_t held = __hip_atomic_load(&header[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (held == 0u) held = atomicCAS(&header[k], 0u, keys[j]);
-                if (held == keys[j] || held == 0u) break;
-            }
-            if (k == TILE_MOVES_MAX) lost = 1u;
-        }
-        if (lost) atomicOr(&header[TILE_MOVES_MAX], 1u);
-    }
 }
 
 // masks[example][move][S]: the nodes where an edge of the move ends.  One workgroup per example; LDS: n * S words.

@@ -2535,6 +2535,27 @@ int fit_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
     return GTM_OK;
 }
 
+// What k_fit_edge_look found in a call's examples; it lies at w.coop_got as well until a launch exchanges rows there.
+struct EdgeLook {
+    bool looked;
+    uint32_t found[TILE_MOVES_HEADER_WORDS];
+};
+int look_at_edges(const gtm_graphs *g, const FitWs &w, int first_example, int n_examples, bool moves, hipStream_t st, EdgeLook *look) {
+    if (look->looked) return GTM_OK;
+    if (!g->number_of_graph_node_edges || !g->edge || !g->edge_index)
+        return fail(GTM_ERR_INVALID, "graphs with edges need number_of_graph_node_edges, edge and edge_index");
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(TPB), 0, st, (int32_t *)w.coop_got, (int64_t)TILE_MOVES_HEADER_WORDS, 0);
+    if (int rc = check_launch("fill")) return rc;
+    hipLaunchKernelGGL(k_fit_edge_look, dim3(n_examples), dim3(256), 0, st, g->number_of_graph_nodes, g->node_index,
+                       g->number_of_graph_node_edges, g->edge_index, g->edge, first_example, moves ? 1 : 0, w.coop_got);
+    if (int rc = check_launch("k_fit_edge_look")) return rc;
+    hipError_t e = hipMemcpyAsync(look->found, w.coop_got, sizeof look->found, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) return fail(GTM_ERR_HIP, "looking at the edges: %s", hipGetErrorString(e));
+    look->looked = true;
+    return GTM_OK;
+}
+
 // `_fit`'s inner loop of a model with message layers as one cooperative launch (fit_deep_persistent.h).
 // Returns GTM_OK with *done = false when this device or shape cannot run it, so that the caller
 // falls back to the launches per example.  GTM_NO_DEEP_PERSISTENT_FIT (tuning aid) turns it off.
@@ -2543,7 +2564,7 @@ int fit_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
 // when a launch gave up (the model is then as it was before that launch).
 int fit_deep_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const gtm_state *s, const TileGeom &tg,
                         const FitWs &w, const int32_t *encoded_Y, int first_example, int n_examples, uint64_t first_step,
-                        hipStream_t st, bool *done, int *examples_done) {
+                        hipStream_t st, EdgeLook *look, bool *done, int *examples_done) {
     *done = false;
     *examples_done = 0;
     if (tune(T_NO_DEEP_PERSISTENT_FIT) || tune(T_NO_PERSISTENT_FIT) || cfg->depth < 2 || d.K > FITD_BLOCK) return GTM_OK;
@@ -2552,8 +2573,6 @@ int fit_deep_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *
     if (hipGetDevice(&dev) != hipSuccess) return GTM_OK;
     if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !coop) return GTM_OK;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) return GTM_OK;
-    if (g->total_edges > 0 && (!g->number_of_graph_node_edges || !g->edge || !g->edge_index))
-        return fail(GTM_ERR_INVALID, "graphs with edges need number_of_graph_node_edges, edge and edge_index");
 
     const int layers = cfg->depth - 1, MW = d.M / 32;
     int per_group = (d.C + cus - 1) / cus;
@@ -2562,19 +2581,11 @@ int fit_deep_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *
     const int NW = d.NC;
     const int rows_words = (cfg->literals + g->number_of_node_types + 1) * NW;
     // the edges of the run's examples: most per graph, largest type, stored node after node?
-    uint32_t limits[3] = {0u, 0u, 0u};
-    if (g->total_edges > 0) {
-        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(TPB), 0, st, (int32_t *)w.coop_got, (int64_t)3, 0);
-        if (int rc = check_launch("fill")) return rc;
-        hipLaunchKernelGGL(k_edge_limits, dim3(n_examples), dim3(256), 0, st, g->number_of_graph_nodes, g->node_index,
-                           g->number_of_graph_node_edges, g->edge_index, g->edge, first_example, w.coop_got);
-        if (int rc = check_launch("k_edge_limits")) return rc;
-        hipError_t e = hipMemcpyAsync(limits, w.coop_got, sizeof(limits), hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
-        if (e != hipSuccess) return fail(GTM_ERR_HIP, "reading the edge limits: %s", hipGetErrorString(e));
-        if (limits[2] != 0u || limits[1] >= (uint32_t)FITD_MAX_EDGE_TYPES || limits[0] > (1u << 20)) return GTM_OK;
-    }
-    const int edge_cap = (int)limits[0], edge_types = (int)limits[1] + 1;
+    if (g->total_edges > 0)
+        if (int rc = look_at_edges(g, w, first_example, n_examples, false, st, look)) return rc;
+    const uint32_t most_edges = look->found[FITD_EDGES_MOST], largest_type = look->found[FITD_EDGES_TYPE];
+    if (look->found[FITD_EDGES_IRREGULAR] != 0u || largest_type >= (uint32_t)FITD_MAX_EDGE_TYPES || most_edges > (1u << 20)) return GTM_OK;
+    const int edge_cap = (int)most_edges, edge_types = (int)largest_type + 1;
     // automata, layer-0 rows and all received rows in LDS where they fit; else automata in memory, rows in
     // place and as wide a window of received rows as fits
     const size_t lds_cap = 158 * 1024;  // of 160 KiB; the kernel has a few words of its own
@@ -2769,7 +2780,7 @@ int fit_deep_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *
 
 // The same for data sets whose edges are a few moves (fit_moves.h).
 int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const gtm_state *s, const TileGeom &tg, const FitWs &w,
-              const int32_t *encoded_Y, int first_example, int n_examples, uint64_t first_step, hipStream_t st, bool *done,
+              const int32_t *encoded_Y, int first_example, int n_examples, uint64_t first_step, hipStream_t st, EdgeLook *look, bool *done,
               int *examples_done) {
     *done = false;
     *examples_done = 0;
@@ -2780,8 +2791,6 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) return GTM_OK;
     if (g->total_edges == 0 || cfg->max_nodes < 2) return GTM_OK;  // nothing to shift: as before
     if (cfg->literals + std::min(d.C, g->number_of_node_types) > 65536) return GTM_OK;  // (the last type row's 16-bit number)
-    if (!g->number_of_graph_node_edges || !g->edge || !g->edge_index)
-        return fail(GTM_ERR_INVALID, "graphs with edges need number_of_graph_node_edges, edge and edge_index");
 
     const int layers = cfg->depth - 1, S = fitl_stride(d.NC), per_group = fit_moves_per_group(d, cus), groups = (d.C + per_group - 1) / per_group;
     if (per_group > 512 || (size_t)groups * per_group > (size_t)d.C + 2048) return GTM_OK;
@@ -2798,16 +2807,9 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
     };
     if (layout_of(0) < 0) return GTM_OK;
 
-    uint32_t found[TILE_MOVES_HEADER_WORDS] = {};
+    if (int rc = look_at_edges(g, w, first_example, n_examples, true, st, look)) return rc;
+    const uint32_t *found = look->found;
     uint32_t *header = w.coop_got;
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(TPB), 0, st, (int32_t *)header, (int64_t)TILE_MOVES_HEADER_WORDS, 0);
-    if (int rc = check_launch("fill")) return rc;
-    hipLaunchKernelGGL(k_fit_edge_moves, dim3(n_examples), dim3(256), 0, st, g->number_of_graph_nodes, g->node_index,
-                       g->number_of_graph_node_edges, g->edge_index, g->edge, first_example, header);
-    if (int rc = check_launch("k_fit_edge_moves")) return rc;
-    hipError_t looked = hipMemcpyAsync(found, header, sizeof found, hipMemcpyDeviceToHost, st);
-    if (looked == hipSuccess) looked = hipStreamSynchronize(st);
-    if (looked != hipSuccess) return fail(GTM_ERR_HIP, "reading the edges' moves: %s", hipGetErrorString(looked));
     if (found[TILE_MOVES_MAX] != 0u || found[0] == 0u) return GTM_OK;
     while (p.moves.n < TILE_MOVES_MAX && found[p.moves.n] != 0u) {
         const uint32_t key = found[p.moves.n];
@@ -2911,7 +2913,7 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
         }
         {
             if (at > 0) {  // (the header lies in the rows that the launch before exchanged)
-                hipError_t e = hipMemcpyAsync(header, found, sizeof found, hipMemcpyHostToDevice, st);
+                hipError_t e = hipMemcpyAsync(header, found, sizeof look->found, hipMemcpyHostToDevice, st);
                 if (e != hipSuccess) return fail(GTM_ERR_HIP, "the edges' moves: %s", hipGetErrorString(e));
             }
             hipLaunchKernelGGL(k_fit_move_masks, dim3(n_now), dim3(256), (size_t)p.moves.n * S * 4, st, g->number_of_graph_nodes, g->node_index,
@@ -3332,11 +3334,13 @@ int gtm_fit(const gtm_config *cfg, const gtm_graphs *graphs, const gtm_state *st
         if (tg.ok && tg.slot_words <= 64 && cfg->max_nodes <= 2048) {  // one lane per word of the graph's nodes
             bool done = false;
             int so_far = 0;  // examples that launches which did not give up have trained on
-            if (int rc = fit_moves(d, cfg, graphs, state, tg, w, encoded_Y, first_example, n_examples, first_step, st, &done, &so_far)) return rc;
+            EdgeLook look{};
+            if (int rc = fit_moves(d, cfg, graphs, state, tg, w, encoded_Y, first_example, n_examples, first_step, st, &look, &done, &so_far))
+                return rc;
             if (done) return GTM_OK;
             first_example += so_far, n_examples -= so_far, first_step += (uint64_t)so_far, h_n += so_far, h_base += so_far;
             if (int rc = fit_deep_persistent(d, cfg, graphs, state, tg, w, encoded_Y, first_example, n_examples, first_step, st,
-                                             &done, &so_far))
+                                             &look, &done, &so_far))
                 return rc;
             if (done) return GTM_OK;
             first_example += so_far, n_examples -= so_far, first_step += (uint64_t)so_far, h_n += so_far, h_base += so_far;

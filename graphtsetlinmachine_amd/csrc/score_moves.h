@@ -34,6 +34,30 @@ __device__ __forceinline__ uint32_t tile_move_key(uint32_t from, uint32_t to, ui
     return to < n && type < TILE_MOVE_TYPES && d - 1u < 2u * TILE_MOVE_OFFSET - 1u ? (type << 16) | d : 0u;
 }
 
+// A key into a workgroup's table in LDS, where it is not there yet; false: it is no key, or there is no room.
+__device__ __forceinline__ bool tile_move_noted(uint32_t *keys, uint32_t key) {
+    if (key == 0u) return false;
+    for (int k = 0; k < TILE_MOVES_MAX; ++k) {
+        uint32_t held = *(volatile uint32_t *)&keys[k];
+        if (held == 0u) held = atomicCAS(&keys[k], 0u, key);
+        if (held == key || held == 0u) return true;
+    }
+    return false;
+}
+// A workgroup's table -> the header in memory (one thread).
+__device__ __forceinline__ void tile_moves_publish(const uint32_t *keys, uint32_t lost, uint32_t *header) {
+    for (int j = 0; j < TILE_MOVES_MAX && keys[j] && !lost; ++j) {
+        int k = 0;
+        for (; k < TILE_MOVES_MAX; ++k) {
+            uint32_t held = __hip_atomic_load(&header[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (held == 0u) held = atomicCAS(&header[k], 0u, keys[j]);
+            if (held == keys[j] || held == 0u) break;
+        }
+        if (k == TILE_MOVES_MAX) lost = 1u;
+    }
+    if (lost) atomicOr(&header[TILE_MOVES_MAX], 1u);
+}
+
 // The node in slot `pos` of a tile: its place in the data set's node arrays, its number in its graph and the graph's
 // nodes and first slot; false when there is none.
 __device__ __forceinline__ bool tile_slot_node(const TileGeom &tg, int tile, int pos, int G, const uint32_t *node_index,
@@ -73,31 +97,11 @@ __global__ __launch_bounds__(TILE_MOVES_BLOCK) void k_edge_moves(TileGeom tg, in
         for (uint32_t e = 0; e < count; ++e) {
             if (*(volatile uint32_t *)&too_many) break;
             const uint2 to = out_edges[e];
-            const uint32_t key = tile_move_key(n, to.x, to.y, nodes);
-            int k = 0;
-            if (key)
-                for (; k < TILE_MOVES_MAX; ++k) {
-                    uint32_t held = *(volatile uint32_t *)&keys[k];
-                    if (held == 0u) held = atomicCAS(&keys[k], 0u, key);
-                    if (held == key || held == 0u) break;
-                }
-            if (key == 0u || k == TILE_MOVES_MAX) too_many = 1u;
+            if (!tile_move_noted(keys, tile_move_key(n, to.x, to.y, nodes))) too_many = 1u;
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t lost = too_many;
-        for (int j = 0; j < TILE_MOVES_MAX && keys[j] && !lost; ++j) {
-            int k = 0;
-            for (; k < TILE_MOVES_MAX; ++k) {
-                uint32_t held = __hip_atomic_load(&header[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (held == 0u) held = atomicCAS(&header[k], 0u, keys[j]);
-                if (held == keys[j] || held == 0u) break;
-            }
-            if (k == TILE_MOVES_MAX) lost = 1u;
-        }
-        if (lost) atomicOr(&header[TILE_MOVES_MAX], 1u);
-    }
+    if (threadIdx.x == 0) tile_moves_publish(keys, too_many, header);
 }
 
 // masks[tile][move][tw]: the slots where an edge of the move ends.  One workgroup per tile at a time; nothing when
