@@ -300,7 +300,7 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_persistent(FitPersistParams 
             } else {
                 const uint2 acc = included < p.lists ? fitl_truth(list, included + 1, col, stride, p.lanes_log, lane)
                                                      : fitl_walk(inc, B, LA, p.filter, p.literals + (one_type ? 0 : c % p.n_types),
-                                                                 ones_row, col, stride, lane);
+                                                                 ones_row, col, stride, p.lanes_log, lane);
                 v = fitl_nodes(acc, fg, p.lanes_log, lane);
             }
             const int node = n_now == 0 ? -1 : fitl_pick_node(v, pick_of[cl], lane);
