@@ -14,8 +14,8 @@
 //   3. decides the feedback and updates its automata and weights in LDS: the
 //      (clause, class) pairs that need Type I bits and the clauses that get any
 //      feedback are listed, so that every thread has a byte to draw or a word to update.
-// Single-node images of 128 literal words, 2,500 clauses: 9.4 us per example before the lists, with every
-// (clause, word) looking at all its classes and a word's four generator calls in one thread; now 6.0.
+// Single-node images of 128 literal words, 2,500 clauses: 14.4 us per example with every (clause, word) looking at all
+// its classes and a word's four generator calls in one thread; now 10.5.
 // Class sums and barrier are one thing: class k has a 64-bit word (kept as
 // FITP_SUM_PARTS partial words that a reader adds up, since the memory system
 // carries out the adds to one word one after the other) to which every
@@ -230,9 +230,7 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_persistent(FitPersistParams 
     lds_barrier();
 
     const int ones_row = p.literals + p.n_types;
-    int quarter_log = 2, word_log = 0;  // 2^quarter_log >= 4 LA lanes draw a clause's Type I bytes for one class, 2^word_log >= LA update its words
-    while ((1 << word_log) < LA && word_log < 10) ++word_log;
-    while ((1 << quarter_log) < 4 * LA && quarter_log < 10) ++quarter_log;
+    const uint32_t by_words = 0xFFFFFFFFu / (uint32_t)LA, by_bytes = 0xFFFFFFFFu / (uint32_t)(4 * LA);  // (a quotient from them is one too low at most)
     FitRowLoader loader{};
     int loader_words = 0;
     // The threads that add the group's votes to the device-wide class sums and then poll for them are the first K
@@ -468,31 +466,31 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_persistent(FitPersistParams 
             if (atomicOr(&stale[cl], 2u) < 2u) busy_list[atomicAdd(&n_busy, 1)] = cl;
         }
         lds_barrier();
-        // a thread per byte of Type I bits, 2^quarter_log threads per pair
-        for (int t = tid; t < n_pairs << quarter_log; t += FITP_BLOCK) {
-            const int j = pair_list[t >> quarter_log], cl = j / K, k = j - cl * K;
-            for (int item = t & ((1 << quarter_log) - 1); item < 4 * LA; item += 1 << quarter_log) {
-                const int w = item >> 2, q = item & 3;
-                ((uint8_t *)&fbits[((size_t)cl * LA + w) * K + k])[q] =
-                    (uint8_t)fitl_feedback_byte(p.k0, p.k1, (uint32_t)(c0 + cl), (uint32_t)w, (uint32_t)q, step, 0u, (uint32_t)k, p.thr16);
-            }
+        // a thread per byte of Type I bits (with 2^n threads per pair and clause, half of them idle just above 128 words, an example of
+        // 150 words and 1,000 clauses took 11.9 us on single nodes, 9.6 now)
+        for (int t = tid; t < n_pairs * 4 * LA; t += FITP_BLOCK) {
+            int pair = (int)__umulhi((uint32_t)t, by_bytes), item = t - pair * 4 * LA;
+            if (item >= 4 * LA) item -= 4 * LA, ++pair;
+            const int j = pair_list[pair], cl = j / K, k = j - cl * K, w = item >> 2, q = item & 3;
+            ((uint8_t *)&fbits[((size_t)cl * LA + w) * K + k])[q] =
+                (uint8_t)fitl_feedback_byte(p.k0, p.k1, (uint32_t)(c0 + cl), (uint32_t)w, (uint32_t)q, step, 0u, (uint32_t)k, p.thr16);
         }
         lds_barrier();
-        for (int t = tid; t < n_busy << word_log; t += FITP_BLOCK) {
-            const int cl = busy_list[t >> word_log];
+        for (int t = tid; t < n_busy * LA; t += FITP_BLOCK) {
+            int at = (int)__umulhi((uint32_t)t, by_words), w = t - at * LA;
+            if (w >= LA) w -= LA, ++at;
+            const int cl = busy_list[at];
             const int node = node_of[cl];
             const bool fired = node != -1;
             const bool learns = fired && incl_of[cl] <= p.max_included;
-            for (int w = t & ((1 << word_log) - 1); w < LA; w += 1 << word_log) {
-                const uint32_t x = fired ? literal_word(cl, node, w) : 0u;
-                fits_word<MAXB, EXACT> word(planes_of(cl, w), B);
-                const uint32_t was = word.top();
-                const uint32_t *fb_of = fbits + ((size_t)cl * LA + w) * K;
-                for (int kw = 0; kw < KW; ++kw)
-                    fitl_feedback(word, pos_of[cl * KW + kw], neg_of[cl * KW + kw], fired, learns, p.boost, x, fb_of + 32 * kw);
-                word.store(planes_of(cl, w));
-                if (word.top() != was) atomicOr(&stale[cl], 1u);
-            }
+            const uint32_t x = fired ? literal_word(cl, node, w) : 0u;
+            fits_word<MAXB, EXACT> word(planes_of(cl, w), B);
+            const uint32_t was = word.top();
+            const uint32_t *fb_of = fbits + ((size_t)cl * LA + w) * K;
+            for (int kw = 0; kw < KW; ++kw)
+                fitl_feedback(word, pos_of[cl * KW + kw], neg_of[cl * KW + kw], fired, learns, p.boost, x, fb_of + 32 * kw);
+            word.store(planes_of(cl, w));
+            if (word.top() != was) atomicOr(&stale[cl], 1u);
         }
         lds_barrier();
         slot = slot == 2 ? 0 : slot + 1;
