@@ -98,7 +98,7 @@ constexpr int FITP_SUM_STRIDE = 16;                      // 64-bit words between
 // reader adds the parts up (the protocol is linear in the word). Adds to one word are carried out
 // one after the other by the memory system, so fewer groups per word shorten the exchange.
 constexpr int FITP_SUM_PARTS = 16;
-constexpr int FITP_DIRECT_NODES = 2;  // data sets whose graphs have at most this many nodes skip the literal rows altogether
+constexpr int FITP_DIRECT_NODES = 32;  // a node of a directly tested graph is a bit of a word
 
 // One 32-bit word per lane from global memory straight into LDS (no register holds it meanwhile):
 // lane l's word lands at dst_of_wave[l]; dst_of_wave must be the same for the whole wave. The words
@@ -281,18 +281,19 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_persistent(FitPersistParams 
             }
             uint2 v;
             if constexpr (DIRECT) {
-                // one or two nodes: the clause against each node's own literal words (kernels.py:443-466 as
+                // a few nodes: the clause against each node's own literal words (kernels.py:443-466 as
                 // it stands), lane w on word w; no literal-major rows are read or staged
-                uint32_t bits = 0u;
-                for (int node = 0; node < n_now; ++node) {
-                    bool violated = false;
-                    for (int w0 = 0; w0 < LA; w0 += 64) {
-                        uint32_t mine = w0 + lane < LA ? inc[(w0 + lane) * B] : 0u;
-                        if (w0 + lane == LA - 1) mine &= p.filter;
-                        const uint32_t xs = w0 + lane < LA ? x_now[node * LA + w0 + lane] : 0xFFFFFFFFu;
-                        violated |= __ballot((mine & ~xs) != 0) != 0;
-                    }
-                    if (!violated && (int)types_lds[i & 1][node] == (one_type ? 0 : c % p.n_types)) bits |= 1u << node;
+                const uint32_t type = lane < n_now ? types_lds[i & 1][lane] : 0xFFFFFFFFu;
+                uint32_t bits = (uint32_t)__ballot((int)type == (one_type ? 0 : c % p.n_types));
+                for (int w0 = 0; w0 < LA && bits != 0u; w0 += 64) {
+                    const bool there = w0 + lane < LA;
+                    uint32_t mine = there ? inc[(w0 + lane) * B] : 0u;
+                    if (w0 + lane == LA - 1) mine &= p.filter;
+                    const uint32_t *xs = x_now + (there ? w0 + lane : 0);
+                    uint32_t violated = 0u;
+#pragma unroll 4
+                    for (int node = 0; node < n_now; ++node) violated |= (uint32_t)(__ballot((mine & ~xs[node * LA]) != 0u) != 0ull) << node;
+                    bits &= ~violated;
                 }
                 v = make_uint2(lane == 0 ? bits : 0u, 0u);
             } else {

@@ -2400,8 +2400,14 @@ int fit_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
 
     FitPersistParams p{};
     p.max_words = tg.slot_words > 0 ? tg.slot_words : 1;
-    // graphs of one or two nodes: the nodes are tested on their own literal words, no rows are staged
-    const bool direct = g->max_number_of_graph_nodes <= FITP_DIRECT_NODES && !tune(T_NO_DIRECT_FIT);
+    // Graphs of one or two nodes: the nodes are tested on their own literal words, no rows are staged.  So are graphs of up to 32
+    // nodes with at least as many literal words, where the words are too many for k_fit_waves: a clause that holds reads a row for
+    // every literal that it includes, and its list is made of all its words, while a node costs a wave's read per 64 words.  us per
+    // example on rows and here, 1,000 clauses: 5 nodes of 2,000 literals 14.7 and 6.7, of 4,800 (their lists do not fit) 33 and
+    // 9.9; 32 nodes of 1,200 10.7 and 7.7, of 600 (19 words) 7.7 and 7.9, late in training 6.9 and 7.9.  9,600 literals: the rows do
+    // not fit, 75 and 14.
+    const int nodes = g->max_number_of_graph_nodes;
+    const bool direct = (nodes <= 2 || (d.LA > FITV_MAX_WORDS && nodes <= std::min(d.LA, FITP_DIRECT_NODES))) && !tune(T_NO_DIRECT_FIT);
     p.node_type = g->node_type;
     p.rows_words = direct ? 0 : (cfg->literals + g->number_of_node_types + 1) * fitl_stride(p.max_words);
     p.x_words = direct ? (g->max_number_of_graph_nodes > 0 ? g->max_number_of_graph_nodes : 1) * d.LA : 0;
@@ -2425,8 +2431,8 @@ int fit_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
     p.lanes_log = fitl_lanes_log(p.max_words);
     p.lists = direct ? 0 : fitl_entries(cfg->literals, p.lanes_log);
     // A wave per clause with its state in registers where the clauses are small enough (us per example, waves against
-    // state in LDS: 361 nodes, 2,500 clauses of 8 words, 10 classes 5.2 against 6.3; 81 nodes, 250 clauses of 4 words 3.3
-    // against 5.1; ragged chains of up to 300 nodes, 150 clauses 4.1 against 6.3); else the state in LDS, and as much of the lists
+    // state in LDS: 361 nodes, 2,500 clauses of 8 words, 10 classes 5.7 against 6.6; 81 nodes, 250 clauses of 4 words 3.6
+    // against 5.3; ragged chains of up to 300 nodes, 150 clauses 3.7 against 5.5); else the state in LDS, and as much of the lists
     // and of the picked nodes' literal words as it has room for (a clause with more literals than its list holds walks
     // its include plane instead).
     const bool waves = !direct && per_group <= FITP_BLOCK / 64 && d.K <= FITV_MAX_CLASSES && d.LA <= FITV_MAX_WORDS &&

@@ -2,6 +2,8 @@
 rows of 1 to 64 words, 16 and 17 literal words, 63 and 64 classes, clauses longer than their list - every split follows
 the oracle bit for bit (whole numbers: no tolerance)."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -62,3 +64,28 @@ def test_feedback_of_many_literal_words(hv_size, max_nodes, s, per_group, tune):
     """Single nodes and pairs of thousands of literals: Type I bits a byte per thread, feedback of the clauses that get any."""
     graphs = helpers.random_graphs(hv_size, n_graphs=30, max_nodes=max_nodes, hv_size=hv_size, n_symbols=40, max_degree=0)
     follow(graphs, tune, {} if per_group is None else {"GTM_FIT_PER_GROUP": per_group}, classes=10, clauses=45, density=0.02, s=s)
+
+
+@pytest.mark.parametrize("sizes,hv_size,clauses,kernel", [
+    ([5, 3, 0, 1, 4], 4800, 20, b"k_fit_persistent"),    # 300 words: rows of as many literals have no room
+    ([3, 5, 2], 3300, 2100, b"k_fit_persistent"),         # nine clauses a workgroup: nor have lists
+    ([32, 31, 7, 0, 1], 512, 21, b"k_fit_persistent"),    # 32 words, 32 nodes: the last graphs tested node by node
+    ([32, 31, 7, 0, 1], 496, 21, b"k_fit_persistent"),    # 31 words: the first on rows
+    ([17, 16, 2], 264, 21, b"k_fit_persistent"),          # 17 words
+    ([17, 16, 2], 256, 21, b"k_fit_waves"),
+], ids=str)
+@pytest.mark.parametrize("density", [0.003, 0.3])
+def test_few_nodes_of_many_literals(sizes, hv_size, clauses, kernel, density, tune):
+    """Graphs of a few nodes whose words are too many for a wave per clause: one launch, whatever the number of literals."""
+    from graphtsetlinmachine_amd import _abi
+
+    graphs = helpers.random_graphs(hv_size, n_graphs=3 * len(sizes), sizes=sizes * 3, hv_size=hv_size, n_symbols=30, max_degree=0,
+                                   node_types=("a", "b", "c"))
+    name, launches, total = ctypes.c_char_p(), ctypes.c_int32(), ctypes.c_double()
+    _abi.call("gtm_profile_enable", 1)
+    try:
+        follow(graphs, tune, {}, classes=3, clauses=clauses, density=density)
+        _abi.call("gtm_profile_read", ctypes.byref(name), ctypes.byref(launches), ctypes.byref(total))
+    finally:
+        _abi.call("gtm_profile_enable", 0)
+    assert name.value == kernel, name.value
