@@ -59,6 +59,14 @@ struct FitMovesParams {
     int max_nodes;
 };
 
+// Do a workgroup's clauses send to so many rows that they meet in them?  ORed into memory one by one, the rows of short messages
+// were a queue of all clauses: us per example with the edges walked, ORed in memory, ORed in LDS first (chains of 20 nodes,
+// two moves, two bits a message): 20,000 clauses, 32-bit messages (316 rows sent by a workgroup) 90, 108, 31; 5,000 clauses, 32 bits
+// 36, 37, 22, 256 bits (80 rows) 34, 22.6, 21.0; 8,000 clauses, 1,024 bits, 100 nodes (128 rows) 79, 48, 50.  Automata in memory only: in
+// registers a workgroup has at most 16 clauses, which are ahead of the walk without (4,000 clauses, 32 bits 32 and 29).  A kernel of
+// its own: the choice inside one cost calls that do not collect up to 4 %.
+inline bool fit_moves_collects(int own, int n_moves, int MB, int M) { return 4 * (int64_t)own * n_moves * MB > M; }
+
 inline size_t fit_moves_lds_words(bool regs, bool rows_lds, int depth, int own, int LA, int MC, int MB, int M, int K, int S, int rows_words,
                                   int list0, int listm, int n_moves) {
     const size_t o = (size_t)own, words = (size_t)LA + (size_t)(depth - 1) * MC;
@@ -128,8 +136,8 @@ __device__ __forceinline__ uint2 fitm_rows(uint2 acc, const uint4 *list, int n8,
 }
 
 // MAXB, EXACT: the planes of an automaton (fits_word).  REGS: automata in registers, lists in LDS.  ROWS_LDS: the graph's layer-0 rows
-// are staged in LDS; else they are read from the tile in place.
-template <int MAXB, bool EXACT, bool REGS, bool ROWS_LDS>
+// are staged in LDS; else they are read from the tile in place.  COLLECT (not REGS): what the workgroup's clauses send is ORed in LDS first.
+template <int MAXB, bool EXACT, bool REGS, bool ROWS_LDS, bool COLLECT>
 __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
     extern __shared__ __align__(16) uint32_t lds[];
     __shared__ int32_t votes[64], sums[64], labels[2][64];
@@ -144,6 +152,7 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
     const int list_entries = p.list0 + L * p.listm;
 
     // LDS carve-up
+    static_assert(!(REGS && COLLECT), "");
     uint32_t *mrows = lds;                                              // [M][S] received rows of the current layer
     uint32_t *rows_both = mrows + (size_t)M * S;                        // ROWS_LDS: [2][rows_words] layer-0 rows of this and the next graph
     uint32_t *lists_lds = rows_both + (ROWS_LDS ? 2 * p.rows_words : 0);  // REGS: [own][list_entries] 16-bit entries
@@ -437,6 +446,11 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
             refresh();
             uint32_t *got_l = got_now + (size_t)l * layer_words;
             if (tid == 0) next_unit = 0, next_words = 0;
+            if constexpr (COLLECT) {  // (the rows received before are not read any more)
+                for (int at = tid; at < layer_words / 2; at += FITP_BLOCK) ((unsigned long long *)mrows)[at] = 0ull;
+                lds_barrier();
+                refresh();
+            }
             // a. what the own clauses make the nodes receive: their truth rows, shifted, where an edge of the move ends
             for (int u = tid >> row_log; u < n_own * NM; u += FITP_BLOCK >> row_log) {
                 const int cl = (u * by_moves) >> 16, k = u - cl * NM, w = SENT * (tid & ((1 << row_log) - 1));
@@ -454,11 +468,21 @@ __global__ __launch_bounds__(FITP_BLOCK) void k_fit_moves(FitMovesParams p) {
                 if (v != 0u)
                     for (int j = 0; j < p.MB; ++j) {
                         uint32_t *at = got_l + send_row[u * p.MB + j] * (uint32_t)S + w;
-                        if constexpr (SENT == 2)
+                        if constexpr (COLLECT)
+                            atomicOr((unsigned long long *)(mrows + (at - got_l)), (unsigned long long)v);
+                        else if constexpr (SENT == 2)
                             __hip_atomic_fetch_or((unsigned long long *)at, (unsigned long long)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                         else
                             __hip_atomic_fetch_or(at, (uint32_t)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     }
+            }
+            if constexpr (COLLECT) {
+                lds_barrier();
+                refresh();
+                for (int at = tid; at < layer_words / 2; at += FITP_BLOCK) {
+                    const unsigned long long v = ((const unsigned long long *)mrows)[at];
+                    if (v != 0ull) __hip_atomic_fetch_or((unsigned long long *)got_l + at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
             }
             __builtin_amdgcn_s_waitcnt(FITP_WAIT_VMEM);  // the ORs have been carried out where every workgroup sees them
             asm volatile("" ::: "memory");

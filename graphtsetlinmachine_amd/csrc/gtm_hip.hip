@@ -2829,12 +2829,14 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
     if (layout < 0) return GTM_OK;
     const bool rows_lds = layout == 0;
     const size_t lds = fit_moves_lds_bytes(d, cfg, per_group, layout < 2, rows_lds ? rows_words : 0, p.moves.n);
-    const int variant = (d.B == 8 ? 0 : 3) + layout;
-    const void *kernels[6] = {(const void *)k_fit_moves<8, true, true, true>,    (const void *)k_fit_moves<8, true, true, false>,
-                              (const void *)k_fit_moves<8, true, false, false>,  (const void *)k_fit_moves<16, false, true, true>,
-                              (const void *)k_fit_moves<16, false, true, false>, (const void *)k_fit_moves<16, false, false, false>};
+    const bool collect = layout == 2 && fit_moves_collects(per_group, p.moves.n, d.MB, d.M);
+    const int variant = (d.B == 8 ? 0 : 4) + layout + collect;
+    const void *kernels[8] = {(const void *)k_fit_moves<8, true, true, true, false>,     (const void *)k_fit_moves<8, true, true, false, false>,
+                              (const void *)k_fit_moves<8, true, false, false, false>,   (const void *)k_fit_moves<8, true, false, false, true>,
+                              (const void *)k_fit_moves<16, false, true, true, false>,   (const void *)k_fit_moves<16, false, true, false, false>,
+                              (const void *)k_fit_moves<16, false, false, false, false>, (const void *)k_fit_moves<16, false, false, false, true>};
     const void *kernel = kernels[variant];
-    static thread_local size_t lds_set_of[6] = {48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024};
+    static thread_local size_t lds_set_of[8] = {48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024};
     if (lds > lds_set_of[variant]) {
         if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
             (void)hipGetLastError();
