@@ -137,6 +137,12 @@ void gtm_pack_numbers(const uint32_t *in, int64_t n, int32_t bytes, void *out) {
     }
 }
 
+/* A new array's pages are made by whoever first writes to them; done by all threads while the device still works on what goes there. */
+void gtm_touch_pages(void *array, int64_t bytes) {
+#pragma omp parallel for schedule(static) if (bytes > 4 * PACK_PARALLEL)
+    for (int64_t at = 0; at < bytes; at += 4096) ((volatile char *)array)[at] = 0;
+}
+
 #define OUTPUTS_4(v) { (v) & 1, ((v) >> 1) & 1, ((v) >> 2) & 1, ((v) >> 3) & 1 }
 /* Clause outputs, which cross the bus as bits: out[i] = bit i % 32 of word i / 32.  Four outputs per table look-up; from
  * PACK_PARALLEL words on by all threads (a new array's pages are then also touched by all of them). */

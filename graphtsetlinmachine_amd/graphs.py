@@ -59,6 +59,8 @@ def _native_encoder():
         lib.gtm_pack_numbers.restype = None
         lib.gtm_pack_numbers.argtypes = [p, i64, i32, p]
         # (tm.py)
+        lib.gtm_touch_pages.restype = None
+        lib.gtm_touch_pages.argtypes = [p, i64]
         lib.gtm_unpack_outputs.restype = None
         lib.gtm_unpack_outputs.argtypes = [p, i64, p]
         _encoder = lib

@@ -48,24 +48,30 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None and t.numel() > 0 else ctypes.c_void_p(0)
 
 
-# Clause outputs from this many on cross the bus as bits and are made numbers again by all threads of the host; below, the launch
-# and the threads' waking take longer than what they save (us per call, bits and numbers: 100,000 outputs 139 and 122, 333,000 149
-# and 208, 1.3 million 265 and 539, 20 million per node 1,617 and 19,720).
+# Clause outputs from this many on cross the bus as bits and are made numbers again by the threads of the host, into an array whose pages
+# are touched while the device works.  us per call, bits and numbers, on a data set scored before and on one that was not:
+# 100,000 outputs 187 and 202, 437 and 431; 263,000 220 and 258, 449 and 496; 1.3 million 278 and 530, 612 and 862; 5.3 million 382 and
+# 5,500, 1,103 and 2,126; 19 million per node 1,443 and 18,700, 1,297 and 4,842 (8 threads; with one thread 263,000 234 and 260, 512 and
+# 553, 5.3 million 868 and 1,521 to 5,520, 2,729 and 3,355).  Pages touched only by the unpacking, data sets not scored before
+# took 538 us where they take 499, 728 (627), 1,250 (1,060): numbers were ahead up to 500,000 outputs.
 OUTPUTS_AS_BITS = 1 << 18
 # Bytes that are fetched through pinned memory, which torch keeps for the next call.
 PINNED_RESULT = 16 << 20
 
 
-def _to_host(t):
-    """t on the host, complete; through pinned memory where it is small and there is some."""
+def _to_host(t, meanwhile):
+    """t on the host, complete; through pinned memory where it is small and there is some.  `meanwhile` is called while the device works."""
     if t.numel() * t.element_size() <= PINNED_RESULT:
         try:
             out = torch.empty(t.shape, dtype=t.dtype, pin_memory=True)
         except RuntimeError:
-            return t.cpu()
-        out.copy_(t, non_blocking=True)
-        torch.cuda.current_stream().synchronize()
-        return out
+            out = None
+        if out is not None:
+            out.copy_(t, non_blocking=True)
+            meanwhile()
+            torch.cuda.current_stream().synchronize()
+            return out
+    meanwhile()
     return t.cpu()
 
 
@@ -618,8 +624,8 @@ class CommonTsetlinMachine:
         shape = (n, C, width) if nodewise else (n, C)
         if native:
             _abi.call("gtm_pack_outputs", _ptr(outputs), outputs.numel(), _ptr(result), _stream())
-            result = _to_host(result)
             out = np.empty(shape, dtype=np.int32)
+            result = _to_host(result, lambda: native.gtm_touch_pages(out.ctypes.data, out.nbytes))
             native.gtm_unpack_outputs(result.data_ptr(), out.size, out.ctypes.data)
             sums = result[words:].numpy().copy()
         else:

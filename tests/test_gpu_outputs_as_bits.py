@@ -20,6 +20,17 @@ def test_bits_become_outputs_again(n):
     assert np.array_equal(out[:n], want) and out[n] == 7
 
 
+@pytest.mark.parametrize("n", [0, 1, 4095, 4096, 4097, 8192, 70000, 1 << 20])
+def test_touching_pages_stays_in_the_array(n):
+    from graphtsetlinmachine_amd.graphs import _native_encoder
+
+    array = np.full(n + 8, 7, dtype=np.uint8)
+    _native_encoder().gtm_touch_pages(array.ctypes.data, n)
+    want = np.full(n + 8, 7, dtype=np.uint8)
+    want[:n:4096] = 0
+    assert np.array_equal(array, want)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 2048 * 1024 + 77])  # the last: more than one turn of the largest grid
 def test_outputs_become_bits(n):
@@ -55,10 +66,24 @@ def test_outputs_whichever_way_they_take(sizes, clauses, depth, monkeypatch):
     model.message_ta_state = [b.reshape(clauses, -1, 8) for b in state.message_ta_state]
     want, want_sums = o.transform(model, graphs)
     want_wide, _ = o.transform(model, graphs, nodewise=True)
+    native, calls = tm_module._native_encoder(), []
+    waited = tm_module.torch.cuda.Stream.synchronize
+
+    class Recorder:
+        def __getattr__(self, name):
+            return lambda *args: (calls.append(name), getattr(native, name)(*args))[1]
+
+    monkeypatch.setattr(tm_module, "_native_encoder", lambda: Recorder())
+    monkeypatch.setattr(tm_module.torch.cuda.Stream, "synchronize", lambda stream: (calls.append("wait"), waited(stream))[1])
     for bits_from, pinned in ((0, 1 << 24), (0, 0), (1 << 40, 0)):
         monkeypatch.setattr(tm_module, "OUTPUTS_AS_BITS", bits_from)
         monkeypatch.setattr(tm_module, "PINNED_RESULT", pinned)
+        calls.clear()
         got, sums = tm.transform(graphs)
+        # (a new array's pages are made while the device works, not after the wait)
+        seen = [c for c in calls if c in ("gtm_touch_pages", "wait", "gtm_unpack_outputs")]
+        want_calls = [] if bits_from else ["gtm_touch_pages"] + ["wait"] * bool(pinned) + ["gtm_unpack_outputs"]
+        assert seen[-len(want_calls):] == want_calls if want_calls else "gtm_unpack_outputs" not in seen
         assert got.dtype == sums.dtype == np.int32 and got.flags.writeable and sums.flags.writeable
         assert np.array_equal(got, want) and np.array_equal(sums, want_sums)
         got, sums = tm.transform_nodewise(graphs)
