@@ -2362,16 +2362,17 @@ int gtm_score_static(const gtm_config *cfg, const gtm_graphs *graphs, const gtm_
 
 namespace {
 
-// How long a device-wide wait of the one-launch training kernels may last: a poll cap that only the
-// tests use (GTM_FIT_SPIN_LIMIT = a number of polls, or "abort" = give up at the first wait whatever
-// it shows) and 5 seconds of the device's wall clock otherwise.
+// How long a device-wide wait of the one-launch training kernels may last: 5 seconds of the device's wall clock.  The tests bound
+// it otherwise (GTM_FIT_SPIN_LIMIT): a number of polls; "abort" = give up at the first wait whatever it shows, and report it; "from
+// N" = launches that start N examples into a kernel's run, or later, give up so, and the next way of training goes on.
 struct WaitBound {
     uint32_t spin_limit;
     unsigned long long wait_ticks;
-    int force_abort;
+    bool abort;
+    int give_up_from;
 };
 WaitBound wait_bound(int dev) {
-    WaitBound b{0xFFFFFFFFu, 0ull, 0};
+    WaitBound b{0xFFFFFFFFu, 0ull, false, INT_MAX};
     int khz = 0;
     if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0) {
         (void)hipGetLastError();
@@ -2379,8 +2380,13 @@ WaitBound wait_bound(int dev) {
     }
     b.wait_ticks = 5ull * 1000ull * (unsigned long long)khz;
     if (const char *e = tune(T_FIT_SPIN_LIMIT)) {
-        b.force_abort = strcmp(e, "abort") == 0;
-        if (!b.force_abort) b.spin_limit = (uint32_t)strtoul(e, nullptr, 10);
+        b.abort = strcmp(e, "abort") == 0;
+        if (b.abort)
+            b.give_up_from = 0;
+        else if (strncmp(e, "from ", 5) == 0)
+            b.give_up_from = atoi(e + 5);
+        else
+            b.spin_limit = (uint32_t)strtoul(e, nullptr, 10);
     }
     return b;
 }
@@ -2503,7 +2509,7 @@ int fit_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
     p.class_sum = (unsigned long long *)w.class_sum;
     p.abort_flag = (uint32_t *)((unsigned long long *)w.class_sum + (size_t)d.K * 3 * FITP_SUM_PARTS * FITP_SUM_STRIDE);
     const WaitBound bound = wait_bound(dev);
-    p.spin_limit = bound.spin_limit, p.wait_ticks = bound.wait_ticks, p.force_abort = bound.force_abort;
+    p.spin_limit = bound.spin_limit, p.wait_ticks = bound.wait_ticks, p.force_abort = bound.give_up_from <= 0;
     // A run that gives up leaves the workgroups at different examples.  The bank and the weights
     // are kept as they were, so that a failed call leaves the model as it found it.
     const size_t bank_bytes = (size_t)d.C * d.LA * d.B * 4, weights_bytes = (size_t)d.K * d.C * 4;
@@ -2533,7 +2539,7 @@ int fit_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
         // The model is as it was.  A wait that really ran out (a GPU shared with other work, a very
         // large graph) is no reason to fail the call: the caller goes on with the launches per example,
         // which wait for nobody.  Only the forced give-up of the tests is reported.
-        if (!p.force_abort) return GTM_OK;  // *done stays false
+        if (!bound.abort) return GTM_OK;  // *done stays false
         return fail(GTM_ERR_HIP, "training kernel gave up waiting at its device-wide barrier (%d workgroups); "
                                  "the model state is as it was before the call", groups);
     }
@@ -2677,7 +2683,7 @@ int fit_deep_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *
     p.class_sum = (unsigned long long *)w.class_sum;
     p.abort_flag = (uint32_t *)((unsigned long long *)w.class_sum + (size_t)d.K * 3 * FITP_SUM_PARTS * FITP_SUM_STRIDE);
     const WaitBound bound = wait_bound(dev);
-    p.spin_limit = bound.spin_limit, p.wait_ticks = bound.wait_ticks, p.force_abort = bound.force_abort;
+    p.spin_limit = bound.spin_limit, p.wait_ticks = bound.wait_ticks;
     p.clauses_per_group = per_group;
     p.NW = NW;
     p.rows_words = big ? 0 : rows_words;
@@ -2707,6 +2713,7 @@ int fit_deep_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *
         const int n_now = std::min(chunk, n_examples - at);
         p.first_example = first_example + at;
         p.n_examples = n_now;
+        p.force_abort = at >= bound.give_up_from;
         p.first_step = (uint32_t)(first_step + (uint64_t)at);
         p.perm = nullptr;
         if (deal) {
@@ -2772,7 +2779,7 @@ int fit_deep_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *
             if (e != hipSuccess)
                 return fail(GTM_ERR_HIP, "training kernel gave up waiting at a device-wide barrier (%d workgroups) and the "
                                          "model state could not be restored: %s", groups, hipGetErrorString(e));
-            if (!p.force_abort) return GTM_OK;  // as in fit_persistent: the launches per example take over
+            if (!bound.abort) return GTM_OK;  // as in fit_persistent: the launches per example take over
             return fail(GTM_ERR_HIP, "training kernel gave up waiting at a device-wide barrier (%d workgroups); "
                                      "the model state is as it was before the call", groups);
         }
@@ -2835,6 +2842,8 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
                               (const void *)k_fit_moves<8, true, false, false, false>,   (const void *)k_fit_moves<8, true, false, false, true>,
                               (const void *)k_fit_moves<16, false, true, true, false>,   (const void *)k_fit_moves<16, false, true, false, false>,
                               (const void *)k_fit_moves<16, false, false, false, false>, (const void *)k_fit_moves<16, false, false, false, true>};
+    static const char *const names[4] = {"k_fit_moves<registers>", "k_fit_moves<registers, rows in place>", "k_fit_moves<in memory>",
+                                         "k_fit_moves<in memory, sent rows in LDS>"};
     const void *kernel = kernels[variant];
     static thread_local size_t lds_set_of[8] = {48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024, 48 * 1024};
     if (lds > lds_set_of[variant]) {
@@ -2883,7 +2892,7 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
     p.class_sum = (unsigned long long *)w.class_sum;
     p.abort_flag = (uint32_t *)((unsigned long long *)w.class_sum + (size_t)d.K * 3 * FITP_SUM_PARTS * FITP_SUM_STRIDE);
     const WaitBound bound = wait_bound(dev);
-    p.spin_limit = bound.spin_limit, p.wait_ticks = bound.wait_ticks, p.force_abort = bound.force_abort;
+    p.spin_limit = bound.spin_limit, p.wait_ticks = bound.wait_ticks;
     p.clauses_per_group = per_group;
     p.lists = w.lists;
     p.lanes_log = fitl_lanes_log(S);
@@ -2905,6 +2914,7 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
         const int n_now = std::min(chunk, n_examples - at);
         p.first_example = first_example + at;
         p.n_examples = n_now;
+        p.force_abort = at >= bound.give_up_from;
         p.first_step = (uint32_t)(first_step + (uint64_t)at);
         p.perm = nullptr;
         if (deal) {
@@ -2947,7 +2957,7 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
         if (e == hipSuccess) e = hipMemcpyAsync(w.weights_backup, s->clause_weights, weights_bytes, hipMemcpyDeviceToDevice, st);
         if (e != hipSuccess) return fail(GTM_ERR_HIP, "keeping a copy of the model state: %s", hipGetErrorString(e));
         void *args[] = {&p};
-        profile_start("k_fit_moves", st);
+        profile_start(names[layout + collect], st);
         e = hipLaunchCooperativeKernel(kernel, dim3(groups), dim3(FITP_BLOCK), args, (unsigned)lds, st);
         if (e != hipSuccess) return fail(GTM_ERR_HIP, "cooperative launch of the training kernel: %s", hipGetErrorString(e));
         profile_stop(st);
@@ -2965,7 +2975,7 @@ int fit_moves(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, const g
             if (e != hipSuccess)
                 return fail(GTM_ERR_HIP, "training kernel gave up waiting at a device-wide barrier (%d workgroups) and the "
                                          "model state could not be restored: %s", groups, hipGetErrorString(e));
-            if (!p.force_abort) return GTM_OK;  // as in fit_persistent: the launches per example take over
+            if (!bound.abort) return GTM_OK;  // as in fit_persistent: the launches per example take over
             return fail(GTM_ERR_HIP, "training kernel gave up waiting at a device-wide barrier (%d workgroups); "
                                      "the model state is as it was before the call", groups);
         }

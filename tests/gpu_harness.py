@@ -2,6 +2,7 @@
 torch-owned device buffers and bring results back as NumPy arrays in the
 oracle's shapes.  Imported only by GPU tests."""
 
+import contextlib
 import ctypes
 
 import numpy as np
@@ -20,6 +21,24 @@ def abi_config(cfg, depth, s, seed):
         max_nodes=cfg.max_nodes, message_size=cfg.message_size, message_bits=cfg.message_bits, depth=depth,
         s=s, seed=seed,
     )
+
+
+@contextlib.contextmanager
+def profiled():
+    """The kernels that the library's profile saw in the block: a function that gives {name: launches}, in the order of first use."""
+    seen = {}
+    _abi.call("gtm_profile_enable", 1)
+    try:
+        yield lambda: seen
+        name, launches, total = ctypes.c_char_p(), ctypes.c_int32(), ctypes.c_double()
+        while True:
+            _abi.call("gtm_profile_read_kernel", len(seen), ctypes.byref(name), ctypes.byref(launches), ctypes.byref(total))
+            if launches.value == 0:
+                break
+            seen[name.value] = launches.value
+        _abi.call("gtm_profile_read", ctypes.byref(name), ctypes.byref(launches), ctypes.byref(total))  # (starts anew)
+    finally:
+        _abi.call("gtm_profile_enable", 0)
 
 
 def dev_u32(shape_or_array):

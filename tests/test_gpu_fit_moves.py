@@ -40,8 +40,7 @@ LAYOUTS = {
 @pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("boost,max_included,state_bits", [(1, None, 8), (0, 9, 5), (1, None, 12)])
 def test_training_by_moves(shape, layout, boost, max_included, state_bits, tune):
-    from graphtsetlinmachine_amd import _abi
-    from tests.gpu_harness import Device
+    from tests.gpu_harness import Device, profiled
 
     name, sizes, moves, hv, sizing, taken = shape
     for switch, value in LAYOUTS[layout].items():
@@ -55,20 +54,98 @@ def test_training_by_moves(shape, layout, boost, max_included, state_bits, tune)
     assert dev.build_tiles()
     G = graphs.number_of_graphs
     Y = o.encode_labels(np.random.default_rng(1).integers(0, cfg.classes, size=G), cfg.classes, cfg.threshold)
-    kernel, launches, total = ctypes.c_char_p(), ctypes.c_int32(), ctypes.c_double()
     for epoch in range(2):
         o.fit(model, graphs, Y)
-        _abi.call("gtm_profile_enable", 1)
-        dev.fit(Y, 0, G // 3, epoch * G)  # the restart from memory is covered, too
-        dev.fit(Y, G // 3, G - G // 3, epoch * G + G // 3)
-        _abi.call("gtm_profile_read", ctypes.byref(kernel), ctypes.byref(launches), ctypes.byref(total))
-        _abi.call("gtm_profile_enable", 0)
-        assert (kernel.value == b"k_fit_moves") == taken, kernel.value
+        with profiled() as kernels:
+            dev.fit(Y, 0, G // 3, epoch * G)  # the restart from memory is covered, too
+            dev.fit(Y, G // 3, G - G // 3, epoch * G + G // 3)
+        assert all(k.startswith(b"k_fit_moves<") == taken for k in kernels()), kernels()
+        if taken and "17" not in layout and layout != "as_it_comes":
+            assert all((b"in memory" in k) == ("memory" in layout or cfg.classes > 63) for k in kernels()), kernels()
         ta, banks, w = dev.download()
         assert np.array_equal(w, model.clause_weights), "weights after epoch %d" % epoch
         assert np.array_equal(ta, model.ta_state), "layer-0 automata after epoch %d" % epoch
         for layer in range(depth - 1):
             assert np.array_equal(banks[layer], model.message_ta_state[layer]), "bank %d epoch %d" % (layer, epoch)
+
+
+# The shares of a workgroup's 16 waves and 128 lanes' words that a clause in registers can have: clauses per workgroup, automaton words per clause
+# (literals / 32 + 2 message banks), hence waves per clause, a lane's words, and whether the rows of two graphs fit in LDS beside the lists.
+REGISTER_SHAPES = [
+    ("two_waves_two_words_rows_in_place", 324, 1024, 1024, 8, b"k_fit_moves<registers, rows in place>"),   # 192 words, 128 lanes
+    ("four_waves_one_word_rows_in_place", 324, 1024, 1024, 4, b"k_fit_moves<registers, rows in place>"),   # 192 words, 256 lanes
+    ("two_waves_two_words_staged_rows", 90, 448, 448, 8, b"k_fit_moves<registers>"),                     
+    ("one_wave_one_word", 90, 256, 256, 16, b"k_fit_moves<registers>"),                                   # 48 words, 64 lanes; the polling wave owns a clause
+    ("one_wave_two_words", 90, 384, 384, 16, b"k_fit_moves<registers>"),                                  # 72 words
+    ("one_wave_all_128_words", 70, 512, 768, 9, b"k_fit_moves<registers>"),                               # 32 + 2 * 48
+    ("one_wave_129_words", 70, 520, 768, 9, b"k_fit_moves<in memory>"),                                   # 33 + 2 * 48: too many
+]
+
+
+@pytest.mark.parametrize("name,nodes,hv,message_size,per_group,kernel", REGISTER_SHAPES, ids=lambda v: v if isinstance(v, str) else "")
+@pytest.mark.parametrize("state_bits", [8, 6])
+def test_clauses_in_registers_at_every_share_of_the_waves(name, nodes, hv, message_size, per_group, kernel, state_bits, tune):
+    from tests.gpu_harness import Device, profiled
+
+    tune("GTM_FIT_DEEP_CLAUSES_PER_GROUP", str(per_group))
+    tune("GTM_NO_SMALL_FIT", "1")
+    moves = GRID if nodes == 324 else CHAIN
+    graphs = _graphs(np.array([nodes, nodes, nodes if nodes == 324 else 33, nodes]), moves, seed=nodes + hv, hv=hv)
+    cfg = helpers.oracle_config(graphs, classes=5, clauses=2 * per_group + 3, depth=3, message_size=message_size, T=30, state_bits=state_bits)
+    model = helpers.random_model(5, cfg, 3, s=(3.0, 2.0, 1.5), include_density=0.004, message_density=0.004)
+    dev = Device(model, graphs)
+    assert dev.build_tiles()
+    Y = o.encode_labels(np.arange(4) % 5, 5, cfg.threshold)
+    for epoch in range(2):
+        o.fit(model, graphs, Y)
+        with profiled() as kernels:
+            dev.fit(Y, 0, 4, epoch * 4)
+        assert list(kernels()) == [kernel], kernels()
+        ta, banks, w = dev.download()
+        assert np.array_equal(w, model.clause_weights) and np.array_equal(ta, model.ta_state)
+        assert all(np.array_equal(a, b) for a, b in zip(banks, model.message_ta_state))
+
+
+@pytest.mark.parametrize("in_memory", [False, True])
+@pytest.mark.parametrize("switches,kernels_expected", [
+    ({"GTM_NO_FIT_MOVES": "1"}, {"k_fit_deep_persistent": 4}),
+    # launches that start three examples into a kernel's run or later give up: each trains on three, the next goes on from there
+    ({"GTM_FIT_SPIN_LIMIT": "from 3"}, {"k_fit_moves": 2, "k_fit_deep_persistent": 2}),
+    ({"GTM_FIT_SPIN_LIMIT": "from 9"}, {"k_fit_moves": 4, "k_fit_deep_persistent": 1}),
+    ({"GTM_FIT_SPIN_LIMIT": "from 0"}, {"k_fit_moves": 1, "k_fit_deep_persistent": 1}),
+], ids=["edges-walked", "both-give-up", "moves-give-up-at-the-end", "both-give-up-at-once"])
+def test_another_kernel_goes_on_where_one_gave_up(switches, kernels_expected, in_memory, tune):
+    """Chains train on k_fit_moves; where it is off or gives up, on the kernel that walks the edges, and where that gives up, on
+    launches per example: the same automata and weights, each example once."""
+    from tests.gpu_harness import Device, profiled
+
+    for name, value in switches.items():
+        tune(name, value)
+    if in_memory:
+        tune("GTM_FIT_DEEP_IN_MEMORY", "1")
+    tune("GTM_FIT_DEEP_CLAUSES_PER_GROUP", "7")  # (clauses are dealt out anew every three examples)
+    tune("GTM_FIT_DEEP_CHUNK", "3")
+    graphs = _graphs(np.array([100, 90, 110, 70, 65, 33, 100, 128, 80, 1, 77]), CHAIN, seed=2)
+    cfg = helpers.oracle_config(graphs, classes=3, clauses=40, depth=3, message_size=64, T=30)
+    model = helpers.random_model(5, cfg, 3, s=(3.0, 2.0, 1.5), include_density=0.02, message_density=0.02)
+    dev = Device(model, graphs)
+    assert dev.build_tiles()
+    Y = o.encode_labels(np.arange(11) % 3, 3, cfg.threshold)
+    for epoch in range(2):
+        o.fit(model, graphs, Y)
+        with profiled() as kernels:
+            dev.fit(Y, 0, 11, epoch * 11)
+        ran = {}
+        for k, launches in kernels().items():
+            one_launch = [n for n in ("k_fit_moves", "k_fit_deep_persistent") if k.startswith(n.encode())]
+            if one_launch:
+                assert (b"in memory" in k) == in_memory
+                ran[one_launch[0]] = launches
+        assert ran == kernels_expected, kernels()
+        ta, banks, w = dev.download()
+        assert np.array_equal(w, model.clause_weights), "weights after epoch %d" % epoch
+        assert np.array_equal(ta, model.ta_state), "automata after epoch %d" % epoch
+        assert all(np.array_equal(a, b) for a, b in zip(banks, model.message_ta_state))
 
 
 @pytest.mark.parametrize("in_memory", [False, True])

@@ -232,11 +232,17 @@ def test_scoring_the_colour_configuration_at_a_trained_state(scoring, tune):
     assert len(np.unique(want.argmax(axis=1))) > 1  # the state tells classes apart
 
 
-@pytest.mark.parametrize("training", ["one-launch", "one-launch-small-windows", "launches-per-example"])
-def test_training_the_colour_configuration_from_a_trained_state(training, tune):
+@pytest.mark.parametrize("training,switches,kernel", [
+    ("moves", {}, b"k_fit_moves<in memory>"),
+    ("edges-walked", {"GTM_NO_FIT_MOVES": "1"}, b"k_fit_deep_persistent<in memory>"),
+    ("edges-walked-small-windows", {"GTM_NO_FIT_MOVES": "1", "GTM_FIT_DEEP_WINDOW_ROWS": "128"}, b"k_fit_deep_persistent<in memory>"),
+    ("launches-per-example", {"GTM_NO_DEEP_PERSISTENT_FIT": "1"}, None),
+], ids=lambda v: v if isinstance(v, str) else "")
+def test_training_the_colour_configuration_from_a_trained_state(training, switches, kernel, tune):
     """48 more examples from the trained state, on every training path this shape can take, against the
     C oracle: all three banks and the weights bit for bit, and the class sums afterwards."""
     from graphtsetlinmachine_amd.tm import MultiClassGraphTsetlinMachine
+    from tests.gpu_harness import profiled
 
     wl, tm, state = trained_colour_state()
     if "model_after" not in TRAINED_COLOUR:
@@ -245,15 +251,18 @@ def test_training_the_colour_configuration_from_a_trained_state(training, tune):
                indices=range(4096, 4096 + 48), threads=min(16, oc.threads_available()))
         TRAINED_COLOUR["model_after"] = model
     model = TRAINED_COLOUR["model_after"]
-    if training == "one-launch-small-windows":
-        tune("GTM_FIT_DEEP_WINDOW_ROWS", "128")
-    elif training == "launches-per-example":
-        tune("GTM_NO_DEEP_PERSISTENT_FIT", "1")
+    for switch, value in switches.items():
+        tune(switch, value)
     np.random.seed(42)
     again = MultiClassGraphTsetlinMachine(**wl.params, seed=1)
     again.load(state)
     assert again.step == 4096 and again.seed == 42
-    again.fit(wl.graphs_train, wl.Y_train, epochs=1, incremental=True, examples=(4096, 48))
+    with profiled() as kernels:
+        again.fit(wl.graphs_train, wl.Y_train, epochs=1, incremental=True, examples=(4096, 48))
+    if kernel is not None:
+        assert kernels() == {kernel: 1}
+    else:
+        assert not any(k.startswith((b"k_fit_moves", b"k_fit_deep_persistent")) for k in kernels())
     saved = again.save()
     assert np.array_equal(saved["clause_weights"].reshape(model.clause_weights.shape), model.clause_weights)
     assert np.array_equal(saved["ta_state"], model.ta_state.reshape(-1))
