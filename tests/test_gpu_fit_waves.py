@@ -2,8 +2,6 @@
 rows of 1 to 64 words, 16 and 17 literal words, 63 and 64 classes, clauses longer than their list - every split follows
 the oracle bit for bit (whole numbers: no tolerance)."""
 
-import ctypes
-
 import numpy as np
 import pytest
 
@@ -13,8 +11,8 @@ from tests import helpers
 pytestmark = pytest.mark.gpu
 
 
-def follow(graphs, tune, switches, classes, clauses, state_bits=8, density=0.05, s=3.0, max_included=None, per_group=None):
-    from tests.gpu_harness import Device
+def follow(graphs, tune, switches, classes, clauses, kernel, state_bits=8, density=0.05, s=3.0, max_included=None):
+    from tests.gpu_harness import Device, profiled
 
     for name, value in switches.items():
         tune(name, value)
@@ -32,7 +30,9 @@ def follow(graphs, tune, switches, classes, clauses, state_bits=8, density=0.05,
     Y = o.encode_labels(rng.integers(0, classes, size=G), classes, cfg.threshold)
     for epoch in range(2):
         o.fit(model, graphs, Y)
-        dev.fit(Y, 0, G, epoch * G)
+        with profiled() as kernels:
+            dev.fit(Y, 0, G, epoch * G)
+        assert kernels() == {kernel: 1}
         ta, _, w = dev.download()
         assert np.array_equal(w, model.clause_weights), "weights after epoch %d" % epoch
         assert np.array_equal(ta, model.ta_state), "automata after epoch %d" % epoch
@@ -54,16 +54,20 @@ def follow(graphs, tune, switches, classes, clauses, state_bits=8, density=0.05,
 def test_lists_of_rows_at_their_edges(sizes, hv_size, classes, switches, state_bits, density, tune):
     graphs = helpers.random_graphs(len(sizes) + hv_size, n_graphs=3 * len(sizes), sizes=sizes * 3, hv_size=hv_size, n_symbols=9, max_degree=0,
                                    node_types=("a", "b") if classes == 3 else ("a",))
-    follow(graphs, tune, switches, classes, clauses=21, state_bits=state_bits, density=density,
+    waves = hv_size <= 256 and classes <= 63 and "GTM_NO_FIT_WAVES" not in switches
+    follow(graphs, tune, switches, classes, clauses=21, kernel=b"k_fit_waves" if waves else b"k_fit_persistent", state_bits=state_bits, density=density,
            max_included=20 if state_bits == 6 else None)
 
 
 @pytest.mark.parametrize("hv_size,max_nodes", [(512, 1), (520, 2), (2048, 1)])
-@pytest.mark.parametrize("s,per_group", [(1.0, None), (5.0, "20")])
+@pytest.mark.parametrize("s,per_group", [(1.0, None), (5.0, "20")])  # (of 128 words 15 fit in LDS)
 def test_feedback_of_many_literal_words(hv_size, max_nodes, s, per_group, tune):
     """Single nodes and pairs of thousands of literals: Type I bits a byte per thread, feedback of the clauses that get any."""
     graphs = helpers.random_graphs(hv_size, n_graphs=30, max_nodes=max_nodes, hv_size=hv_size, n_symbols=40, max_degree=0)
-    follow(graphs, tune, {} if per_group is None else {"GTM_FIT_PER_GROUP": per_group}, classes=10, clauses=45, density=0.02, s=s)
+    if per_group is not None and hv_size == 2048:
+        per_group = "15"
+    follow(graphs, tune, {} if per_group is None else {"GTM_FIT_PER_GROUP": per_group}, classes=10, clauses=45, kernel=b"k_fit_persistent",
+           density=0.02, s=s)
 
 
 @pytest.mark.parametrize("sizes,hv_size,clauses,kernel", [
@@ -77,15 +81,6 @@ def test_feedback_of_many_literal_words(hv_size, max_nodes, s, per_group, tune):
 @pytest.mark.parametrize("density", [0.003, 0.3])
 def test_few_nodes_of_many_literals(sizes, hv_size, clauses, kernel, density, tune):
     """Graphs of a few nodes whose words are too many for a wave per clause: one launch, whatever the number of literals."""
-    from graphtsetlinmachine_amd import _abi
-
     graphs = helpers.random_graphs(hv_size, n_graphs=3 * len(sizes), sizes=sizes * 3, hv_size=hv_size, n_symbols=30, max_degree=0,
                                    node_types=("a", "b", "c"))
-    name, launches, total = ctypes.c_char_p(), ctypes.c_int32(), ctypes.c_double()
-    _abi.call("gtm_profile_enable", 1)
-    try:
-        follow(graphs, tune, {}, classes=3, clauses=clauses, density=density)
-        _abi.call("gtm_profile_read", ctypes.byref(name), ctypes.byref(launches), ctypes.byref(total))
-    finally:
-        _abi.call("gtm_profile_enable", 0)
-    assert name.value == kernel, name.value
+    follow(graphs, tune, {}, classes=3, clauses=clauses, kernel=kernel, density=density)
