@@ -16,9 +16,9 @@
 //     the class sums travel.
 // Bound by the two or three device-wide exchanges per example (few clauses), or by the generator calls of the Type I
 // feedback and the copies of the received rows (thousands of clauses).  us per example, edges walked and clauses' include
-// planes walked (fit_deep_persistent.h) -> here: 1,000-node chains, 200 clauses 20.5 -> 11; chains of 10 to 40 nodes, 333 clauses,
-// three layers 26 -> 15.9; 324-node grids, 2,000 clauses, three layers 54 -> 22.4; 841-node grids, 8,000 clauses, three layers
-// 170 -> 61, of which the slowest workgroup's evaluation, for which all others waited, was more than half.
+// planes walked (fit_deep_persistent.h) -> here: 1,000-node chains, 200 clauses 20.5 -> 11 to 11.7; chains of 10 to 40 nodes, 333 clauses,
+// three layers 26 -> 15.7; 324-node grids, 2,000 clauses, three layers of 1,024 bits 55 -> 27.6 (256 bits: 21.5); 841-node grids, 8,000
+// clauses, three layers 170 -> 61, of which the slowest workgroup's evaluation, for which all others waited, was more than half.
 #pragma once
 
 constexpr int FITM_MAX_CLASSES = 64;

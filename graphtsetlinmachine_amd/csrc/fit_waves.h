@@ -11,10 +11,10 @@
 // the words of the picked node arrive meanwhile, a list is made anew from the include words in registers, and
 // nothing that the step needs is divided, looked up twice or fetched from memory on that chain.
 //
-// 361 nodes, 2,500 clauses of 8 words on 250 workgroups: 10.1 us per example with the clauses' state in LDS, their include
-// planes walked on the scalar unit and the whole graph's literal words staged; 3.9 now (8 to 16 clauses per workgroup
-// alike), of which about 2.5 are the exchange - an add and a look at memory that all XCDs share, and the slowest of
-// 250 workgroups.  32 workgroups take 3.2.
+// 361 nodes, 2,500 clauses of 8 words on 250 workgroups, us per example in the first epochs of 3,000 and over 60,000 examples: 10.1 and 9.5
+// with the clauses' state in LDS, their include planes walked on the scalar unit and the whole graph's literal words staged; 3.9 and
+// 4.1 now (8 to 16 clauses per workgroup alike), of which about 2.5 are the exchange - an add and a look at memory that all XCDs
+// share, and the slowest of 250 workgroups.  32 workgroups take 3.2.
 #pragma once
 
 constexpr int FITV_MAX_WORDS = 16;    // automaton words: four lanes draw the Type I bits of one

@@ -2437,8 +2437,8 @@ int fit_persistent(const Dims &d, const gtm_config *cfg, const gtm_graphs *g, co
     p.lanes_log = fitl_lanes_log(p.max_words);
     p.lists = direct ? 0 : fitl_entries(cfg->literals, p.lanes_log);
     // A wave per clause with its state in registers where the clauses are small enough (us per example, waves against
-    // state in LDS: 361 nodes, 2,500 clauses of 8 words, 10 classes 5.7 against 6.6; 81 nodes, 250 clauses of 4 words 3.6
-    // against 5.3; ragged chains of up to 300 nodes, 150 clauses 3.7 against 5.5); else the state in LDS, and as much of the lists
+    // state in LDS: 361 nodes, 2,500 clauses of 8 words, 10 classes 4.1 against 5.7; 81 nodes, 250 clauses of 4 words 3.2
+    // against 4.8; ragged chains of up to 300 nodes, 150 clauses 3.9 against 5.9); else the state in LDS, and as much of the lists
     // and of the picked nodes' literal words as it has room for (a clause with more literals than its list holds walks
     // its include plane instead).
     const bool waves = !direct && per_group <= FITP_BLOCK / 64 && d.K <= FITV_MAX_CLASSES && d.LA <= FITV_MAX_WORDS &&

@@ -34,8 +34,9 @@ GTM_HD uint32_t gtm_mulhi32(uint32_t a, uint32_t b) {
 }
 
 // WHOLE: a product's halves by one instruction (v_mad_u64_u32); else by two, as slow each but sooner done when nothing
-// else is there to issue.  Many waves per SIMD gain from the first (361-node images at depth 1 5.23 -> 5.10 us per example, ragged chains
-// 4.11 -> 3.98), the one workgroup of k_fit_small from the second (3.61 against 3.69).
+// else is there to issue.  Many waves per SIMD gain from the first (us per example, two instructions and one: 361-node images at depth 1
+// 4.14 and 4.08, ragged chains 4.03 and 3.90, 324-node grids of three layers 29.0 and 27.5; single-node images 4.04 and 4.11), the one
+// workgroup of k_fit_small from the second (3.60, with one 3.69).
 template <bool WHOLE = true>
 GTM_HD philox_out philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0, uint32_t k1) {
     const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u;

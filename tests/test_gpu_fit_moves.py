@@ -40,6 +40,8 @@ LAYOUTS = {
 @pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("boost,max_included,state_bits", [(1, None, 8), (0, 9, 5), (1, None, 12)])
 def test_training_by_moves(shape, layout, boost, max_included, state_bits, tune):
+    import torch
+
     from tests.gpu_harness import Device, profiled
 
     name, sizes, moves, hv, sizing, taken = shape
@@ -62,6 +64,9 @@ def test_training_by_moves(shape, layout, boost, max_included, state_bits, tune)
         assert all(k.startswith(b"k_fit_moves<") == taken for k in kernels()), kernels()
         if taken and "17" not in layout and layout != "as_it_comes":
             assert all((b"in memory" in k) == ("memory" in layout or cfg.classes > 63) for k in kernels()), kernels()
+        own = max(-(-cfg.clauses // torch.cuda.get_device_properties(0).multi_processor_count), int(LAYOUTS[layout].get("GTM_FIT_DEEP_CLAUSES_PER_GROUP", 1)))
+        collected = 4 * own * len(moves) * cfg.message_bits > cfg.message_size
+        assert all((b"sent rows in LDS" in k) == (b"in memory" in k and collected) for k in kernels() if taken), kernels()
         ta, banks, w = dev.download()
         assert np.array_equal(w, model.clause_weights), "weights after epoch %d" % epoch
         assert np.array_equal(ta, model.ta_state), "layer-0 automata after epoch %d" % epoch
