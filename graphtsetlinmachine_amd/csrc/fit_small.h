@@ -200,14 +200,16 @@ struct fits_word {
 // Four waves work, the fifth (`helper`) fetches: each has a loop of its own over the examples, with the same barriers.
 template <int MAXB, bool EXACT, bool HALVES>
 __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
-    extern __shared__ __align__(16) uint32_t lds[];
+    // An array of its own name, so that the other kernels' `lds`, which is known to lie on 16 bytes, is not taken for it: an automaton word's planes
+    // in two 128-bit accesses, 32 bytes from lane to lane, make an example longer than in four pairs of words (49 clauses 6.83 us, 6.59 in pairs).
+    extern __shared__ uint32_t fits_lds[];
     const int tid = threadIdx.x;
     const int C = p.C, LA = p.LA, MC = p.MC, MW = p.MW, B = EXACT ? MAXB : p.B, K = p.K, layers = p.depth - 1;
 
     // LDS carve-up: bank 0, then the message banks (all of one size), then the rest
     const size_t bank0_words = (size_t)C * LA * B, message_bank_words = (size_t)C * MC * B;
-    auto bank_of = [&](int l) { return l == 0 ? lds : lds + bank0_words + (size_t)(l - 1) * message_bank_words; };
-    int32_t *wts = (int32_t *)(lds + bank0_words + (size_t)layers * message_bank_words);  // [K][C]
+    auto bank_of = [&](int l) { return l == 0 ? fits_lds : fits_lds + bank0_words + (size_t)(l - 1) * message_bank_words; };
+    int32_t *wts = (int32_t *)(fits_lds + bank0_words + (size_t)layers * message_bank_words);  // [K][C]
     uint32_t *hv = (uint32_t *)(wts + K * C);      // [C][MB]
     // per example, double-buffered: literal words [nodes][LA]; node type, edge count, first edge
     // [3][nodes]; labels [FITS_Y_LDS]; node count and first node of the example after
@@ -228,7 +230,7 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
     uint32_t *magic_of = info_both + 8;            // [FITS_EDGES_LDS + 1]
     // the include planes, every bank's words in order: a copy, so that lanes read neighbouring words, or in place
     uint32_t *inc_copy = magic_of + FITS_EDGES_LDS + 1;
-    const uint32_t *inc_words = p.inc_copy ? inc_copy : lds + (B - 1);
+    const uint32_t *inc_words = p.inc_copy ? inc_copy : fits_lds + (B - 1);
     const int inc_stride = p.inc_copy ? 1 : B;
     const int all_words = C * (LA + layers * MC);
     const int lane = tid & 63;
@@ -625,7 +627,7 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
 #pragma unroll
             for (int t = 1; t < GTM_MAX_DEPTH; ++t)
                 if (t == l) thr16 = p.thr16[t];
-            fits_word<MAXB, EXACT> word(lds + j * B, B);
+            fits_word<MAXB, EXACT> word(fits_lds + j * B, B);
             for (int k = 0; k < K; ++k) {
                 const int now = u;
                 if (k + 1 < K) u = u_of[k + 1];
@@ -639,7 +641,7 @@ __global__ __launch_bounds__(FITS_THREADS) void k_fit_small(FitSmallParams p) {
                 }
                 word.count(up, down);
             }
-            word.store(lds + j * B);
+            word.store(fits_lds + j * B);
             if (p.inc_copy) inc_copy[j] = word.top();
         }
         // the next example's random numbers: the first 64 are the helper's
