@@ -55,6 +55,8 @@ def _ptr(t):
 # 553, 5.3 million 868 and 1,521 to 5,520, 2,729 and 3,355).  Pages touched only by the unpacking, data sets not scored before
 # took 538 us where they take 499, 728 (627), 1,250 (1,060): numbers were ahead up to 500,000 outputs.
 OUTPUTS_AS_BITS = 1 << 18
+# Bytes of workspace up to which a scoring call takes all graphs at once.
+SCORE_WORKSPACE = 4 << 30
 # Bytes that are fetched through pinned memory, which torch keeps for the next call.
 PINNED_RESULT = 16 << 20
 
@@ -578,13 +580,16 @@ class CommonTsetlinMachine:
             dg.require_made()
         if tiles:
             dg.ensure_moves(cfg)
-        if batch is None:
-            # as many graphs per launch group as fit in 4 GiB of workspace beyond its fixed part
-            size = lambda b: _abi.lib.gtm_score_workspace_bytes(ctypes.byref(cfg), ctypes.byref(desc), b)
+        size = lambda b: _abi.lib.gtm_score_workspace_bytes(ctypes.byref(cfg), ctypes.byref(desc), b)
+        asked = batch is not None
+        if not asked:
+            batch = max(1, min(n, 1 << 16))
+        need = size(batch)
+        if not asked and need > SCORE_WORKSPACE:  # as many graphs per launch group as fit beyond the workspace's fixed part
             fixed = size(1)
             per_graph = max(1.0, (size(1025) - fixed) / 1024.0)
-            batch = int(max(1, min(n, ((4 << 30) - fixed) // per_graph, 1 << 16)))
-        need = _abi.lib.gtm_score_workspace_bytes(ctypes.byref(cfg), ctypes.byref(desc), batch)
+            batch = int(max(1, min(batch, (SCORE_WORKSPACE - fixed) // per_graph)))
+            need = size(batch)
         ws = self._workspace_of(need)
         out = torch.empty(n * self.number_of_outputs, dtype=torch.int32, device=_device())
         _abi.call(

@@ -135,6 +135,23 @@ def test_ragged_multi_type_graphs_depth3_match_oracle():
     assert np.array_equal(tm.score(test), o.score(model, test))
 
 
+@pytest.mark.parametrize("limit", [4 << 30, 1 << 20, 1])
+def test_scoring_asks_for_all_graphs_workspace_and_cuts_what_is_too_much(limit, monkeypatch):
+    from graphtsetlinmachine_amd import tm as tm_module
+
+    graphs = helpers.random_graphs(9, n_graphs=700, max_nodes=40, hv_size=64)
+    np.random.seed(5)
+    tm = tm_module.MultiClassGraphTsetlinMachine(200, 300, 3.0, depth=2, message_size=64, message_bits=2, seed=3)
+    tm.fit(graphs, np.arange(700) % 3, epochs=1, examples=(0, 30))
+    batches = []
+    want = tm.score_device(graphs, batch=64).cpu().numpy()
+    call = tm_module._abi.call
+    monkeypatch.setattr(tm_module._abi, "call", lambda name, *args: (batches.append(args[5]) if name == "gtm_score" else None, call(name, *args))[1])
+    monkeypatch.setattr(tm_module, "SCORE_WORKSPACE", limit)
+    assert np.array_equal(tm.score_device(graphs).cpu().numpy(), want)
+    assert batches == [700] if limit == 4 << 30 else 1 <= batches[0] < 700
+
+
 def test_fit_not_incremental_resets_layer_zero_only():
     """tm.py:524-526: a second fit(incremental=False) re-runs `prepare` only."""
     from graphtsetlinmachine_amd.tm import MultiClassGraphTsetlinMachine
